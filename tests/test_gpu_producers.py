@@ -1,0 +1,48 @@
+"""The kernels that produce a 4-bit model's tensors, where their paths change: scales and weights outside of what the
+quantiser's three-instruction quotient covers, the transforms' types and widths, the column transform."""
+import numpy as np
+import pytest
+import torch
+
+from oracle import uniql_oracle as O
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("given", [False, True])
+def test_quantize_outside_the_fast_quotient(gpu, given):
+    """Columns with zero, negative, subnormal, tiny or huge scales, infinite weights and quotients at both ends of fp16,
+    ties included, beside ordinary ones: bit for bit the oracle's arithmetic."""
+    from uniql_amd import ops
+    g = torch.Generator().manual_seed(17)
+    n, k = 192, 392
+    w = (torch.randn(n, k, generator=g) * 0.05).half()
+    w[5, 130:250] = 0
+    w[6] = 0
+    w[7] *= 2.0 ** -20
+    w[8, 3] = float("inf")
+    w[9] = (torch.arange(k) % 31 - 15).half() * 0.25          # quotients on the halves
+    w[10] = 60000.0
+    scales = None
+    if given:
+        scales = (torch.rand(4, n, generator=g) * 0.02 + 0.004).half()
+        scales[1, 5] = 0
+        scales[:, 9] = 0.5
+        scales[0, 11], scales[1, 11], scales[2, 11], scales[3, 11] = -0.01, 2.0 ** -24, 2.0 ** -14, 1000.0
+        scales[:, 10] = torch.tensor([1.0, 1.5, 0.5, 1.9]).half()   # quotients 60000, 40000, overflow, 31578
+        w[12] = 30000.0
+        scales[:, 12] = torch.tensor([0.9, 0.92, 0.5, 0.45]).half()
+    _, o_packed, o_scale = O.w4a16_quantize(w.t().contiguous(), 128, scales, 64)
+    packed, scale = ops.w4a16_quantize(w.to(gpu), None if scales is None else scales.to(gpu), pad_out=64)
+    assert torch.equal(packed.cpu(), o_packed)
+    assert np.array_equal(scale.cpu().numpy().view(np.uint16), o_scale.numpy().view(np.uint16))
+
+
+@pytest.mark.parametrize("view", ["offset", "odd_stride"])
+def test_quantize_rows_that_are_not_16_byte_aligned(gpu, view):
+    from uniql_amd import ops
+    g = torch.Generator().manual_seed(3)
+    big = (torch.randn(128, 517, generator=g) * 0.1).half().to(gpu)
+    w = big[:, 3:387] if view == "offset" else big[:, :384]
+    got, want = ops.w4a16_quantize(w), ops.w4a16_quantize(w.contiguous())
+    assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])

@@ -1,8 +1,7 @@
 // Producer side of the packed layout on the device: group-128 quantisation of an fp16 weight
 // matrix into int4 codes + fp16 scales, and the packing of codes into the kernel's word order.
-// Offline operations (run once per layer): written for clarity and bit-exactness with the
-// host arithmetic of the reference (fp16 tensors on the CPU: every operation rounds its fp32
-// result to fp16), not for the last GB/s.
+// Bit-exact with the host arithmetic of the reference (fp16 tensors on the CPU: every operation rounds its
+// fp32 result to fp16).
 #include "common.hpp"
 
 namespace uniql {
@@ -14,36 +13,6 @@ __device__ __forceinline__ half_t half_div(half_t a, half_t b) { return (half_t)
 // Position of column n's scale inside a permuted scale row (group-128 case): inside every 64
 // columns, position 8 i + j holds column i + 8 j.
 __device__ __forceinline__ int64_t group_scale_pos(int n) { return (n & ~63) + 8 * (n & 7) + ((n & 63) >> 3); }
-
-// One wavefront per (group g, output row n): scale = fp16(max |w| * (2/15)) over the 128 K values
-// of the group (zero beyond in_features and for n >= out_features), written at the permuted
-// position.  With `given` the scales are copied from a natural-order [groups][out_features] array.
-__global__ __launch_bounds__(256) void w4a16_group_scales_kernel(const half_t* __restrict__ W, int64_t ldw,
-                                                                const half_t* __restrict__ given,
-                                                                half_t* __restrict__ S, int out_features,
-                                                                int in_features, int n_pad, int groups) {
-    const int lane = threadIdx.x & 63;
-    const int64_t wave = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (wave >= (int64_t)groups * n_pad) return;
-    const int g = (int)(wave / n_pad), n = (int)(wave % n_pad);
-    half_t scale = (half_t)0.0f;
-    if (n < out_features) {
-        if (given) {
-            scale = given[(size_t)g * out_features + n];
-        } else {
-            float amax = 0.f;
-#pragma unroll
-            for (int i = 0; i < 2; ++i) {
-                const int k = 128 * g + 2 * lane + i;
-                if (k < in_features) amax = fmaxf(amax, fabsf((float)W[(size_t)n * ldw + k]));
-            }
-#pragma unroll
-            for (int d = 1; d < 64; d <<= 1) amax = fmaxf(amax, __shfl_xor(amax, d, kWave));
-            scale = scaled_to_half(amax, (float)(2.0 / 15.0));   // fp32 product, then one rounding to fp16
-        }
-    }
-    if (lane == 0) S[(size_t)g * n_pad + group_scale_pos(n)] = scale;
-}
 
 // code of one weight; `gptq`: the scales were handed over and the reference computes
 // round(w / s + 8) (quantize_helpers.py:216-217) instead of round(w / s) + 8 (:114).
@@ -63,16 +32,136 @@ __device__ __forceinline__ uint32_t quantize_code(half_t w, half_t s, bool gptq)
     return (uint32_t)fminf(fmaxf(r, 0.0f), 15.0f);
 }
 
-// One thread per packed 32-bit word.  Word j of piece (c8, kq) of chunk c of packed row r holds,
-// in nibble 4 lo + 2 blk + hi, K row 16 r + 2 kq + 8 hi + lo of column 64 c + 16 j + 8 blk + c8.
-// SRC 0: quantise fp16 weights W[n][k] (row stride ldw) with the scales already in S (permuted);
-// SRC 1: take ready codes[k][n].
-template <int SRC>
-__global__ __launch_bounds__(256) void w4a16_pack_kernel(const half_t* __restrict__ W, int64_t ldw,
-                                                        const uint8_t* __restrict__ codes,
-                                                        const half_t* __restrict__ S, uint32_t* __restrict__ B,
-                                                        int out_features, int in_features, int n_pad, int k_pad,
-                                                        int gptq) {
+// One workgroup quantises 64 columns (one chunk of the packed layout) x one group of 128 K values in one pass:
+// every weight is read once, 32 bytes per column and thread, and stays in registers between the group's
+// maximum and its codes.  Thread t takes packed row r = t % 8 of the columns 16 j + c8 and 16 j + 8 + c8
+// (c8 = (t / 8) % 8, j = t / 64): their 2 x 16 values are exactly the four words (j of the pieces (c8, kq),
+// kq = 0..3) of that row, and the eight threads of a column pair are neighbours, so a group's maximum is three lane
+// exchanges.  The words leave through LDS as whole 16-byte pieces.
+//
+// Bound by memory: 14336 x 4096 (150 MB) takes 32 us = 4.7 TB/s, the rate of a large copy; a kernel for the scales (one wave
+// per group, 107 us) and one for the words (each gathering its eight weights, 71 us) took 178.  The quotient decides that: the
+// compiler's correctly rounded fp32 division costs ten instructions per weight, more than the memory time, where
+// three give the same fp16 quotient.  With w and s of 11 bits and m a midpoint of two fp16 numbers (12 bits),
+// w / s differs from m by at least 2^-23 of itself (|w - m s| is at least one unit of a product below 2^23, and never
+// zero: an odd 12-bit m times s has more than 11 bits), so every approximation closer than that rounds to the same fp16
+// number: the product with a reciprocal refined once, corrected by its own remainder, is within 2^-24 and a bit.
+// Columns with a scale or weights outside of what that covers (zero, negative or non-finite scales, non-finite
+// weights, quotients that leave fp16) take the plain division.
+constexpr int kPackLdsRow = 132;  // words per packed row in LDS: 128 + 4, rows on different banks
+
+// 16 codes (bits 4 lo .. of two words' worth of one column are placed by the caller) of 16 weights w with scale s
+template <bool GPTQ>
+__device__ __forceinline__ void quantize_sixteen(const h8 (&w)[2], half_t s, bool fast, float rcp, uint32_t (&code)[8]) {
+    // code[p]: codes of K values 2 p (low half) and 2 p + 1 (high half)
+#pragma unroll
+    for (int p = 0; p < 8; ++p) {
+        const half_t w0 = w[p >> 2][2 * (p & 3)], w1 = w[p >> 2][2 * (p & 3) + 1];
+        if (fast) {
+            const float f0 = (float)w0, f1 = (float)w1, sf = (float)s;
+            float q0 = f0 * rcp, q1 = f1 * rcp;
+            q0 = __builtin_fmaf(__builtin_fmaf(-q0, sf, f0), rcp, q0);
+            q1 = __builtin_fmaf(__builtin_fmaf(-q1, sf, f1), rcp, q1);
+            h2 q = h2{(half_t)q0, (half_t)q1};
+            // clamping first, then adding 1536 (spacing 1: the addition rounds to the nearest integer, ties to even)
+            // gives clamp(rint(q) + 8) or, with the scales handed over, clamp(rint(fp16(q + 8))) in the low bits
+            if (GPTQ) {
+                q = q + h2{(half_t)8.0f, (half_t)8.0f};
+                q = __builtin_elementwise_min(__builtin_elementwise_max(q, h2{(half_t)0.0f, (half_t)0.0f}), h2{(half_t)15.0f, (half_t)15.0f});
+                q = q + h2{(half_t)1536.0f, (half_t)1536.0f};
+            } else {
+                q = __builtin_elementwise_min(__builtin_elementwise_max(q, h2{(half_t)-8.0f, (half_t)-8.0f}), h2{(half_t)7.0f, (half_t)7.0f});
+                q = q + h2{(half_t)1544.0f, (half_t)1544.0f};
+            }
+            code[p] = h2_to_bits(q) & 0x000f000fu;
+        } else {
+            code[p] = quantize_code(w0, s, GPTQ) | (quantize_code(w1, s, GPTQ) << 16);
+        }
+    }
+}
+
+template <bool GPTQ>
+__global__ __launch_bounds__(256) void w4a16_quantize_kernel(const half_t* __restrict__ W, int64_t ldw, int vec_ok,
+                                                            const half_t* __restrict__ given, half_t* __restrict__ S,
+                                                            uint32_t* __restrict__ B, int out_features, int in_features,
+                                                            int n_pad, int groups) {
+    __shared__ __attribute__((aligned(16))) uint32_t words[8 * kPackLdsRow];
+    __shared__ __attribute__((aligned(16))) half_t scales[64];
+    const int tid = threadIdx.x;
+    const int r = tid & 7, c8 = (tid >> 3) & 7, j = tid >> 6;
+    const int g = blockIdx.x % groups, chunk = blockIdx.x / groups;  // neighbours read on along the same rows
+    const int k0 = 128 * g + 16 * r;
+    uint32_t out[4] = {0u, 0u, 0u, 0u};
+#pragma unroll
+    for (int blk = 0; blk < 2; ++blk) {
+        const int n = 64 * chunk + 16 * j + 8 * blk + c8;
+        h8 w[2];
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            const half_t* src = W + (size_t)n * ldw + k0 + 8 * i;
+            if (n < out_features && k0 + 8 * i + 8 <= in_features && vec_ok) {
+                w[i] = *reinterpret_cast<const h8*>(src);
+            } else {
+#pragma unroll
+                for (int e = 0; e < 8; ++e) w[i][e] = n < out_features && k0 + 8 * i + e < in_features ? src[e] : (half_t)0.0f;
+            }
+        }
+        h2 m = h2{(half_t)0.0f, (half_t)0.0f};
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int e = 0; e < 8; e += 2) m = __builtin_elementwise_max(m, __builtin_elementwise_abs(h2{w[i][e], w[i][e + 1]}));
+        float own = fmaxf((float)m.x, (float)m.y);
+        bool finite = true;
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            const u32x4 bits = __builtin_bit_cast(u32x4, w[i]);
+#pragma unroll
+            for (int e = 0; e < 4; ++e)  // an exponent of all ones in either half carries into bit 15 of that half
+                finite = finite && (((bits[e] & 0x7c007c00u) + 0x04000400u) & 0x80008000u) == 0u;
+        }
+        half_t s = (half_t)0.0f;
+        if (GPTQ) {
+            if (n < out_features) s = given[(size_t)g * out_features + n];
+        } else {
+            float amax = own;
+#pragma unroll
+            for (int d = 1; d < 8; d <<= 1) amax = fmaxf(amax, __shfl_xor(amax, d, kWave));
+            s = scaled_to_half(amax, (float)(2.0 / 15.0));   // fp32 product, then one rounding to fp16
+        }
+        if (n >= out_features) s = (half_t)0.0f;
+        if (r == 0) scales[8 * c8 + 2 * j + blk] = s;
+        const float sf = (float)s;
+        const bool fast = finite && sf > 0.0f && sf <= 65504.0f && own <= 32768.0f * sf;
+        float rcp = __builtin_amdgcn_rcpf(fast ? sf : 1.0f);
+        rcp = __builtin_fmaf(__builtin_fmaf(-sf, rcp, 1.0f), rcp, rcp);
+        uint32_t code[8];
+        if (n < out_features) {
+            if (__builtin_expect(fast, 1)) quantize_sixteen<GPTQ>(w, s, true, rcp, code);
+            else quantize_sixteen<GPTQ>(w, s, false, rcp, code);
+        } else {  // padding columns: code 0 (and scale 0)
+#pragma unroll
+            for (int p = 0; p < 8; ++p) code[p] = 0u;
+        }
+        // word kq: K values 2 kq, 2 kq + 1 (code[kq]) at bits 8 blk and 16 + 8 blk, 2 kq + 8, 2 kq + 9 (code[kq + 4]) four bits up
+#pragma unroll
+        for (int kq = 0; kq < 4; ++kq) out[kq] |= (code[kq] | (code[kq + 4] << 4)) << (8 * blk);
+    }
+#pragma unroll
+    for (int kq = 0; kq < 4; ++kq) words[r * kPackLdsRow + (4 * c8 + kq) * 4 + j] = out[kq];
+    __syncthreads();
+    // eight packed rows x 512 bytes, 16 bytes per thread; the chunk's 64 scales
+    const int row = tid >> 5, piece = tid & 31;
+    const u32x4 v = *reinterpret_cast<const u32x4*>(words + row * kPackLdsRow + 4 * piece);
+    *reinterpret_cast<u32x4*>(B + (size_t)(8 * g + row) * 2 * n_pad + 128 * (size_t)chunk + 4 * piece) = v;
+    if (tid < 8)
+        *reinterpret_cast<u32x4*>(S + (size_t)g * n_pad + 64 * (size_t)chunk + 8 * tid) = *reinterpret_cast<const u32x4*>(scales + 8 * tid);
+}
+
+// Ready codes[k][n] -> packed words, one thread per 32-bit word.  Word j of piece (c8, kq) of chunk c of packed row r
+// holds, in nibble 4 lo + 2 blk + hi, K row 16 r + 2 kq + 8 hi + lo of column 64 c + 16 j + 8 blk + c8.
+__global__ __launch_bounds__(256) void w4a16_pack_kernel(const uint8_t* __restrict__ codes, uint32_t* __restrict__ B,
+                                                        int out_features, int in_features, int n_pad, int k_pad) {
     const int64_t words_per_row = 2 * (int64_t)n_pad;
     const int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (idx >= (int64_t)(k_pad >> 4) * words_per_row) return;
@@ -80,27 +169,17 @@ __global__ __launch_bounds__(256) void w4a16_pack_kernel(const half_t* __restric
     const int c = (int)(idx % words_per_row);
     const int chunk = c >> 7, piece = (c >> 2) & 31, j = c & 3;
     const int c8 = piece >> 2, kq = piece & 3;
-    const int g = r >> 3;
     uint32_t word = 0u;
 #pragma unroll
     for (int blk = 0; blk < 2; ++blk) {
         const int n = 64 * chunk + 16 * j + 8 * blk + c8;
-        half_t s = (half_t)0.0f;
-        if (SRC == 0) s = S[(size_t)g * n_pad + group_scale_pos(n)];
 #pragma unroll
         for (int hi = 0; hi < 2; ++hi) {
 #pragma unroll
             for (int lo = 0; lo < 2; ++lo) {
                 const int k = 16 * r + 2 * kq + 8 * hi + lo;
                 uint32_t code = 0u;  // columns past out_features: code 0 (and scale 0)
-                if (n < out_features) {
-                    if (SRC == 0) {
-                        const half_t w = k < in_features ? W[(size_t)n * ldw + k] : (half_t)0.0f;
-                        code = quantize_code(w, s, gptq != 0);
-                    } else {
-                        code = k < in_features ? (uint32_t)(codes[(size_t)k * out_features + n] & 15u) : 8u;
-                    }
-                }
+                if (n < out_features) code = k < in_features ? (uint32_t)(codes[(size_t)k * out_features + n] & 15u) : 8u;
                 word |= code << (4 * (4 * lo + 2 * blk + hi));
             }
         }
@@ -121,15 +200,13 @@ __global__ __launch_bounds__(256) void w4a16_permute_scales_kernel(const half_t*
 int quantize_launch(const void* W, int64_t ldw, const void* given_scales, void* B, void* S, int out_features,
                     int in_features, int n_pad, int k_pad, hipStream_t stream) {
     const int groups = k_pad / 128;
-    const int64_t waves = (int64_t)groups * n_pad;
-    hipLaunchKernelGGL(w4a16_group_scales_kernel, dim3((unsigned)((waves + 3) / 4)), dim3(256), 0, stream,
-                       reinterpret_cast<const half_t*>(W), ldw, reinterpret_cast<const half_t*>(given_scales),
-                       reinterpret_cast<half_t*>(S), out_features, in_features, n_pad, groups);
-    const int64_t words = (int64_t)(k_pad / 16) * 2 * n_pad;
-    hipLaunchKernelGGL(w4a16_pack_kernel<0>, dim3((unsigned)((words + 255) / 256)), dim3(256), 0, stream,
-                       reinterpret_cast<const half_t*>(W), ldw, (const uint8_t*)nullptr,
-                       reinterpret_cast<const half_t*>(S), reinterpret_cast<uint32_t*>(B), out_features,
-                       in_features, n_pad, k_pad, given_scales ? 1 : 0);
+    const int64_t grid = (int64_t)groups * (n_pad / 64);
+    if (grid > 0x7fffffffLL) return UNIQL_E_SHAPE;
+    const int vec_ok = ldw % 8 == 0 && (reinterpret_cast<uintptr_t>(W) & 15u) == 0 ? 1 : 0;
+    auto kern = given_scales ? &w4a16_quantize_kernel<true> : &w4a16_quantize_kernel<false>;
+    hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(256), 0, stream, reinterpret_cast<const half_t*>(W), ldw, vec_ok,
+                       reinterpret_cast<const half_t*>(given_scales), reinterpret_cast<half_t*>(S),
+                       reinterpret_cast<uint32_t*>(B), out_features, in_features, n_pad, groups);
     return hipGetLastError() == hipSuccess ? UNIQL_OK : UNIQL_E_LAUNCH;
 }
 
@@ -140,9 +217,8 @@ int pack_launch(const uint8_t* codes, const void* scales, void* B, void* S, int 
     hipLaunchKernelGGL(w4a16_permute_scales_kernel, dim3((unsigned)((sc + 255) / 256)), dim3(256), 0, stream,
                        reinterpret_cast<const half_t*>(scales), reinterpret_cast<half_t*>(S), n, n_pad, groups);
     const int64_t words = (int64_t)(k_pad / 16) * 2 * n_pad;
-    hipLaunchKernelGGL(w4a16_pack_kernel<1>, dim3((unsigned)((words + 255) / 256)), dim3(256), 0, stream,
-                       (const half_t*)nullptr, (int64_t)0, codes, (const half_t*)nullptr,
-                       reinterpret_cast<uint32_t*>(B), n, k, n_pad, k_pad, 0);
+    hipLaunchKernelGGL(w4a16_pack_kernel, dim3((unsigned)((words + 255) / 256)), dim3(256), 0, stream, codes,
+                       reinterpret_cast<uint32_t*>(B), n, k, n_pad, k_pad);
     return hipGetLastError() == hipSuccess ? UNIQL_OK : UNIQL_E_LAUNCH;
 }
 
