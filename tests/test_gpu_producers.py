@@ -46,3 +46,30 @@ def test_quantize_rows_that_are_not_16_byte_aligned(gpu, view):
     w = big[:, 3:387] if view == "offset" else big[:, :384]
     got, want = ops.w4a16_quantize(w), ops.w4a16_quantize(w.contiguous())
     assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
+
+
+def _as(t, dtype):
+    """numpy float32 of what the kernel's rounding to `dtype` gives for a float32 tensor"""
+    return t.to(dtype).float().numpy()
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("block", [64, 128, 256, 2048, 4096, 8192, 16384, 32768])
+def test_transform_in_every_type_and_width(gpu, dtype, block):
+    from uniql_amd import ops
+    x = torch.randn(3, 2 * block if block <= 4096 else block, generator=torch.Generator().manual_seed(block)).to(dtype)
+    y = ops.hadamard_blockwise(x.to(gpu), block ** -0.5, block)
+    want = torch.from_numpy(O.fwht(x.float().numpy(), 1.0, block=block)) * torch.tensor(block ** -0.5, dtype=torch.float32)
+    assert np.array_equal(y.float().cpu().numpy(), _as(want, dtype))
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("dim", [12 * 128, 12 * 2048, 20 * 64, 20 * 1024, 28 * 128, 28 * 1024, 40 * 512, 40 * 1024])
+def test_composite_transform_widths(gpu, dtype, dim):
+    """The smallest and largest width of the vector kernel for each base, and one of the kernel it leaves the rest to."""
+    from uniql_amd import ops
+    base, scale = O.had_variant(dim)
+    x = torch.randn(5, dim, generator=torch.Generator().manual_seed(dim)).to(dtype)
+    y = ops.hadamard_composite(x.to(gpu), scale, base)
+    want = torch.from_numpy(O.fwht_composite(x.float().numpy(), 1.0, base)) * torch.tensor(scale, dtype=torch.float32)
+    assert np.array_equal(y.float().cpu().numpy(), _as(want, dtype))

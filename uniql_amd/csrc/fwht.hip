@@ -1,38 +1,119 @@
-// Walsh-Hadamard transform of fp16 rows: y = fp16((x . H_block) * scale), H the
+// Walsh-Hadamard transform of fp16 / bf16 / fp32 rows: y = T((x . H_block) * scale), H the
 // Sylvester (natural-order) matrix, applied to consecutive `block`-wide pieces.
-// Butterflies run in fp32, lowest index bit first, one rounding to fp16 at the end.
+// Butterflies run in fp32, lowest index bit first, one rounding to T at the end.
+#include <atomic>
+
 #include "common.hpp"
 #include "fwht_device.hpp"
 #include "hadamard_base.hpp"
 
 namespace uniql {
 
+// ---- values in memory <-> fp32 ----------------------------------------------------------------
+// Eight consecutive values as raw 16-byte words (fp32: two of them), so that a load can be issued long before the
+// conversion; results are rounded once (see scaled_to_half: multiply and rounding stay separate).
+template <typename T>
+struct RowIo;
+template <>
+struct RowIo<half_t> {
+    struct Raw { u32x4 a; };
+    static __device__ __forceinline__ Raw load(const half_t* p) { return Raw{*reinterpret_cast<const u32x4*>(p)}; }
+    static __device__ __forceinline__ void unpack(const Raw& r, float (&f)[8]) {
+#pragma unroll
+        for (int p = 0; p < 4; ++p) {
+            const h2 hv = bits_to_h2(r.a[p]);
+            f[2 * p] = (float)hv.x;
+            f[2 * p + 1] = (float)hv.y;
+        }
+    }
+    static __device__ __forceinline__ uint32_t pair(float a, float b, float scale) {
+        h2 r;
+        r.x = scaled_to_half(a, scale);
+        r.y = scaled_to_half(b, scale);
+        return h2_to_bits(r);
+    }
+    static __device__ __forceinline__ void store2(half_t* p, float a, float b, float scale) {
+        *reinterpret_cast<uint32_t*>(p) = pair(a, b, scale);
+    }
+    static __device__ __forceinline__ void store8(half_t* p, const float (&f)[8], float scale) {
+        *reinterpret_cast<u32x4*>(p) =
+            u32x4{pair(f[0], f[1], scale), pair(f[2], f[3], scale), pair(f[4], f[5], scale), pair(f[6], f[7], scale)};
+    }
+};
+template <>
+struct RowIo<__bf16> {
+    struct Raw { u32x4 a; };
+    static __device__ __forceinline__ Raw load(const __bf16* p) { return Raw{*reinterpret_cast<const u32x4*>(p)}; }
+    static __device__ __forceinline__ void unpack(const Raw& r, float (&f)[8]) {
+#pragma unroll
+        for (int p = 0; p < 4; ++p) {
+            f[2 * p] = __uint_as_float(r.a[p] << 16);
+            f[2 * p + 1] = __uint_as_float(r.a[p] & 0xffff0000u);
+        }
+    }
+    static __device__ __forceinline__ uint32_t pair(float a, float b, float scale) {
+        float p = a * scale, q = b * scale;
+        asm volatile("" : "+v"(p), "+v"(q));
+        const __bf16 lo = (__bf16)p, hi = (__bf16)q;
+        return (uint32_t)__builtin_bit_cast(uint16_t, lo) | ((uint32_t)__builtin_bit_cast(uint16_t, hi) << 16);
+    }
+    static __device__ __forceinline__ void store2(__bf16* p, float a, float b, float scale) {
+        *reinterpret_cast<uint32_t*>(p) = pair(a, b, scale);
+    }
+    static __device__ __forceinline__ void store8(__bf16* p, const float (&f)[8], float scale) {
+        *reinterpret_cast<u32x4*>(p) =
+            u32x4{pair(f[0], f[1], scale), pair(f[2], f[3], scale), pair(f[4], f[5], scale), pair(f[6], f[7], scale)};
+    }
+};
+template <>
+struct RowIo<float> {
+    struct Raw { f4 a, b; };
+    static __device__ __forceinline__ Raw load(const float* p) {
+        return Raw{*reinterpret_cast<const f4*>(p), *reinterpret_cast<const f4*>(p + 4)};
+    }
+    static __device__ __forceinline__ void unpack(const Raw& r, float (&f)[8]) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            f[i] = r.a[i];
+            f[4 + i] = r.b[i];
+        }
+    }
+    static __device__ __forceinline__ void store2(float* p, float a, float b, float scale) {
+        *reinterpret_cast<float2*>(p) = make_float2(a * scale, b * scale);
+    }
+    static __device__ __forceinline__ void store8(float* p, const float (&f)[8], float scale) {
+        *reinterpret_cast<f4*>(p) = f4{f[0] * scale, f[1] * scale, f[2] * scale, f[3] * scale};
+        *reinterpret_cast<f4*>(p + 4) = f4{f[4] * scale, f[5] * scale, f[6] * scale, f[7] * scale};
+    }
+};
+
+// index bits 0..2 of eight consecutive values
+__device__ __forceinline__ void wht8(float (&f)[8]) {
+#pragma unroll
+    for (int h = 1; h < 8; h <<= 1) {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            if ((i & h) == 0) {
+                const float p = f[i], q = f[i + h];
+                f[i] = p + q;
+                f[i + h] = p - q;
+            }
+        }
+    }
+}
+
 // ---- block == 128: one 16-lane group per piece, all in registers ------------------
-__global__ __launch_bounds__(256) void fwht128_kernel(const u32x4* __restrict__ x, u32x4* __restrict__ y,
-                                                     int64_t pieces, float scale) {
+template <typename T>
+__global__ __launch_bounds__(256) void fwht128_kernel(const T* __restrict__ x, T* __restrict__ y, int64_t pieces, float scale) {
     const int64_t piece = (int64_t)blockIdx.x * 16 + (threadIdx.x >> 4);
     const int seg = threadIdx.x & 15;
     // every lane of a 16-lane group shares `piece`, so the exchange below never
     // crosses into a group that has left
     if (piece >= pieces) return;
-    const u32x4 v = x[piece * 16 + seg];
     float f[8];
-#pragma unroll
-    for (int p = 0; p < 4; ++p) {
-        const h2 hv = bits_to_h2(v[p]);
-        f[2 * p] = (float)hv.x;
-        f[2 * p + 1] = (float)hv.y;
-    }
+    RowIo<T>::unpack(RowIo<T>::load(x + (piece * 16 + seg) * 8), f);
     wht128_row16(f, seg);
-    u32x4 o;
-#pragma unroll
-    for (int p = 0; p < 4; ++p) {
-        h2 hv;
-        hv.x = scaled_to_half(f[2 * p], scale);
-        hv.y = scaled_to_half(f[2 * p + 1], scale);
-        o[p] = h2_to_bits(hv);
-    }
-    y[piece * 16 + seg] = o;
+    RowIo<T>::store8(y + (piece * 16 + seg) * 8, f, scale);
 }
 
 // ---- general power of two: one workgroup per piece, fp32 image in LDS --------------
@@ -96,72 +177,57 @@ __global__ __launch_bounds__(256) void fwht_lds_kernel(const T* __restrict__ x, 
     }
 }
 
-// ---- fp16, power of two >= 256: vector loads, index bits 0..2 in registers, LDS passes of
-// up to four bits (fwht_row_to_lds), vector stores ----------------------------------------------
-__global__ __launch_bounds__(1024) void fwht_f16_kernel(const u32x4* __restrict__ x, u32x4* __restrict__ y, int L,
-                                                       int log2L, float scale) {
+// ---- power of two >= 256: vector loads, index bits 0..2 in registers, LDS passes of
+// up to four bits, vector stores ----------------------------------------------
+template <typename T>
+__global__ __launch_bounds__(256) void fwht_vec_kernel(const T* __restrict__ x, T* __restrict__ y, int L, int log2L, float scale) {
     extern __shared__ __attribute__((aligned(16))) float fbuf[];
     const int tid = threadIdx.x, nthreads = blockDim.x;
     const int chunks = L >> 3;
-    const u32x4* xp = x + (size_t)blockIdx.x * chunks;
-    u32x4* yp = y + (size_t)blockIdx.x * chunks;
-    fwht_row_to_lds(xp, fbuf, L, log2L, tid, nthreads);
+    const T* xp = x + (size_t)blockIdx.x * L;
+    T* yp = y + (size_t)blockIdx.x * L;
+    for (int c = tid; c < chunks; c += nthreads) {
+        float f[8];
+        RowIo<T>::unpack(RowIo<T>::load(xp + 8 * c), f);
+        wht8(f);
+        float* dst = fbuf + fwht_pad(8 * c);
+        *reinterpret_cast<f4*>(dst) = f4{f[0], f[1], f[2], f[3]};
+        *reinterpret_cast<f4*>(dst + 4) = f4{f[4], f[5], f[6], f[7]};
+    }
+    __syncthreads();
+    fwht_passes_from_bit3(fbuf, 1, 0, L, log2L, tid, nthreads);
     for (int c = tid; c < chunks; c += nthreads) {
         const float* src = fbuf + fwht_pad(8 * c);
         const f4 a = *reinterpret_cast<const f4*>(src), b = *reinterpret_cast<const f4*>(src + 4);
-        h2 r0, r1, r2, r3;
-        r0.x = scaled_to_half(a[0], scale);
-        r0.y = scaled_to_half(a[1], scale);
-        r1.x = scaled_to_half(a[2], scale);
-        r1.y = scaled_to_half(a[3], scale);
-        r2.x = scaled_to_half(b[0], scale);
-        r2.y = scaled_to_half(b[1], scale);
-        r3.x = scaled_to_half(b[2], scale);
-        r3.y = scaled_to_half(b[3], scale);
-        yp[c] = u32x4{h2_to_bits(r0), h2_to_bits(r1), h2_to_bits(r2), h2_to_bits(r3)};
+        const float f[8] = {a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]};
+        RowIo<T>::store8(yp + 8 * c, f, scale);
     }
 }
 
-// Long rows (L >= 4096), fp16: two LDS exchanges instead of one per four index bits.
+// Long rows (L >= 4096): two LDS exchanges instead of one per four index bits.
 //   load    every thread takes L/8/T sixteen-byte chunks (consecutive lanes on consecutive chunks),
 //           transforms index bits 0..2 in registers and writes fp32 to LDS;
 //   middle  index bits 3 .. n-6 in passes of up to five bits (32 values per task in registers);
 //   final   the top five bits: a thread reads two neighbouring values at 32 strides of L/32,
-//           transforms, scales, rounds and stores 4 bytes per stride: consecutive lanes store
-//           consecutive words, no trip back through LDS.
+//           transforms, scales, rounds and stores a pair per stride: consecutive lanes store
+//           consecutive pairs, no trip back through LDS.
 // The stages run in ascending bit order like everywhere else, so the fp32 sums are associated
-// the same way and the result is the same bit for bit.  T = L / 64 threads per row.
-__global__ __launch_bounds__(512) void fwht_f16_wide_kernel(const u32x4* __restrict__ x, uint32_t* __restrict__ y,
-                                                           int L, int log2L, float scale) {
+// the same way and the result is the same bit for bit.  L / 64 threads per row.
+template <typename T>
+__global__ __launch_bounds__(512) void fwht_wide_kernel(const T* __restrict__ x, T* __restrict__ y, int L, int log2L, float scale) {
     extern __shared__ __attribute__((aligned(16))) float fbuf[];
     const int tid = threadIdx.x, nthreads = blockDim.x;
-    const int chunks = L >> 3;
-    const u32x4* xp = x + (size_t)blockIdx.x * chunks;
-    uint32_t* yp = y + (size_t)blockIdx.x * (L >> 1);
+    const T* xp = x + (size_t)blockIdx.x * L;
+    T* yp = y + (size_t)blockIdx.x * L;
     constexpr int kChunksPerThread = 8;  // chunks / nthreads = (L / 8) / (L / 64)
-    u32x4 v[kChunksPerThread];
+    typename RowIo<T>::Raw v[kChunksPerThread];
 #pragma unroll
-    for (int i = 0; i < kChunksPerThread; ++i) v[i] = xp[tid + i * nthreads];
+    for (int i = 0; i < kChunksPerThread; ++i) v[i] = RowIo<T>::load(xp + 8 * (tid + i * nthreads));
 #pragma unroll
     for (int i = 0; i < kChunksPerThread; ++i) {
         float f[8];
-#pragma unroll
-        for (int p = 0; p < 4; ++p) {
-            const h2 hv = bits_to_h2(v[i][p]);
-            f[2 * p] = (float)hv.x;
-            f[2 * p + 1] = (float)hv.y;
-        }
-#pragma unroll
-        for (int h = 1; h < 8; h <<= 1) {
-#pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                if ((e & h) == 0) {
-                    const float p = f[e], q = f[e + h];
-                    f[e] = p + q;
-                    f[e + h] = p - q;
-                }
-            }
-        }
+        RowIo<T>::unpack(v[i], f);
+        wht8(f);
         float* dst = fbuf + fwht_pad(8 * (tid + i * nthreads));
         *reinterpret_cast<f4*>(dst) = f4{f[0], f[1], f[2], f[3]};
         *reinterpret_cast<f4*>(dst + 4) = f4{f[4], f[5], f[6], f[7]};
@@ -209,33 +275,36 @@ __global__ __launch_bounds__(512) void fwht_f16_wide_kernel(const u32x4* __restr
         }
     }
 #pragma unroll
-    for (int j = 0; j < 32; ++j) {
-        h2 r;
-        r.x = scaled_to_half(a[j], scale);
-        r.y = scaled_to_half(b[j], scale);
-        yp[tid + j * (stride >> 1)] = h2_to_bits(r);
-    }
+    for (int j = 0; j < 32; ++j) RowIo<T>::store2(yp + 2 * tid + j * stride, a[j], b[j], scale);
 }
 
-static int fwht_f16_launch(const void* x, void* y, int64_t pieces, int block, float scale, hipStream_t stream) {
+// more than 64 KB of LDS: a property of (kernel, device), set on the first launch there
+template <typename K>
+static bool allow_lds(K kern, size_t bytes, std::atomic<unsigned long long>& done) {
+    if (bytes <= 64 * 1024) return true;
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return false;
+    if ((done.load(std::memory_order_acquire) >> dev) & 1ull) return true;
+    if (hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024) != hipSuccess)
+        return false;
+    done.fetch_or(1ull << dev, std::memory_order_release);
+    return true;
+}
+
+template <typename T>
+static int fwht_vec_launch(const void* x, void* y, int64_t pieces, int block, float scale, hipStream_t stream) {
     int log2L = 0;
     while ((1 << log2L) < block) ++log2L;
     const size_t shmem = (size_t)(block + (block >> 7) * 8) * sizeof(float);
-    if (shmem > 64 * 1024) {
-        if (hipFuncSetAttribute(reinterpret_cast<const void*>(&fwht_f16_kernel),
-                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)shmem) != hipSuccess ||
-            hipFuncSetAttribute(reinterpret_cast<const void*>(&fwht_f16_wide_kernel),
-                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)shmem) != hipSuccess)
-            return UNIQL_E_LAUNCH;
-    }
     if (block >= 4096) {
-        hipLaunchKernelGGL(fwht_f16_wide_kernel, dim3((unsigned)pieces), dim3(block / 64), shmem, stream,
-                           reinterpret_cast<const u32x4*>(x), reinterpret_cast<uint32_t*>(y), block, log2L, scale);
+        static std::atomic<unsigned long long> done{0};
+        if (!allow_lds(&fwht_wide_kernel<T>, shmem, done)) return UNIQL_E_LAUNCH;
+        hipLaunchKernelGGL(fwht_wide_kernel<T>, dim3((unsigned)pieces), dim3(block / 64), shmem, stream,
+                           reinterpret_cast<const T*>(x), reinterpret_cast<T*>(y), block, log2L, scale);
         return UNIQL_OK;
     }
-    const int threads = block / 8 < 1024 ? block / 8 : 1024;
-    hipLaunchKernelGGL(fwht_f16_kernel, dim3((unsigned)pieces), dim3(threads), shmem, stream,
-                       reinterpret_cast<const u32x4*>(x), reinterpret_cast<u32x4*>(y), block, log2L, scale);
+    hipLaunchKernelGGL(fwht_vec_kernel<T>, dim3((unsigned)pieces), dim3(block / 8), shmem, stream,
+                       reinterpret_cast<const T*>(x), reinterpret_cast<T*>(y), block, log2L, scale);
     return UNIQL_OK;
 }
 
@@ -287,18 +356,99 @@ __global__ __launch_bounds__(256) void fwht_composite_kernel(const T* __restrict
     }
 }
 
+// The same for P >= 128, at the memory rate: 16-byte loads with index bits 0..2 in registers, padded LDS passes of up
+// to four bits, then the base matrix with its signs as constants, one addition per term (the mask bits tested at run
+// time are three instructions per term, 34 us of vector time at 1024 rows of 14336 against 12 us of memory
+// time), on pairs of neighbouring columns.  1024 rows of 14336 fp16: 23 us, against 65 us of fwht_composite_kernel;
+// 4096 rows: 84 against 230.  From BASE = 20 on two halves of the workgroup take half of the
+// outputs each (a lane would otherwise hold the only use of its SIMD for BASE^2 dependent additions).
+// The terms are added in ascending order, starting from zero, as fwht_composite_kernel does: the same bits.
+template <int BASE>
+struct BaseTable;
+template <> struct BaseTable<12> { static constexpr const uint64_t (&mask)[12] = kHadamard12; };
+template <> struct BaseTable<20> { static constexpr const uint64_t (&mask)[20] = kHadamard20; };
+template <> struct BaseTable<28> { static constexpr const uint64_t (&mask)[28] = kHadamard28; };
+template <> struct BaseTable<40> { static constexpr const uint64_t (&mask)[40] = kHadamard40; };
+
+template <int BASE, int C, int CP>
+__device__ __forceinline__ void base_terms(const float2 (&z)[BASE], float& a, float& b) {
+    if constexpr (CP < BASE) {
+        constexpr bool minus = (BaseTable<BASE>::mask[C] >> CP) & 1ull;
+        a = minus ? a - z[CP].x : a + z[CP].x;
+        b = minus ? b - z[CP].y : b + z[CP].y;
+        base_terms<BASE, C, CP + 1>(z, a, b);
+    }
+}
+template <typename T, int BASE, int C, int END>
+__device__ __forceinline__ void base_outputs(const float2 (&z)[BASE], T* yp, int P, float scale) {
+    if constexpr (C < END) {
+        float a = 0.f, b = 0.f;
+        base_terms<BASE, C, 0>(z, a, b);
+        RowIo<T>::store2(yp + C * P, a, b, scale);
+        base_outputs<T, BASE, C + 1, END>(z, yp, P, scale);
+    }
+}
+
+template <typename T, int BASE>
+__global__ __launch_bounds__(512) void fwht_composite_vec_kernel(const T* __restrict__ x, T* __restrict__ y, int P, int log2P,
+                                                                float scale) {
+    extern __shared__ __attribute__((aligned(16))) float fbuf[];
+    const int tid = threadIdx.x, nthreads = blockDim.x;
+    const int L = BASE * P, chunks = L >> 3;
+    const T* xp = x + (size_t)blockIdx.x * L;
+    T* yp = y + (size_t)blockIdx.x * L;
+    constexpr int kAhead = 4;  // chunks requested before the first is used
+    for (int c0 = tid; c0 < chunks; c0 += kAhead * nthreads) {
+        typename RowIo<T>::Raw v[kAhead];
+#pragma unroll
+        for (int i = 0; i < kAhead; ++i)
+            if (c0 + i * nthreads < chunks) v[i] = RowIo<T>::load(xp + 8 * (c0 + i * nthreads));
+#pragma unroll
+        for (int i = 0; i < kAhead; ++i) {
+            const int c = c0 + i * nthreads;
+            if (c >= chunks) break;
+            float f[8];
+            RowIo<T>::unpack(v[i], f);
+            wht8(f);
+            float* dst = fbuf + fwht_pad(8 * c);
+            *reinterpret_cast<f4*>(dst) = f4{f[0], f[1], f[2], f[3]};
+            *reinterpret_cast<f4*>(dst + 4) = f4{f[4], f[5], f[6], f[7]};
+        }
+    }
+    __syncthreads();
+    fwht_passes_from_bit3(fbuf, 1, 0, L, log2P, tid, nthreads);
+    constexpr int kHalves = BASE >= 20 ? 2 : 1;
+    const int pairs = P >> 1;  // a multiple of 64: a wave's lanes share the half
+    for (int item = tid; item < kHalves * pairs; item += nthreads) {
+        const int half = __builtin_amdgcn_readfirstlane(item >= pairs ? 1 : 0);
+        const int i = 2 * (item - half * pairs);
+        float2 z[BASE];
+#pragma unroll
+        for (int c = 0; c < BASE; ++c) z[c] = *reinterpret_cast<const float2*>(fbuf + fwht_pad(c * P + i));
+        if (half == 0) base_outputs<T, BASE, 0, BASE / kHalves>(z, yp + i, P, scale);
+        else base_outputs<T, BASE, BASE / kHalves, BASE>(z, yp + i, P, scale);
+    }
+}
+
 template <typename T, int BASE>
 static int fwht_composite_go(const void* x, void* y, int64_t rows, int P, float scale, hipStream_t stream) {
     int log2P = 0;
     while ((1 << log2P) < P) ++log2P;
-    const size_t shmem = (size_t)BASE * P * sizeof(float);
-    auto kern = &fwht_composite_kernel<T, BASE>;
-    if (shmem > 64 * 1024 &&
-        hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
-                            (int)shmem) != hipSuccess)
-        return UNIQL_E_LAUNCH;
-    hipLaunchKernelGGL(kern, dim3((unsigned)rows), dim3(256), shmem, stream, reinterpret_cast<const T*>(x),
-                       reinterpret_cast<T*>(y), P, log2P, scale);
+    const int L = BASE * P;
+    const size_t padded = (size_t)(L + (L >> 7) * 8) * sizeof(float);
+    if (P >= 128 && padded <= 160 * 1024) {
+        static std::atomic<unsigned long long> done{0};
+        if (!allow_lds(&fwht_composite_vec_kernel<T, BASE>, padded, done)) return UNIQL_E_LAUNCH;
+        const int threads = P >= 512 ? 512 : 256;
+        hipLaunchKernelGGL((fwht_composite_vec_kernel<T, BASE>), dim3((unsigned)rows), dim3(threads), padded, stream,
+                           reinterpret_cast<const T*>(x), reinterpret_cast<T*>(y), P, log2P, scale);
+        return hipGetLastError() == hipSuccess ? UNIQL_OK : UNIQL_E_LAUNCH;
+    }
+    const size_t shmem = (size_t)L * sizeof(float);
+    static std::atomic<unsigned long long> done{0};
+    if (!allow_lds(&fwht_composite_kernel<T, BASE>, shmem, done)) return UNIQL_E_LAUNCH;
+    hipLaunchKernelGGL((fwht_composite_kernel<T, BASE>), dim3((unsigned)rows), dim3(256), shmem, stream,
+                       reinterpret_cast<const T*>(x), reinterpret_cast<T*>(y), P, log2P, scale);
     return hipGetLastError() == hipSuccess ? UNIQL_OK : UNIQL_E_LAUNCH;
 }
 
@@ -324,16 +474,19 @@ int fwht_composite_launch(const void* x, void* y, int64_t rows, int dim, int bas
 }
 
 template <typename T>
-static int fwht_lds_launch(const void* x, void* y, int64_t pieces, int block, float scale, hipStream_t stream) {
+static int fwht_typed_launch(const void* x, void* y, int64_t pieces, int block, float scale, hipStream_t stream) {
+    if (block == 128) {
+        const int64_t grid = (pieces + 15) / 16;
+        if (grid > 0x7fffffffLL) return UNIQL_E_SHAPE;
+        hipLaunchKernelGGL(fwht128_kernel<T>, dim3((unsigned)grid), dim3(256), 0, stream, reinterpret_cast<const T*>(x),
+                           reinterpret_cast<T*>(y), pieces, scale);
+        return UNIQL_OK;
+    }
+    if (pieces > 0x7fffffffLL) return UNIQL_E_SHAPE;
+    if (block >= 256) return fwht_vec_launch<T>(x, y, pieces, block, scale, stream);
     int log2L = 0;
     while ((1 << log2L) < block) ++log2L;
-    const size_t shmem = (size_t)block * sizeof(float);
-    if (shmem > 64 * 1024) {
-        if (hipFuncSetAttribute(reinterpret_cast<const void*>(&fwht_lds_kernel<T>),
-                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)shmem) != hipSuccess)
-            return UNIQL_E_LAUNCH;
-    }
-    hipLaunchKernelGGL((fwht_lds_kernel<T>), dim3((unsigned)pieces), dim3(256), shmem, stream,
+    hipLaunchKernelGGL((fwht_lds_kernel<T>), dim3((unsigned)pieces), dim3(256), (size_t)block * sizeof(float), stream,
                        reinterpret_cast<const T*>(x), reinterpret_cast<T*>(y), block, log2L, scale);
     return UNIQL_OK;
 }
@@ -342,20 +495,10 @@ int fwht_launch(const void* x, void* y, int64_t rows, int dim, int block, float 
                 hipStream_t stream) {
     const int64_t pieces = rows * (dim / block);
     if (pieces == 0) return UNIQL_OK;
-    if (block == 128 && dtype == UNIQL_DT_F16) {
-        const int64_t grid = (pieces + 15) / 16;
-        if (grid > 0x7fffffffLL) return UNIQL_E_SHAPE;
-        hipLaunchKernelGGL(fwht128_kernel, dim3((unsigned)grid), dim3(256), 0, stream,
-                           reinterpret_cast<const u32x4*>(x), reinterpret_cast<u32x4*>(y), pieces, scale);
-    } else {
-        if (pieces > 0x7fffffffLL) return UNIQL_E_SHAPE;
-        int rc;
-        if (dtype == UNIQL_DT_F16 && block >= 256) rc = fwht_f16_launch(x, y, pieces, block, scale, stream);
-        else if (dtype == UNIQL_DT_F16) rc = fwht_lds_launch<half_t>(x, y, pieces, block, scale, stream);
-        else if (dtype == UNIQL_DT_BF16) rc = fwht_lds_launch<__bf16>(x, y, pieces, block, scale, stream);
-        else rc = fwht_lds_launch<float>(x, y, pieces, block, scale, stream);
-        if (rc != UNIQL_OK) return rc;
-    }
+    const int rc = dtype == UNIQL_DT_F16    ? fwht_typed_launch<half_t>(x, y, pieces, block, scale, stream)
+                   : dtype == UNIQL_DT_BF16 ? fwht_typed_launch<__bf16>(x, y, pieces, block, scale, stream)
+                                            : fwht_typed_launch<float>(x, y, pieces, block, scale, stream);
+    if (rc != UNIQL_OK) return rc;
     return hipGetLastError() == hipSuccess ? UNIQL_OK : UNIQL_E_LAUNCH;
 }
 

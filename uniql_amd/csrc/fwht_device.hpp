@@ -102,40 +102,6 @@ __device__ __forceinline__ void fwht_passes_from_bit3(float* images, int rows, i
     }
 }
 
-// One fp16 row of L = 2^log2L values (L >= 8) -> its unscaled transform as a padded fp32 image in
-// LDS (L + L/16 floats), by all `nthreads` threads of the workgroup together: 16-byte loads, index
-// bits 0..2 in registers, then LDS passes of up to four bits, lowest bit first.  Ends with a
-// workgroup barrier; every thread of the workgroup must call it.
-__device__ __forceinline__ void fwht_row_to_lds(const u32x4* xp, float* fbuf, int L, int log2L, int tid, int nthreads) {
-    const int chunks = L >> 3;
-    for (int c = tid; c < chunks; c += nthreads) {
-        const u32x4 v = xp[c];
-        float f[8];
-#pragma unroll
-        for (int p = 0; p < 4; ++p) {
-            const h2 hv = bits_to_h2(v[p]);
-            f[2 * p] = (float)hv.x;
-            f[2 * p + 1] = (float)hv.y;
-        }
-#pragma unroll
-        for (int h = 1; h < 8; h <<= 1) {
-#pragma unroll
-            for (int i = 0; i < 8; ++i) {
-                if ((i & h) == 0) {
-                    const float p = f[i], q = f[i + h];
-                    f[i] = p + q;
-                    f[i + h] = p - q;
-                }
-            }
-        }
-        float* dst = fbuf + fwht_pad(8 * c);
-        *reinterpret_cast<f4*>(dst) = f4{f[0], f[1], f[2], f[3]};
-        *reinterpret_cast<f4*>(dst + 4) = f4{f[4], f[5], f[6], f[7]};
-    }
-    __syncthreads();
-    fwht_passes_from_bit3(fbuf, 1, 0, L, log2L, tid, nthreads);
-}
-
 // ---- M rows at once, for a caller that has other memory requests to place between the loads and
 // the first use of their data.  fwht_rows_load fetches the chunks (16 bytes) tid, tid + nthreads,
 // ... of the M K / 8 chunks of all rows (at most MAXC per thread); fwht_rows_to_lds finishes the
