@@ -326,6 +326,17 @@ int uniql_fwht(const void* x, void* y, int64_t rows, int dim, int block,
 int uniql_fwht_composite(const void* x, void* y, int64_t rows, int dim, int base,
                          float scale, int dtype, void* stream);
 
+/*
+ * The power-of-two transform down the columns of a row-major [rows, cols] matrix:
+ * y[:, c] = T((H_rows . x[:, c]) * scale), the same values as transposing, uniql_fwht along the
+ * rows, and transposing back.  The output side of HadLinear.fuse_hadamard
+ * (quantize/quant_linear_layers.py:159-167).
+ *   rows 1024, 2048 or 4096 (UNIQL_E_UNSUPPORTED otherwise), cols % 8 == 0, x and y 16-byte aligned;
+ *   y must not overlap x
+ */
+int uniql_fwht_columns(const void* x, void* y, int rows, int cols, float scale, int dtype, void* stream);
+
+
 #ifdef __cplusplus
 }
 #endif

@@ -64,6 +64,17 @@ def test_transform_in_every_type_and_width(gpu, dtype, block):
 
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("rows,cols", [(1024, 8), (1024, 264), (2048, 8), (2048, 1048), (4096, 8), (4096, 136)])
+def test_column_transform(gpu, dtype, rows, cols):
+    """One tile and less, tiles that do not divide the width, more tiles than XCDs: the row transform of the transpose."""
+    from uniql_amd import ops
+    x = torch.randn(rows, cols, generator=torch.Generator().manual_seed(rows + cols)).to(dtype).to(gpu)
+    y = ops.hadamard_columns(x, rows ** -0.5)
+    assert torch.equal(y, ops.fast_hadamard_transform(x.t().contiguous(), rows ** -0.5).t())
+    assert ops.hadamard_columns(x[:, :4].contiguous(), 1.0) is None and ops.hadamard_columns(x[:512].contiguous(), 1.0) is None
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("dim", [12 * 128, 12 * 2048, 20 * 64, 20 * 1024, 28 * 128, 28 * 1024, 40 * 512, 40 * 1024])
 def test_composite_transform_widths(gpu, dtype, dim):
     """The smallest and largest width of the vector kernel for each base, and one of the kernel it leaves the rest to."""
@@ -73,3 +84,17 @@ def test_composite_transform_widths(gpu, dtype, dim):
     y = ops.hadamard_composite(x.to(gpu), scale, base)
     want = torch.from_numpy(O.fwht_composite(x.float().numpy(), 1.0, base)) * torch.tensor(scale, dtype=torch.float32)
     assert np.array_equal(y.float().cpu().numpy(), _as(want, dtype))
+
+
+def test_hadlinear_leaves_the_layer_it_is_made_from_alone(gpu):
+    from uniql_amd.quantize.quant_linear_layers import HadLinear
+    g = torch.Generator().manual_seed(2)
+    lin = torch.nn.Linear(256, 1024, bias=False).half().to(gpu)
+    lin.weight.data = torch.randn(1024, 256, generator=g).half().to(gpu)
+    before = lin.weight.data.clone()
+    fused = HadLinear(lin, input_transform=True, output_transform=True, fuse_had=True)
+    want = O.hadlinear_fused_weight(before.cpu().numpy(), True, True)
+    assert np.array_equal(fused.weight.data.cpu().numpy().view(np.uint16), want.view(np.uint16))
+    plain = HadLinear(lin, input_transform=False, output_transform=False, fuse_had=True)
+    assert torch.equal(plain.weight.data, before) and plain.weight.data_ptr() != lin.weight.data_ptr()
+    assert torch.equal(lin.weight.data, before)

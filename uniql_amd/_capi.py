@@ -56,6 +56,7 @@ SIGNATURES = {
                                    c_void_p, c_int, c_int64, c_int, c_int, c_int, c_int, c_int, c_int, c_void_p]),
     "uniql_fwht": (c_int, [c_void_p, c_void_p, c_int64, c_int, c_int, c_float, c_int, c_void_p]),
     "uniql_fwht_composite": (c_int, [c_void_p, c_void_p, c_int64, c_int, c_int, c_float, c_int, c_void_p]),
+    "uniql_fwht_columns": (c_int, [c_void_p, c_void_p, c_int, c_int, c_float, c_int, c_void_p]),
 }
 
 _lib = None

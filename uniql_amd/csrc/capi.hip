@@ -38,6 +38,7 @@ int fwht_launch(const void* x, void* y, int64_t rows, int dim, int block, float 
                 hipStream_t stream);
 int fwht_composite_launch(const void* x, void* y, int64_t rows, int dim, int base, float scale, int dtype,
                           hipStream_t stream);
+int fwht_columns_launch(const void* x, void* y, int rows, int cols, float scale, int dtype, hipStream_t stream);
 int quantize_launch(const void* W, int64_t ldw, const void* given_scales, void* B, void* S, int out_features,
                     int in_features, int n_pad, int k_pad, hipStream_t stream);
 int pack_launch(const uint8_t* codes, const void* scales, void* B, void* S, int n, int k, int n_pad, int k_pad,
@@ -455,6 +456,15 @@ int uniql_fwht_composite(const void* x, void* y, int64_t rows, int dim, int base
     if (rows == 0) return UNIQL_OK;
     if (!x || !y) return UNIQL_E_NULL;
     return fwht_composite_launch(x, y, rows, dim, base, scale, dtype, reinterpret_cast<hipStream_t>(stream));
+}
+
+int uniql_fwht_columns(const void* x, void* y, int rows, int cols, float scale, int dtype, void* stream) {
+    if (dtype != UNIQL_DT_F16 && dtype != UNIQL_DT_BF16 && dtype != UNIQL_DT_F32) return UNIQL_E_UNSUPPORTED;
+    if (rows != 1024 && rows != 2048 && rows != 4096) return UNIQL_E_UNSUPPORTED;
+    if (cols <= 0 || cols % 8 != 0) return UNIQL_E_SHAPE;
+    if (!x || !y) return UNIQL_E_NULL;
+    if (!aligned16(x) || !aligned16(y)) return UNIQL_E_ALIGN;
+    return fwht_columns_launch(x, y, rows, cols, scale, dtype, reinterpret_cast<hipStream_t>(stream));
 }
 
 }  // extern "C"

@@ -308,6 +308,139 @@ static int fwht_vec_launch(const void* x, void* y, int64_t pieces, int block, fl
     return UNIQL_OK;
 }
 
+// ---- down the columns of a row-major matrix: y = T((H_L . x) * scale), L = 1024, 2048 or 4096 rows ------------
+// The output side of a weight rotation without the two transposed copies around the row transform.  A workgroup
+// takes 32768 / L neighbouring columns over all rows as one fp32 image in LDS (136 KB with its padding: four floats
+// per 64), so that a value is read and written once:
+//   load    a thread reads eight consecutive rows x eight columns (16 bytes of fp16 per row): index bits 0..2;
+//   middle  bits 3 .. n-5, one column of 2^(n-7) rows per task;
+//   final   the top four bits of two neighbouring columns, scaled, rounded and stored.
+// Same butterfly order as the row transform: the same values as transposing twice.  A row of a tile is only
+// 16 to 128 bytes, so neighbouring tiles share cache lines: the tiles of one XCD (workgroups i, i + 8, i + 16, ...) are
+// neighbours, and run at the same time, so a line is fetched and written back once per second-level cache.
+// 4096 x 14336 fp16: 98 us, against 504 us for two transposed copies (230 each) and the row transform (44).
+__device__ __forceinline__ int fwht_pad64(int idx) { return idx + ((idx >> 6) << 2); }
+
+template <typename T, int LOG2L>
+__global__ __launch_bounds__(512) void fwht_columns_kernel(const T* __restrict__ x, T* __restrict__ y, int cols, int tiles, float scale) {
+    extern __shared__ __attribute__((aligned(16))) float fbuf[];
+    constexpr int L = 1 << LOG2L, CT = 32768 >> LOG2L, LOG2CT = 15 - LOG2L, CHUNKS = CT / 8;
+    const int tid = threadIdx.x;
+    const int per_xcd = (tiles + 7) >> 3;
+    const int tile = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
+    if (tile >= tiles) return;  // uniform
+    const int col0 = tile * CT;
+    {
+        const int chunk = tid & (CHUNKS - 1), row0 = (tid / CHUNKS) * 8;
+        const bool real = col0 + 8 * chunk < cols;  // cols is a multiple of eight: a chunk exists or it does not
+        typename RowIo<T>::Raw raw[8];
+        if (real) {
+#pragma unroll
+            for (int i = 0; i < 8; ++i) raw[i] = RowIo<T>::load(x + (size_t)(row0 + i) * cols + col0 + 8 * chunk);
+            float f[8][8];
+#pragma unroll
+            for (int i = 0; i < 8; ++i) RowIo<T>::unpack(raw[i], f[i]);
+#pragma unroll
+            for (int h = 1; h < 8; h <<= 1)
+#pragma unroll
+                for (int i = 0; i < 8; ++i)
+                    if ((i & h) == 0) {
+#pragma unroll
+                        for (int e = 0; e < 8; ++e) {
+                            const float p = f[i][e], q = f[i + h][e];
+                            f[i][e] = p + q;
+                            f[i + h][e] = p - q;
+                        }
+                    }
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                float* dst = fbuf + fwht_pad64((row0 + i) * CT + 8 * chunk);
+                *reinterpret_cast<f4*>(dst) = f4{f[i][0], f[i][1], f[i][2], f[i][3]};
+                *reinterpret_cast<f4*>(dst + 4) = f4{f[i][4], f[i][5], f[i][6], f[i][7]};
+            }
+        }
+    }
+    __syncthreads();
+    {
+        constexpr int PB = LOG2L - 7, E = 1 << PB, LO = 3;
+        constexpr int LOWS = 8 * CT;  // (row bits 0..2, column): one run of consecutive floats
+#pragma unroll
+        for (int task = tid; task < 32768 / E; task += 512) {
+            const int low = task & (LOWS - 1), high = task / LOWS;  // high: row bits LO + PB ..
+            const int base = (high << (LO + PB + LOG2CT)) + low;
+            float v[E];
+#pragma unroll
+            for (int i = 0; i < E; ++i) v[i] = fbuf[fwht_pad64(base + (i << (LO + LOG2CT)))];
+#pragma unroll
+            for (int h = 1; h < E; h <<= 1)
+#pragma unroll
+                for (int i = 0; i < E; ++i)
+                    if ((i & h) == 0) {
+                        const float p = v[i], q = v[i + h];
+                        v[i] = p + q;
+                        v[i + h] = p - q;
+                    }
+#pragma unroll
+            for (int i = 0; i < E; ++i) fbuf[fwht_pad64(base + (i << (LO + LOG2CT)))] = v[i];
+        }
+    }
+    __syncthreads();
+    {
+        constexpr int LO = LOG2L - 4;
+#pragma unroll
+        for (int task = tid; task < 1024; task += 512) {
+            const int c = 2 * (task & (CT / 2 - 1)), row = task / (CT / 2);  // row bits 0 .. LO - 1
+            if (col0 + c >= cols) continue;
+            float a[16], b[16];
+#pragma unroll
+            for (int i = 0; i < 16; ++i) {
+                const float2 v = *reinterpret_cast<const float2*>(fbuf + fwht_pad64(((i << LO) + row) * CT + c));
+                a[i] = v.x;
+                b[i] = v.y;
+            }
+#pragma unroll
+            for (int h = 1; h < 16; h <<= 1)
+#pragma unroll
+                for (int i = 0; i < 16; ++i)
+                    if ((i & h) == 0) {
+                        const float p = a[i], q = a[i + h], r = b[i], t = b[i + h];
+                        a[i] = p + q;
+                        a[i + h] = p - q;
+                        b[i] = r + t;
+                        b[i + h] = r - t;
+                    }
+#pragma unroll
+            for (int i = 0; i < 16; ++i) RowIo<T>::store2(y + (size_t)((i << LO) + row) * cols + col0 + c, a[i], b[i], scale);
+        }
+    }
+}
+
+template <typename T, int LOG2L>
+static int fwht_columns_go(const void* x, void* y, int cols, float scale, hipStream_t stream) {
+    constexpr int CT = 32768 >> LOG2L;
+    constexpr size_t shmem = (32768 + 32768 / 16) * sizeof(float);
+    static std::atomic<unsigned long long> done{0};
+    if (!allow_lds(&fwht_columns_kernel<T, LOG2L>, shmem, done)) return UNIQL_E_LAUNCH;
+    const int tiles = (cols + CT - 1) / CT;
+    hipLaunchKernelGGL((fwht_columns_kernel<T, LOG2L>), dim3((unsigned)((tiles + 7) / 8 * 8)), dim3(512), shmem, stream,
+                       reinterpret_cast<const T*>(x), reinterpret_cast<T*>(y), cols, tiles, scale);
+    return hipGetLastError() == hipSuccess ? UNIQL_OK : UNIQL_E_LAUNCH;
+}
+template <typename T>
+static int fwht_columns_rows(const void* x, void* y, int rows, int cols, float scale, hipStream_t stream) {
+    switch (rows) {
+        case 1024: return fwht_columns_go<T, 10>(x, y, cols, scale, stream);
+        case 2048: return fwht_columns_go<T, 11>(x, y, cols, scale, stream);
+        case 4096: return fwht_columns_go<T, 12>(x, y, cols, scale, stream);
+        default: return UNIQL_E_UNSUPPORTED;
+    }
+}
+int fwht_columns_launch(const void* x, void* y, int rows, int cols, float scale, int dtype, hipStream_t stream) {
+    if (dtype == UNIQL_DT_F16) return fwht_columns_rows<half_t>(x, y, rows, cols, scale, stream);
+    if (dtype == UNIQL_DT_BF16) return fwht_columns_rows<__bf16>(x, y, rows, cols, scale, stream);
+    return fwht_columns_rows<float>(x, y, rows, cols, scale, stream);
+}
+
 // ---- composite widths: dim = BASE * P with P a power of two -----------------------------------
 // The row is BASE chunks of P values: every chunk gets the P-point transform (LDS passes over
 // the whole row touch only index bits below log2 P, so the chunks stay apart), then the BASE x BASE

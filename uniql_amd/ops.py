@@ -21,7 +21,8 @@ from . import _capi
 __all__ = [
     "w4a16o16_gemm", "w4a16_gemm_ex", "w4a16_gemm_static", "w4a16_linear", "prepare_linear", "linear_prepared",
     "w4a16_dequant", "w4a16_embedding_lookup",
-    "fast_hadamard_transform", "hadamard_blockwise", "hadamard_composite", "composite_hadamard_variant",
+    "fast_hadamard_transform", "hadamard_blockwise", "hadamard_composite", "hadamard_columns",
+    "composite_hadamard_variant",
     "w4a16_read_floor", "w4a16_quantize", "w4a16_pack", "w4a16_unpack", "w4_embedding_quantize", "rope_indices_",
 ]
 
@@ -593,6 +594,27 @@ def hadamard_composite(x: torch.Tensor, scale: float, base: int) -> torch.Tensor
         code = lib.uniql_fwht_composite(xc.data_ptr(), y.data_ptr(), rows, dim, base, float(scale),
                                         dtypes[x.dtype], _stream_ptr(dev))
     _capi.check(code, "uniql_fwht_composite")
+    return y
+
+
+_COLUMN_ROWS = (1024, 2048, 4096)   # heights uniql_fwht_columns takes
+
+
+def hadamard_columns(x: torch.Tensor, scale: float) -> torch.Tensor | None:
+    """(H_rows . x) * scale for a contiguous matrix x [rows, cols]: fast_hadamard_transform(x.t(), scale).t() without
+    the transposed copies, a new contiguous tensor; None where the kernel does not take the shape."""
+    _require_gpu(x, "x")
+    dtypes = {torch.float16: _capi.DT_F16, torch.bfloat16: _capi.DT_BF16, torch.float32: _capi.DT_F32}
+    if x.dim() != 2 or x.dtype not in dtypes or not x.is_contiguous() or x.shape[0] not in _COLUMN_ROWS or x.shape[1] == 0 \
+            or x.shape[1] % 8 or x.data_ptr() % 16:
+        return None
+    lib = _capi.load()
+    dev = x.device
+    with _device_guard(dev):
+        y = torch.empty_like(x)
+        code = lib.uniql_fwht_columns(x.data_ptr(), y.data_ptr(), x.shape[0], x.shape[1], float(scale), dtypes[x.dtype],
+                                      _stream_ptr(dev))
+    _capi.check(code, "uniql_fwht_columns")
     return y
 
 

@@ -139,39 +139,43 @@ class HadLinear(nn.Linear):
 
     def __init__(self, originalLayer: nn.Linear, input_transform=True, output_transform=False, fuse_had=False):
         assert originalLayer.weight.is_cuda, "Hadamard transform must be on CUDA"
-        has_bias = originalLayer.bias is not None
-        super().__init__(originalLayer.in_features, originalLayer.out_features, has_bias,
-                         originalLayer.weight.device, originalLayer.weight.dtype)
+        # (nn.Linear's own constructor would allocate and randomly initialise a weight that is replaced at once)
+        nn.Module.__init__(self)
+        self.in_features, self.out_features = originalLayer.in_features, originalLayer.out_features
+        self.weight = nn.Parameter(originalLayer.weight.data)
+        if originalLayer.bias is not None:
+            assert not output_transform, "Bias is not supported for output_transform"
+            self.bias = nn.Parameter(originalLayer.bias.data)
+        else:
+            self.register_parameter("bias", None)
         self.input_transform = input_transform
         self.output_transform = output_transform
         if input_transform:
             self.input_transform_fn, self.Nin, self.had_scale_in = get_had_fn(originalLayer.in_features)
         if output_transform:
             self.output_transform_fn, self.Nout, self.had_scale_out = get_had_fn(originalLayer.out_features)
-        self.weight.data = originalLayer.weight.data
-        if has_bias:
-            assert not output_transform, "Bias is not supported for output_transform"
-            self.bias.data = originalLayer.bias.data
         self.fuse_had = False
         if fuse_had:
             self.fuse_hadamard()
 
     def _rotated(self, w):
+        """A new tensor (the transforms never write their input), `w` itself when neither side is rotated."""
         if self.input_transform:
             w = self.input_transform_fn(w, self.had_scale_in)
         if self.output_transform:
-            w = self.output_transform_fn(w.t(), self.had_scale_out).t()
+            # power-of-two heights go down the columns; the others through two transposed copies
+            rotated = ops.hadamard_columns(w, self.had_scale_out) if self.Nout == 2 else None
+            w = self.output_transform_fn(w.t(), self.had_scale_out).t() if rotated is None else rotated
         return w
 
     def fuse_hadamard(self):
-        self.weight.data = self._rotated(self.weight.data.clone()).contiguous()
+        w = self.weight.data
+        rotated = self._rotated(w)
+        self.weight.data = rotated.contiguous() if rotated is not w else w.clone()
         self.fuse_had = True
 
     def forward(self, x):
-        w = self.weight.clone()
-        if not self.fuse_had:
-            w = self._rotated(w)
-        return F.linear(x, w, self.bias)
+        return F.linear(x, self.weight if self.fuse_had else self._rotated(self.weight), self.bias)
 
     def __repr__(self):
         return (f"HadLinear(in_features={self.in_features}, out_features={self.out_features}, "
