@@ -250,6 +250,31 @@ int uniql_w4a16_pack(const uint8_t* codes, const void* scales, void* B, void* S,
                      void* stream);
 
 /*
+ * Keeps columns of a packed matrix (group-128 scales) without unpacking it: what the slicing functions of
+ * modeling/modeling_helpers.py:361-757 get by unpacking, indexing and packing on the CPU.
+ *   B, S      device, int32 [k/16, 2 n] and fp16 [k/128, n], permuted
+ *   runs      HOST, int[6 n_runs] (1 <= n_runs <= 5): {base, units, full, kept, split, skip}, one after the other; a run
+ *             keeps the columns base + u full + i (+ skip from i = split on) for u < units, i < kept, in that order
+ *   k_real    rows from here on get code 0
+ *   n_scaled  output columns from here on get scale 0 (their codes stay)
+ *   B_out     device out, int32 [k/16, 2 n_pad];  S_out  device out, fp16 [k/128, n_pad], permuted
+ *   n_pad >= the number of kept columns, n_pad % 128 == 0 (padding columns: code 0, scale 0)
+ */
+int uniql_w4a16_cut_columns(const void* B, const void* S, int n, int k, int k_real, const int* runs, int n_runs,
+                            int n_scaled, void* B_out, void* S_out, int n_pad, void* stream);
+
+/*
+ * Keeps rows of a packed matrix and quantises them again in their new groups: uniql_w4a16_dequant, the kept rows of its
+ * result, uniql_w4a16_quantize of their transpose, in one kernel and with the same results bit for bit
+ * (modeling/modeling_helpers.py:600-656,809-867).
+ *   B, S    device, int32 [k/16, 2 n] and fp16 [groups, n], permuted (groups == k/128 or 1)
+ *   kept rows: u full + i for u < units, i < kept, in that order; more than 128 of them
+ *   n_real  output columns that exist (<= n); B_out, S_out, n_pad >= n_real as above, k_pad = units kept rounded up to 128
+ */
+int uniql_w4a16_cut_rows(const void* B, const void* S, int n, int k, int groups, int units, int full, int kept, int n_real,
+                         void* B_out, void* S_out, int n_pad, void* stream);
+
+/*
  * out[t, :] = fp16_rn((code - 8) * scales[ids[t]]) for t < ntokens.
  * Replaces quant_embedding_cuda.w4a16_embedding_lookup
  * (csrc/embedding/quant_embedding_kernel.cuh:80-166).

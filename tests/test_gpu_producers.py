@@ -1,5 +1,6 @@
 """The kernels that produce a 4-bit model's tensors, where their paths change: scales and weights outside of what the
-quantiser's three-instruction quotient covers, the transforms' types and widths, the column transform."""
+quantiser's three-instruction quotient covers, the transforms' types and widths, the column transform, the cuts of packed
+matrices."""
 import numpy as np
 import pytest
 import torch
@@ -98,3 +99,62 @@ def test_hadlinear_leaves_the_layer_it_is_made_from_alone(gpu):
     plain = HadLinear(lin, input_transform=False, output_transform=False, fuse_had=True)
     assert torch.equal(plain.weight.data, before) and plain.weight.data_ptr() != lin.weight.data_ptr()
     assert torch.equal(lin.weight.data, before)
+
+
+def _packed_layer(gpu, k, n, g):
+    from uniql_amd import ops
+    codes = torch.randint(0, 16, (k, n), generator=g).to(torch.uint8).to(gpu)
+    scales = (torch.rand(k // 128, n, generator=g) * 0.02 + 0.004).half().to(gpu)
+    scales[:, 3] = 0
+    return ops.w4a16_pack(codes, scales), codes, scales
+
+
+@pytest.mark.parametrize("k,k_real", [(128, 128), (256, 250), (1408, 1399)])
+@pytest.mark.parametrize("runs,n_scaled,pad", [
+    ([(0, 1, 256, 256, 256, 0)], 200, 0),                          # a prefix: whole chunks
+    ([(64, 1, 320, 320, 320, 0)], 320, 64),                        # whole chunks from the second one on
+    ([(0, 3, 100, 38, 19, 31)], 114, 14),                          # two pieces of every head
+    ([(0, 2, 33, 17, 17, 0), (5, 0, 9, 3, 3, 0), (66, 4, 40, 40, 20, 0), (511, 1, 1, 1, 1, 0), (300, 1, 11, 6, 2, -3)], 201, 55),
+])
+def test_cut_columns(gpu, k, k_real, runs, n_scaled, pad):
+    """Rows that do not end with a group, runs inside and across chunks, padding: packing the indexed codes."""
+    from uniql_amd import ops
+    (w, s), codes, scales = _packed_layer(gpu, k, 512, torch.Generator().manual_seed(k))
+    cols = [base + u * full + i + (skip if i >= split else 0)
+            for base, units, full, kept, split, skip in runs for u in range(units) for i in range(kept)]
+    kept_codes, kept_scales = codes[:, cols], scales[:, cols]
+    kept_codes[k_real:] = 0
+    kept_scales[:, n_scaled:] = 0
+    want = ops.w4a16_pack(kept_codes, kept_scales, pad_out=pad)
+    got = ops.w4a16_cut_columns(w, s, 512, k, runs, k_real=k_real, n_scaled=n_scaled, pad_out=pad)
+    assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
+    with pytest.raises(RuntimeError):
+        ops.w4a16_cut_columns(w, s, 512, k, [(1, 1, 512, 512, 512, 0)])
+
+
+def test_cut_columns_many_groups_per_workgroup(gpu):
+    from uniql_amd import ops
+    k, n = 128 * 131, 4096
+    (w, s), codes, scales = _packed_layer(gpu, k, n, torch.Generator().manual_seed(5))
+    runs = [(0, 32, 128, 126, 63, 1)]
+    cols = torch.tensor([128 * u + i + (i >= 63) for u in range(32) for i in range(126)], device=gpu)
+    want = ops.w4a16_pack(codes[:, cols], scales[:, cols], pad_out=64)
+    got = ops.w4a16_cut_columns(w, s, n, k, runs, pad_out=64)
+    assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
+
+
+@pytest.mark.parametrize("n,n_real,pad", [(128, 128, 0), (256, 200, 56), (256, 130, 126), (256, 60, 324)])
+@pytest.mark.parametrize("k,units,full,kept", [(256, 1, 0, 129), (512, 4, 128, 108), (1280, 10, 128, 77), (1280, 37, 33, 31)])
+@pytest.mark.parametrize("per_column", [False, True])
+def test_cut_rows(gpu, n, n_real, pad, k, units, full, kept, per_column):
+    """Kept rows over group and word boundaries, odd widths: quantising the gathered dequantised rows."""
+    from uniql_amd import ops
+    (w, s), _, _ = _packed_layer(gpu, k, n, torch.Generator().manual_seed(n + k))
+    if per_column:
+        s = s[:1].contiguous()
+    rows = torch.tensor([u * full + i for u in range(units) for i in range(kept)], device=gpu)
+    want = ops.w4a16_quantize(ops.w4a16_dequant(w, s, n, k)[rows][:, :n_real].t().contiguous(), None, pad_out=pad)
+    got = ops.w4a16_cut_rows(w, s, n, k, units, full, kept, n_real, pad_out=pad)
+    assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
+    with pytest.raises(RuntimeError):
+        ops.w4a16_cut_rows(w, s, n, k, 2, k, 100, n_real, pad_out=pad)

@@ -43,6 +43,10 @@ int quantize_launch(const void* W, int64_t ldw, const void* given_scales, void* 
                     int in_features, int n_pad, int k_pad, hipStream_t stream);
 int pack_launch(const uint8_t* codes, const void* scales, void* B, void* S, int n, int k, int n_pad, int k_pad,
                 hipStream_t stream);
+int cut_columns_launch(const void* B, const void* S, int n, int k, int k_real, const int* runs, int n_runs, int n_scaled,
+                       void* B_out, void* S_out, int n_pad, hipStream_t stream);
+int cut_rows_launch(const void* B, const void* S, int n, int groups_in, int units, int full, int kept, int n_real, void* B_out,
+                    void* S_out, int n_pad, hipStream_t stream);
 }  // namespace uniql
 
 using namespace uniql;
@@ -397,6 +401,43 @@ int uniql_w4a16_pack(const uint8_t* codes, const void* scales, void* B, void* S,
     if (n <= 0 || k <= 0 || k % 128 != 0 || n_pad < n || n_pad % 128 != 0) return UNIQL_E_SHAPE;
     if ((int64_t)(k / 16) * 2 * n_pad > 0x7fffffffLL * 256) return UNIQL_E_SHAPE;
     return pack_launch(codes, scales, B, S, n, k, n_pad, k, reinterpret_cast<hipStream_t>(stream));
+}
+
+int uniql_w4a16_cut_columns(const void* B, const void* S, int n, int k, int k_real, const int* runs, int n_runs, int n_scaled,
+                            void* B_out, void* S_out, int n_pad, void* stream) {
+    const int rc = check_linear_shape(1, n, k, k / 128);
+    if (rc != UNIQL_OK) return rc;
+    if (!B || !S || !runs || !B_out || !S_out) return UNIQL_E_NULL;
+    if (n_runs < 1 || n_runs > 5 || k_real < 0 || k_real > k) return UNIQL_E_SHAPE;
+    int64_t total = 0;
+    for (int i = 0; i < n_runs; ++i) {
+        const int64_t base = runs[6 * i], units = runs[6 * i + 1], full = runs[6 * i + 2], kept = runs[6 * i + 3];
+        const int64_t split = runs[6 * i + 4], skip = runs[6 * i + 5];
+        if (base < 0 || units < 0 || full < 0 || kept < 0 || split < 0 || split > kept) return UNIQL_E_SHAPE;
+        if (units * kept == 0) continue;
+        const int64_t last_unit = base + (units - 1) * full;
+        if (last_unit + split > n) return UNIQL_E_SHAPE;
+        if (split < kept && (base + split + skip < 0 || last_unit + kept + skip > n)) return UNIQL_E_SHAPE;
+        total += units * kept;
+    }
+    if (total <= 0 || n_pad <= 0 || n_pad < total || n_pad % 128 != 0 || n_scaled < 0) return UNIQL_E_SHAPE;
+    if (!aligned16(B) || !aligned16(B_out)) return UNIQL_E_ALIGN;
+    return cut_columns_launch(B, S, n, k, k_real, runs, n_runs, n_scaled, B_out, S_out, n_pad,
+                              reinterpret_cast<hipStream_t>(stream));
+}
+
+int uniql_w4a16_cut_rows(const void* B, const void* S, int n, int k, int groups, int units, int full, int kept, int n_real,
+                         void* B_out, void* S_out, int n_pad, void* stream) {
+    const int rc = check_linear_shape(1, n, k, groups);
+    if (rc != UNIQL_OK) return rc;
+    if (!B || !S || !B_out || !S_out) return UNIQL_E_NULL;
+    if (units < 1 || full < 0 || kept < 1 || (int64_t)(units - 1) * full + kept > k) return UNIQL_E_SHAPE;
+    if (n_real < 1 || n_real > n || n_pad < n_real || n_pad % 128 != 0) return UNIQL_E_SHAPE;
+    if ((int64_t)units * kept <= 128) return UNIQL_E_UNSUPPORTED;
+    if ((int64_t)units * kept > 0x7fffffffLL - 128) return UNIQL_E_SHAPE;
+    if (!aligned16(B) || !aligned16(B_out) || !aligned16(S_out)) return UNIQL_E_ALIGN;
+    return cut_rows_launch(B, S, n, groups, units, full, kept, n_real, B_out, S_out, n_pad,
+                           reinterpret_cast<hipStream_t>(stream));
 }
 
 int uniql_w4_embedding_lookup(const int64_t* ids, int64_t ntokens, const void* weight, const void* scales,

@@ -80,32 +80,20 @@ __device__ __forceinline__ void quantize_sixteen(const h8 (&w)[2], half_t s, boo
     }
 }
 
-template <bool GPTQ>
-__global__ __launch_bounds__(256) void w4a16_quantize_kernel(const half_t* __restrict__ W, int64_t ldw, int vec_ok,
-                                                            const half_t* __restrict__ given, half_t* __restrict__ S,
-                                                            uint32_t* __restrict__ B, int out_features, int in_features,
-                                                            int n_pad, int groups) {
-    __shared__ __attribute__((aligned(16))) uint32_t words[8 * kPackLdsRow];
-    __shared__ __attribute__((aligned(16))) half_t scales[64];
+// Quantises and stores one tile; load(n, w) fetches the thread's 16 K values (from 128 g + 16 r on) of column n, zeros
+// where there is none.
+template <bool GPTQ, class Load>
+__device__ __forceinline__ void quantize_tile(const Load& load, uint32_t* words, half_t* scales, const half_t* __restrict__ given,
+                                              half_t* __restrict__ S, uint32_t* __restrict__ B, int out_features, int n_pad,
+                                              int g, int chunk) {
     const int tid = threadIdx.x;
     const int r = tid & 7, c8 = (tid >> 3) & 7, j = tid >> 6;
-    const int g = blockIdx.x % groups, chunk = blockIdx.x / groups;  // neighbours read on along the same rows
-    const int k0 = 128 * g + 16 * r;
     uint32_t out[4] = {0u, 0u, 0u, 0u};
 #pragma unroll
     for (int blk = 0; blk < 2; ++blk) {
         const int n = 64 * chunk + 16 * j + 8 * blk + c8;
         h8 w[2];
-#pragma unroll
-        for (int i = 0; i < 2; ++i) {
-            const half_t* src = W + (size_t)n * ldw + k0 + 8 * i;
-            if (n < out_features && k0 + 8 * i + 8 <= in_features && vec_ok) {
-                w[i] = *reinterpret_cast<const h8*>(src);
-            } else {
-#pragma unroll
-                for (int e = 0; e < 8; ++e) w[i][e] = n < out_features && k0 + 8 * i + e < in_features ? src[e] : (half_t)0.0f;
-            }
-        }
+        load(n, w);
         h2 m = h2{(half_t)0.0f, (half_t)0.0f};
 #pragma unroll
         for (int i = 0; i < 2; ++i)
@@ -156,6 +144,164 @@ __global__ __launch_bounds__(256) void w4a16_quantize_kernel(const half_t* __res
     *reinterpret_cast<u32x4*>(B + (size_t)(8 * g + row) * 2 * n_pad + 128 * (size_t)chunk + 4 * piece) = v;
     if (tid < 8)
         *reinterpret_cast<u32x4*>(S + (size_t)g * n_pad + 64 * (size_t)chunk + 8 * tid) = *reinterpret_cast<const u32x4*>(scales + 8 * tid);
+}
+
+template <bool GPTQ>
+__global__ __launch_bounds__(256) void w4a16_quantize_kernel(const half_t* __restrict__ W, int64_t ldw, int vec_ok,
+                                                            const half_t* __restrict__ given, half_t* __restrict__ S,
+                                                            uint32_t* __restrict__ B, int out_features, int in_features,
+                                                            int n_pad, int groups) {
+    __shared__ __attribute__((aligned(16))) uint32_t words[8 * kPackLdsRow];
+    __shared__ __attribute__((aligned(16))) half_t scales[64];
+    const int g = blockIdx.x % groups, chunk = blockIdx.x / groups;  // neighbours read on along the same rows
+    const int k0 = 128 * g + 16 * (threadIdx.x & 7);
+    const auto load = [&](int n, h8 (&w)[2]) {
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            const half_t* src = W + (size_t)n * ldw + k0 + 8 * i;
+            if (n < out_features && k0 + 8 * i + 8 <= in_features && vec_ok) {
+                w[i] = *reinterpret_cast<const h8*>(src);
+            } else {
+#pragma unroll
+                for (int e = 0; e < 8; ++e) w[i][e] = n < out_features && k0 + 8 * i + e < in_features ? src[e] : (half_t)0.0f;
+            }
+        }
+    };
+    quantize_tile<GPTQ>(load, words, scales, given, S, B, out_features, n_pad, g, chunk);
+}
+
+// Keeps rows of a packed matrix that no longer line up with the groups, and quantises them again: what dequantising, gathering
+// the rows, transposing and the kernel above give, without the fp16 matrix and its two copies (4096 x 4096, 32 heads of 128
+// cut to 108 rows: 14.3 us).  Kept row i is row (i / kept) full + i % kept.  One workgroup takes 64 columns x one group of the
+// OUTPUT: 1024 tasks of one kept row x eight columns (one 16-byte piece holds them; neighbouring rows read the same
+// pieces, from the first-level cache) expand into LDS, from where every thread takes its 2 x 16 values.
+constexpr int kCutLdsRow = 136;  // fp16 values per column in LDS: 128 + 8, 16-byte reads of eight columns on different banks
+
+__global__ __launch_bounds__(256) void w4a16_cut_rows_kernel(const uint32_t* __restrict__ Bin, const half_t* __restrict__ Sin,
+                                                            half_t* __restrict__ S, uint32_t* __restrict__ B, int n, int k_kept,
+                                                            int full, int kept, int per_column, int vec_ok, int n_real,
+                                                            int n_pad, int groups) {
+    __shared__ __attribute__((aligned(16))) uint32_t words[8 * kPackLdsRow];
+    __shared__ __attribute__((aligned(16))) half_t scales[64];
+    __shared__ __attribute__((aligned(16))) half_t values[64 * kCutLdsRow];
+    const int g = blockIdx.x % groups, chunk = blockIdx.x / groups;
+    const int tid = threadIdx.x, c8 = tid & 7;
+    if (64 * chunk < n_real) {  // n_real <= n: the chunk exists in the source
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+            const int row = 32 * t + (tid >> 3), i = 128 * g + row;
+            h8 v = {};
+            if (i < k_kept) {
+                const int k = (i / kept) * full + i % kept;
+                const u32x4 q4 = *reinterpret_cast<const u32x4*>(Bin + (size_t)(k >> 4) * 2 * n + 128 * (size_t)chunk + 16 * c8 +
+                                                                 4 * ((k >> 1) & 3));
+                const int bit = 16 * (k & 1) + 4 * ((k >> 3) & 1);
+                const half_t* sp = Sin + (per_column ? 0 : (size_t)(k >> 7) * n);
+                h8 s;
+                if (!per_column && vec_ok) {
+                    s = *reinterpret_cast<const h8*>(sp + 64 * chunk + 8 * c8);
+                } else {
+#pragma unroll
+                    for (int e = 0; e < 8; ++e)
+                        s[e] = per_column ? sp[single_scale_pos(64 * chunk + 8 * e + c8)] : sp[64 * chunk + 8 * c8 + e];
+                }
+#pragma unroll
+                for (int e = 0; e < 8; ++e)  // column 8 e + c8: word e / 2, bits 8 (e % 2) up
+                    v[e] = (half_t)(float)((int)((q4[e >> 1] >> (bit + 8 * (e & 1))) & 15u) - 8);
+                v *= s;
+            }
+#pragma unroll
+            for (int e = 0; e < 8; ++e) values[(8 * e + c8) * kCutLdsRow + row] = v[e];
+        }
+    }
+    __syncthreads();
+    const int r = tid & 7;
+    const auto load = [&](int col, h8 (&w)[2]) {
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+            w[i] = col < n_real ? *reinterpret_cast<const h8*>(values + (col & 63) * kCutLdsRow + 16 * r + 8 * i) : h8{};
+    };
+    quantize_tile<false>(load, words, scales, nullptr, S, B, n_real, n_pad, g, chunk);
+}
+
+// Keeps columns of a packed matrix, as they are: kept columns are up to five runs of `units` x (`kept` of every `full`
+// columns, from `base` on: the first `split`, and the others `skip` columns further on); columns behind them have code 0, those from n_scaled on scale 0; rows from k_real on get
+// code 0.  A column's four codes of a word are two of its bytes, so nothing is unpacked: a 16-byte piece of the output
+// takes eight 4-byte loads and a byte selection each, or, where its 64 columns are one source chunk (a kept prefix),
+// one load.  A workgroup resolves its chunk's 64 source columns once and keeps them for `per` groups of 128 rows.
+// Bound by memory and, for the small projections, by the launch (4096 x 14336 cut to 12160, 53 MB: 12.2 us = 4.3 TB/s,
+// 1024 columns: 5.4; the seven cuts of a decoder layer with their host calls 912 -> 86 us).
+struct ColumnRuns {
+    int count;
+    int base[5], units[5], full[5], kept[5], split[5], skip[5];
+};
+
+__global__ __launch_bounds__(256) void w4a16_cut_columns_kernel(const uint32_t* __restrict__ Bin, const half_t* __restrict__ Sin,
+                                                               uint32_t* __restrict__ B, half_t* __restrict__ S, int n,
+                                                               int groups, int k_real, ColumnRuns runs, int n_scaled, int n_pad,
+                                                               int per) {
+    __shared__ int source[64];
+    __shared__ int whole_chunk;
+    const int tid = threadIdx.x;
+    const int steps = (groups + per - 1) / per;
+    const int chunk = blockIdx.x / steps, g0 = (blockIdx.x % steps) * per;
+    if (tid < 64) {
+        int i = 64 * chunk + tid, col = -1;
+#pragma unroll
+        for (int s = 0; s < 5; ++s) {
+            if (s < runs.count && col < 0) {
+                const int len = runs.units[s] * runs.kept[s];
+                if (i < len) {
+                    const int at = i % runs.kept[s];
+                    col = runs.base[s] + (i / runs.kept[s]) * runs.full[s] + at + (at >= runs.split[s] ? runs.skip[s] : 0);
+                }
+                i -= len;
+            }
+        }
+        source[tid] = col;
+        const int first = __shfl(col, 0, kWave);
+        const bool same = first >= 0 && (first & 63) == 0 && col - tid == first;
+        const unsigned long long all = __ballot(same);
+        if (tid == 0) whole_chunk = all == ~0ull ? first >> 6 : -1;
+    }
+    __syncthreads();
+    const int piece = tid & 31, row = tid >> 5, c8 = piece >> 2, kq = piece & 3;
+    const int from = whole_chunk;
+    int word[8], shift[8];       // columns 8 e + c8: word of a packed row and bits to go down; -1: none
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+        const int col = source[8 * e + c8];
+        word[e] = col < 0 ? -1 : 128 * (col >> 6) + 16 * (col & 7) + 4 * kq + ((col & 63) >> 4);
+        shift[e] = 8 * ((col >> 3) & 1);
+    }
+    int scale_from = -1;
+    if (tid < 64) {  // the scale at position tid of a chunk belongs to column (tid / 8) + 8 (tid % 8)
+        const int at = 8 * (tid & 7) + (tid >> 3), col = source[at];
+        if (col >= 0 && 64 * chunk + at < n_scaled) scale_from = (int)group_scale_pos(col);
+    }
+    const int g1 = g0 + per < groups ? g0 + per : groups;
+    for (int g = g0; g < g1; ++g) {
+        const uint32_t* src = Bin + (size_t)(8 * g + row) * 2 * n;
+        u32x4 v;
+        if (from >= 0) {
+            v = *reinterpret_cast<const u32x4*>(src + 128 * (size_t)from + 4 * piece);
+        } else {
+            uint32_t q[8];
+#pragma unroll
+            for (int e = 0; e < 8; ++e) q[e] = word[e] >= 0 ? (src[word[e]] >> shift[e]) & 0x00ff00ffu : 0u;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) v[j] = q[2 * j] | (q[2 * j + 1] << 8);
+        }
+        const int k0 = 128 * g + 16 * row + 2 * kq;  // K rows k0, k0 + 1 (nibbles 0 and 4 of a 16-bit half's pairs), k0 + 8, k0 + 9
+        if (k0 + 9 >= k_real) {
+            const uint32_t mask = (k0 < k_real ? 0x00000f0fu : 0u) | (k0 + 1 < k_real ? 0x0f0f0000u : 0u) |
+                                  (k0 + 8 < k_real ? 0x0000f0f0u : 0u) | (k0 + 9 < k_real ? 0xf0f00000u : 0u);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) v[j] &= mask;
+        }
+        *reinterpret_cast<u32x4*>(B + (size_t)(8 * g + row) * 2 * n_pad + 128 * (size_t)chunk + 4 * piece) = v;
+        if (tid < 64) S[(size_t)g * n_pad + 64 * (size_t)chunk + tid] = scale_from >= 0 ? Sin[(size_t)g * n + scale_from] : (half_t)0.0f;
+    }
 }
 
 // Ready codes[k][n] -> packed words, one thread per 32-bit word.  Word j of piece (c8, kq) of chunk c of packed row r
@@ -219,6 +365,42 @@ int pack_launch(const uint8_t* codes, const void* scales, void* B, void* S, int 
     const int64_t words = (int64_t)(k_pad / 16) * 2 * n_pad;
     hipLaunchKernelGGL(w4a16_pack_kernel, dim3((unsigned)((words + 255) / 256)), dim3(256), 0, stream, codes,
                        reinterpret_cast<uint32_t*>(B), n, k, n_pad, k_pad);
+    return hipGetLastError() == hipSuccess ? UNIQL_OK : UNIQL_E_LAUNCH;
+}
+
+int cut_rows_launch(const void* B, const void* S, int n, int groups_in, int units, int full, int kept, int n_real, void* B_out,
+                    void* S_out, int n_pad, hipStream_t stream) {
+    const int k_kept = units * kept, groups = (k_kept + 127) / 128;
+    const int64_t grid = (int64_t)groups * (n_pad / 64);
+    if (grid > 0x7fffffffLL) return UNIQL_E_SHAPE;
+    hipLaunchKernelGGL(w4a16_cut_rows_kernel, dim3((unsigned)grid), dim3(256), 0, stream, reinterpret_cast<const uint32_t*>(B),
+                       reinterpret_cast<const half_t*>(S), reinterpret_cast<half_t*>(S_out), reinterpret_cast<uint32_t*>(B_out),
+                       n, k_kept, full, kept, groups_in == 1 ? 1 : 0, (reinterpret_cast<uintptr_t>(S) & 15u) == 0 ? 1 : 0,
+                       n_real, n_pad, groups);
+    return hipGetLastError() == hipSuccess ? UNIQL_OK : UNIQL_E_LAUNCH;
+}
+
+int cut_columns_launch(const void* B, const void* S, int n, int k, int k_real, const int* runs, int n_runs, int n_scaled,
+                       void* B_out, void* S_out, int n_pad, hipStream_t stream) {
+    ColumnRuns r = {};
+    r.count = n_runs;
+    for (int i = 0; i < n_runs; ++i) {
+        r.base[i] = runs[6 * i];
+        r.units[i] = runs[6 * i + 1];
+        r.full[i] = runs[6 * i + 2];
+        r.kept[i] = runs[6 * i + 3];
+        r.split[i] = runs[6 * i + 4];
+        r.skip[i] = runs[6 * i + 5];
+    }
+    const int groups = k / 128;
+    const int64_t tiles = (int64_t)groups * (n_pad / 64);
+    // Four groups per workgroup share the resolved columns once the chip (2048 workgroups at a time) is filled all the same.
+    const int per = tiles >= 4 * 2048 ? 4 : 1;
+    const int64_t grid = (int64_t)((groups + per - 1) / per) * (n_pad / 64);
+    if (grid > 0x7fffffffLL) return UNIQL_E_SHAPE;
+    hipLaunchKernelGGL(w4a16_cut_columns_kernel, dim3((unsigned)grid), dim3(256), 0, stream, reinterpret_cast<const uint32_t*>(B),
+                       reinterpret_cast<const half_t*>(S), reinterpret_cast<uint32_t*>(B_out), reinterpret_cast<half_t*>(S_out),
+                       n, groups, k_real, r, n_scaled, n_pad, per);
     return hipGetLastError() == hipSuccess ? UNIQL_OK : UNIQL_E_LAUNCH;
 }
 

@@ -23,7 +23,8 @@ __all__ = [
     "w4a16_dequant", "w4a16_embedding_lookup",
     "fast_hadamard_transform", "hadamard_blockwise", "hadamard_composite", "hadamard_columns",
     "composite_hadamard_variant",
-    "w4a16_read_floor", "w4a16_quantize", "w4a16_pack", "w4a16_unpack", "w4_embedding_quantize", "rope_indices_",
+    "w4a16_read_floor", "w4a16_quantize", "w4a16_pack", "w4a16_unpack", "w4a16_cut_columns",
+    "w4a16_cut_rows", "w4_embedding_quantize", "rope_indices_",
 ]
 
 
@@ -450,6 +451,54 @@ def w4a16_unpack(B: torch.Tensor, s: torch.Tensor, size_n: int, size_k: int):
     n = torch.arange(size_n, device=B.device)
     pos = (n & ~63) + 8 * (n & 7) + ((n & 63) >> 3)
     return codes, s[:, pos].contiguous()
+
+
+def _require_packed(B: torch.Tensor, s: torch.Tensor, size_n: int, size_k: int) -> None:
+    _require_gpu(B, "B")
+    _require_gpu(s, "s")
+    if B.dtype != torch.int32 or s.dtype != torch.float16 or not (B.is_contiguous() and s.is_contiguous()):
+        raise RuntimeError("B must be contiguous int32 and s contiguous float16")
+    if tuple(B.shape) != (size_k // 16, 2 * size_n) or s.dim() != 2 or s.shape[1] != size_n:
+        raise RuntimeError("B / s shapes do not match size_k, size_n")
+
+
+def w4a16_cut_columns(B: torch.Tensor, s: torch.Tensor, size_n: int, size_k: int, runs, k_real: int | None = None,
+                      n_scaled: int | None = None, pad_out: int = 0):
+    """Keeps columns of a packed group-128 matrix: w4a16_pack of the kept columns of w4a16_unpack, straight from packed to
+    packed.  runs: up to five (base, units, full, kept, split, skip), each `kept` of every `full` columns from `base` on, `units`
+    times: the first `split`, and the others `skip` columns further on.  Rows from k_real on get code 0; kept columns from n_scaled on get scale 0; pad_out padding columns follow."""
+    _require_packed(B, s, size_n, size_k)
+    if s.shape[0] != size_k // 128:
+        raise RuntimeError("scales must be [k/128, n]")
+    n_pad = sum(run[1] * run[3] for run in runs) + pad_out
+    flat = [int(v) for run in runs for v in run]
+    lib = _capi.load()
+    dev = B.device
+    with _device_guard(dev):
+        B_out = torch.empty((size_k // 16, 2 * n_pad), dtype=torch.int32, device=dev)
+        S_out = torch.empty((size_k // 128, n_pad), dtype=torch.float16, device=dev)
+        code = lib.uniql_w4a16_cut_columns(B.data_ptr(), s.data_ptr(), size_n, size_k, size_k if k_real is None else k_real,
+                                           (ctypes.c_int * len(flat))(*flat), len(runs), n_pad if n_scaled is None else n_scaled,
+                                           B_out.data_ptr(), S_out.data_ptr(), n_pad, _stream_ptr(dev))
+    _capi.check(code, "uniql_w4a16_cut_columns")
+    return B_out, S_out
+
+
+def w4a16_cut_rows(B: torch.Tensor, s: torch.Tensor, size_n: int, size_k: int, units: int, full: int, kept: int, n_real: int,
+                   pad_out: int = 0):
+    """Keeps the first `kept` of every `full` rows, `units` times, of a packed matrix's first n_real columns and quantises them
+    in their new groups: w4a16_quantize of the kept rows of w4a16_dequant, in one kernel."""
+    _require_packed(B, s, size_n, size_k)
+    k_pad, n_pad = (units * kept + 127) // 128 * 128, n_real + pad_out
+    lib = _capi.load()
+    dev = B.device
+    with _device_guard(dev):
+        B_out = torch.empty((k_pad // 16, 2 * n_pad), dtype=torch.int32, device=dev)
+        S_out = torch.empty((k_pad // 128, n_pad), dtype=torch.float16, device=dev)
+        code = lib.uniql_w4a16_cut_rows(B.data_ptr(), s.data_ptr(), size_n, size_k, s.shape[0], units, full, kept, n_real,
+                                        B_out.data_ptr(), S_out.data_ptr(), n_pad, _stream_ptr(dev))
+    _capi.check(code, "uniql_w4a16_cut_rows")
+    return B_out, S_out
 
 
 def w4a16_embedding_lookup(input: torch.Tensor, weight: torch.Tensor, scale: torch.Tensor) -> torch.Tensor:

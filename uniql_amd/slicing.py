@@ -2,9 +2,9 @@
 
 UniQL stores one full-size quantised model and cuts every layer down to the pruned size
 when it is loaded (modeling/modeling_helpers.py:235-867).  The reference does this on the
-CPU in numpy: unpack the Marlin layout, cut, pack again.  Here the same three steps run on
-the device (uniql_w4a16_dequant's code output, a tensor slice, uniql_w4a16_pack), with the
-reference's function names, argument order and results.
+CPU in numpy: unpack the Marlin layout, cut, pack again.  Here one kernel takes the packed tensors
+to the cut packed tensors (uniql_w4a16_cut_columns moves columns, uniql_w4a16_cut_rows quantises
+rows in new groups), with the reference's function names, argument order and results.
 """
 from __future__ import annotations
 
@@ -37,10 +37,8 @@ def slice_w4a16_up_gate_proj(weight, scale, workspace, hidden_size, intermediate
     size_k, size_n = hidden_size + pad_k, intermediate_size + pad_n
     keep = reduced_intermediate_size + reduced_pad_n
     assert size_n >= keep, "Reduced size shape exceeds recovered weight"
-    codes, scales = ops.w4a16_unpack(weight, scale, size_n, size_k)
-    cut_scales = scales[:, :keep].clone()
-    cut_scales[:, reduced_intermediate_size:] = 0
-    new_weight, new_scale = ops.w4a16_pack(codes[:, :keep], cut_scales)
+    new_weight, new_scale = ops.w4a16_cut_columns(weight, scale, size_n, size_k, [(0, 1, keep, keep, keep, 0)],
+                                                  n_scaled=reduced_intermediate_size)
     new_workspace = workspace[:(keep // MIN_THREAD_N) * MAX_PARALLEL].contiguous()
     return new_weight, new_scale, new_workspace
 
@@ -69,16 +67,11 @@ def _workspace_for(size_n: int, workspace):
     return workspace[:(size_n // MIN_THREAD_N) * MAX_PARALLEL].contiguous()
 
 
-def _gather_columns(weight, scale, workspace, size_k, size_n, rows_real, cols: torch.Tensor, pad_n_new: int):
-    """Unpacks [size_k, size_n], keeps the real K rows and the columns `cols`, pads the rows back
-    to size_k with code 0 as the reference's torch.nn.functional.pad does, and packs with
-    pad_n_new padding columns (code 0, scale 0)."""
-    codes, scales = ops.w4a16_unpack(weight, scale, size_n, size_k)
-    cut = codes[:rows_real][:, cols]
-    if rows_real < size_k:
-        cut = torch.cat([cut, cut.new_zeros(size_k - rows_real, cut.shape[1])], dim=0)
-    new_weight, new_scale = ops.w4a16_pack(cut.contiguous(), scales[:, cols].contiguous(), pad_out=pad_n_new)
-    return new_weight, new_scale, _workspace_for(cols.numel() + pad_n_new, workspace)
+def _keep_columns(weight, scale, workspace, size_k, size_n, rows_real, runs, pad_n_new: int):
+    """Keeps the columns of `runs` (as ops.w4a16_cut_columns takes them) and appends pad_n_new padding columns (code 0,
+    scale 0); rows from rows_real on get code 0, as the reference's torch.nn.functional.pad gives them."""
+    new_weight, new_scale = ops.w4a16_cut_columns(weight, scale, size_n, size_k, runs, k_real=rows_real, pad_out=pad_n_new)
+    return new_weight, new_scale, _workspace_for(new_scale.shape[1], workspace)
 
 
 def _rope_half_columns(nheads, head_dim, reduced_head_dim, device):
@@ -104,10 +97,11 @@ def slice_w4a16_qk_proj(weight, bias, scale, workspace, hidden_size, nheads, hea
     pad_n = _pad_to(nheads * head_dim, 256)
     reduced_pad_n = _pad_to(nheads * reduced_head_dim, 256)
     assert load_shape[0] == weight.shape[0], "hidden_size dimension mismatch"
-    cols = _rope_half_columns(nheads, head_dim, reduced_head_dim, weight.device)
-    new_weight, new_scale, new_workspace = _gather_columns(
-        weight, scale, workspace, hidden_size + pad_k, nheads * head_dim + pad_n, hidden_size, cols, reduced_pad_n)
-    new_bias = None if bias is None else bias[cols.to(bias.device)]
+    half, kept = head_dim // 2, reduced_head_dim // 2
+    runs = [(0, nheads, head_dim, 2 * kept, kept, half - kept)]
+    new_weight, new_scale, new_workspace = _keep_columns(
+        weight, scale, workspace, hidden_size + pad_k, nheads * head_dim + pad_n, hidden_size, runs, reduced_pad_n)
+    new_bias = None if bias is None else bias[_rope_half_columns(nheads, head_dim, reduced_head_dim, bias.device)]
     return new_weight, new_bias, new_scale, new_workspace
 
 
@@ -121,27 +115,23 @@ def slice_w4a16_v_proj(weight, scale, workspace, hidden_size, nheads, head_dim, 
     pad_n = _pad_to(nheads * head_dim, 256)
     reduced_pad_n = _pad_to(nheads * reduced_head_dim, 256)
     assert load_shape[0] == weight.shape[0], "hidden_size dimension mismatch"
-    cols = _head_prefix(nheads, head_dim, reduced_head_dim, weight.device)
-    return _gather_columns(weight, scale, workspace, hidden_size + pad_k, nheads * head_dim + pad_n, hidden_size,
-                           cols, reduced_pad_n)
+    return _keep_columns(weight, scale, workspace, hidden_size + pad_k, nheads * head_dim + pad_n, hidden_size,
+                         [(0, nheads, head_dim, reduced_head_dim, reduced_head_dim, 0)], reduced_pad_n)
 
 
 def slice_w4a16_o_proj(weight, scale, workspace, hidden_size, nheads, head_dim, reduced_head_dim,
                        load_shape, num_bits=4, group_size=128):
     """Output projection [nheads * head_dim -> hidden_size]: the kept input rows do not line up
     with the groups of 128 any more, so the reference dequantises, keeps every head's first
-    reduced_head_dim rows and quantises again (modeling_helpers.py:600-656); the same here with
-    the device kernels (bit-exact fp16 weights out of uniql_w4a16_dequant, uniql_w4a16_quantize)."""
+    reduced_head_dim rows and quantises again (modeling_helpers.py:600-656); the same here."""
     assert num_bits == 4, "Only support 4-bit quantization for now"
     assert group_size == 128, "Only group_size 128 is supported on the device"
     pad_k = _pad_to(nheads * head_dim, group_size)
     pad_n = _pad_to(hidden_size, 256)
     assert load_shape[1] == weight.shape[1], "hidden_size dimension mismatch"
     size_k, size_n = nheads * head_dim + pad_k, hidden_size + pad_n
-    w_full = ops.w4a16_dequant(weight, scale, size_n, size_k)              # fp16 (code - 8) * scale, [k, n]
-    rows = _head_prefix(nheads, head_dim, reduced_head_dim, weight.device)
-    kept = w_full[rows][:, :hidden_size]                                  # [nheads * reduced_head_dim, hidden]
-    new_weight, new_scale = ops.w4a16_quantize(kept.t().contiguous(), None, pad_out=pad_n)
+    new_weight, new_scale = ops.w4a16_cut_rows(weight, scale, size_n, size_k, nheads, head_dim, reduced_head_dim, hidden_size,
+                                               pad_out=pad_n)
     return new_weight, new_scale, workspace
 
 
@@ -176,18 +166,16 @@ def slice_w4a16_in_proj(weight, scale, workspace, hidden_size, n_groups, num_hea
     pad_n = _pad_to(projection_size, 256)
     reduced_pad_n = _pad_to(reduced_projection_size, 256)
     assert load_shape[0] == weight.shape[0], "hidden_size dimension mismatch"
-    dev = weight.device
-    heads = get_topk_head_indices(n_groups, num_heads, intermediate_size // num_heads,
-                                  load_intermediate_size // num_heads, dev)
-    states = get_topk_ssm_state_indices(n_groups, ssm_state_size, load_ssm_state_size, dev)
+    kept = load_intermediate_size // num_heads
+    heads = (num_heads, intermediate_size // num_heads, kept, kept, 0)
+    states = (n_groups, ssm_state_size, load_ssm_state_size, load_ssm_state_size, 0)
     x_start = intermediate_size
     b_start = x_start + intermediate_size
     c_start = b_start + n_groups * ssm_state_size
     dt_start = c_start + n_groups * ssm_state_size
-    cols = torch.cat([heads, x_start + heads, b_start + states, c_start + states,
-                      torch.arange(dt_start, projection_size, device=dev)])
-    return _gather_columns(weight, scale, workspace, hidden_size + pad_k, projection_size + pad_n, hidden_size,
-                           cols, reduced_pad_n)
+    runs = [(0, *heads), (x_start, *heads), (b_start, *states), (c_start, *states), (dt_start, 1, num_heads, num_heads, num_heads, 0)]
+    return _keep_columns(weight, scale, workspace, hidden_size + pad_k, projection_size + pad_n, hidden_size, runs,
+                         reduced_pad_n)
 
 
 def slice_w4a16_out_proj(weight, scale, workspace, hidden_size, n_groups, num_heads, intermediate_size,
@@ -199,11 +187,9 @@ def slice_w4a16_out_proj(weight, scale, workspace, hidden_size, n_groups, num_he
     pad_k = _pad_to(intermediate_size, group_size)
     pad_n = _pad_to(hidden_size, 256)
     assert load_shape[1] == weight.shape[1], "hidden_size dimension mismatch"
-    w_full = ops.w4a16_dequant(weight, scale, hidden_size + pad_n, intermediate_size + pad_k)
-    rows = get_topk_head_indices(n_groups, num_heads, intermediate_size // num_heads,
-                                 load_intermediate_size // num_heads, weight.device)
-    kept = w_full[rows][:, :hidden_size]
-    new_weight, new_scale = ops.w4a16_quantize(kept.t().contiguous(), None, pad_out=pad_n)
+    new_weight, new_scale = ops.w4a16_cut_rows(weight, scale, hidden_size + pad_n, intermediate_size + pad_k, num_heads,
+                                               intermediate_size // num_heads, load_intermediate_size // num_heads, hidden_size,
+                                               pad_out=pad_n)
     return new_weight, new_scale, workspace
 
 
