@@ -99,6 +99,8 @@ int uniql_clear(void* p, size_t bytes, void* stream);
  *              (<= 32768, dividing k), and every rotation for larger m, runs the
  *              transform kernel into `temp` first.  Same values either way.
  *   k % 128 == 0, n % 128 == 0 (the module pads n to 256).
+ *   Calls of more than 128 rows may run as two launches over consecutive rows (on the same stream,
+ *   sharing accum and temp); the kernels are chosen from m, n, k.
  *
  * Partial sums that meet in the streaming kernel's `accum` words are rounded to multiples of
  * 2^-24 and clamped to +-2^18 (beyond the fp16 range of D, so an infinite partial sum still

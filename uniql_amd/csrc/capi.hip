@@ -24,7 +24,8 @@ size_t tile_accum_bytes(int m, int n, int k, unsigned tune = 0);
 int wide_launch(const void* A, int64_t lda, const void* B, const void* S, void* D, const Epilogue& epi, int m, int n,
                 int k, int groups, hipStream_t stream);
 bool wide_shape_ok(int m, int n, int k, int groups, int64_t ldx);
-bool wide_preferred(int m, int n, int k, unsigned tune);
+double wide_us(int m, int n, int k);
+unsigned tile_choose(int m, int n, int k, size_t part_cap, double* us);
 int dequant_launch(const void* B, const void* S, void* W, uint8_t* codes, int n, int k, int groups,
                    hipStream_t stream);
 int embedding_launch(const int64_t* ids, int64_t ntokens, const void* weight, const void* scales, void* out,
@@ -122,19 +123,101 @@ static size_t activation_copy_bytes(int m, int k, int k_in, int had_block, bool 
     return (rotate_first || pad_first) ? round256((size_t)m * k * sizeof(half_t)) : 0;
 }
 
+static constexpr size_t kStaticAccumBytes = (size_t)4 << 20;   // the static area: exchange words, 16 rows x 32768 columns
+static constexpr size_t kStaticTempBytes = (size_t)12 << 20;   //                  rotated rows / partial tiles
+
+// How the tiled kernels run the rows of a call: one launch, or two over consecutive rows.  `tune` holds the 128-column
+// kernel's tuning fields with the whole plan in them; row tiles = 8 stands for the 256 x 256 kernel.
+struct RowPart {
+    int rows;
+    unsigned tune;
+    bool wide() const { return ((tune >> 8) & 0xfu) == 8; }
+};
+struct LinearPlan {
+    int parts;
+    RowPart part[2];
+};
+
+// The faster of the two kernels for m rows in one launch, by their expected times.  The 4 %: most layer calls cut, add or
+// gate their outputs, which the 256 x 256 kernel does at next to no cost and the tall tiles of the other with 3 to 8 %
+// (4096 -> 18560 of 18688 at 565 rows: 101 us against 107, expected of the plain product 101.5 and 100.5).
+static RowPart best_launch(int m, int n, int k, bool wide_ok, size_t part_cap, double* us) {
+    RowPart p = {m, tile_choose(m, n, k, part_cap, us)};
+    const double w = wide_ok ? wide_us(m, n, k) : 1e30;
+    if (w < 1.04 * *us) {
+        *us = w;
+        p.tune = 8u << 8;
+    }
+    return p;
+}
+
+// wide_ok: the 256 x 256 kernel can take the call.  part_cap: the most bytes of partial tiles a plan may ask for.
+// A last round of workgroups that leaves most of the chip idle costs as much as a full one, so the rows behind the
+// last 128-row boundaries are also tried as a launch of their own (shorter tiles, K split): 4096 -> 28672 at 1100
+// rows is 1024 on the 256 x 256 kernel and 76 on 96-row tiles, 240 us instead of 297 in one launch.
+// Up to 128 rows there is nothing to split (a second launch costs 2 us).
+static LinearPlan linear_plan(int m, int n, int k, bool wide_ok, size_t part_cap, unsigned tune) {
+    LinearPlan plan;
+    plan.parts = 1;
+    const unsigned forced_rows = (tune >> 8) & 0xfu;
+    if ((tune & 0x3fffu) != 0) {  // a plan asked for by the caller, as far as the kernels can follow it
+        plan.part[0] = RowPart{m, tune};
+        if (forced_rows == 8 && !wide_ok) plan.part[0].tune = tune & ~0xf00u;
+        return plan;
+    }
+    double us;
+    plan.part[0] = best_launch(m, n, k, wide_ok, part_cap, &us);
+    int j = (m - 1) / 128;
+    for (int tries = 0; j > 0 && tries < 8; --j, ++tries) {
+        double head_us, tail_us;
+        const RowPart head = best_launch(128 * j, n, k, wide_ok, part_cap, &head_us);
+        if (head_us + 2.0 >= us) continue;
+        const RowPart tail = best_launch(m - 128 * j, n, k, wide_ok, part_cap, &tail_us);
+        if (head_us + tail_us + 2.0 < 0.97 * us) {
+            us = (head_us + tail_us + 2.0) / 0.97;
+            plan.parts = 2;
+            plan.part[0] = head;
+            plan.part[1] = tail;
+        }
+    }
+    return plan;
+}
+static size_t plan_accum_bytes(const LinearPlan& plan, int n, int k) {
+    size_t most = 0;
+    for (int i = 0; i < plan.parts; ++i) {
+        const size_t b = plan.part[i].wide() ? 0 : tile_accum_bytes(plan.part[i].rows, n, k, plan.part[i].tune);
+        most = b > most ? b : most;
+    }
+    return most;
+}
+static size_t plan_part_bytes(const LinearPlan& plan, int n, int k) {
+    size_t most = 0;
+    for (int i = 0; i < plan.parts; ++i) {
+        const size_t b = plan.part[i].wide() ? 0 : tile_part_bytes(plan.part[i].rows, n, k, plan.part[i].tune);
+        most = b > most ? b : most;
+    }
+    return most;
+}
+// Partial tiles of any call fit the static area (with more splits than that the exchange costs more than it gives);
+// the static entry asks for less where the copy of the activations needs the room.
+static constexpr size_t kPartialCap = kStaticTempBytes;
+
 // What one layer call needs, decided in ONE place for the argument checks, the launch and the
-// entry point that brings its own scratch memory: which kernel takes the call, whether the
+// entry point that brings its own scratch memory: which kernels take the call, whether the
 // activations are copied (rotated / zero-padded) into `temp` first, and the bytes of `accum` and
-// `temp` that follow from that.  The 256 x 256 kernel needs neither buffer.
+// `temp` that follow from that.  The 256 x 256 kernel needs neither buffer; two launches of the 128-column
+// kernel run one after the other and share theirs.
 struct LinearNeeds {
-    bool use_stream, use_wide, rotate_first, pad_first;
+    bool use_stream, rotate_first, pad_first;
     int had_mode;
     int64_t ld_kernel;   // row stride the product kernel will see
+    LinearPlan plan;     // of the tiled kernels
     size_t accum_bytes;  // rounded to 256
     size_t act_bytes;    // copy of the activations at the start of temp (rounded to 256), or 0
     size_t part_bytes;   // the tiled kernel's partial tiles behind it, or 0
 };
-static LinearNeeds linear_needs(int m, int n, int k, int k_in, int64_t lda, int groups, int had_block, unsigned flags) {
+static LinearNeeds linear_needs(int m, int n, int k, int k_in, int64_t lda, int groups, int had_block, unsigned flags,
+                                size_t part_cap = kPartialCap) {
     LinearNeeds q;
     const unsigned tune = flags >> 8;
     q.use_stream = takes_stream_kernel(m, flags);
@@ -144,12 +227,28 @@ static LinearNeeds linear_needs(int m, int n, int k, int k_in, int64_t lda, int 
     // (and zero-padded) into the temporary buffer, then rotated there in place
     q.pad_first = q.rotate_first ? (k_in != k || lda != k) : (k_in != k && !q.use_stream);
     q.ld_kernel = (q.rotate_first || q.pad_first) ? (int64_t)k : lda;
-    // large M: the 256 x 256 kernel where it is the faster one and can take the call
-    q.use_wide = !q.use_stream && wide_preferred(m, n, k, tune) && wide_shape_ok(m, n, k, groups, q.ld_kernel);
-    q.accum_bytes = round256(q.use_stream ? stream_accum_bytes(m, n, k) : q.use_wide ? 0 : tile_accum_bytes(m, n, k, tune));
     q.act_bytes = (q.rotate_first || q.pad_first) ? round256((size_t)m * k * sizeof(half_t)) : 0;
-    q.part_bytes = (q.use_stream || q.use_wide) ? 0 : tile_part_bytes(m, n, k, tune);
+    q.plan.parts = 0;
+    if (q.use_stream) {
+        q.accum_bytes = round256(stream_accum_bytes(m, n, k));
+        q.part_bytes = 0;
+    } else {
+        q.plan = linear_plan(m, n, k, wide_shape_ok(m, n, k, groups, q.ld_kernel), part_cap, tune);
+        q.accum_bytes = round256(plan_accum_bytes(q.plan, n, k));
+        q.part_bytes = plan_part_bytes(q.plan, n, k);
+    }
     return q;
+}
+
+// The most the tiled kernels may ask for, whether or not the call's scales and strides let the 256 x 256 kernel take part.
+static void tiled_workspace(int m, int n, int k, unsigned tune, size_t* accum, size_t* part) {
+    *accum = *part = 0;
+    for (int wide = 0; wide < 2; ++wide) {
+        const LinearPlan plan = linear_plan(m, n, k, wide != 0 && wide_shape_ok(m, n, k, k / 128, k), kPartialCap, tune);
+        const size_t a = plan_accum_bytes(plan, n, k), p = plan_part_bytes(plan, n, k);
+        *accum = a > *accum ? a : *accum;
+        *part = p > *part ? p : *part;
+    }
 }
 
 int uniql_w4a16_linear_workspace(int m, int n, int k, int k_in, int had_block, unsigned flags, size_t* accum_bytes,
@@ -159,22 +258,23 @@ int uniql_w4a16_linear_workspace(int m, int n, int k, int k_in, int had_block, u
     if (m < 0 || n <= 0 || k <= 0 || n % 128 != 0 || k % 128 != 0) return UNIQL_E_SHAPE;
     if (m == 0) return UNIQL_OK;
     const bool use_stream = takes_stream_kernel(m, flags);
-    const unsigned tune = flags >> 8;
-    // (the 256 x 256 kernel needs neither buffer; the sizes are the 128 x 128 kernel's, which takes
-    // the call when the scales are per column)
-    *accum_bytes = round256(use_stream ? stream_accum_bytes(m, n, k) : tile_accum_bytes(m, n, k, tune));
     // a strided input ahead of a separate rotation is compacted into the copy as well: count it
     const size_t act = had_block != 0 && fused_rotation(m, k, k_in, had_block, use_stream, flags) == 0
                            ? round256((size_t)m * k * sizeof(half_t))
                            : activation_copy_bytes(m, k, k_in, had_block, use_stream, flags);
-    *temp_bytes = act + (use_stream ? 0 : round256(tile_part_bytes(m, n, k, tune)));
+    size_t accum = stream_accum_bytes(m, n, k), part = 0;
+    if (!use_stream) tiled_workspace(m, n, k, flags >> 8, &accum, &part);
+    *accum_bytes = round256(accum);
+    *temp_bytes = act + round256(part);
     return UNIQL_OK;
 }
 
 size_t uniql_w4a16_gemm_accum_bytes(int m, int n, int k) {
     if (m <= 0 || n <= 0 || k <= 0 || n % 128 != 0 || k % 128 != 0) return 0;
     // enough for either kernel with its own plan (forced tuning fields: uniql_w4a16_linear_workspace)
-    const size_t a = stream_accum_bytes(m, n, k), b = tile_accum_bytes(m, n, k);
+    const size_t a = stream_accum_bytes(m, n, k);
+    size_t b, part;
+    tiled_workspace(m, n, k, 0, &b, &part);
     return round256(a > b ? a : b);
 }
 
@@ -183,7 +283,9 @@ size_t uniql_w4a16_linear_temp_bytes(int m, int n, int k, int k_in, int had_bloc
     // the copy of the activations (as if the tiled kernel took the call: the larger case) and the
     // partial tiles of the tiled kernel's own plan
     const size_t act = (had_block != 0 || k_in != k) ? round256((size_t)m * k * sizeof(half_t)) : 0;
-    return act + (takes_stream_kernel(m, 0) ? 0 : round256(tile_part_bytes(m, n, k, 0)));
+    size_t accum = 0, part = 0;
+    if (!takes_stream_kernel(m, 0)) tiled_workspace(m, n, k, 0, &accum, &part);
+    return act + round256(part);
 }
 
 size_t uniql_w4a16_gemm_temp_bytes(int m, int n, int k, int had_block) {
@@ -196,7 +298,7 @@ static int linear_impl(const void* A, int64_t lda, int k_in, const void* B, cons
                        const int32_t* workspace,
                        int64_t workspace_len, void* accum, size_t accum_bytes, void* temp, size_t temp_bytes, int m,
                        int n, int k, int groups, int had_block, float had_scale, unsigned flags, void* stream,
-                       bool check_only) {
+                       bool check_only, size_t part_cap) {
     const int rc = check_linear_shape(m, n, k, groups);
     if (rc != UNIQL_OK) return rc;
     const bool transpose = (flags & UNIQL_F_TRANSPOSE_OUT) != 0;
@@ -223,8 +325,8 @@ static int linear_impl(const void* A, int64_t lda, int k_in, const void* B, cons
     if ((accum && !aligned16(accum)) || (temp && !aligned16(temp))) return UNIQL_E_ALIGN;
     hipStream_t st = reinterpret_cast<hipStream_t>(stream);
     const unsigned tune = flags >> 8;  // tuning fields, see the header
-    const LinearNeeds q = linear_needs(m, n, k, k_in, lda, groups, had_block, flags);
-    const bool use_stream = q.use_stream, use_wide = q.use_wide, rotate_first = q.rotate_first, pad_first = q.pad_first;
+    const LinearNeeds q = linear_needs(m, n, k, k_in, lda, groups, had_block, flags, part_cap);
+    const bool use_stream = q.use_stream, rotate_first = q.rotate_first, pad_first = q.pad_first;
     const int had_mode = q.had_mode;
     const int64_t ld_kernel = q.ld_kernel;
     const void* Ain = A;
@@ -237,7 +339,8 @@ static int linear_impl(const void* A, int64_t lda, int k_in, const void* B, cons
     if (act_bytes + part_bytes > 0 && (!temp || temp_bytes < act_bytes + part_bytes)) return UNIQL_E_WORKSPACE;
     void* part = part_bytes ? reinterpret_cast<char*>(temp) + act_bytes : nullptr;
     // last check before the first kernel is enqueued: whether the tiled kernel can take the shape
-    if (!use_stream && !use_wide && !tile_shape_ok(m, n, k, ld_kernel, tune)) return UNIQL_E_SHAPE;
+    for (int i = 0; i < q.plan.parts; ++i)
+        if (!q.plan.part[i].wide() && !tile_shape_ok(q.plan.part[i].rows, n, k, ld_kernel, q.plan.part[i].tune)) return UNIQL_E_SHAPE;
     if (use_stream && !stream_shape_ok(k, ld_kernel)) return UNIQL_E_SHAPE;
     if (check_only) return UNIQL_OK;
     if (pad_first) {
@@ -266,8 +369,18 @@ static int linear_impl(const void* A, int64_t lda, int k_in, const void* B, cons
     epi.vec_ok = (!transpose && ldd % 8 == 0 && aligned16(D)) ? 1 : 0;
     if (use_stream)
         return stream_launch(Ain, ld, k_valid, B, S, D, epi, accum, m, n, k, groups, had_mode, had_scale, tune, st);
-    if (use_wide) return wide_launch(Ain, ld, B, S, D, epi, m, n, k, groups, st);
-    return tile_launch(Ain, ld, B, S, D, epi, accum, accum_bytes, part, part_bytes, m, n, k, groups, tune, st);
+    int m0 = 0;
+    for (int i = 0; i < q.plan.parts; ++i) {
+        const RowPart& p = q.plan.part[i];
+        const char* x = reinterpret_cast<const char*>(Ain) + (size_t)m0 * ld * sizeof(half_t);
+        char* d = reinterpret_cast<char*>(D) + (size_t)m0 * (transpose ? 1 : ldd) * (out_f32 ? 4 : 2);
+        epi.residual = residual ? reinterpret_cast<const half_t*>(residual) + (size_t)m0 * ldr : nullptr;
+        const int e = p.wide() ? wide_launch(x, ld, B, S, d, epi, p.rows, n, k, groups, st)
+                               : tile_launch(x, ld, B, S, d, epi, accum, accum_bytes, part, part_bytes, p.rows, n, k, groups, p.tune, st);
+        if (e != UNIQL_OK) return e;
+        m0 += p.rows;
+    }
+    return UNIQL_OK;
 }
 
 int uniql_w4a16_linear(const void* A, int64_t lda, int k_in, const void* B, const void* S, const void* bias,
@@ -276,26 +389,26 @@ int uniql_w4a16_linear(const void* A, int64_t lda, int k_in, const void* B, cons
                        int64_t workspace_len, void* accum, size_t accum_bytes, void* temp, size_t temp_bytes, int m,
                        int n, int k, int groups, int had_block, float had_scale, unsigned flags, void* stream) {
     return linear_impl(A, lda, k_in, B, S, bias, residual, ldr, D, ldd, n_out, epilogue, workspace, workspace_len, accum,
-                       accum_bytes, temp, temp_bytes, m, n, k, groups, had_block, had_scale, flags, stream, false);
+                       accum_bytes, temp, temp_bytes, m, n, k, groups, had_block, had_scale, flags, stream, false, kPartialCap);
 }
 
 static int gemm_impl(const void* A, int64_t lda, const void* B, const void* S, void* D, const int32_t* workspace,
                      int64_t workspace_len, void* accum, size_t accum_bytes, void* temp, size_t temp_bytes, int m,
                      int n, int k, int groups, int had_block, float had_scale, unsigned flags, void* stream,
-                     bool check_only) {
+                     bool check_only, size_t part_cap) {
     if (D && !aligned16(D)) return UNIQL_E_ALIGN;
     // transposed: D is [n, m8] with m8 = m rounded up to 8, as the reference allocates it
     // (marlin_gemm_kernel.cuh:1023-1026)
     const int64_t ldd = (flags & UNIQL_F_TRANSPOSE_OUT) ? (int64_t)((m + 7) / 8) * 8 : n;
     return linear_impl(A, lda, k, B, S, nullptr, nullptr, 0, D, ldd, n, UNIQL_EPI_NONE, workspace, workspace_len, accum,
-                       accum_bytes, temp, temp_bytes, m, n, k, groups, had_block, had_scale, flags, stream, check_only);
+                       accum_bytes, temp, temp_bytes, m, n, k, groups, had_block, had_scale, flags, stream, check_only, part_cap);
 }
 
 int uniql_w4a16_gemm(const void* A, int64_t lda, const void* B, const void* S, void* D, const int32_t* workspace,
                      int64_t workspace_len, void* accum, size_t accum_bytes, void* temp, size_t temp_bytes, int m,
                      int n, int k, int groups, int had_block, float had_scale, unsigned flags, void* stream) {
     return gemm_impl(A, lda, B, S, D, workspace, workspace_len, accum, accum_bytes, temp, temp_bytes, m, n, k, groups,
-                     had_block, had_scale, flags, stream, false);
+                     had_block, had_scale, flags, stream, false, kPartialCap);
 }
 
 // ---- the entry point that allocates nothing --------------------------------------------------
@@ -303,8 +416,6 @@ int uniql_w4a16_gemm(const void* A, int64_t lda, const void* B, const void* S, v
 // temporary area) lives in one array in this library's device image.  Each GPU holds its own copy
 // at its own address; the name below is only a host-side handle for hipGetSymbolAddress, never a
 // device address, so every use goes through the per-device pointer looked up once.
-static constexpr size_t kStaticAccumBytes = (size_t)4 << 20;   // exchange words: 16 rows x 32768 columns
-static constexpr size_t kStaticTempBytes = (size_t)12 << 20;   // rotated rows / partial tiles
 static __device__ __align__(256) unsigned char scratch[kStaticAccumBytes + kStaticTempBytes];
 
 static constexpr int kMaxDevices = 64;
@@ -336,7 +447,13 @@ int uniql_w4a16_gemm_static(const void* A, int64_t lda, const void* B, const voi
     if (m == 0) return UNIQL_OK;
     // (the sizes of the kernel that will really take the call: a long prefill on the 256 x 256 kernel needs
     // no scratch at all, whatever the 128-column kernel would have asked for)
-    const LinearNeeds q = linear_needs(m, n, k, k, lda, groups, had_block, flags);
+    size_t part_cap = kPartialCap;
+    LinearNeeds q = linear_needs(m, n, k, k, lda, groups, had_block, flags, part_cap);
+    if (q.act_bytes < kStaticTempBytes && q.act_bytes + round256(q.part_bytes) > kStaticTempBytes) {
+        // the copy of the activations leaves less room for partial tiles: fewer K splits
+        part_cap = kStaticTempBytes - q.act_bytes;
+        q = linear_needs(m, n, k, k, lda, groups, had_block, flags, part_cap);
+    }
     const size_t need_accum = q.accum_bytes, need_temp = q.act_bytes + round256(q.part_bytes);
     if (need_accum > kStaticAccumBytes || need_temp > kStaticTempBytes) return UNIQL_E_STATIC_LIMIT;
     if (!A || !B || !S || !D) return UNIQL_E_NULL;
@@ -346,7 +463,7 @@ int uniql_w4a16_gemm_static(const void* A, int64_t lda, const void* B, const voi
     void* temp = need_temp ? base + kStaticAccumBytes : nullptr;
     // every argument check of the product first: nothing is enqueued for a call that will be refused
     const int crc = gemm_impl(A, lda, B, S, D, workspace, workspace_len, accum, need_accum, temp, need_temp, m, n, k,
-                              groups, had_block, had_scale, flags, stream, true);
+                              groups, had_block, had_scale, flags, stream, true, part_cap);
     if (crc != UNIQL_OK) return crc;
     // The exchange words must be zero on entry.  The kernels leave them zero, but the array is
     // shared by every call on this GPU, so the part this call uses is cleared by a small kernel
@@ -356,7 +473,7 @@ int uniql_w4a16_gemm_static(const void* A, int64_t lda, const void* B, const voi
         if (e != UNIQL_OK) return e;
     }
     return gemm_impl(A, lda, B, S, D, workspace, workspace_len, accum, need_accum, temp, need_temp, m, n, k, groups,
-                     had_block, had_scale, flags, stream, false);
+                     had_block, had_scale, flags, stream, false, part_cap);
 }
 
 int uniql_w4a16_read_floor(const void* B, const void* S, void* sink, size_t sink_bytes, int m, int n, int k,

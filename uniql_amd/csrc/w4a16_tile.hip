@@ -1,6 +1,6 @@
 // Tiled W4A16 kernel for M > 16 (prefill): D[M,N] = X[M,K] . dequant(B)[K,N].
 //
-// A workgroup of four wavefronts owns a (32 MT) x 128 output tile (MT = 1, 2 or 4) and a
+// A workgroup of four wavefronts owns a (32 MT) x 128 output tile (MT = 1 to 4) and a
 // range of 128-wide K groups.  The four waves split K: of the eight packed rows (16 K
 // values each) of a group, wave w takes rows w and w + 4 and accumulates the WHOLE tile
 // for them with v_mfma_f32_32x32x16_f16, so every weight of the tile is expanded to fp16
@@ -315,7 +315,7 @@ __global__ __launch_bounds__(256 * KW, 1) void w4a16_tile_kernel(const TileArgs 
                 const int slot_i = op * MT + mt;
                 acc[mt][op] = __builtin_amdgcn_mfma_f32_32x32x16_f16(bw, xa[mt], acc[mt][op], 0, 0, 0);
 #pragma unroll
-                for (int q = mt * (4 / MT); q < (mt + 1) * (4 / MT); ++q) {
+                for (int q = mt * 4 / MT; q < (mt + 1) * 4 / MT; ++q) {
                     // the empty asm pins the quarter to this slot: it cannot sink below the slot's
                     // closing barrier
                     uint32_t bits = h2_to_bits(expand_quarter(nset, nblock, q));
@@ -325,7 +325,7 @@ __global__ __launch_bounds__(256 * KW, 1) void w4a16_tile_kernel(const TileArgs 
                 if (slot_i % kDmaStride == 0 && slot_i / kDmaStride < dma_count)
                     issue_piece(next_g, next_ring, dma_first + slot_i / kDmaStride);
                 lds_reads(slot_i);
-                if (MT == 4) {
+                if (MT >= 3) {
                     // inside the slot: the first two operations of the quarter, the MFMA, the rest;
                     // the MFMA between the fp16 add and the dependent multiply fills the wait
                     // state that would otherwise cost an s_nop
@@ -560,11 +560,12 @@ static inline int ceil_div_i(int a, int b) { return (a + b - 1) / b; }
 struct TilePlan {
     int mtiles, splits, gps;
     int quartets;  // wave quartets per workgroup (1 or 2)
+    double us;     // what tile_us expects of it
 };
-static TilePlan tile_plan(int m, int n, int k, int splits_override, int mt_override = 0, int kw_override = 0);
+static TilePlan tile_plan(int m, int n, int k, int splits_override, int mt_override, int kw_override, size_t part_cap);
 
 static TilePlan tile_plan_tuned(int m, int n, int k, unsigned tune) {
-    return tile_plan(m, n, k, (int)(tune & 0xffu), (int)((tune >> 8) & 0xfu), (int)((tune >> 12) & 0x3u));
+    return tile_plan(m, n, k, (int)(tune & 0xffu), (int)((tune >> 8) & 0xfu), (int)((tune >> 12) & 0x3u), (size_t)-1);
 }
 
 // What a plan that splits K over workgroups needs (tune: the same fields as tile_launch takes):
@@ -582,66 +583,97 @@ size_t tile_part_bytes(int m, int n, int k, unsigned tune) {
     return tiles * plan.splits * (32 * plan.mtiles * 128) * sizeof(float);
 }
 
-// Measured on MI355X, in units of the time one MT = 4 workgroup takes for its K loop when every
-// compute unit has one ("a round"):
-//   * MT = 4: one workgroup per compute unit, every started round of 256 costs 1;
-//   * MT = 2: two workgroups share a compute unit; a full round of 512 costs 1.08 (every weight
-//     is expanded twice per 128 rows), a last round of at most 256 costs 0.85;
-//   * MT = 1: up to four share a compute unit: 0.62 for at most 256 workgroups, 0.88 for at most
-//     512, 1.62 per started round of 1024;
-//   * a grid that gives a compute unit at most one MT = 1 or MT = 2 workgroup runs faster with two
-//     wave quartets per workgroup (factors 0.85 and 0.92);
-//   * K split over workgroups: every workgroup writes its fp32 partial tile to scratch memory and
-//     the last one to arrive adds them (about 1 to 1.5 us per MB of partial tiles).
-// So: the MT with the cheapest grid; K splits while the grid stays within one workgroup per compute
-// unit and the partial tiles stay small against the weights; two quartets whenever the final
-// grid has at most 256 workgroups of MT <= 2 and every workgroup gets an even number of groups.
-static TilePlan tile_plan(int m, int n, int k, int splits_override, int mt_override, int kw_override) {
-    TilePlan p;
+// Time of a launch of `wgs` workgroups that walk `g` K groups each, in us, on 256 compute units.
+// Workgroups run in rounds: one per compute unit with 96- and 128-row tiles (LDS) or two quartets, two with
+// 64-row tiles, four with 32-row tiles.  A round costs a prologue and an epilogue (6 us) and a time per group that
+// grows once more than half of the chip is busy (the clock falls with the matrix load).  Fitted to forced
+// launches of nine shapes (K 4096 to 14336, N 4096 to 28672) at 96 to 4096 rows, within 5 % of all but the
+// 32-row tiles from 600 workgroups on; e.g. 4096 -> 4096, 256 tiles of 128 rows 35.6 us (model 35.0), of 96 rows 29.7
+// (29.4), 14336 -> 4096 106 (104) and 89.8 (87.8).
+static double ramp(double lo, double hi, int64_t x, int64_t x0, int64_t x1) {
+    return x <= x0 ? lo : lo + (hi - lo) * (double)(x - x0) / (double)(x1 - x0);
+}
+static double tile_us(int mt, int quartets, int64_t wgs, int g) {
+    const int64_t per_round = quartets == 2 || mt >= 3 ? 256 : (mt == 2 ? 512 : 1024);
+    const double full = (double)(wgs / per_round);
+    const int64_t rest = wgs % per_round;
+    double us = 0.0;
+    if (quartets == 2 && mt == 2) {
+        us = full * (5.7 + 0.536 * g);
+        if (rest) us += 5.7 + g * (rest <= 192 ? ramp(0.375, 0.447, rest, 64, 192) : ramp(0.447, 0.536, rest, 192, 256));
+    } else if (quartets == 2) {
+        us = full * (3.9 + 0.40 * g) + (rest ? 3.9 + g * ramp(0.30, 0.40, rest, 64, 256) : 0.0);
+    } else if (mt == 4) {
+        us = full * (6.5 + 0.875 * g) + (rest ? 6.5 + g * ramp(0.60, 0.86, rest, 128, 256) : 0.0);
+    } else if (mt == 3) {
+        us = full * (6.0 + 0.73 * g) + (rest ? 6.0 + g * ramp(0.53, 0.73, rest, 128, 256) : 0.0);
+    } else if (mt == 2) {
+        us = full * (6.5 + 1.02 * g);
+        if (rest > 256) us += 6.0 + g * ramp(0.75, 1.02, rest, 256, 512);
+        else if (rest) us += full > 0 ? 4.0 + g * ramp(0.33, 0.49, rest, 0, 256) : 6.5 + 0.55 * g;  // starts before the round ends
+    } else {
+        us = full * (5.0 + 1.5 * g);
+        if (rest > 512) us += 5.0 + g * ramp(0.85, 1.5, rest, 512, 1024);
+        else if (rest > 256) us += 5.0 + g * ramp(0.55, 0.75, rest, 256, 512);
+        else if (rest) us += full > 0 ? 4.0 + 0.35 * g : 5.0 + 0.5 * g;
+    }
+    return us;
+}
+
+// What the exchange between the splits of a tile adds: the partial tiles' stores, the count, and the last workgroup's
+// reading of all of them (forced splits of 1 to 8 on six shapes at 24 to 192 rows).
+static double exchange_us(int mt, int splits) {
+    if (mt == 1) return 2.2 + 0.08 * splits * splits;
+    if (mt == 2) return 3.0 + 0.11 * splits * splits;
+    return mt == 3 ? 3.0 + 1.8 * splits : 6.0 + 2.1 * splits;
+}
+
+// Height of the tiles, K splits and quartets with the smallest expected time.  K is split over workgroups while the
+// grid stays within one workgroup per compute unit, every workgroup keeps at least 8 groups and the
+// partial tiles fit part_cap bytes.  Two quartets whenever the grid has at most 256 workgroups of at most 64 rows
+// and every workgroup gets an even number of groups.
+// The 96-row tiles are there for the rounds: 14336 -> 4096 at 333 rows runs as 256 workgroups of them in 51.3 us
+// (128 rows: 54.1, 64 rows: 54.5, the rule of thumb this search replaced: 57-63), 4096 -> 24576 at 333 rows as three
+// whole rounds (87.0 against 93.3).
+static TilePlan tile_plan(int m, int n, int k, int splits_override, int mt_override, int kw_override, size_t part_cap) {
+    TilePlan best = {4, 1, k / 128, 1, 1e30};
     const int strips = n / 128, G = k / 128;
     const bool even_g = G % 2 == 0;
-    const int64_t t4 = (int64_t)strips * ceil_div_i(m, 128), t2 = (int64_t)strips * ceil_div_i(m, 64);
-    const int64_t t1 = (int64_t)strips * ceil_div_i(m, 32);
-    const double cost4 = (double)((t4 + 255) / 256);
-    const int64_t rem2 = t2 % 512;
-    double cost2 = 1.08 * (double)(t2 / 512) + (rem2 == 0 ? 0.0 : (rem2 <= 256 ? 0.85 : 1.08));
-    double cost1 = t1 <= 256 ? 0.62 : (t1 <= 512 ? 0.88 : 1.62 * (double)((t1 + 1023) / 1024));
-    if (even_g && t2 <= 256) cost2 *= 0.92;
-    if (even_g && t1 <= 256) cost1 *= 0.85;
-    p.mtiles = 4;
-    if (cost2 < cost4 && cost2 <= cost1) p.mtiles = 2;
-    else if (cost1 < cost4) p.mtiles = 1;
-    if (m <= 32) p.mtiles = 1;
-    // a long K loop over few 64-row tiles: two K splits of 64-row tiles beat 32-row tiles (every
-    // weight is expanded for twice the rows; down_proj at M = 256: 545 -> 650 TFLOP/s)
-    if (p.mtiles == 1 && G >= 64 && m >= 64 && t2 <= 128) p.mtiles = 2;
-    if (mt_override == 1 || mt_override == 2 || mt_override == 4) p.mtiles = mt_override;
-    const int64_t tiles = (int64_t)strips * ceil_div_i(m, 32 * p.mtiles);
-    int splits = 1;
-    if (splits_override > 0) {
-        splits = splits_override;
-    } else {
-        // K splits while the grid stays within one workgroup per compute unit, every workgroup
-        // keeps at least 8 groups, and the partial tiles (m x n x 4 bytes per split, written and
-        // read once) stay below a quarter of the packed weights the launch streams
-        while (tiles * (2 * splits) <= 256 && G / (2 * splits) >= 8 && (int64_t)(2 * splits) * m * 16 <= k) splits *= 2;
-    }
-    if (splits > G) splits = G;
-    if (splits > 255) splits = 255;
-    p.gps = ceil_div_i(G, splits);
-    p.splits = ceil_div_i(G, p.gps);
-    // two quartets take alternate groups: every workgroup's range must hold an even number
-    p.quartets = 1;
-    const bool want2 = kw_override == 2 || (kw_override == 0 && tiles * p.splits <= 256);
-    if (want2 && p.mtiles <= 2 && even_g) {
-        const int gps2 = p.gps + (p.gps & 1);
-        if (splits_override == 0 || gps2 == p.gps) {
-            p.gps = gps2;
+    for (int mt = 1; mt <= 4; ++mt) {
+        if (mt_override >= 1 && mt_override <= 4 && mt != mt_override) continue;
+        const int64_t tiles = (int64_t)strips * ceil_div_i(m, 32 * mt);
+        for (int s = 1; s <= 255; ++s) {
+            if (splits_override > 0) s = splits_override;
+            else if (s > 1 && (tiles * s > 256 || G / s < 8)) break;
+            TilePlan p;
+            p.mtiles = mt;
+            p.gps = ceil_div_i(G, s > G ? G : s);
             p.splits = ceil_div_i(G, p.gps);
-            p.quartets = 2;
+            p.quartets = 1;
+            // two quartets take alternate groups: every workgroup's range must hold an even number
+            if ((kw_override == 2 || (kw_override == 0 && tiles * p.splits <= 256)) && mt <= 2 && even_g) {
+                const int gps2 = p.gps + (p.gps & 1);
+                if (splits_override == 0 || gps2 == p.gps) {
+                    p.gps = gps2;
+                    p.splits = ceil_div_i(G, p.gps);
+                    p.quartets = 2;
+                }
+            }
+            p.us = tile_us(mt, p.quartets, tiles * p.splits, p.gps);
+            if (p.splits > 1) p.us += exchange_us(mt, p.splits);
+            const bool fits = p.splits == 1 || splits_override > 0 || (size_t)tiles * p.splits * mt * (32 * 128 * 4) <= part_cap;
+            if (fits && p.us < best.us) best = p;
+            if (splits_override > 0) break;
         }
     }
-    return p;
+    return best;
+}
+
+// The plan for m rows as the tuning fields that force it, and its expected time.
+unsigned tile_choose(int m, int n, int k, size_t part_cap, double* us) {
+    const TilePlan p = tile_plan(m, n, k, 0, 0, 0, part_cap);
+    *us = p.us;
+    return (unsigned)p.splits | ((unsigned)p.mtiles << 8) | ((unsigned)p.quartets << 12);
 }
 
 // Whether tile_launch can take the call: grid size, and the 32-bit offsets of the loads (128 rows of
@@ -713,6 +745,8 @@ int tile_launch(const void* A, int64_t lda, const void* B, const void* S, void* 
         e = plan.quartets == 2 ? tile_launch_ext<1, 2>(a, ext, (int)grid, stream) : tile_launch_ext<1, 1>(a, ext, (int)grid, stream);
     else if (plan.mtiles == 2)
         e = plan.quartets == 2 ? tile_launch_ext<2, 2>(a, ext, (int)grid, stream) : tile_launch_ext<2, 1>(a, ext, (int)grid, stream);
+    else if (plan.mtiles == 3)
+        e = tile_launch_ext<3, 1>(a, ext, (int)grid, stream);
     else
         e = tile_launch_ext<4, 1>(a, ext, (int)grid, stream);
     return e == hipSuccess ? UNIQL_OK : UNIQL_E_LAUNCH;

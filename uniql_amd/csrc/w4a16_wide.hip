@@ -19,7 +19,7 @@
 // weights) a weight is expanded once per 256 rows instead of once per 128, an X element is loaded
 // once per 256 columns instead of once per 128, and the weights no longer pass through the vector
 // ALU of the wave that multiplies them.  The price is the 256 x 256 granularity: the kernel is
-// chosen only where the grid still fills the chip (see wide_preferred).
+// chosen only where the grid still fills the chip (by expected time, see linear_plan).
 //
 // LDS operand layout.  Weights: element (column x, k) of a block lives in 16-byte unit
 // 4 x + ((k / 8) ^ sw(x)); activations: element (row x, k) of a pair of blocks in unit
@@ -486,20 +486,14 @@ bool wide_shape_ok(int m, int n, int k, int groups, int64_t ldx) {
            (int64_t)(n / 256) * ((m + 255) / 256) <= 0x7fffffffLL;
 }
 
-// Whether the entry point sends a call of the tiled path here.  tune: the tiled kernel's fields;
-// 8 in its "row tiles of 32 per workgroup" field (bits 8..11) asks for this kernel, any other
-// non-zero value there for the 128 x 128 one.
-// Without a forced choice: measured on the Llama and Mamba2 shapes at 256 to 8192 rows, the
-// 256 x 256 tiles win (by 5 to 30 %) where their grid keeps the chip busy: the share of real
-// output in the tile slots of its rounds of 256 workgroups is at least 0.62.
-bool wide_preferred(int m, int n, int k, unsigned tune) {
-    if (m <= 0 || n % 256 != 0 || k % 128 != 0 || k < 256) return false;
-    const int mt = (int)((tune >> 8) & 0xfu);
-    if (mt != 0) return mt == 8;
-    if ((tune & 0xffu) != 0 || ((tune >> 12) & 3u) != 0) return false;  // forced K splits or quartets: the 128 x 128 kernel's
+// Expected time in us (fitted like the 128-column kernel's: forced launches of nine shapes at 96 to 4096 rows, within 5 %):
+// rounds of 256 workgroups, the time per K group growing with the busy part of the chip.
+double wide_us(int m, int n, int k) {
     const int64_t tiles = (int64_t)(n / 256) * ((m + 255) / 256);
-    const int64_t rounds = (tiles + 255) / 256;
-    return (double)m * n / 65536.0 >= 0.62 * 256.0 * (double)rounds;
+    const int g = k / 128;
+    const int64_t rest = tiles % 256;
+    const double slow = rest > 120 ? 1.08 * (double)(rest - 120) / 136.0 : 0.0;
+    return (double)(tiles / 256) * (9.0 + 3.2 * g) + (rest ? 8.5 + g * (2.12 + slow) : 0.0);
 }
 
 static hipError_t wide_launch_one(const WideArgs& a, int grid, hipStream_t stream) {
