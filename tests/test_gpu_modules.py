@@ -162,3 +162,59 @@ def test_empty_inputs(gpu):
     x = torch.randn(2, 200).half().to(gpu)
     assert torch.isfinite(q(x)).all()
     torch.cuda.synchronize()
+
+
+def test_native_host_path_keeps_the_modules_forms(gpu):
+    """ranks, strides, empty inputs, gradients switched on, copies and pickles of a layer that has run"""
+    import copy
+    import io
+    from uniql_amd import ops
+    from uniql_amd.quantize.quant_embedding_layers import W4O16Embedding
+    from uniql_amd.quantize.quant_linear_layers import W4A16B16O16Linear
+    torch.manual_seed(3)
+    lin = torch.nn.Linear(384, 200, bias=True, device=gpu, dtype=torch.float16)
+    layer = W4A16B16O16Linear.from_fp16(lin)
+    x = torch.randn(2, 3, 4, 384, device=gpu).half()
+    y = layer(x)
+    assert y.shape == (2, 3, 4, 200) and not y.requires_grad and y.is_contiguous()
+    rows = layer(x.reshape(24, 384))
+    assert torch.equal(y.reshape(24, 200), rows) and torch.equal(layer(x[0, 0, 0]), layer(x[0, 0, 0][None])[0])
+    strided = x.transpose(0, 2)                                        # rows not evenly spaced: copied
+    assert torch.equal(layer(strided), y.transpose(0, 2))
+    inner = x.reshape(24, 384).t().contiguous().t()                    # unit stride along the other axis
+    assert torch.equal(layer(inner), rows)
+    odd = torch.zeros(24, 385, device=gpu, dtype=torch.float16)[:, 1:]  # rows off the 16-byte grid
+    odd.copy_(x.reshape(24, 384))
+    assert torch.equal(layer(odd), rows)
+    assert layer(x[:, :0]).shape == (2, 0, 4, 200) and layer(x[:0].reshape(0, 384)).shape == (0, 200)
+    res = torch.randn(2, 3, 4, 200, device=gpu).half()
+    want = layer(x, residual=res)
+    assert torch.equal(layer(x, residual=res.transpose(0, 1).contiguous().transpose(0, 1)), want)
+    grad = layer(x.clone().requires_grad_(), residual=res.clone().requires_grad_())
+    assert torch.equal(grad, want) and grad.grad_fn is None
+    for bad in (dict(x=x.float()), dict(x=x[..., :200]), dict(x=x, residual=res[..., :8]), dict(x=x.cpu()),
+                dict(x=x, residual=res, activation="relu2"), dict(x=x, residual=res.cpu())):
+        with pytest.raises(RuntimeError):
+            layer(**bad)
+    twin = copy.deepcopy(layer)
+    assert torch.equal(twin(x), y) and twin.weight.data_ptr() != layer.weight.data_ptr()
+    blob = io.BytesIO()
+    torch.save(layer, blob)
+    blob.seek(0)
+    assert torch.equal(torch.load(blob, weights_only=False)(x), y)
+    layer.weight = layer.weight.clone()                                # a replaced buffer is prepared again
+    layer.scale = layer.scale * 2
+    assert torch.equal(layer(x).float(), ops.w4a16_linear(x.reshape(24, 384), layer.weight, layer.scale, layer.workspace, 256,
+                                                           384, out_features=200, bias=layer.bias.data).reshape(y.shape).float())
+    table = W4O16Embedding.from_fp16(torch.nn.Embedding(40, 64, device=gpu, dtype=torch.float16))
+    ids = torch.arange(40, device=gpu).reshape(5, 8)
+    out = table(ids)
+    assert out.shape == (5, 8, 64) and torch.equal(table(ids.t()), out.transpose(0, 1)) and table(ids[:0]).shape == (0, 8, 64)
+    for bad in (ids.int(), ids[None], ids.cpu()):
+        with pytest.raises(RuntimeError):
+            table(bad)
+    h = torch.randn(6, 256, device=gpu).requires_grad_()
+    rotated = ops.fast_hadamard_transform(h, 0.5)
+    assert not rotated.requires_grad and torch.equal(ops.fast_hadamard_transform(h.t().contiguous().t(), 0.5), rotated)
+    with pytest.raises(RuntimeError):
+        ops.hadamard_blockwise(h.double(), 1.0)

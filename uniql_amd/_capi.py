@@ -10,7 +10,7 @@ import ctypes
 import os
 from ctypes import c_char_p, c_float, c_int, c_int64, c_size_t, c_uint, c_void_p
 
-from .build import LIB_PATH
+from .build import HOST_PATH, LIB_PATH
 
 OK = 0
 F_OUT_F32 = 1 << 0
@@ -98,3 +98,25 @@ def check(code: int, what: str) -> None:
     if code != OK:
         msg = load().uniql_status_string(code).decode()
         raise RuntimeError(f"{what}: {msg} (code {code})")
+
+
+_host = None
+
+
+def host():
+    """The native binding of the calls a token is made of (lib/_host.so), bound to the loaded library."""
+    global _host
+    if _host is not None:
+        return _host
+    from importlib import util
+    lib = load()
+    if not os.path.exists(HOST_PATH):
+        raise UniqlLibraryError(f"{HOST_PATH} not found: build it with `python -m uniql_amd.build`")
+    spec = util.spec_from_file_location("uniql_amd._host", HOST_PATH)
+    module = util.module_from_spec(spec)
+    spec.loader.exec_module(module)
+    module.bind(*(ctypes.cast(fn, ctypes.c_void_p).value
+                  for fn in (lib.uniql_w4a16_linear, lib.uniql_w4a16_linear_workspace, lib.uniql_w4_embedding_lookup,
+                             lib.uniql_fwht, lib.uniql_fwht_composite, lib.uniql_status_string)))
+    _host = module
+    return module

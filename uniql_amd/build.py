@@ -1,4 +1,5 @@
-"""Compiles the HIP sources under csrc/ into lib/libuniql_amd.so for gfx950.
+"""Compiles the HIP sources under csrc/ into lib/libuniql_amd.so for gfx950, and csrc/host.cpp, the binding
+between torch's tensors and that library, into lib/_host.so.
 
     python -m uniql_amd.build
 
@@ -18,6 +19,7 @@ CSRC = os.path.join(PKG_DIR, "csrc")
 INCLUDE = os.path.join(os.path.dirname(PKG_DIR), "include")
 LIB_DIR = os.path.join(PKG_DIR, "lib")
 LIB_PATH = os.path.join(LIB_DIR, "libuniql_amd.so")
+HOST_PATH = os.path.join(LIB_DIR, "_host.so")
 
 ARCH = "gfx950"
 HIPCC_FLAGS = [
@@ -51,6 +53,18 @@ def _run(cmd: list[str], verbose: bool) -> None:
         print(err, file=sys.stderr)
 
 
+def _host_command(dst: str) -> list[str]:
+    import sysconfig
+
+    import torch
+    from torch.utils import cpp_extension
+    includes = [INCLUDE, sysconfig.get_paths()["include"], *cpp_extension.include_paths()]
+    libs = os.path.join(os.path.dirname(torch.__file__), "lib")
+    return ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", "-DTORCH_EXTENSION_NAME=_host",
+            f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", *[f"-I{d}" for d in includes],
+            os.path.join(CSRC, "host.cpp"), "-o", dst, f"-L{libs}", "-ltorch_python", "-ltorch", "-ltorch_cpu", "-lc10"]
+
+
 def build(verbose: bool = True, jobs: int | None = None) -> str:
     """Always recompiles every source (one hipcc per file, a few at a time, into a temporary
     directory), links, and returns the path of the shared library."""
@@ -63,12 +77,16 @@ def build(verbose: bool = True, jobs: int | None = None) -> str:
     jobs = jobs or max(1, min(len(srcs), (os.cpu_count() or 2) // 2, 8))
     with tempfile.TemporaryDirectory(prefix="uniql_build_") as tmpdir:
         objs = [os.path.join(tmpdir, os.path.basename(src)[:-4] + ".o") for src in srcs]
+        host = HOST_PATH + ".tmp"
         with ThreadPoolExecutor(max_workers=jobs) as pool:
+            host_done = pool.submit(_run, _host_command(host), verbose)
             list(pool.map(lambda so: _run([hipcc, *compile_flags, f"-I{INCLUDE}", f"-I{CSRC}", "-c", so[0], "-o", so[1]],
                                           verbose), zip(srcs, objs)))
         tmp = LIB_PATH + ".tmp"
         _run([hipcc, f"--offload-arch={ARCH}", "-shared", "-fPIC", *objs, "-o", tmp], verbose)
+        host_done.result()
     os.replace(tmp, LIB_PATH)
+    os.replace(host, HOST_PATH)
     return LIB_PATH
 
 

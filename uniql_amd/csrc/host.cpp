@@ -1,0 +1,223 @@
+// The host side of the calls that a token is made of - layer, embedding lookup, rotation - between torch and the C
+// ABI, in one native step per call: argument checks, the output's allocation and the launch.
+//
+// Bound by what it costs to get a launch out: at one token the kernels take 4-5 us, and the same checks in Python with
+// a ctypes call of 26 arguments took 14.2 us per W4A16B16O16Linear call, 10.9 per embedding lookup and 9.6 per
+// rotation.  The checks, their messages and the order in which they are made are those of uniql_amd.ops, which
+// validates a layer's own tensors once (prepare_linear) and hands the functions' addresses over (bind).
+// Nothing of a call is kept: no address of an input, no check, no output.  A layer's sizes -> scratch sizes map belongs to
+// the layer's handle and is a pure function of its key.  The interpreter lock is held except across the launch itself,
+// which may wait for room in the queue.
+#include <torch/extension.h>
+
+#include <map>
+#include <optional>
+#include <stdexcept>
+#include <string>
+#include <tuple>
+
+#include "uniql_amd.h"
+
+namespace {
+
+namespace py = pybind11;
+using at::Tensor;
+
+decltype(&uniql_w4a16_linear) p_linear = nullptr;
+decltype(&uniql_w4a16_linear_workspace) p_workspace = nullptr;
+decltype(&uniql_w4_embedding_lookup) p_embedding = nullptr;
+decltype(&uniql_fwht) p_fwht = nullptr;
+decltype(&uniql_fwht_composite) p_composite = nullptr;
+decltype(&uniql_status_string) p_status = nullptr;
+
+void bind(uintptr_t linear, uintptr_t workspace, uintptr_t embedding, uintptr_t fwht, uintptr_t composite, uintptr_t status) {
+    p_linear = reinterpret_cast<decltype(p_linear)>(linear);
+    p_workspace = reinterpret_cast<decltype(p_workspace)>(workspace);
+    p_embedding = reinterpret_cast<decltype(p_embedding)>(embedding);
+    p_fwht = reinterpret_cast<decltype(p_fwht)>(fwht);
+    p_composite = reinterpret_cast<decltype(p_composite)>(composite);
+    p_status = reinterpret_cast<decltype(p_status)>(status);
+}
+
+[[noreturn]] void fail(const std::string& what) { throw std::runtime_error(what); }
+void check(int code, const char* what) {
+    if (code != UNIQL_OK) fail(std::string(what) + ": " + p_status(code) + " (code " + std::to_string(code) + ")");
+}
+void require_gpu(const Tensor& t, const char* name) {
+    if (!t.is_cuda()) fail(std::string(name) + " must be a GPU tensor (this package has no CPU path)");
+}
+Tensor new_output(at::IntArrayRef sizes, at::ScalarType type, const Tensor& like) {
+    return at::empty(sizes, like.options().dtype(type).requires_grad(false).memory_format(std::nullopt));
+}
+
+struct Linear {
+    Tensor B, s, workspace;   // held so that the addresses below stay valid
+    std::optional<Tensor> bias;
+    int size_n, size_k, n_out, groups, had_block;
+    float had_scale;
+    bool silu_mul;
+    std::map<std::tuple<int64_t, int64_t, unsigned>, std::pair<size_t, size_t>> needs;   // (m, k_in, flags) -> accum, temp bytes
+};
+
+// The call on x [m, k_in]; `sizes`: the shape of a new output.
+Tensor run(Linear& p, Tensor x, std::optional<Tensor> residual, bool relu2, bool out_f32, std::optional<Tensor> out,
+           unsigned flags, uintptr_t stream, const py::object& accumulator, std::optional<std::vector<int64_t>> sizes) {
+    if (!x.is_cuda()) fail("x must be a GPU tensor (this package has no CPU path)");
+    if (x.scalar_type() != at::kHalf) fail("x and s must be float16");
+    if (x.dim() != 2 || x.stride(1) != 1) fail("x must be 2-D with unit stride along K");
+    const int64_t m = x.size(0);
+    int64_t k_in = x.size(1);
+    if (!(p.size_k - 128 < k_in && k_in <= p.size_k))
+        fail("x has " + std::to_string(k_in) + " columns, the packed weights cover " + std::to_string(p.size_k));
+    if (m > 0x7fffffff) fail("x has more rows than a call can take");
+    if (p.silu_mul && relu2) fail("silu_mul and relu2 are different epilogues: choose one");
+    const int64_t n_out = p.n_out;
+    const void* res_ptr = nullptr;
+    int64_t ldr = 0;
+    if (residual) {
+        require_gpu(*residual, "residual");
+        if (p.silu_mul || relu2) fail("a residual cannot be combined with an activation epilogue");
+        if (residual->scalar_type() != at::kHalf || residual->dim() != 2 || residual->size(0) != m || residual->size(1) != n_out ||
+            residual->stride(1) != 1)
+            fail("residual must be float16 [m, out_features] with unit inner stride");
+        res_ptr = residual->data_ptr();
+        ldr = m > 1 ? residual->stride(0) : n_out;
+    }
+    if (k_in % 8 || (m > 1 && x.stride(0) % 8) || reinterpret_cast<uintptr_t>(x.data_ptr()) % 16) {
+        // rare: rows that cannot be read in 16-byte pieces are copied (and padded) here
+        x = at::constant_pad_nd(x, {0, p.size_k - k_in});
+        k_in = p.size_k;
+    }
+    const c10::DeviceGuard guard(x.device());
+    const at::ScalarType type = out_f32 ? at::kFloat : at::kHalf;
+    Tensor y;
+    int64_t ldd = n_out;
+    if (!out) {
+        y = sizes ? new_output(*sizes, type, x) : new_output({m, n_out}, type, x);
+    } else {
+        if (out->scalar_type() != type || out->dim() != 2 || out->size(0) != m || out->size(1) != n_out || out->stride(1) != 1 ||
+            out->device() != x.device())
+            fail("out must be a [m, out_features] view with unit inner stride on x's device");
+        y = *out;
+        if (m > 1) ldd = y.stride(0);
+    }
+    if (m == 0) return y;
+    if (out_f32) flags |= UNIQL_F_OUT_F32;
+    const auto key = std::make_tuple(m, k_in, flags);
+    auto hit = p.needs.find(key);
+    if (hit == p.needs.end()) {
+        size_t accum = 0, temp = 0;
+        check(p_workspace((int)m, p.size_n, p.size_k, (int)k_in, p.had_block, flags, &accum, &temp), "uniql_w4a16_linear_workspace");
+        if (p.needs.size() > 4096) p.needs.clear();
+        hit = p.needs.emplace(key, std::make_pair(accum, temp)).first;
+    }
+    const size_t need_acc = hit->second.first, need_tmp = hit->second.second;
+    Tensor accum, temp;
+    if (need_acc) accum = accumulator(py::cast(x.device()), need_acc, stream).cast<Tensor>();
+    if (need_tmp) temp = new_output({(int64_t)need_tmp}, at::kByte, x);
+    const int64_t lda = m > 1 ? x.stride(0) : std::max<int64_t>((k_in + 7) / 8 * 8, 8);
+    int code;
+    {
+        const py::gil_scoped_release release;
+        code = p_linear(x.data_ptr(), lda, (int)k_in, p.B.data_ptr(), p.s.data_ptr(), p.bias ? p.bias->data_ptr() : nullptr, res_ptr,
+                        ldr, y.data_ptr(), ldd, (int)n_out,
+                        p.silu_mul ? UNIQL_EPI_SILU_MUL : (relu2 ? UNIQL_EPI_RELU2 : UNIQL_EPI_NONE),
+                        p.workspace.data_ptr<int32_t>(), p.workspace.numel(), need_acc ? accum.data_ptr() : nullptr,
+                        need_acc ? (size_t)accum.numel() * 8 : 0, need_tmp ? temp.data_ptr() : nullptr, need_tmp, (int)m, p.size_n,
+                        p.size_k, p.groups, p.had_block, p.had_scale, flags, reinterpret_cast<void*>(stream));
+    }
+    check(code, "uniql_w4a16_linear");
+    return y;
+}
+
+// rows x [..., k] as a matrix with unit inner stride (copied only where it has to be)
+Tensor as_rows(const Tensor& x, int64_t columns) {
+    Tensor r = x.dim() == 2 ? x : x.reshape({-1, columns});
+    return r.stride(-1) == 1 ? r : r.contiguous();
+}
+
+// a layer module's forward: x [..., in_features], residual of the result's shape
+Tensor forward(Linear& p, const Tensor& x, const std::optional<Tensor>& residual, bool relu2, uintptr_t stream,
+               const py::object& accumulator) {
+    const at::NoGradGuard no_grad;
+    if (x.dim() == 0) fail("x must have at least one dimension");
+    std::optional<Tensor> res;
+    if (residual) res = residual->reshape({-1, p.n_out});
+    std::vector<int64_t> sizes = x.sizes().vec();
+    sizes.back() = p.n_out;
+    return run(p, as_rows(x, x.size(-1)), res, relu2, false, std::nullopt, 0, stream, accumulator, sizes);
+}
+
+Tensor prepared(Linear& p, const Tensor& x, const std::optional<Tensor>& residual, bool relu2, bool out_f32,
+                const std::optional<Tensor>& out, unsigned flags, uintptr_t stream, const py::object& accumulator) {
+    return run(p, x, residual, relu2, out_f32, out, flags, stream, accumulator, std::nullopt);
+}
+
+Tensor embedding(const Tensor& ids_in, const Tensor& weight, const Tensor& scale, uintptr_t stream) {
+    const at::NoGradGuard no_grad;
+    if (weight.dim() != 2) fail("weight must be 2-D");
+    require_gpu(weight, "weight");
+    if (weight.scalar_type() != at::kInt) fail("weight's dtype must be int32");
+    const int64_t vocab = weight.size(0), dim = weight.size(1) * 8;
+    if (scale.dim() != 1) fail("scale must be 1-D");
+    require_gpu(scale, "scale");
+    if (scale.scalar_type() != at::kHalf) fail("scale's dtype must be float16");
+    if (scale.numel() != vocab) fail("scale must have one entry per vocabulary row");
+    if (ids_in.dim() != 1 && ids_in.dim() != 2) fail("input must be a 1D or 2D tensor");
+    require_gpu(ids_in, "input");
+    if (ids_in.scalar_type() != at::kLong) fail("input's dtype must be int64");
+    const Tensor ids = ids_in.contiguous();
+    if (!weight.is_contiguous() || !scale.is_contiguous()) fail("weight and scale must be contiguous");
+    const c10::DeviceGuard guard(ids.device());
+    std::vector<int64_t> sizes = ids.sizes().vec();
+    sizes.push_back(dim);
+    Tensor y = new_output(sizes, at::kHalf, ids);
+    int code;
+    {
+        const py::gil_scoped_release release;
+        code = p_embedding(ids.data_ptr<int64_t>(), ids.numel(), weight.data_ptr(), scale.data_ptr(), y.data_ptr(), vocab, (int)dim,
+                           reinterpret_cast<void*>(stream));
+    }
+    check(code, "uniql_w4_embedding_lookup");
+    return y;
+}
+
+// base 0: blocks of `block` values; else the composite transform of width base * 2^k.  New tensor.
+Tensor hadamard(const Tensor& x_in, int64_t block, int base, double scale, uintptr_t stream) {
+    const at::NoGradGuard no_grad;
+    require_gpu(x_in, "x");
+    const at::ScalarType t = x_in.scalar_type();
+    if (t != at::kHalf && t != at::kBFloat16 && t != at::kFloat)
+        fail("hadamard transform supports float16 / bfloat16 / float32, got " + std::string(c10::toString(t)));
+    const int type = t == at::kHalf ? UNIQL_DT_F16 : (t == at::kBFloat16 ? UNIQL_DT_BF16 : UNIQL_DT_F32);
+    const Tensor x = x_in.contiguous();
+    const int64_t dim = x.size(-1), rows = dim ? x.numel() / dim : 0;
+    if (dim > 0x7fffffff || block > 0x7fffffff) fail("the last axis is too wide");
+    const c10::DeviceGuard guard(x.device());
+    Tensor y = at::empty_like(x);
+    int code;
+    {
+        const py::gil_scoped_release release;
+        code = base == 0 ? p_fwht(x.data_ptr(), y.data_ptr(), rows, (int)dim, (int)block, (float)scale, type, reinterpret_cast<void*>(stream))
+                         : p_composite(x.data_ptr(), y.data_ptr(), rows, (int)dim, base, (float)scale, type, reinterpret_cast<void*>(stream));
+    }
+    check(code, base == 0 ? "uniql_fwht" : "uniql_fwht_composite");
+    return y;
+}
+
+}  // namespace
+
+PYBIND11_MODULE(_host, module) {
+    py::class_<Linear>(module, "Linear")
+        .def(py::init([](Tensor B, Tensor s, Tensor workspace, std::optional<Tensor> bias, int size_n, int size_k, int n_out,
+                         int had_block, double had_scale, bool silu_mul) {
+            const int groups = (int)s.size(0);
+            return Linear{std::move(B), std::move(s), std::move(workspace), std::move(bias), size_n, size_k, n_out, groups,
+                          had_block, (float)had_scale, silu_mul, {}};
+        }))
+        .def("forward", &forward)
+        .def("prepared", &prepared);
+    module.def("bind", &bind);
+    module.def("embedding", &embedding);
+    module.def("hadamard", &hadamard);
+}

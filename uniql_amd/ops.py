@@ -45,6 +45,12 @@ def _stream_ptr(device: torch.device) -> int:
     return torch.cuda.current_stream(device).cuda_stream
 
 
+def _stream_of(t: torch.Tensor, name: str) -> int:
+    if not t.is_cuda:
+        raise RuntimeError(f"{name} must be a GPU tensor (this package has no CPU path)")
+    return _stream_ptr(t.device)
+
+
 # Zero-in / zero-out accumulator words of the split-K exchange, one buffer per
 # (device, stream): kernels on one stream run in order, so they can share it; work on
 # different streams may overlap and must not.
@@ -212,10 +218,12 @@ def w4a16_gemm_static(A: torch.Tensor, B: torch.Tensor, s: torch.Tensor, workspa
 
 class PreparedLinear:
     """What a layer call needs that does not change from call to call, validated once
-    (prepare_linear): the packed tensors, their addresses and sizes, bias, rotation, epilogue.
-    The tensors are held so that the addresses stay valid."""
-    __slots__ = ("B", "s", "workspace", "bias", "b_ptr", "s_ptr", "ws_ptr", "ws_len", "bias_ptr", "size_n", "size_k",
-                 "n_out", "groups", "had_block", "had_scale", "silu_mul", "dev", "needs")
+    (prepare_linear) and held by a native handle: the packed tensors, bias, rotation, epilogue.
+    Copies and pickles of it are None (the addresses are this process's): prepare again."""
+    __slots__ = ("host", "__weakref__")
+
+    def __reduce__(self):
+        return type(None), ()
 
 
 def prepare_linear(B: torch.Tensor, s: torch.Tensor, workspace: torch.Tensor, size_n: int, size_k: int, *,
@@ -241,13 +249,8 @@ def prepare_linear(B: torch.Tensor, s: torch.Tensor, workspace: torch.Tensor, si
         if bias.dtype != torch.float16 or not bias.is_contiguous() or bias.numel() != (2 if silu_mul else 1) * n_out:
             raise RuntimeError("bias must be contiguous float16 with one entry per output column")
     p = PreparedLinear()
-    p.B, p.s, p.workspace, p.bias = B, s, workspace, bias
-    p.b_ptr, p.s_ptr, p.ws_ptr, p.ws_len = B.data_ptr(), s.data_ptr(), workspace.data_ptr(), workspace.numel()
-    p.bias_ptr = bias.data_ptr() if bias is not None else None
-    p.size_n, p.size_k, p.n_out, p.groups = int(size_n), int(size_k), n_out, s.shape[0]
-    p.had_block, p.had_scale, p.silu_mul = int(had_block), float(had_scale), bool(silu_mul)
-    p.dev = B.device
-    p.needs = {}   # (m, k_in, flags) -> (accum bytes, temp bytes)
+    p.host = _capi.host().Linear(B, s, workspace, bias, int(size_n), int(size_k), n_out, int(had_block), float(had_scale),
+                                 bool(silu_mul))
     return p
 
 
@@ -255,65 +258,13 @@ def linear_prepared(p: PreparedLinear, x: torch.Tensor, *, residual: torch.Tenso
                     out_f32: bool = False, out: torch.Tensor | None = None, flags: int = 0) -> torch.Tensor:
     """The per-call half of w4a16_linear: checks on the activations (and residual / out), the
     output's allocation, one call into the library."""
-    if not x.is_cuda:
-        raise RuntimeError("x must be a GPU tensor (this package has no CPU path)")
-    if x.dtype != torch.float16:
-        raise RuntimeError("x and s must be float16")
-    if x.dim() != 2 or x.stride(1) != 1:
-        raise RuntimeError("x must be 2-D with unit stride along K")
-    m, k_in = x.shape
-    size_k, n_out = p.size_k, p.n_out
-    if not (size_k - 128 < k_in <= size_k):
-        raise RuntimeError(f"x has {k_in} columns, the packed weights cover {size_k}")
-    if p.silu_mul and relu2:
-        raise RuntimeError("silu_mul and relu2 are different epilogues: choose one")
-    res_ptr, ldr = None, 0
-    if residual is not None:
-        _require_gpu(residual, "residual")
-        if p.silu_mul or relu2:
-            raise RuntimeError("a residual cannot be combined with an activation epilogue")
-        if residual.dtype != torch.float16 or tuple(residual.shape) != (m, n_out) or residual.stride(1) != 1:
-            raise RuntimeError("residual must be float16 [m, out_features] with unit inner stride")
-        res_ptr, ldr = residual.data_ptr(), (residual.stride(0) if m > 1 else n_out)
-    x_ptr = x.data_ptr()
-    if k_in % 8 or (m > 1 and x.stride(0) % 8) or x_ptr % 16:
-        # rare: rows that cannot be read in 16-byte pieces are copied (and padded) here
-        x = torch.nn.functional.pad(x, (0, size_k - k_in))
-        k_in = size_k
-        x_ptr = x.data_ptr()
-    lib = _capi.load()
-    dev = x.device
-    out_dtype = torch.float32 if out_f32 else torch.float16
-    with _device_guard(dev):
-        if out is None:
-            out = torch.empty((m, n_out), dtype=out_dtype, device=dev)
-        elif out.dtype != out_dtype or tuple(out.shape) != (m, n_out) or out.stride(1) != 1 or out.device != dev:
-            raise RuntimeError("out must be a [m, out_features] view with unit inner stride on x's device")
-        if m == 0:
-            return out
-        if out_f32:
-            flags |= _capi.F_OUT_F32
-        key = (m, k_in, flags)
-        need = p.needs.get(key)
-        if need is None:
-            need = p.needs[key] = _workspace(lib, m, p.size_n, size_k, k_in, p.had_block, flags)
-        need_acc, need_tmp = need
-        stream = _stream_ptr(dev)
-        accum = _accumulator(dev, need_acc, stream) if need_acc else None
-        temp = torch.empty(need_tmp, dtype=torch.uint8, device=dev) if need_tmp else None
-        lda = x.stride(0) if m > 1 else max(k_in + (-k_in) % 8, 8)
-        ldd = out.stride(0) if m > 1 else n_out
-        code = lib.uniql_w4a16_linear(
-            x_ptr, lda, k_in, p.b_ptr, p.s_ptr, p.bias_ptr, res_ptr, ldr,
-            out.data_ptr(), ldd, n_out,
-            _capi.EPI_SILU_MUL if p.silu_mul else (_capi.EPI_RELU2 if relu2 else _capi.EPI_NONE),
-            p.ws_ptr, p.ws_len,
-            accum.data_ptr() if accum is not None else None, accum.numel() * 8 if accum is not None else 0,
-            temp.data_ptr() if temp is not None else None, need_tmp,
-            m, p.size_n, size_k, p.groups, p.had_block, p.had_scale, flags, stream)
-    if code:
-        _capi.check(code, "uniql_w4a16_linear")
-    return out
+    return p.host.prepared(x, residual, relu2, out_f32, out, flags, _stream_of(x, "x"), _accumulator)
+
+
+def layer_forward(p: PreparedLinear, x: torch.Tensor, residual: torch.Tensor | None = None, relu2: bool = False) -> torch.Tensor:
+    """linear_prepared for a layer module: x of any rank (its rows along the last axis), residual and
+    result of x's leading shape."""
+    return p.host.forward(x, residual, relu2, _stream_of(x, "x"), _accumulator)
 
 
 def w4a16_linear(x: torch.Tensor, B: torch.Tensor, s: torch.Tensor, workspace: torch.Tensor, size_n: int,
@@ -503,37 +454,7 @@ def w4a16_cut_rows(B: torch.Tensor, s: torch.Tensor, size_n: int, size_k: int, u
 
 def w4a16_embedding_lookup(input: torch.Tensor, weight: torch.Tensor, scale: torch.Tensor) -> torch.Tensor:
     """out[..., :] = (code - 8) * scale[id].  Checks follow quant_embedding_kernel.cuh:121-134."""
-    if weight.dim() != 2:
-        raise RuntimeError("weight must be 2-D")
-    _require_gpu(weight, "weight")
-    if weight.dtype != torch.int32:
-        raise RuntimeError("weight's dtype must be int32")
-    vocab, words = weight.shape
-    dim = words * 8
-    if scale.dim() != 1:
-        raise RuntimeError("scale must be 1-D")
-    _require_gpu(scale, "scale")
-    if scale.dtype != torch.float16:
-        raise RuntimeError("scale's dtype must be float16")
-    if scale.numel() != vocab:
-        raise RuntimeError("scale must have one entry per vocabulary row")
-    if input.dim() not in (1, 2):
-        raise RuntimeError("input must be a 1D or 2D tensor")
-    _require_gpu(input, "input")
-    if input.dtype != torch.int64:
-        raise RuntimeError("input's dtype must be int64")
-    lib = _capi.load()
-    dev = input.device
-    ids = input.contiguous()
-    weight_c = weight.detach()
-    if not weight_c.is_contiguous() or not scale.is_contiguous():
-        raise RuntimeError("weight and scale must be contiguous")
-    with _device_guard(dev):
-        out = torch.empty((*ids.shape, dim), dtype=torch.float16, device=dev)
-        code = lib.uniql_w4_embedding_lookup(ids.data_ptr(), ids.numel(), weight_c.data_ptr(), scale.data_ptr(),
-                                             out.data_ptr(), vocab, dim, _stream_ptr(dev))
-    _capi.check(code, "uniql_w4_embedding_lookup")
-    return out
+    return _capi.host().embedding(input, weight, scale, _stream_of(input, "input"))
 
 
 def w4_embedding_quantize(weight: torch.Tensor):
@@ -600,22 +521,7 @@ def rope_indices_(q: torch.Tensor, k: torch.Tensor, cos: torch.Tensor, sin: torc
 
 def hadamard_blockwise(x: torch.Tensor, scale: float, block: int | None = None) -> torch.Tensor:
     """(x . H_block) * scale on consecutive block-wide pieces of the last axis; new tensor."""
-    _require_gpu(x, "x")
-    dim = x.shape[-1]
-    block = dim if block is None else block
-    dtypes = {torch.float16: _capi.DT_F16, torch.bfloat16: _capi.DT_BF16, torch.float32: _capi.DT_F32}
-    if x.dtype not in dtypes:
-        raise RuntimeError(f"hadamard transform supports float16 / bfloat16 / float32, got {x.dtype}")
-    lib = _capi.load()
-    xc = x.contiguous()
-    dev = x.device
-    with _device_guard(dev):
-        y = torch.empty_like(xc)
-        rows = xc.numel() // dim if dim else 0
-        code = lib.uniql_fwht(xc.data_ptr(), y.data_ptr(), rows, dim, block, float(scale),
-                              dtypes[x.dtype], _stream_ptr(dev))
-    _capi.check(code, "uniql_fwht")
-    return y
+    return _capi.host().hadamard(x, x.shape[-1] if block is None else block, 0, scale, _stream_of(x, "x"))
 
 
 def fast_hadamard_transform(x: torch.Tensor, scale: float = 1.0) -> torch.Tensor:
@@ -629,21 +535,7 @@ def fast_hadamard_transform(x: torch.Tensor, scale: float = 1.0) -> torch.Tensor
 def hadamard_composite(x: torch.Tensor, scale: float, base: int) -> torch.Tensor:
     """(x . (H_base (x) H_P)) * scale along the last axis of width base * P, P a power of two
     (uniql_fwht_composite); new tensor."""
-    _require_gpu(x, "x")
-    dim = x.shape[-1]
-    dtypes = {torch.float16: _capi.DT_F16, torch.bfloat16: _capi.DT_BF16, torch.float32: _capi.DT_F32}
-    if x.dtype not in dtypes:
-        raise RuntimeError(f"hadamard transform supports float16 / bfloat16 / float32, got {x.dtype}")
-    lib = _capi.load()
-    xc = x.contiguous()
-    dev = x.device
-    with _device_guard(dev):
-        y = torch.empty_like(xc)
-        rows = xc.numel() // dim if dim else 0
-        code = lib.uniql_fwht_composite(xc.data_ptr(), y.data_ptr(), rows, dim, base, float(scale),
-                                        dtypes[x.dtype], _stream_ptr(dev))
-    _capi.check(code, "uniql_fwht_composite")
-    return y
+    return _capi.host().hadamard(x, x.shape[-1], base, scale, _stream_of(x, "x"))
 
 
 _COLUMN_ROWS = (1024, 2048, 4096)   # heights uniql_fwht_columns takes

@@ -35,7 +35,6 @@ class W4O16Embedding(nn.Module):
         q.weight.data = packed.to(w.device)
         return q
 
-    @torch.no_grad()
     def forward(self, x):
         return ops.w4a16_embedding_lookup(x, self.weight, self.scales)
 

@@ -18,9 +18,8 @@ class Hadamard(torch.nn.Module):
         super().to(*args, **kwargs)
         return self
 
-    @torch.no_grad()
     def forward(self, x):
-        return self.transform_fn(x.contiguous(), self.had_scale)
+        return self.transform_fn(x, self.had_scale)   # (a strided input is copied inside; nothing is recorded for autograd)
 
     def __repr__(self):
         return f"Hadamard(dim={self.dim})"

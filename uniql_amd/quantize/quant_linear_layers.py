@@ -94,7 +94,6 @@ class W4A16B16O16Linear(nn.Module):
         self.had_scale = float(scale) if scale is not None else (block ** -0.5 if block else 1.0)
         return self
 
-    @torch.no_grad()
     def forward(self, x, residual=None, activation=None):
         """Padding of the input, the product, the cut of the padded output columns and the bias
         (quant_linear_layers.py:92-114) happen inside one kernel call.  Beyond the reference:
@@ -103,13 +102,7 @@ class W4A16B16O16Linear(nn.Module):
         of the un-gated MLP (nemotron_h_qblocks.py:588: act_fn(up_proj(x))) to the result."""
         if activation not in (None, "relu2"):
             raise ValueError(f"unsupported activation {activation!r} (None or 'relu2')")
-        x2 = x if x.dim() == 2 else x.reshape(-1, x.shape[-1])
-        if x2.stride(-1) != 1:
-            x2 = x2.contiguous()
-        y = ops.linear_prepared(self._prepared(), x2,
-                                residual=None if residual is None else residual.reshape(-1, self.out_features),
-                                relu2=activation == "relu2")
-        return y if x.dim() == 2 else y.view(*x.shape[:-1], self.out_features)
+        return ops.layer_forward(self._prepared(), x, residual, activation == "relu2")
 
     def _prepared(self):
         """The layer's side of the call, validated once and kept until a buffer is replaced
@@ -120,7 +113,7 @@ class W4A16B16O16Linear(nn.Module):
         key = (weight.data_ptr(), scale.data_ptr(), workspace.data_ptr(), None if bias is None else bias.data_ptr(),
                self.had_block, self.had_scale, self.size_n, self.size_k, self.out_features)
         cached = self.__dict__.get("_prep")
-        if cached is None or cached[0] != key:
+        if cached is None or cached[0] != key or cached[1] is None:
             prep = ops.prepare_linear(weight, scale, workspace, self.size_n, self.size_k, out_features=self.out_features,
                                       bias=None if bias is None else bias.data, had_block=self.had_block,
                                       had_scale=self.had_scale)
