@@ -610,12 +610,13 @@ static double tile_us(int mt, int quartets, int64_t wgs, int g) {
     } else if (mt == 2) {
         us = full * (6.5 + 1.02 * g);
         if (rest > 256) us += 6.0 + g * ramp(0.75, 1.02, rest, 256, 512);
-        else if (rest) us += full > 0 ? 4.0 + g * ramp(0.33, 0.49, rest, 0, 256) : 6.5 + 0.55 * g;  // starts before the round ends
+        else if (rest) us += full > 0 ? 4.0 + g * ramp(0.33, 0.49, rest, 0, 256)  // starts before the round ends
+                                  : 5.1 + g * ramp(0.46, 0.55, rest, 128, 256);
     } else {
         us = full * (5.0 + 1.5 * g);
         if (rest > 512) us += 5.0 + g * ramp(0.85, 1.5, rest, 512, 1024);
         else if (rest > 256) us += 5.0 + g * ramp(0.55, 0.75, rest, 256, 512);
-        else if (rest) us += full > 0 ? 4.0 + 0.35 * g : 5.0 + 0.5 * g;
+        else if (rest) us += full > 0 ? 4.0 + 0.35 * g : 3.1 + g * ramp(0.395, 0.45, rest, 128, 256);
     }
     return us;
 }
