@@ -154,6 +154,23 @@ def test_static_entry_uses_the_needs_of_the_kernel_that_takes_the_call(lib):
     assert st(None, 4096, None, None, None, None, 0, 4096, 28672, 4096, 32, 0, 1.0, 0, None) == -1
 
 
+def test_static_entry_with_the_copy_of_the_activations_filling_its_area(lib):
+    """Rotated rows of exactly the static area's size: the plan has to leave K unsplit (no room for partial tiles),
+    and the call passes the limit check."""
+    st = lib.uniql_w4a16_gemm_static
+    limit = lib.uniql_w4a16_gemm_static_limit(1)
+    split = 0
+    for k in (1024, 2048, 4096, 8192):
+        for n in (512, 1024, 4096, 6144, 14336):
+            m = limit // (2 * k)
+            acc, tmp = ctypes.c_size_t(0), ctypes.c_size_t(0)
+            assert lib.uniql_w4a16_linear_workspace(m, n, k, k, k, 0, ctypes.byref(acc), ctypes.byref(tmp)) == 0
+            split += tmp.value > limit
+            assert st(None, k, None, None, None, None, 0, m, n, k, k // 128, k, 1.0, 0, None) == -1, (m, n, k)
+            assert st(None, k, None, None, None, None, 0, m + 1, n, k, k // 128, k, 1.0, 0, None) == -7, (m, n, k)
+    assert split > 0   # some of these plans split K where there is room
+
+
 def test_argument_checks_need_no_gpu(lib):
     """Shape errors are reported before anything touches the device."""
     f = lib.uniql_w4a16_gemm

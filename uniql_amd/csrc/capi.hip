@@ -449,7 +449,7 @@ int uniql_w4a16_gemm_static(const void* A, int64_t lda, const void* B, const voi
     // no scratch at all, whatever the 128-column kernel would have asked for)
     size_t part_cap = kPartialCap;
     LinearNeeds q = linear_needs(m, n, k, k, lda, groups, had_block, flags, part_cap);
-    if (q.act_bytes < kStaticTempBytes && q.act_bytes + round256(q.part_bytes) > kStaticTempBytes) {
+    if (q.act_bytes <= kStaticTempBytes && q.act_bytes + round256(q.part_bytes) > kStaticTempBytes) {
         // the copy of the activations leaves less room for partial tiles: fewer K splits
         part_cap = kStaticTempBytes - q.act_bytes;
         q = linear_needs(m, n, k, k, lda, groups, had_block, flags, part_cap);
