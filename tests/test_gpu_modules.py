@@ -218,3 +218,21 @@ def test_native_host_path_keeps_the_modules_forms(gpu):
     assert not rotated.requires_grad and torch.equal(ops.fast_hadamard_transform(h.t().contiguous().t(), 0.5), rotated)
     with pytest.raises(RuntimeError):
         ops.hadamard_blockwise(h.double(), 1.0)
+
+
+@pytest.mark.parametrize("fuse", [False, True])
+def test_had_linear_weight_updated_between_forward_and_backward(gpu, fuse):
+    """the product recorded for the backward has a weight of its own"""
+    from uniql_amd.quantize.quant_linear_layers import HadLinear
+    torch.manual_seed(5)
+    lin = torch.nn.Linear(256, 128, bias=False, device=gpu, dtype=torch.float32)
+    layer = HadLinear(lin, input_transform=fuse, fuse_had=fuse)
+    x = torch.randn(4, 256, device=gpu, requires_grad=True)
+    before = layer.weight.detach().clone()
+    y = layer(x)
+    with torch.no_grad():
+        layer.weight.mul_(2.0)
+    y.sum().backward()
+    want = before.double().sum(0)
+    assert ((x.grad[0].double() - want).norm() / want.norm()).item() < 1e-5   # 128 fp32 terms: 128 x 2^-24
+    assert layer.weight.grad is not None

@@ -168,7 +168,10 @@ class HadLinear(nn.Linear):
         self.fuse_had = True
 
     def forward(self, x):
-        return F.linear(x, self.weight if self.fuse_had else self._rotated(self.weight), self.bias)
+        w = self.weight if self.fuse_had else self._rotated(self.weight)
+        if w is self.weight and torch.is_grad_enabled():
+            w = w.clone()   # a recorded product keeps its own weight: the layer's may be updated before the backward
+        return F.linear(x, w, self.bias)
 
     def __repr__(self):
         return (f"HadLinear(in_features={self.in_features}, out_features={self.out_features}, "
