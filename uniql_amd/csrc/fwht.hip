@@ -563,13 +563,19 @@ __global__ __launch_bounds__(512) void fwht_composite_vec_kernel(const T* __rest
     }
 }
 
+// The vector kernels move 16 bytes at a time; rows that start elsewhere (a contiguous view with an offset) take the kernels
+// that move single values.  Both give the same bits.
+static bool rows_aligned(const void* x, const void* y) {
+    return ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(y)) & 15u) == 0;
+}
+
 template <typename T, int BASE>
 static int fwht_composite_go(const void* x, void* y, int64_t rows, int P, float scale, hipStream_t stream) {
     int log2P = 0;
     while ((1 << log2P) < P) ++log2P;
     const int L = BASE * P;
     const size_t padded = (size_t)(L + (L >> 7) * 8) * sizeof(float);
-    if (P >= 128 && padded <= 160 * 1024) {
+    if (P >= 128 && padded <= 160 * 1024 && rows_aligned(x, y)) {
         static std::atomic<unsigned long long> done{0};
         if (!allow_lds(&fwht_composite_vec_kernel<T, BASE>, padded, done)) return UNIQL_E_LAUNCH;
         const int threads = P >= 512 ? 512 : 256;
@@ -608,7 +614,8 @@ int fwht_composite_launch(const void* x, void* y, int64_t rows, int dim, int bas
 
 template <typename T>
 static int fwht_typed_launch(const void* x, void* y, int64_t pieces, int block, float scale, hipStream_t stream) {
-    if (block == 128) {
+    const bool vec = rows_aligned(x, y);
+    if (block == 128 && vec) {
         const int64_t grid = (pieces + 15) / 16;
         if (grid > 0x7fffffffLL) return UNIQL_E_SHAPE;
         hipLaunchKernelGGL(fwht128_kernel<T>, dim3((unsigned)grid), dim3(256), 0, stream, reinterpret_cast<const T*>(x),
@@ -616,9 +623,11 @@ static int fwht_typed_launch(const void* x, void* y, int64_t pieces, int block, 
         return UNIQL_OK;
     }
     if (pieces > 0x7fffffffLL) return UNIQL_E_SHAPE;
-    if (block >= 256) return fwht_vec_launch<T>(x, y, pieces, block, scale, stream);
+    if (block >= 256 && vec) return fwht_vec_launch<T>(x, y, pieces, block, scale, stream);
     int log2L = 0;
     while ((1 << log2L) < block) ++log2L;
+    static std::atomic<unsigned long long> done{0};
+    if (!allow_lds(&fwht_lds_kernel<T>, (size_t)block * sizeof(float), done)) return UNIQL_E_LAUNCH;
     hipLaunchKernelGGL((fwht_lds_kernel<T>), dim3((unsigned)pieces), dim3(256), (size_t)block * sizeof(float), stream,
                        reinterpret_cast<const T*>(x), reinterpret_cast<T*>(y), block, log2L, scale);
     return UNIQL_OK;
