@@ -49,6 +49,24 @@ def test_quantize_rows_that_are_not_16_byte_aligned(gpu, view):
     assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
 
 
+@pytest.mark.parametrize("given", [False, True])
+def test_quantize_into_buffers_off_the_16_byte_grid(gpu, given):
+    """the C entry asks for 4-byte words and 2-byte scales only"""
+    from uniql_amd import _capi, ops
+    g = torch.Generator().manual_seed(4)
+    n, k = 192, 392
+    w = (torch.randn(n, k, generator=g) * 0.1).half().to(gpu)
+    scales = (torch.rand(4, n, generator=g) * 0.02 + 0.004).half().to(gpu) if given else None
+    packed, scale = ops.w4a16_quantize(w, scales, pad_out=64)
+    words = torch.full((packed.numel() + 2,), 7, dtype=torch.int32, device=gpu)
+    halves = torch.full((scale.numel() + 2,), 7, dtype=torch.float16, device=gpu)
+    code = _capi.load().uniql_w4a16_quantize(w.data_ptr(), k, scales.data_ptr() if given else None, words[1:].data_ptr(),
+                                             halves[1:].data_ptr(), n, k, 256, 512, torch.cuda.current_stream().cuda_stream)
+    assert code == 0
+    assert torch.equal(words[1:-1], packed.flatten()) and torch.equal(halves[1:-1], scale.flatten())
+    assert words[0] == words[-1] == 7 and halves[0] == halves[-1] == 7
+
+
 def _as(t, dtype):
     """numpy float32 of what the kernel's rounding to `dtype` gives for a float32 tensor"""
     return t.to(dtype).float().numpy()

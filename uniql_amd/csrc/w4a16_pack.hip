@@ -85,7 +85,7 @@ __device__ __forceinline__ void quantize_sixteen(const h8 (&w)[2], half_t s, boo
 template <bool GPTQ, class Load>
 __device__ __forceinline__ void quantize_tile(const Load& load, uint32_t* words, half_t* scales, const half_t* __restrict__ given,
                                               half_t* __restrict__ S, uint32_t* __restrict__ B, int out_features, int n_pad,
-                                              int g, int chunk) {
+                                              int g, int chunk, bool out_ok) {
     const int tid = threadIdx.x;
     const int r = tid & 7, c8 = (tid >> 3) & 7, j = tid >> 6;
     uint32_t out[4] = {0u, 0u, 0u, 0u};
@@ -141,16 +141,23 @@ __device__ __forceinline__ void quantize_tile(const Load& load, uint32_t* words,
     // eight packed rows x 512 bytes, 16 bytes per thread; the chunk's 64 scales
     const int row = tid >> 5, piece = tid & 31;
     const u32x4 v = *reinterpret_cast<const u32x4*>(words + row * kPackLdsRow + 4 * piece);
-    *reinterpret_cast<u32x4*>(B + (size_t)(8 * g + row) * 2 * n_pad + 128 * (size_t)chunk + 4 * piece) = v;
-    if (tid < 8)
-        *reinterpret_cast<u32x4*>(S + (size_t)g * n_pad + 64 * (size_t)chunk + 8 * tid) = *reinterpret_cast<const u32x4*>(scales + 8 * tid);
+    uint32_t* to = B + (size_t)(8 * g + row) * 2 * n_pad + 128 * (size_t)chunk + 4 * piece;
+    half_t* scale_to = S + (size_t)g * n_pad + 64 * (size_t)chunk;
+    if (out_ok) {
+        *reinterpret_cast<u32x4*>(to) = v;
+        if (tid < 8) *reinterpret_cast<u32x4*>(scale_to + 8 * tid) = *reinterpret_cast<const u32x4*>(scales + 8 * tid);
+    } else {  // a caller's buffers off the 16-byte grid
+#pragma unroll
+        for (int i = 0; i < 4; ++i) to[i] = v[i];
+        if (tid < 64) scale_to[tid] = scales[tid];
+    }
 }
 
 template <bool GPTQ>
 __global__ __launch_bounds__(256) void w4a16_quantize_kernel(const half_t* __restrict__ W, int64_t ldw, int vec_ok,
                                                             const half_t* __restrict__ given, half_t* __restrict__ S,
                                                             uint32_t* __restrict__ B, int out_features, int in_features,
-                                                            int n_pad, int groups) {
+                                                            int n_pad, int groups, int out_ok) {
     __shared__ __attribute__((aligned(16))) uint32_t words[8 * kPackLdsRow];
     __shared__ __attribute__((aligned(16))) half_t scales[64];
     const int g = blockIdx.x % groups, chunk = blockIdx.x / groups;  // neighbours read on along the same rows
@@ -167,7 +174,7 @@ __global__ __launch_bounds__(256) void w4a16_quantize_kernel(const half_t* __res
             }
         }
     };
-    quantize_tile<GPTQ>(load, words, scales, given, S, B, out_features, n_pad, g, chunk);
+    quantize_tile<GPTQ>(load, words, scales, given, S, B, out_features, n_pad, g, chunk, out_ok != 0);
 }
 
 // Keeps rows of a packed matrix that no longer line up with the groups, and quantises them again: what dequantising, gathering
@@ -221,7 +228,7 @@ __global__ __launch_bounds__(256) void w4a16_cut_rows_kernel(const uint32_t* __r
         for (int i = 0; i < 2; ++i)
             w[i] = col < n_real ? *reinterpret_cast<const h8*>(values + (col & 63) * kCutLdsRow + 16 * r + 8 * i) : h8{};
     };
-    quantize_tile<false>(load, words, scales, nullptr, S, B, n_real, n_pad, g, chunk);
+    quantize_tile<false>(load, words, scales, nullptr, S, B, n_real, n_pad, g, chunk, true);
 }
 
 // Keeps columns of a packed matrix, as they are: kept columns are up to five runs of `units` x (`kept` of every `full`
@@ -349,10 +356,11 @@ int quantize_launch(const void* W, int64_t ldw, const void* given_scales, void* 
     const int64_t grid = (int64_t)groups * (n_pad / 64);
     if (grid > 0x7fffffffLL) return UNIQL_E_SHAPE;
     const int vec_ok = ldw % 8 == 0 && (reinterpret_cast<uintptr_t>(W) & 15u) == 0 ? 1 : 0;
+    const int out_ok = ((reinterpret_cast<uintptr_t>(B) | reinterpret_cast<uintptr_t>(S)) & 15u) == 0 ? 1 : 0;
     auto kern = given_scales ? &w4a16_quantize_kernel<true> : &w4a16_quantize_kernel<false>;
     hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(256), 0, stream, reinterpret_cast<const half_t*>(W), ldw, vec_ok,
                        reinterpret_cast<const half_t*>(given_scales), reinterpret_cast<half_t*>(S),
-                       reinterpret_cast<uint32_t*>(B), out_features, in_features, n_pad, groups);
+                       reinterpret_cast<uint32_t*>(B), out_features, in_features, n_pad, groups, out_ok);
     return hipGetLastError() == hipSuccess ? UNIQL_OK : UNIQL_E_LAUNCH;
 }
 
