@@ -619,8 +619,8 @@ def main():
             "unit": "TFLOP/s", "us_per_layer": round(tot_sec * 1e6, 2), "per_linear": per_shape,
             "roofline": {"bound": "mfma", "achieved": round(tot_flops / tot_sec / 1e12, 1), "peak": MFMA_F16_PEAK_TFLOPS,
                          "unit": "TFLOP/s", "frac": round(tot_flops / tot_sec / 1e12 / MFMA_F16_PEAK_TFLOPS, 4),
-                         "kernel": "w4a16_wide_kernel (256 x 256 tiles) for gate_up, w4a16_tile_kernel<MT> (MT = 4, or 2 "
-                                   "for the 6144-wide qkv) for the other three"}}
+                         "kernel": "w4a16_wide_kernel (256 x 256 tiles) or w4a16_tile_kernel<MT> (32 MT x 128 tiles), in one "
+                                   "launch or two, by expected time"}}
         result["library_fp16_gemm_m1024"] = {
             "what": "torch.matmul(x[1024, k] fp16, w[k, n] fp16) on the same weights dequantised beforehand (its "
                     "dequantisation pass not counted), same graph timing",
