@@ -1,0 +1,69 @@
+"""The tiled kernels' plans (csrc/tile_plan.hpp, plain host C++): what is chosen can be run as it is."""
+import ctypes
+import os
+import shutil
+import subprocess
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+
+SOURCE = r"""
+#include "tile_plan.hpp"
+using namespace uniql;
+
+static bool runnable(const TilePlan& p, int k) {
+    const int G = k / 128;
+    if (p.mtiles < 1 || p.mtiles > 4 || p.splits < 1 || p.gps < 1) return false;
+    if ((p.splits - 1) * p.gps >= G || p.splits * p.gps < G) return false;   // every split has groups, none is left over
+    if (p.quartets == 2) return p.mtiles <= 2 && G % 2 == 0 && p.gps % 2 == 0;  // even ranges, the last one too
+    return p.quartets == 1;
+}
+
+// Rows lo..hi of one layer: how many launches are not what the search chose once its fields are asked for, or cannot run.
+extern "C" int plans_off(int n, int k, int lo, int hi, int wide_ok, int* launches) {
+    int off = 0;
+    *launches = 0;
+    for (int m = lo; m <= hi; ++m) {
+        const LinearPlan plan = linear_plan(m, n, k, wide_ok != 0, (size_t)12 << 20, 0);
+        int rows = 0;
+        for (int i = 0; i < plan.parts; ++i) {
+            const RowPart& part = plan.part[i];
+            rows += part.rows;
+            if (part.wide) continue;
+            ++*launches;
+            const TilePlan& p = part.tile;
+            const unsigned tune = (unsigned)p.splits | ((unsigned)p.mtiles << 8) | ((unsigned)p.quartets << 12);
+            const TilePlan q = linear_plan(part.rows, n, k, false, 0, tune).part[0].tile;
+            off += !runnable(p, k) || q.mtiles != p.mtiles || q.splits != p.splits || q.gps != p.gps || q.quartets != p.quartets;
+        }
+        off += rows != m;
+    }
+    return off;
+}
+"""
+
+
+@pytest.fixture(scope="module")
+def plans(tmp_path_factory):
+    if shutil.which("g++") is None:
+        pytest.skip("g++ not available")
+    d = tmp_path_factory.mktemp("tile_plan")
+    (d / "plans.cpp").write_text(SOURCE)
+    subprocess.run(["g++", "-O2", "-std=c++17", "-Wall", "-Wno-unused-function", "-shared", "-fPIC",
+                    f"-I{os.path.join(ROOT, 'uniql_amd', 'csrc')}", str(d / "plans.cpp"), "-o", str(d / "plans.so")], check=True)
+    return ctypes.CDLL(str(d / "plans.so"))
+
+
+@pytest.mark.parametrize("n", [256, 1024, 4096, 6144, 18688, 28672])
+def test_the_plan_that_is_chosen_is_the_plan_that_its_fields_ask_for(plans, n):
+    """a field set that names a choice (K splits, tile height, quartets) leads back to that choice, group count per
+    split included: 10496 -> 4096 at 65 rows wants two splits of 42 groups for two quartets, not of 41"""
+    launches = ctypes.c_int(0)
+    total = 0
+    for k in list(range(128, 2048, 384)) + list(range(2048, 14337, 128)):
+        for lo, hi in ((17, 200), (320, 340), (1090, 1110), (4090, 4096)):
+            for wide_ok in (0, 1):
+                assert plans.plans_off(n, k, lo, hi, wide_ok, ctypes.byref(launches)) == 0, (n, k, lo, hi, wide_ok)
+                total += launches.value
+    assert total > 10000

@@ -3,6 +3,7 @@
 #include <mutex>
 
 #include "common.hpp"
+#include "tile_plan.hpp"
 #include "uniql_amd_diag.h"
 
 namespace uniql {
@@ -15,17 +16,13 @@ bool stream_shape_ok(int k, int64_t lda);
 int read_floor_launch(const void* B, const void* S, void* sink, int m, int n, int k, unsigned tune, hipStream_t stream);
 size_t read_floor_sink_bytes(int m, int n, int k, unsigned tune);
 int tile_launch(const void* A, int64_t lda, const void* B, const void* S, void* D, const Epilogue& epi, void* accum,
-                size_t accum_bytes, void* part, size_t part_bytes, int m, int n, int k, int groups, unsigned tune,
+                size_t accum_bytes, void* part, size_t part_bytes, int m, int n, int k, int groups, const TilePlan& plan,
                 hipStream_t stream);
-size_t tile_part_bytes(int m, int n, int k, unsigned tune);
-bool tile_shape_ok(int m, int n, int k, int64_t ldx, unsigned tune);
+bool tile_shape_ok(int m, int n, int k, int64_t ldx, const TilePlan& plan);
 int pad_rows_launch(const void* A, int64_t lda, int k_in, void* dst, int k, int m, hipStream_t stream);
-size_t tile_accum_bytes(int m, int n, int k, unsigned tune = 0);
 int wide_launch(const void* A, int64_t lda, const void* B, const void* S, void* D, const Epilogue& epi, int m, int n,
                 int k, int groups, hipStream_t stream);
 bool wide_shape_ok(int m, int n, int k, int groups, int64_t ldx);
-double wide_us(int m, int n, int k);
-unsigned tile_choose(int m, int n, int k, size_t part_cap, double* us);
 int dequant_launch(const void* B, const void* S, void* W, uint8_t* codes, int n, int k, int groups,
                    hipStream_t stream);
 int embedding_launch(const int64_t* ids, int64_t ntokens, const void* weight, const void* scales, void* out,
@@ -126,78 +123,6 @@ static size_t activation_copy_bytes(int m, int k, int k_in, int had_block, bool 
 static constexpr size_t kStaticAccumBytes = (size_t)4 << 20;   // the static area: exchange words, 16 rows x 32768 columns
 static constexpr size_t kStaticTempBytes = (size_t)12 << 20;   //                  rotated rows / partial tiles
 
-// How the tiled kernels run the rows of a call: one launch, or two over consecutive rows.  `tune` holds the 128-column
-// kernel's tuning fields with the whole plan in them; row tiles = 8 stands for the 256 x 256 kernel.
-struct RowPart {
-    int rows;
-    unsigned tune;
-    bool wide() const { return ((tune >> 8) & 0xfu) == 8; }
-};
-struct LinearPlan {
-    int parts;
-    RowPart part[2];
-};
-
-// The faster of the two kernels for m rows in one launch, by their expected times.  The 4 %: most layer calls cut, add or
-// gate their outputs, which the 256 x 256 kernel does at next to no cost and the tall tiles of the other with 3 to 8 %
-// (4096 -> 18560 of 18688 at 565 rows: 101 us against 107, expected of the plain product 101.5 and 100.5).
-static RowPart best_launch(int m, int n, int k, bool wide_ok, size_t part_cap, double* us) {
-    RowPart p = {m, tile_choose(m, n, k, part_cap, us)};
-    const double w = wide_ok ? wide_us(m, n, k) : 1e30;
-    if (w < 1.04 * *us) {
-        *us = w;
-        p.tune = 8u << 8;
-    }
-    return p;
-}
-
-// wide_ok: the 256 x 256 kernel can take the call.  part_cap: the most bytes of partial tiles a plan may ask for.
-// A last round of workgroups that leaves most of the chip idle costs as much as a full one, so the rows behind the
-// last 128-row boundaries are also tried as a launch of their own (shorter tiles, K split): 4096 -> 28672 at 1100
-// rows is 1024 on the 256 x 256 kernel and 76 on 96-row tiles, 240 us instead of 297 in one launch.
-// Up to 128 rows there is nothing to split (a second launch costs 2 us).
-static LinearPlan linear_plan(int m, int n, int k, bool wide_ok, size_t part_cap, unsigned tune) {
-    LinearPlan plan;
-    plan.parts = 1;
-    const unsigned forced_rows = (tune >> 8) & 0xfu;
-    if ((tune & 0x3fffu) != 0) {  // a plan asked for by the caller, as far as the kernels can follow it
-        plan.part[0] = RowPart{m, tune};
-        if (forced_rows == 8 && !wide_ok) plan.part[0].tune = tune & ~0xf00u;
-        return plan;
-    }
-    double us;
-    plan.part[0] = best_launch(m, n, k, wide_ok, part_cap, &us);
-    int j = (m - 1) / 128;
-    for (int tries = 0; j > 0 && tries < 8; --j, ++tries) {
-        double head_us, tail_us;
-        const RowPart head = best_launch(128 * j, n, k, wide_ok, part_cap, &head_us);
-        if (head_us + 2.0 >= us) continue;
-        const RowPart tail = best_launch(m - 128 * j, n, k, wide_ok, part_cap, &tail_us);
-        if (head_us + tail_us + 2.0 < 0.97 * us) {
-            us = (head_us + tail_us + 2.0) / 0.97;
-            plan.parts = 2;
-            plan.part[0] = head;
-            plan.part[1] = tail;
-        }
-    }
-    return plan;
-}
-static size_t plan_accum_bytes(const LinearPlan& plan, int n, int k) {
-    size_t most = 0;
-    for (int i = 0; i < plan.parts; ++i) {
-        const size_t b = plan.part[i].wide() ? 0 : tile_accum_bytes(plan.part[i].rows, n, k, plan.part[i].tune);
-        most = b > most ? b : most;
-    }
-    return most;
-}
-static size_t plan_part_bytes(const LinearPlan& plan, int n, int k) {
-    size_t most = 0;
-    for (int i = 0; i < plan.parts; ++i) {
-        const size_t b = plan.part[i].wide() ? 0 : tile_part_bytes(plan.part[i].rows, n, k, plan.part[i].tune);
-        most = b > most ? b : most;
-    }
-    return most;
-}
 // Partial tiles of any call fit the static area (with more splits than that the exchange costs more than it gives);
 // the static entry asks for less where the copy of the activations needs the room.
 static constexpr size_t kPartialCap = kStaticTempBytes;
@@ -234,8 +159,8 @@ static LinearNeeds linear_needs(int m, int n, int k, int k_in, int64_t lda, int 
         q.part_bytes = 0;
     } else {
         q.plan = linear_plan(m, n, k, wide_shape_ok(m, n, k, groups, q.ld_kernel), part_cap, tune);
-        q.accum_bytes = round256(plan_accum_bytes(q.plan, n, k));
-        q.part_bytes = plan_part_bytes(q.plan, n, k);
+        q.accum_bytes = round256(plan_accum_bytes(q.plan, n));
+        q.part_bytes = plan_part_bytes(q.plan, n);
     }
     return q;
 }
@@ -245,7 +170,7 @@ static void tiled_workspace(int m, int n, int k, unsigned tune, size_t* accum, s
     *accum = *part = 0;
     for (int wide = 0; wide < 2; ++wide) {
         const LinearPlan plan = linear_plan(m, n, k, wide != 0 && wide_shape_ok(m, n, k, k / 128, k), kPartialCap, tune);
-        const size_t a = plan_accum_bytes(plan, n, k), p = plan_part_bytes(plan, n, k);
+        const size_t a = plan_accum_bytes(plan, n), p = plan_part_bytes(plan, n);
         *accum = a > *accum ? a : *accum;
         *part = p > *part ? p : *part;
     }
@@ -340,7 +265,7 @@ static int linear_impl(const void* A, int64_t lda, int k_in, const void* B, cons
     void* part = part_bytes ? reinterpret_cast<char*>(temp) + act_bytes : nullptr;
     // last check before the first kernel is enqueued: whether the tiled kernel can take the shape
     for (int i = 0; i < q.plan.parts; ++i)
-        if (!q.plan.part[i].wide() && !tile_shape_ok(q.plan.part[i].rows, n, k, ld_kernel, q.plan.part[i].tune)) return UNIQL_E_SHAPE;
+        if (!q.plan.part[i].wide && !tile_shape_ok(q.plan.part[i].rows, n, k, ld_kernel, q.plan.part[i].tile)) return UNIQL_E_SHAPE;
     if (use_stream && !stream_shape_ok(k, ld_kernel)) return UNIQL_E_SHAPE;
     if (check_only) return UNIQL_OK;
     if (pad_first) {
@@ -375,8 +300,8 @@ static int linear_impl(const void* A, int64_t lda, int k_in, const void* B, cons
         const char* x = reinterpret_cast<const char*>(Ain) + (size_t)m0 * ld * sizeof(half_t);
         char* d = reinterpret_cast<char*>(D) + (size_t)m0 * (transpose ? 1 : ldd) * (out_f32 ? 4 : 2);
         epi.residual = residual ? reinterpret_cast<const half_t*>(residual) + (size_t)m0 * ldr : nullptr;
-        const int e = p.wide() ? wide_launch(x, ld, B, S, d, epi, p.rows, n, k, groups, st)
-                               : tile_launch(x, ld, B, S, d, epi, accum, accum_bytes, part, part_bytes, p.rows, n, k, groups, p.tune, st);
+        const int e = p.wide ? wide_launch(x, ld, B, S, d, epi, p.rows, n, k, groups, st)
+                               : tile_launch(x, ld, B, S, d, epi, accum, accum_bytes, part, part_bytes, p.rows, n, k, groups, p.tile, st);
         if (e != UNIQL_OK) return e;
         m0 += p.rows;
     }

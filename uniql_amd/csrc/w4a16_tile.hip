@@ -36,6 +36,7 @@
 #include <atomic>
 
 #include "common.hpp"
+#include "tile_plan.hpp"
 
 namespace uniql {
 
@@ -555,133 +556,10 @@ __global__ __launch_bounds__(256 * KW, 1) void w4a16_tile_kernel(const TileArgs 
 }
 
 // ---------------------------------------------------------------------------------
-static inline int ceil_div_i(int a, int b) { return (a + b - 1) / b; }
-
-struct TilePlan {
-    int mtiles, splits, gps;
-    int quartets;  // wave quartets per workgroup (1 or 2)
-    double us;     // what tile_us expects of it
-};
-static TilePlan tile_plan(int m, int n, int k, int splits_override, int mt_override, int kw_override, size_t part_cap);
-
-static TilePlan tile_plan_tuned(int m, int n, int k, unsigned tune) {
-    return tile_plan(m, n, k, (int)(tune & 0xffu), (int)((tune >> 8) & 0xfu), (int)((tune >> 12) & 0x3u), (size_t)-1);
-}
-
-// What a plan that splits K over workgroups needs (tune: the same fields as tile_launch takes):
-// one arrival count per output tile in `accum` (zero on entry, zero again on exit) and one fp32
-// partial tile per (tile, split) in a scratch area whose contents do not matter.
-size_t tile_accum_bytes(int m, int n, int k, unsigned tune) {
-    const TilePlan plan = tile_plan_tuned(m, n, k, tune);
-    if (plan.splits <= 1) return 0;
-    return (size_t)(n / 128) * ceil_div_i(m, 32 * plan.mtiles) * sizeof(unsigned long long);
-}
-size_t tile_part_bytes(int m, int n, int k, unsigned tune) {
-    const TilePlan plan = tile_plan_tuned(m, n, k, tune);
-    if (plan.splits <= 1) return 0;
-    const size_t tiles = (size_t)(n / 128) * ceil_div_i(m, 32 * plan.mtiles);
-    return tiles * plan.splits * (32 * plan.mtiles * 128) * sizeof(float);
-}
-
-// Time of a launch of `wgs` workgroups that walk `g` K groups each, in us, on 256 compute units.
-// Workgroups run in rounds: one per compute unit with 96- and 128-row tiles (LDS) or two quartets, two with
-// 64-row tiles, four with 32-row tiles.  A round costs a prologue and an epilogue (6 us) and a time per group that
-// grows once more than half of the chip is busy (the clock falls with the matrix load).  Fitted to forced
-// launches of nine shapes (K 4096 to 14336, N 4096 to 28672) at 96 to 4096 rows, within 5 % of all but the
-// 32-row tiles from 600 workgroups on; e.g. 4096 -> 4096, 256 tiles of 128 rows 35.6 us (model 35.0), of 96 rows 29.7
-// (29.4), 14336 -> 4096 106 (104) and 89.8 (87.8).
-static double ramp(double lo, double hi, int64_t x, int64_t x0, int64_t x1) {
-    return x <= x0 ? lo : lo + (hi - lo) * (double)(x - x0) / (double)(x1 - x0);
-}
-static double tile_us(int mt, int quartets, int64_t wgs, int g) {
-    const int64_t per_round = quartets == 2 || mt >= 3 ? 256 : (mt == 2 ? 512 : 1024);
-    const double full = (double)(wgs / per_round);
-    const int64_t rest = wgs % per_round;
-    double us = 0.0;
-    if (quartets == 2 && mt == 2) {
-        us = full * (5.7 + 0.536 * g);
-        if (rest) us += 5.7 + g * (rest <= 192 ? ramp(0.375, 0.447, rest, 64, 192) : ramp(0.447, 0.536, rest, 192, 256));
-    } else if (quartets == 2) {
-        us = full * (3.9 + 0.40 * g) + (rest ? 3.9 + g * ramp(0.30, 0.40, rest, 64, 256) : 0.0);
-    } else if (mt == 4) {
-        us = full * (6.5 + 0.875 * g) + (rest ? 6.5 + g * ramp(0.60, 0.86, rest, 128, 256) : 0.0);
-    } else if (mt == 3) {
-        us = full * (6.0 + 0.73 * g) + (rest ? 6.0 + g * ramp(0.53, 0.73, rest, 128, 256) : 0.0);
-    } else if (mt == 2) {
-        us = full * (6.5 + 1.02 * g);
-        if (rest > 256) us += 6.0 + g * ramp(0.75, 1.02, rest, 256, 512);
-        else if (rest) us += full > 0 ? 4.0 + g * ramp(0.33, 0.49, rest, 0, 256)  // starts before the round ends
-                                  : 5.1 + g * ramp(0.46, 0.55, rest, 128, 256);
-    } else {
-        us = full * (5.0 + 1.5 * g);
-        if (rest > 512) us += 5.0 + g * ramp(0.85, 1.5, rest, 512, 1024);
-        else if (rest > 256) us += 5.0 + g * ramp(0.55, 0.75, rest, 256, 512);
-        else if (rest) us += full > 0 ? 4.0 + 0.35 * g : 3.1 + g * ramp(0.395, 0.45, rest, 128, 256);
-    }
-    return us;
-}
-
-// What the exchange between the splits of a tile adds: the partial tiles' stores, the count, and the last workgroup's
-// reading of all of them (forced splits of 1 to 8 on six shapes at 24 to 192 rows).
-static double exchange_us(int mt, int splits) {
-    if (mt == 1) return 2.2 + 0.08 * splits * splits;
-    if (mt == 2) return 3.0 + 0.11 * splits * splits;
-    return mt == 3 ? 3.0 + 1.8 * splits : 6.0 + 2.1 * splits;
-}
-
-// Height of the tiles, K splits and quartets with the smallest expected time.  K is split over workgroups while the
-// grid stays within one workgroup per compute unit, every workgroup keeps at least 8 groups and the
-// partial tiles fit part_cap bytes.  Two quartets whenever the grid has at most 256 workgroups of at most 64 rows
-// and every workgroup gets an even number of groups.
-// The 96-row tiles are there for the rounds: 14336 -> 4096 at 333 rows runs as 256 workgroups of them in 51.3 us
-// (128 rows: 54.1, 64 rows: 54.5, the rule of thumb this search replaced: 57-63), 4096 -> 24576 at 333 rows as three
-// whole rounds (87.0 against 93.3).
-static TilePlan tile_plan(int m, int n, int k, int splits_override, int mt_override, int kw_override, size_t part_cap) {
-    TilePlan best = {4, 1, k / 128, 1, 1e30};
-    const int strips = n / 128, G = k / 128;
-    const bool even_g = G % 2 == 0;
-    for (int mt = 1; mt <= 4; ++mt) {
-        if (mt_override >= 1 && mt_override <= 4 && mt != mt_override) continue;
-        const int64_t tiles = (int64_t)strips * ceil_div_i(m, 32 * mt);
-        for (int s = 1; s <= 255; ++s) {
-            if (splits_override > 0) s = splits_override;
-            else if (s > 1 && (tiles * s > 256 || G / s < 8)) break;
-            TilePlan p;
-            p.mtiles = mt;
-            p.gps = ceil_div_i(G, s > G ? G : s);
-            p.splits = ceil_div_i(G, p.gps);
-            p.quartets = 1;
-            // two quartets take alternate groups: every workgroup's range must hold an even number
-            if ((kw_override == 2 || (kw_override == 0 && tiles * p.splits <= 256)) && mt <= 2 && even_g) {
-                const int gps2 = p.gps + (p.gps & 1);
-                if (splits_override == 0 || gps2 == p.gps) {
-                    p.gps = gps2;
-                    p.splits = ceil_div_i(G, p.gps);
-                    p.quartets = 2;
-                }
-            }
-            p.us = tile_us(mt, p.quartets, tiles * p.splits, p.gps);
-            if (p.splits > 1) p.us += exchange_us(mt, p.splits);
-            const bool fits = p.splits == 1 || splits_override > 0 || (size_t)tiles * p.splits * mt * (32 * 128 * 4) <= part_cap;
-            if (fits && p.us < best.us) best = p;
-            if (splits_override > 0) break;
-        }
-    }
-    return best;
-}
-
-// The plan for m rows as the tuning fields that force it, and its expected time.
-unsigned tile_choose(int m, int n, int k, size_t part_cap, double* us) {
-    const TilePlan p = tile_plan(m, n, k, 0, 0, 0, part_cap);
-    *us = p.us;
-    return (unsigned)p.splits | ((unsigned)p.mtiles << 8) | ((unsigned)p.quartets << 12);
-}
-
 // Whether tile_launch can take the call: grid size, and the 32-bit offsets of the loads (128 rows of
 // ldx elements, 2 bytes each, and the packed weights must stay below 2^32 bytes).  Checked by the entry point
 // before anything is enqueued.
-bool tile_shape_ok(int m, int n, int k, int64_t ldx, unsigned tune) {
-    const TilePlan plan = tile_plan_tuned(m, n, k, tune);
+bool tile_shape_ok(int m, int n, int k, int64_t ldx, const TilePlan& plan) {
     const int64_t grid = (int64_t)(n / 128) * ceil_div_i(m, 32 * plan.mtiles) * plan.splits;
     return grid <= 0x7fffffffLL && ldx < (1LL << 24) && (int64_t)k * n / 2 < (1LL << 32);
 }
@@ -711,14 +589,11 @@ static hipError_t tile_launch_ext(const TileArgs& a, bool ext, int grid, hipStre
     return ext ? tile_launch_one<MT, true, KW>(a, grid, stream) : tile_launch_one<MT, false, KW>(a, grid, stream);
 }
 
-// tune: bits 0..7 force the number of K splits, bits 8..11 the number of 32-row M tiles per
-// workgroup, bits 12..13 the number of wave quartets (0 = choose)
 int tile_launch(const void* A, int64_t lda, const void* B, const void* S, void* D, const Epilogue& epi, void* accum,
-                size_t accum_bytes, void* part, size_t part_bytes, int m, int n, int k, int groups, unsigned tune,
+                size_t accum_bytes, void* part, size_t part_bytes, int m, int n, int k, int groups, const TilePlan& plan,
                 hipStream_t stream) {
-    const TilePlan plan = tile_plan_tuned(m, n, k, tune);
-    if (plan.splits > 1 && (!accum || accum_bytes < tile_accum_bytes(m, n, k, tune) || !part ||
-                            part_bytes < tile_part_bytes(m, n, k, tune)))
+    if (plan.splits > 1 && (!accum || accum_bytes < tile_accum_bytes(m, n, plan) || !part ||
+                            part_bytes < tile_part_bytes(m, n, plan)))
         return UNIQL_E_WORKSPACE;
     TileArgs a;
     a.part = reinterpret_cast<float*>(part);

@@ -486,16 +486,6 @@ bool wide_shape_ok(int m, int n, int k, int groups, int64_t ldx) {
            (int64_t)(n / 256) * ((m + 255) / 256) <= 0x7fffffffLL;
 }
 
-// Expected time in us (fitted like the 128-column kernel's: forced launches of nine shapes at 96 to 4096 rows, within 5 %):
-// rounds of 256 workgroups, the time per K group growing with the busy part of the chip.
-double wide_us(int m, int n, int k) {
-    const int64_t tiles = (int64_t)(n / 256) * ((m + 255) / 256);
-    const int g = k / 128;
-    const int64_t rest = tiles % 256;
-    const double slow = rest > 120 ? 1.08 * (double)(rest - 120) / 136.0 : 0.0;
-    return (double)(tiles / 256) * (9.0 + 3.2 * g) + (rest ? 8.5 + g * (2.12 + slow) : 0.0);
-}
-
 static hipError_t wide_launch_one(const WideArgs& a, int grid, hipStream_t stream) {
     auto kern = &w4a16_wide_kernel;
     static std::atomic<unsigned long long> done{0};  // the attribute is set once per device
