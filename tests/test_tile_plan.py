@@ -41,6 +41,32 @@ extern "C" int plans_off(int n, int k, int lo, int hi, int wide_ok, int* launche
     }
     return off;
 }
+
+// Rows lo..hi: in how many the search leaves a plan that it rates (a height, a split count, one or two quartets) below its choice.
+extern "C" int plans_missed(int n, int k, int lo, int hi) {
+    int missed = 0;
+    for (int m = lo; m <= hi; ++m) {
+        const TilePlan best = tile_plan(m, n, k, 0, 0, 0, (size_t)12 << 20);
+        for (int mt = 1; mt <= 4; ++mt) {
+            for (int kw = 1; kw <= 2; ++kw) {
+                const TilePlan p = tile_plan(m, n, k, 0, mt, kw, (size_t)12 << 20);
+                const bool rated = p.quartets == 1 || (int64_t)(n / 128) * ceil_div_i(m, 32 * mt) * p.splits <= 256;
+                missed += rated && p.us < best.us;
+            }
+        }
+    }
+    return missed;
+}
+
+// Rows lo..hi: in how many the launch that is taken is neither the rule's nor faster than it by its expected time.
+extern "C" int rule_left_for_nothing(int n, int k, int lo, int hi) {
+    int bad = 0;
+    for (int m = lo; m <= hi; ++m) {
+        const RowPart rule = rule_launch(m, n, k, n % 256 == 0), p = best_launch(m, n, k, n % 256 == 0, (size_t)-1);
+        bad += p.tile.us > rule.tile.us || !(p.wide || runnable(p.tile, k)) || !(rule.wide || runnable(rule.tile, k));
+    }
+    return bad;
+}
 """
 
 
@@ -67,3 +93,11 @@ def test_the_plan_that_is_chosen_is_the_plan_that_its_fields_ask_for(plans, n):
                 assert plans.plans_off(n, k, lo, hi, wide_ok, ctypes.byref(launches)) == 0, (n, k, lo, hi, wide_ok)
                 total += launches.value
     assert total > 10000
+
+
+@pytest.mark.parametrize("n", [256, 1024, 4096, 6144, 28672])
+def test_the_search_rates_one_and_two_quartets(plans, n):
+    """4096 -> 1024 at 97 rows: one quartet is the faster of the two where both fit"""
+    for k in (128, 512, 1280, 2688, 4096, 7424, 10496, 14336):
+        assert plans.plans_missed(n, k, 17, 1100) == 0, (n, k)
+        assert plans.rule_left_for_nothing(n, k, 17, 1100) == 0, (n, k)

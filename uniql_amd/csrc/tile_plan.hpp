@@ -28,101 +28,84 @@ static inline size_t tile_part_bytes(int m, int n, const TilePlan& plan) {
     return (size_t)(n / 128) * ceil_div_i(m, 32 * plan.mtiles) * plan.splits * (32 * plan.mtiles * 128) * sizeof(float);
 }
 
-// Time of a launch of `wgs` workgroups that walk `g` K groups each, in us, on 256 compute units.
-// Workgroups run in rounds: one per compute unit with 96- and 128-row tiles (LDS) or two quartets, two with
-// 64-row tiles, four with 32-row tiles.  A round costs a prologue and an epilogue (6 us) and a time per group that
-// grows once more than half of the chip is busy (the clock falls with the matrix load).  Fitted to forced
-// launches of nine shapes (K 4096 to 14336, N 4096 to 28672) at 96 to 4096 rows, within 5 % of all but the
-// 32-row tiles from 600 workgroups on; e.g. 4096 -> 4096, 256 tiles of 128 rows 35.6 us (model 35.0), of 96 rows 29.7
-// (29.4), 14336 -> 4096 106 (104) and 89.8 (87.8).
-static inline double ramp(double lo, double hi, int64_t x, int64_t x0, int64_t x1) {
-    return x <= x0 ? lo : lo + (hi - lo) * (double)(x - x0) / (double)(x1 - x0);
+// Time in us of a launch of `wgs` workgroups that walk `g` K groups each, on 256 compute units.  Workgroups run in
+// rounds: one per compute unit with two quartets, 96-, 128-row and 256 x 256 tiles (LDS), two with 64-row tiles, four with
+// 32-row tiles.  A launch costs a constant (prologue, epilogue, start) and a time per K group, which steps with the number of
+// workgroups on the fullest compute unit and grows with the busy part of the chip inside a step (the clock falls with the matrix load).
+// Fitted to 6250 drawn layer calls (N 256 to 28672, K 256 to 14336, 17 to 4096 rows, plain, cut, gated and with a residual), each
+// with every plan inside 1.5 x of the best: half of the times are within 3.5 % of these, nine in ten within 12 %.  What
+// is off is mostly the epilogue, which a plan must not depend on (a layer's sum is the same with and without a residual):
+// adding one costs the tall tiles 4 to 8 us a round.  Of another 6250 calls the plan with the smallest time here took 1.003 x
+// the best plan's time on average.
+struct LaunchFit {
+    double full, full_g;        // a whole round: constant, per K group
+    double split, split_each;   // the exchange between K splits (partial tiles' stores, count, the last one's reading of all of them)
+    double after;               // what is left behind whole rounds, a constant
+    int levels;                 // workgroups per compute unit and round
+    struct {                    // i + 1 workgroups on the fullest unit in what is left:
+        double alone;           //   its constant if that is the whole launch
+        double behind;          //   factor on the times per group behind whole rounds
+        double g[3];            //   time per K group with the level nearly empty, half full, full
+    } level[4];
+};
+static const LaunchFit kLaunchFits[7] = {
+    {8.65, 1.351, 0.537, 0.77, 4.03, 4, {{5.34, 0.814, 0.391, 0.355, 0.404}, {5.78, 1.127, 0.581, 0.639, 0.715},
+     {6.82, 1.054, 1.019, 1.032, 1.138}, {8.86, 1.117, 1.304, 1.379, 1.453}}},  // 32 rows, one quartet
+    {5.29, 0.35, 0.763, 0.547, 5.46, 1, {{5.46, 1.0, 0.279, 0.282, 0.339}}},  // 32 rows, two quartets
+    {5.59, 1.001, 1.509, 1.112, 5.58, 2, {{6.82, 0.989, 0.447, 0.452, 0.577}, {7.16, 1.085, 0.8, 0.938, 1.074}}},  // 64 rows, one quartet
+    {7.46, 0.521, 0.852, 0.935, 7.15, 1, {{7.15, 1.0, 0.365, 0.381, 0.498}}},  // 64 rows, two quartets
+    {6.97, 0.74, 2.88, 1.858, 4.67, 1, {{6.35, 1.083, 0.478, 0.604, 0.743}}},  // 96 rows
+    {5.98, 0.95, 1.877, 2.68, 7.49, 1, {{8.94, 1.043, 0.493, 0.692, 0.9}}},  // 128 rows
+    {7.65, 3.39, 0.0, 0.0, 4.41, 1, {{13.28, 1.095, 2.15, 2.64, 3.29}}},  // 256 x 256
+};
+static inline double launch_us(const LaunchFit& f, int64_t wgs, int g, int splits) {
+    const int64_t per_round = 256 * (int64_t)f.levels, full = wgs / per_round, rest = wgs % per_round;
+    double us = (double)full * (f.full + f.full_g * g) + (splits > 1 ? f.split + f.split_each * splits : 0.0);
+    if (rest == 0) return us;
+    const auto& l = f.level[(rest - 1) / 256];
+    const double x = (double)((rest - 1) % 256 + 1) / 128.0;   // 0 to 2 inside the level
+    const double per_g = x < 1.0 ? l.g[0] + (l.g[1] - l.g[0]) * x : l.g[1] + (l.g[2] - l.g[1]) * (x - 1.0);
+    return us + (full > 0 ? f.after + l.behind * per_g * g : l.alone + per_g * g);
 }
-static inline double tile_us(int mt, int quartets, int64_t wgs, int g) {
-    const int64_t per_round = quartets == 2 || mt >= 3 ? 256 : (mt == 2 ? 512 : 1024);
-    const double full = (double)(wgs / per_round);
-    const int64_t rest = wgs % per_round;
-    double us = 0.0;
-    if (quartets == 2 && mt == 2) {
-        us = full * (5.7 + 0.536 * g);
-        if (rest) us += 5.7 + g * (rest <= 192 ? ramp(0.375, 0.447, rest, 64, 192) : ramp(0.447, 0.536, rest, 192, 256));
-    } else if (quartets == 2) {
-        us = full * (3.9 + 0.40 * g) + (rest ? 3.9 + g * ramp(0.30, 0.40, rest, 64, 256) : 0.0);
-    } else if (mt == 4) {
-        us = full * (6.5 + 0.875 * g) + (rest ? 6.5 + g * ramp(0.60, 0.86, rest, 128, 256) : 0.0);
-    } else if (mt == 3) {
-        us = full * (6.0 + 0.73 * g) + (rest ? 6.0 + g * ramp(0.53, 0.73, rest, 128, 256) : 0.0);
-    } else if (mt == 2) {
-        us = full * (6.5 + 1.02 * g);
-        if (rest > 256) us += 6.0 + g * ramp(0.75, 1.02, rest, 256, 512);
-        else if (rest) us += full > 0 ? 4.0 + g * ramp(0.33, 0.49, rest, 0, 256)  // starts before the round ends
-                                  : 5.1 + g * ramp(0.46, 0.55, rest, 128, 256);
-    } else {
-        us = full * (5.0 + 1.5 * g);
-        if (rest > 512) us += 5.0 + g * ramp(0.85, 1.5, rest, 512, 1024);
-        else if (rest > 256) us += 5.0 + g * ramp(0.55, 0.75, rest, 256, 512);
-        else if (rest) us += full > 0 ? 4.0 + 0.35 * g : 3.1 + g * ramp(0.395, 0.45, rest, 128, 256);
-    }
-    return us;
+static inline int fit_index(int mt, int quartets) { return mt <= 2 ? 2 * (mt - 1) + (quartets - 1) : mt + 1; }
+static inline double tile_us(int mt, int quartets, int64_t wgs, int g, int splits) {
+    return launch_us(kLaunchFits[fit_index(mt, quartets)], wgs, g, splits);
 }
-
-// What the exchange between the splits of a tile adds: the partial tiles' stores, the count, and the last workgroup's
-// reading of all of them (forced splits of 1 to 8 on six shapes at 24 to 192 rows).
-static inline double exchange_us(int mt, int splits) {
-    if (mt == 1) return 2.2 + 0.08 * splits * splits;
-    if (mt == 2) return 3.0 + 0.11 * splits * splits;
-    return mt == 3 ? 3.0 + 1.8 * splits : 6.0 + 2.1 * splits;
+static inline double wide_us(int m, int n, int k) {
+    return launch_us(kLaunchFits[6], (int64_t)(n / 256) * ((m + 255) / 256), k / 128, 1);
 }
 
 // Height of the tiles, K splits and quartets with the smallest expected time.  K is split over workgroups while the
 // grid stays within one workgroup per compute unit, every workgroup keeps at least 8 groups and the
-// partial tiles fit part_cap bytes.  Two quartets whenever the grid has at most 256 workgroups of at most 64 rows
+// partial tiles fit part_cap bytes.  Two quartets are rated where the grid has at most 256 workgroups of at most 64 rows
 // and every workgroup can get an even number of groups.  Overrides: 0 = choose.
 // The 96-row tiles are there for the rounds: 14336 -> 4096 at 333 rows runs as 256 workgroups of them in 51.3 us
-// (128 rows: 54.1, 64 rows: 54.5, the rule of thumb this search replaced: 57-63), 4096 -> 24576 at 333 rows as three
+// (128 rows: 54.1, 64 rows: 54.5, the plan of rule_launch: 57-63), 4096 -> 24576 at 333 rows as three
 // whole rounds (87.0 against 93.3).
 static inline TilePlan tile_plan(int m, int n, int k, int splits_override, int mt_override, int kw_override, size_t part_cap) {
     TilePlan best = {4, 1, k / 128, 1, 1e30};
     const int strips = n / 128, G = k / 128;
-    const bool even_g = G % 2 == 0;
     for (int mt = 1; mt <= 4; ++mt) {
         if (mt_override >= 1 && mt_override <= 4 && mt != mt_override) continue;
         const int64_t tiles = (int64_t)strips * ceil_div_i(m, 32 * mt);
         for (int s = 1; s <= 255; ++s) {
             if (splits_override > 0) s = splits_override;
             else if (s > 1 && (tiles * s > 256 || G / s < 8)) break;
-            TilePlan p;
-            p.mtiles = mt;
-            p.gps = ceil_div_i(G, s > G ? G : s);
-            p.splits = ceil_div_i(G, p.gps);
-            p.quartets = 1;
+            const int gps1 = ceil_div_i(G, s > G ? G : s), splits = ceil_div_i(G, gps1);
             // two quartets take alternate groups: every workgroup's range must hold an even number
-            if ((kw_override == 2 || (kw_override == 0 && tiles * p.splits <= 256)) && mt <= 2 && even_g) {
-                const int gps2 = p.gps + (p.gps & 1);
-                if (splits_override == 0 || ceil_div_i(G, gps2) == p.splits) {
-                    p.gps = gps2;
-                    p.splits = ceil_div_i(G, p.gps);
-                    p.quartets = 2;
-                }
+            const int gps2 = gps1 + (gps1 & 1);
+            const bool two_ok = mt <= 2 && G % 2 == 0 && ceil_div_i(G, gps2) == splits && (kw_override == 2 || tiles * splits <= 256);
+            for (int kw = 1; kw <= 2; ++kw) {
+                if (kw == 2 ? !two_ok || (kw_override & 1) : two_ok && kw_override == 2) continue;
+                TilePlan p = {mt, splits, kw == 2 ? gps2 : gps1, kw, 0.0};
+                p.us = tile_us(mt, kw, tiles * splits, p.gps, splits);
+                const bool fits = splits == 1 || splits_override > 0 || tile_part_bytes(m, n, p) <= part_cap;
+                if (fits && p.us < best.us) best = p;
             }
-            p.us = tile_us(mt, p.quartets, tiles * p.splits, p.gps);
-            if (p.splits > 1) p.us += exchange_us(mt, p.splits);
-            const bool fits = p.splits == 1 || splits_override > 0 || tile_part_bytes(m, n, p) <= part_cap;
-            if (fits && p.us < best.us) best = p;
             if (splits_override > 0) break;
         }
     }
     return best;
-}
-
-// Expected time of the 256 x 256 kernel in us (fitted like the 128-column kernel's: forced launches of nine shapes at 96 to
-// 4096 rows, within 5 %): rounds of 256 workgroups, the time per K group growing with the busy part of the chip.
-static inline double wide_us(int m, int n, int k) {
-    const int64_t tiles = (int64_t)(n / 256) * ((m + 255) / 256);
-    const int g = k / 128;
-    const int64_t rest = tiles % 256;
-    const double slow = rest > 120 ? 1.08 * (double)(rest - 120) / 136.0 : 0.0;
-    return (double)(tiles / 256) * (9.0 + 3.2 * g) + (rest ? 8.5 + g * (2.12 + slow) : 0.0);
 }
 
 // How the tiled kernels run the rows of a call: one launch, or two over consecutive rows.
@@ -136,17 +119,58 @@ struct LinearPlan {
     RowPart part[2];
 };
 
-// The faster of the two kernels for m rows in one launch, by their expected times.  The 4 %: most layer calls cut, add or
-// gate their outputs, which the 256 x 256 kernel does at next to no cost and the tall tiles of the other with 3 to 8 %
-// (4096 -> 18560 of 18688 at 565 rows: 101 us against 107, expected of the plain product 101.5 and 100.5).
+// The plan for m rows in one launch by the order of the tile heights alone.  In
+// units of the time one 128-row workgroup takes for its K loop when every compute unit has one: 128 rows 1 per started
+// round of 256; 64 rows 1.08 per round of 512 (every weight is expanded twice per 128 rows), 0.85 for a last round of at most
+// 256; 32 rows 0.62 for at most 256 workgroups, 0.88 for at most 512, 1.62 per started round of 1024; two quartets, at most
+// one workgroup per compute unit, 0.85 and 0.92 of it.  A long K loop over few 64-row tiles prefers those with K split (every weight
+// is expanded for twice the rows).  K splits double while the grid stays within one workgroup per compute unit, every
+// workgroup keeps at least 8 groups and the partial tiles stay below a quarter of the packed weights.  The 256 x 256
+// kernel wherever the real output fills at least 0.62 of the tile slots of its rounds of 256 workgroups.
+static inline RowPart rule_launch(int m, int n, int k, bool wide_ok) {
+    const int64_t wide_rounds = ((int64_t)(n / 256) * ((m + 255) / 256) + 255) / 256;
+    if (wide_ok && (double)m * n / 65536.0 >= 0.62 * 256.0 * (double)wide_rounds)
+        return RowPart{m, true, TilePlan{0, 1, k / 128, 1, wide_us(m, n, k)}};
+    const int strips = n / 128, G = k / 128;
+    const bool even_g = G % 2 == 0;
+    const int64_t t4 = (int64_t)strips * ceil_div_i(m, 128), t2 = (int64_t)strips * ceil_div_i(m, 64);
+    const int64_t t1 = (int64_t)strips * ceil_div_i(m, 32), rest2 = t2 % 512;
+    const double cost4 = (double)((t4 + 255) / 256);
+    const double cost2 = (1.08 * (double)(t2 / 512) + (rest2 == 0 ? 0.0 : (rest2 <= 256 ? 0.85 : 1.08))) * (even_g && t2 <= 256 ? 0.92 : 1.0);
+    const double cost1 = (t1 <= 256 ? 0.62 : (t1 <= 512 ? 0.88 : 1.62 * (double)((t1 + 1023) / 1024))) * (even_g && t1 <= 256 ? 0.85 : 1.0);
+    TilePlan p;
+    p.mtiles = m <= 32 ? 1 : (cost2 < cost4 && cost2 <= cost1 ? 2 : (cost1 < cost4 ? 1 : 4));
+    if (p.mtiles == 1 && G >= 64 && m >= 64 && t2 <= 128) p.mtiles = 2;
+    const int64_t tiles = (int64_t)strips * ceil_div_i(m, 32 * p.mtiles);
+    int splits = 1;
+    while (tiles * (2 * splits) <= 256 && G / (2 * splits) >= 8 && (int64_t)(2 * splits) * m * 16 <= k) splits *= 2;
+    p.gps = ceil_div_i(G, splits);
+    p.quartets = even_g && p.mtiles <= 2 && tiles * ceil_div_i(G, p.gps) <= 256 ? 2 : 1;
+    if (p.quartets == 2) p.gps += p.gps & 1;
+    p.splits = ceil_div_i(G, p.gps);
+    p.us = tile_us(p.mtiles, p.quartets, tiles * p.splits, p.gps, p.splits);
+    return RowPart{m, false, p};
+}
+
+// Whether all workgroups of a launch of the 128-column kernel are on the chip at once.
+static inline bool one_round(int m, int n, const TilePlan& p) {
+    return (int64_t)(n / 128) * ceil_div_i(m, 32 * p.mtiles) * p.splits <= 256 * (int64_t)kLaunchFits[fit_index(p.mtiles, p.quartets)].levels;
+}
+
+// One launch for m rows: what the search expects to be fastest, if that beats the rule's plan by 2 %.  Between two launches
+// of one round each, whose expected times are the most exact, any gain is enough.  Of 6250 calls the search alone is 1.7 %
+// faster than the rule and slower by more than 2 % in 113; with these margins it is 1.7 % faster and slower in 31.
 static inline RowPart best_launch(int m, int n, int k, bool wide_ok, size_t part_cap) {
+    const RowPart rule = rule_launch(m, n, k, wide_ok);
     RowPart p = {m, false, tile_plan(m, n, k, 0, 0, 0, part_cap)};
-    const double w = wide_ok ? wide_us(m, n, k) : 1e30;
-    if (w < 1.04 * p.tile.us) {
+    const double wide = wide_ok ? wide_us(m, n, k) : p.tile.us;
+    if (wide < p.tile.us) {
         p.wide = true;
-        p.tile.us = w;
+        p.tile.us = wide;
     }
-    return p;
+    if (!rule.wide && tile_part_bytes(m, n, rule.tile) > part_cap) return p;
+    const bool exact = !p.wide && !rule.wide && one_round(m, n, p.tile) && one_round(m, n, rule.tile);
+    return p.tile.us < (exact ? 1.0 : 0.98) * rule.tile.us ? p : rule;
 }
 
 // wide_ok: the 256 x 256 kernel can take the call.  part_cap: the most bytes of partial tiles a plan may ask for.
@@ -155,7 +179,9 @@ static inline RowPart best_launch(int m, int n, int k, bool wide_ok, size_t part
 // A last round of workgroups that leaves most of the chip idle costs as much as a full one, so the rows behind the
 // last 128-row boundaries are also tried as a launch of their own (shorter tiles, K split): 4096 -> 28672 at 1100
 // rows is 1024 on the 256 x 256 kernel and 76 on 96-row tiles, 240 us instead of 297 in one launch.
-// Up to 128 rows there is nothing to split (a second launch costs 2 us).
+// Up to 128 rows there is nothing to split.  The 2 us: two launches of different kernels take that much longer than each
+// behind its like (4096 -> 28672 at 200 rows: 69.5 us, 65.1 expected of 128 and 72 rows alone); the 2 %: what the expected times may be
+// off together.
 static inline LinearPlan linear_plan(int m, int n, int k, bool wide_ok, size_t part_cap, unsigned tune) {
     LinearPlan plan;
     plan.parts = 1;
@@ -173,8 +199,8 @@ static inline LinearPlan linear_plan(int m, int n, int k, bool wide_ok, size_t p
         if (head.tile.us + 2.0 >= us) continue;
         const RowPart tail = best_launch(m - 128 * j, n, k, wide_ok, part_cap);
         const double both = head.tile.us + tail.tile.us + 2.0;
-        if (both < 0.97 * us) {
-            us = both / 0.97;
+        if (both < 0.98 * us) {
+            us = both / 0.98;
             plan.parts = 2;
             plan.part[0] = head;
             plan.part[1] = tail;
