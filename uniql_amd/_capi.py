@@ -8,6 +8,7 @@ from __future__ import annotations
 
 import ctypes
 import os
+import threading
 from ctypes import c_char_p, c_float, c_int, c_int64, c_size_t, c_uint, c_void_p
 
 from .build import HOST_PATH, LIB_PATH
@@ -101,6 +102,7 @@ def check(code: int, what: str) -> None:
 
 
 _host = None
+_host_lock = threading.Lock()
 
 
 def host():
@@ -108,15 +110,17 @@ def host():
     global _host
     if _host is not None:
         return _host
-    from importlib import util
-    lib = load()
-    if not os.path.exists(HOST_PATH):
-        raise UniqlLibraryError(f"{HOST_PATH} not found: build it with `python -m uniql_amd.build`")
-    spec = util.spec_from_file_location("uniql_amd._host", HOST_PATH)
-    module = util.module_from_spec(spec)
-    spec.loader.exec_module(module)
-    module.bind(*(ctypes.cast(fn, ctypes.c_void_p).value
-                  for fn in (lib.uniql_w4a16_linear, lib.uniql_w4a16_linear_workspace, lib.uniql_w4_embedding_lookup,
-                             lib.uniql_fwht, lib.uniql_fwht_composite, lib.uniql_status_string)))
-    _host = module
-    return module
+    with _host_lock:   # a second thread that came in first would see the module before its functions are there
+        if _host is None:
+            from importlib import util
+            lib = load()
+            if not os.path.exists(HOST_PATH):
+                raise UniqlLibraryError(f"{HOST_PATH} not found: build it with `python -m uniql_amd.build`")
+            spec = util.spec_from_file_location("uniql_amd._host", HOST_PATH)
+            module = util.module_from_spec(spec)
+            spec.loader.exec_module(module)
+            module.bind(*(ctypes.cast(fn, ctypes.c_void_p).value
+                          for fn in (lib.uniql_w4a16_linear, lib.uniql_w4a16_linear_workspace, lib.uniql_w4_embedding_lookup,
+                                     lib.uniql_fwht, lib.uniql_fwht_composite, lib.uniql_status_string)))
+            _host = module
+    return _host
