@@ -6,8 +6,8 @@
 // rotation.  The checks, their messages and the order in which they are made are those of uniql_amd.ops, which
 // validates a layer's own tensors once (prepare_linear) and hands the functions' addresses over (bind).
 // Nothing of a call is kept: no address of an input, no check, no output.  A layer's sizes -> scratch sizes map belongs to
-// the layer's handle and is a pure function of its key.  The interpreter lock is held except across the launch itself,
-// which may wait for room in the queue.
+// the layer's handle and is a pure function of its key.  The interpreter lock is given up for the whole call - copies of
+// strided rows, allocations and launches may all wait for the device - but for that map and the accumulator's lookup.
 #include <torch/extension.h>
 
 #include <map>
@@ -59,7 +59,7 @@ struct Linear {
     std::map<std::tuple<int64_t, int64_t, unsigned>, std::pair<size_t, size_t>> needs;   // (m, k_in, flags) -> accum, temp bytes
 };
 
-// The call on x [m, k_in]; `sizes`: the shape of a new output.
+// The call on x [m, k_in]; `sizes`: the shape of a new output.  Without the interpreter lock.
 Tensor run(Linear& p, Tensor x, std::optional<Tensor> residual, bool relu2, bool out_f32, std::optional<Tensor> out,
            unsigned flags, uintptr_t stream, const py::object& accumulator, std::optional<std::vector<int64_t>> sizes) {
     if (!x.is_cuda()) fail("x must be a GPU tensor (this package has no CPU path)");
@@ -103,29 +103,30 @@ Tensor run(Linear& p, Tensor x, std::optional<Tensor> residual, bool relu2, bool
     }
     if (m == 0) return y;
     if (out_f32) flags |= UNIQL_F_OUT_F32;
-    const auto key = std::make_tuple(m, k_in, flags);
-    auto hit = p.needs.find(key);
-    if (hit == p.needs.end()) {
-        size_t accum = 0, temp = 0;
-        check(p_workspace((int)m, p.size_n, p.size_k, (int)k_in, p.had_block, flags, &accum, &temp), "uniql_w4a16_linear_workspace");
-        if (p.needs.size() > 4096) p.needs.clear();
-        hit = p.needs.emplace(key, std::make_pair(accum, temp)).first;
-    }
-    const size_t need_acc = hit->second.first, need_tmp = hit->second.second;
+    size_t need_acc, need_tmp;
     Tensor accum, temp;
-    if (need_acc) accum = accumulator(py::cast(x.device()), need_acc, stream).cast<Tensor>();
+    {
+        const py::gil_scoped_acquire lock;
+        const auto key = std::make_tuple(m, k_in, flags);
+        auto hit = p.needs.find(key);
+        if (hit == p.needs.end()) {
+            size_t acc = 0, tmp = 0;
+            check(p_workspace((int)m, p.size_n, p.size_k, (int)k_in, p.had_block, flags, &acc, &tmp), "uniql_w4a16_linear_workspace");
+            if (p.needs.size() > 4096) p.needs.clear();
+            hit = p.needs.emplace(key, std::make_pair(acc, tmp)).first;
+        }
+        need_acc = hit->second.first;
+        need_tmp = hit->second.second;
+        if (need_acc) accum = accumulator(py::cast(x.device()), need_acc, stream).cast<Tensor>();
+    }
     if (need_tmp) temp = new_output({(int64_t)need_tmp}, at::kByte, x);
     const int64_t lda = m > 1 ? x.stride(0) : std::max<int64_t>((k_in + 7) / 8 * 8, 8);
-    int code;
-    {
-        const py::gil_scoped_release release;
-        code = p_linear(x.data_ptr(), lda, (int)k_in, p.B.data_ptr(), p.s.data_ptr(), p.bias ? p.bias->data_ptr() : nullptr, res_ptr,
-                        ldr, y.data_ptr(), ldd, (int)n_out,
-                        p.silu_mul ? UNIQL_EPI_SILU_MUL : (relu2 ? UNIQL_EPI_RELU2 : UNIQL_EPI_NONE),
-                        p.workspace.data_ptr<int32_t>(), p.workspace.numel(), need_acc ? accum.data_ptr() : nullptr,
-                        need_acc ? (size_t)accum.numel() * 8 : 0, need_tmp ? temp.data_ptr() : nullptr, need_tmp, (int)m, p.size_n,
-                        p.size_k, p.groups, p.had_block, p.had_scale, flags, reinterpret_cast<void*>(stream));
-    }
+    const int code = p_linear(x.data_ptr(), lda, (int)k_in, p.B.data_ptr(), p.s.data_ptr(), p.bias ? p.bias->data_ptr() : nullptr, res_ptr,
+                              ldr, y.data_ptr(), ldd, (int)n_out,
+                              p.silu_mul ? UNIQL_EPI_SILU_MUL : (relu2 ? UNIQL_EPI_RELU2 : UNIQL_EPI_NONE),
+                              p.workspace.data_ptr<int32_t>(), p.workspace.numel(), need_acc ? accum.data_ptr() : nullptr,
+                              need_acc ? (size_t)accum.numel() * 8 : 0, need_tmp ? temp.data_ptr() : nullptr, need_tmp, (int)m, p.size_n,
+                              p.size_k, p.groups, p.had_block, p.had_scale, flags, reinterpret_cast<void*>(stream));
     check(code, "uniql_w4a16_linear");
     return y;
 }
@@ -139,6 +140,7 @@ Tensor as_rows(const Tensor& x, int64_t columns) {
 // a layer module's forward: x [..., in_features], residual of the result's shape
 Tensor forward(Linear& p, const Tensor& x, const std::optional<Tensor>& residual, bool relu2, uintptr_t stream,
                const py::object& accumulator) {
+    const py::gil_scoped_release release;
     const at::NoGradGuard no_grad;
     if (x.dim() == 0) fail("x must have at least one dimension");
     std::optional<Tensor> res;
@@ -150,10 +152,12 @@ Tensor forward(Linear& p, const Tensor& x, const std::optional<Tensor>& residual
 
 Tensor prepared(Linear& p, const Tensor& x, const std::optional<Tensor>& residual, bool relu2, bool out_f32,
                 const std::optional<Tensor>& out, unsigned flags, uintptr_t stream, const py::object& accumulator) {
+    const py::gil_scoped_release release;
     return run(p, x, residual, relu2, out_f32, out, flags, stream, accumulator, std::nullopt);
 }
 
 Tensor embedding(const Tensor& ids_in, const Tensor& weight, const Tensor& scale, uintptr_t stream) {
+    const py::gil_scoped_release release;
     const at::NoGradGuard no_grad;
     if (weight.dim() != 2) fail("weight must be 2-D");
     require_gpu(weight, "weight");
@@ -172,18 +176,15 @@ Tensor embedding(const Tensor& ids_in, const Tensor& weight, const Tensor& scale
     std::vector<int64_t> sizes = ids.sizes().vec();
     sizes.push_back(dim);
     Tensor y = new_output(sizes, at::kHalf, ids);
-    int code;
-    {
-        const py::gil_scoped_release release;
-        code = p_embedding(ids.data_ptr<int64_t>(), ids.numel(), weight.data_ptr(), scale.data_ptr(), y.data_ptr(), vocab, (int)dim,
-                           reinterpret_cast<void*>(stream));
-    }
+    const int code = p_embedding(ids.data_ptr<int64_t>(), ids.numel(), weight.data_ptr(), scale.data_ptr(), y.data_ptr(), vocab,
+                                 (int)dim, reinterpret_cast<void*>(stream));
     check(code, "uniql_w4_embedding_lookup");
     return y;
 }
 
 // base 0: blocks of `block` values; else the composite transform of width base * 2^k.  New tensor.
 Tensor hadamard(const Tensor& x_in, int64_t block, int base, double scale, uintptr_t stream) {
+    const py::gil_scoped_release release;
     const at::NoGradGuard no_grad;
     require_gpu(x_in, "x");
     const at::ScalarType t = x_in.scalar_type();
@@ -195,12 +196,9 @@ Tensor hadamard(const Tensor& x_in, int64_t block, int base, double scale, uintp
     if (dim > 0x7fffffff || block > 0x7fffffff) fail("the last axis is too wide");
     const c10::DeviceGuard guard(x.device());
     Tensor y = at::empty_like(x);
-    int code;
-    {
-        const py::gil_scoped_release release;
-        code = base == 0 ? p_fwht(x.data_ptr(), y.data_ptr(), rows, (int)dim, (int)block, (float)scale, type, reinterpret_cast<void*>(stream))
-                         : p_composite(x.data_ptr(), y.data_ptr(), rows, (int)dim, base, (float)scale, type, reinterpret_cast<void*>(stream));
-    }
+    void* const st = reinterpret_cast<void*>(stream);
+    const int code = base == 0 ? p_fwht(x.data_ptr(), y.data_ptr(), rows, (int)dim, (int)block, (float)scale, type, st)
+                               : p_composite(x.data_ptr(), y.data_ptr(), rows, (int)dim, base, (float)scale, type, st);
     check(code, base == 0 ? "uniql_fwht" : "uniql_fwht_composite");
     return y;
 }
