@@ -236,3 +236,30 @@ def test_had_linear_weight_updated_between_forward_and_backward(gpu, fuse):
     want = before.double().sum(0)
     assert ((x.grad[0].double() - want).norm() / want.norm()).item() < 1e-5   # 128 fp32 terms: 128 x 2^-24
     assert layer.weight.grad is not None
+
+
+def test_copies_of_a_prepared_layer(gpu):
+    """a handle's copy, deep copy and pickle give its results, on tensors of their own; its fields can be read"""
+    import copy
+    import pickle
+    from uniql_amd import ops
+    from uniql_amd.quantize.quant_linear_layers import W4A16B16O16Linear
+    torch.manual_seed(11)
+    layer = W4A16B16O16Linear.from_fp16(torch.nn.Linear(384, 200, bias=True, device=gpu, dtype=torch.float16))
+    x = torch.randn(5, 384, device=gpu).half()
+    p = ops.prepare_linear(layer.weight.clone(), layer.scale.clone(), layer.workspace.clone(), 256, 384, out_features=200,
+                           bias=layer.bias.data, had_block=128, had_scale=128 ** -0.5)
+    want = ops.linear_prepared(p, x)
+    assert (p.n_out, p.size_n, p.size_k, p.groups, p.had_block, p.silu_mul) == (200, 256, 384, 3, 128, False)
+    assert torch.equal(p.B, layer.weight) and torch.equal(p.bias, layer.bias.data)
+    shallow, deep, saved = copy.copy(p), copy.deepcopy(p), pickle.dumps(p)
+    later = copy.deepcopy(deep)                       # a copy of a copy that has not run
+    assert torch.equal(ops.linear_prepared(shallow, x), want)
+    p.B.zero_()                                       # the deep copies' weights are their own
+    for q in (deep, later, pickle.loads(saved)):
+        assert torch.equal(ops.linear_prepared(q, x), want)
+    with pytest.raises(AttributeError):
+        p.nothing
+    layer(x)                                          # a layer that has run keeps no handle in its copies
+    assert "_prep" in layer.__dict__ and "_prep" not in copy.deepcopy(layer).__dict__
+    assert torch.equal(copy.copy(layer)(x), layer(x))

@@ -1,7 +1,10 @@
 """The native binding of the layer, lookup and rotation calls (csrc/host.cpp) as far as it needs no GPU."""
 import os
+import pickle
 import subprocess
 import sys
+
+import torch
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
@@ -73,3 +76,28 @@ def test_other_threads_run_while_a_call_waits():
     """the interpreter lock is given up for a call's own copies too, not only for its launch"""
     done = subprocess.run([sys.executable, "-c", OTHER_THREADS.format(root=ROOT)], capture_output=True, text=True, timeout=300)
     assert done.returncode == 0, done.stderr[-2000:]
+
+
+class _SlotsState:
+    """pickles like a PreparedLinear whose fields were slots of its own"""
+
+    def __init__(self, **fields):
+        self.fields = fields
+
+    def __reduce_ex__(self, protocol):
+        from uniql_amd.ops import PreparedLinear
+        return object.__new__, (PreparedLinear,), (None, self.fields)
+
+
+def test_earlier_pickles_of_a_handle_load():
+    """the tensors come back whatever device they are mapped to; validation waits for the first use"""
+    import copy
+    n = k = 256
+    fields = dict(B=torch.arange(k // 16 * 2 * n, dtype=torch.int32).reshape(k // 16, 2 * n), s=torch.ones(k // 128, n).half(),
+                  workspace=torch.zeros(64, dtype=torch.int32), bias=None, b_ptr=1, s_ptr=2, ws_ptr=3, ws_len=64, bias_ptr=None,
+                  size_n=n, size_k=k, n_out=200, groups=2, had_block=128, had_scale=0.25, silu_mul=False, needs={})
+    handle = pickle.loads(pickle.dumps(_SlotsState(**fields)))
+    for again in (handle, copy.copy(handle), copy.deepcopy(handle), pickle.loads(pickle.dumps(handle))):
+        state = again.__getstate__()
+        assert torch.equal(state["B"], fields["B"]) and state["n_out"] == 200 and state["had_scale"] == 0.25
+        assert "b_ptr" not in state

@@ -213,6 +213,17 @@ PYBIND11_MODULE(_host, module) {
             return Linear{std::move(B), std::move(s), std::move(workspace), std::move(bias), size_n, size_k, n_out, groups,
                           had_block, (float)had_scale, silu_mul, {}};
         }))
+        .def_readonly("B", &Linear::B)
+        .def_readonly("s", &Linear::s)
+        .def_readonly("workspace", &Linear::workspace)
+        .def_readonly("bias", &Linear::bias)
+        .def_readonly("size_n", &Linear::size_n)
+        .def_readonly("size_k", &Linear::size_k)
+        .def_readonly("n_out", &Linear::n_out)
+        .def_readonly("groups", &Linear::groups)
+        .def_readonly("had_block", &Linear::had_block)
+        .def_readonly("had_scale", &Linear::had_scale)
+        .def_readonly("silu_mul", &Linear::silu_mul)
         .def("forward", &forward)
         .def("prepared", &prepared);
     module.def("bind", &bind);

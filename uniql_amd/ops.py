@@ -219,11 +219,32 @@ def w4a16_gemm_static(A: torch.Tensor, B: torch.Tensor, s: torch.Tensor, workspa
 class PreparedLinear:
     """What a layer call needs that does not change from call to call, validated once
     (prepare_linear) and held by a native handle: the packed tensors, bias, rotation, epilogue.
-    Copies and pickles of it are None (the addresses are this process's): prepare again."""
-    __slots__ = ("host", "__weakref__")
+    Copies and pickles hold tensors of their own and are validated at their first use (the handle's addresses
+    belong to one process and one set of tensors)."""
+    _FIELDS = ("B", "s", "workspace", "bias", "size_n", "size_k", "n_out", "groups", "had_block", "had_scale", "silu_mul")
+    __slots__ = ("host", "_state", "__weakref__")
 
-    def __reduce__(self):
-        return type(None), ()
+    def __getattr__(self, name):   # only what the slots do not hold
+        if name == "host":
+            t = self._state
+            self.host = prepare_linear(t["B"], t["s"], t["workspace"], t["size_n"], t["size_k"], out_features=t["n_out"],
+                                       bias=t["bias"], silu_mul=t["silu_mul"], had_block=t["had_block"],
+                                       had_scale=t["had_scale"]).host
+            return self.host
+        if name in PreparedLinear._FIELDS:
+            return getattr(self.host, name)
+        raise AttributeError(f"PreparedLinear has no attribute {name!r}")
+
+    def __getstate__(self):
+        try:
+            return self._state
+        except AttributeError:
+            return {name: getattr(self, name) for name in PreparedLinear._FIELDS}
+
+    def __setstate__(self, state):
+        if isinstance(state, tuple):   # pickles of handles whose fields were the object's own slots
+            state = state[1]
+        self._state = {name: state[name] for name in PreparedLinear._FIELDS}
 
 
 def prepare_linear(B: torch.Tensor, s: torch.Tensor, workspace: torch.Tensor, size_n: int, size_k: int, *,

@@ -113,12 +113,19 @@ class W4A16B16O16Linear(nn.Module):
         key = (weight.data_ptr(), scale.data_ptr(), workspace.data_ptr(), None if bias is None else bias.data_ptr(),
                self.had_block, self.had_scale, self.size_n, self.size_k, self.out_features)
         cached = self.__dict__.get("_prep")
-        if cached is None or cached[0] != key or cached[1] is None:
+        if cached is None or cached[0] != key:
             prep = ops.prepare_linear(weight, scale, workspace, self.size_n, self.size_k, out_features=self.out_features,
                                       bias=None if bias is None else bias.data, had_block=self.had_block,
                                       had_scale=self.had_scale)
             cached = self.__dict__["_prep"] = (key, prep)
         return cached[1]
+
+    # copies and pickles prepare their own handle
+    def __getstate__(self):
+        return {name: value for name, value in self.__dict__.items() if name != "_prep"}
+
+    def __setstate__(self, state):
+        super().__setstate__({name: value for name, value in state.items() if name != "_prep"})
 
     def __repr__(self):
         return (f"W4A16B16O16Linear(in_features={self.in_features}, out_features={self.out_features}, "
