@@ -4,6 +4,7 @@ import pickle
 import subprocess
 import sys
 
+import pytest
 import torch
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
@@ -101,3 +102,30 @@ def test_earlier_pickles_of_a_handle_load():
         state = again.__getstate__()
         assert torch.equal(state["B"], fields["B"]) and state["n_out"] == 200 and state["had_scale"] == 0.25
         assert "b_ptr" not in state
+
+
+@pytest.mark.parametrize("missing", ["compiler", "torch"])
+def test_the_library_is_installed_without_the_binding(tmp_path, monkeypatch, missing):
+    """a build where only the binding fails leaves the new library, says so, and leaves no binding of another build"""
+    from uniql_amd import build as B
+    lib, host = tmp_path / "libuniql_amd.so", tmp_path / "_host.so"
+    lib.write_text("old")
+    host.write_text("old")
+
+    def run(cmd, verbose):
+        if cmd[0] == "g++":
+            raise RuntimeError("g++: not found")
+        open(cmd[cmd.index("-o") + 1], "w").write("new")
+
+    def no_torch(dst):
+        raise ImportError("No module named 'torch'")
+
+    monkeypatch.setattr(B, "LIB_DIR", str(tmp_path))
+    monkeypatch.setattr(B, "LIB_PATH", str(lib))
+    monkeypatch.setattr(B, "HOST_PATH", str(host))
+    monkeypatch.setattr(B, "_run", run)
+    if missing == "torch":
+        monkeypatch.setattr(B, "_host_command", no_torch)
+    with pytest.raises(RuntimeError, match="_host.so"):
+        B.build(verbose=False)
+    assert lib.read_text() == "new" and sorted(os.listdir(tmp_path)) == ["libuniql_amd.so"]

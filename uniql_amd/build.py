@@ -48,7 +48,7 @@ def _run(cmd: list[str], verbose: bool) -> None:
     noise = "is not a recognized feature for this target"
     err = "\n".join(l for l in proc.stderr.splitlines() if noise not in l)
     if proc.returncode != 0:
-        raise RuntimeError(f"hipcc failed ({proc.returncode}):\n{err}")
+        raise RuntimeError(f"{os.path.basename(cmd[0])} failed ({proc.returncode}):\n{err}")
     if verbose and err.strip():
         print(err, file=sys.stderr)
 
@@ -67,7 +67,9 @@ def _host_command(dst: str) -> list[str]:
 
 def build(verbose: bool = True, jobs: int | None = None) -> str:
     """Always recompiles every source (one hipcc per file, a few at a time, into a temporary
-    directory), links, and returns the path of the shared library."""
+    directory), links, and returns the path of the shared library.  The library needs neither torch nor
+    Python: where the binding (g++, torch's and Python's headers) cannot be built, the library is installed all the
+    same before that is reported, and a binding of an earlier build is removed."""
     import tempfile
     from concurrent.futures import ThreadPoolExecutor
     os.makedirs(LIB_DIR, exist_ok=True)
@@ -79,13 +81,19 @@ def build(verbose: bool = True, jobs: int | None = None) -> str:
         objs = [os.path.join(tmpdir, os.path.basename(src)[:-4] + ".o") for src in srcs]
         host = HOST_PATH + ".tmp"
         with ThreadPoolExecutor(max_workers=jobs) as pool:
-            host_done = pool.submit(_run, _host_command(host), verbose)
+            host_done = pool.submit(lambda: _run(_host_command(host), verbose))
             list(pool.map(lambda so: _run([hipcc, *compile_flags, f"-I{INCLUDE}", f"-I{CSRC}", "-c", so[0], "-o", so[1]],
                                           verbose), zip(srcs, objs)))
         tmp = LIB_PATH + ".tmp"
         _run([hipcc, f"--offload-arch={ARCH}", "-shared", "-fPIC", *objs, "-o", tmp], verbose)
-        host_done.result()
     os.replace(tmp, LIB_PATH)
+    try:
+        host_done.result()
+    except Exception as e:
+        for stale in (host, HOST_PATH):
+            if os.path.exists(stale):
+                os.remove(stale)
+        raise RuntimeError(f"{LIB_PATH} is built; the binding for torch, {HOST_PATH}, is not: {e}") from e
     os.replace(host, HOST_PATH)
     return LIB_PATH
 
