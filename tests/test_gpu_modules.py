@@ -263,3 +263,17 @@ def test_copies_of_a_prepared_layer(gpu):
     layer(x)                                          # a layer that has run keeps no handle in its copies
     assert "_prep" in layer.__dict__ and "_prep" not in copy.deepcopy(layer).__dict__
     assert torch.equal(copy.copy(layer)(x), layer(x))
+
+
+@pytest.mark.parametrize("fuse", [False, True])
+def test_had_linear_weight_updated_under_autocast(gpu, fuse):
+    """the product uses the weight as it is now, whatever autocast has cast before"""
+    from uniql_amd.quantize.quant_linear_layers import HadLinear
+    torch.manual_seed(6)
+    lin = torch.nn.Linear(256, 128, bias=False, device=gpu, dtype=torch.float32)
+    layer = HadLinear(lin, input_transform=fuse, fuse_had=fuse)
+    x = torch.randn(4, 256, device=gpu)
+    with torch.no_grad(), torch.autocast("cuda", dtype=torch.float16):
+        before = layer(x)
+        layer.weight.mul_(2.0)
+        assert torch.equal(layer(x), before * 2)      # a power of two: the same roundings

@@ -176,8 +176,10 @@ class HadLinear(nn.Linear):
 
     def forward(self, x):
         w = self.weight if self.fuse_had else self._rotated(self.weight)
-        if w is self.weight and torch.is_grad_enabled():
-            w = w.clone()   # a recorded product keeps its own weight: the layer's may be updated before the backward
+        if w is self.weight:
+            # a recorded product keeps its own weight: the layer's may be updated before the backward; and autocast
+            # keeps its cast of a parameter, but not of a detached weight, beyond an update
+            w = w.clone() if torch.is_grad_enabled() else w.detach()
         return F.linear(x, w, self.bias)
 
     def __repr__(self):
