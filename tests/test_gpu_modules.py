@@ -278,3 +278,16 @@ def test_had_linear_weight_updated_under_autocast(gpu, fuse):
         layer.weight.neg_()
         # the sign goes through every rounding (a factor of two would not: fp16 subnormals round differently)
         assert torch.equal(layer(x), -before)
+
+
+def test_had_linear_of_a_layer_made_in_inference_mode(gpu):
+    """a weight that is an inference tensor is wrapped outside of that mode too"""
+    from uniql_amd.quantize.quant_linear_layers import HadLinear
+    torch.manual_seed(8)
+    with torch.inference_mode():
+        lin = torch.nn.Linear(256, 128, bias=True, device=gpu, dtype=torch.float16)
+    layer = HadLinear(lin, input_transform=False)
+    x = torch.randn(4, 256, device=gpu).half()
+    with torch.no_grad():
+        assert torch.equal(layer(x), torch.nn.functional.linear(x, lin.weight, lin.bias))
+    assert layer.weight.data_ptr() == lin.weight.data_ptr() and layer.weight.requires_grad and layer.bias.requires_grad

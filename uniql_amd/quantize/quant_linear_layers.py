@@ -139,13 +139,16 @@ class HadLinear(nn.Linear):
 
     def __init__(self, originalLayer: nn.Linear, input_transform=True, output_transform=False, fuse_had=False):
         assert originalLayer.weight.is_cuda, "Hadamard transform must be on CUDA"
-        # (nn.Linear's own constructor would allocate and randomly initialise a weight that is replaced at once)
+        # (nn.Linear's own constructor would allocate and randomly initialise a weight that is replaced at once; the data
+        # is set afterwards because an inference tensor cannot become a parameter itself)
         nn.Module.__init__(self)
         self.in_features, self.out_features = originalLayer.in_features, originalLayer.out_features
-        self.weight = nn.Parameter(originalLayer.weight.data)
+        self.weight = nn.Parameter(originalLayer.weight.new_empty(0))
+        self.weight.data = originalLayer.weight.data
         if originalLayer.bias is not None:
             assert not output_transform, "Bias is not supported for output_transform"
-            self.bias = nn.Parameter(originalLayer.bias.data)
+            self.bias = nn.Parameter(originalLayer.bias.new_empty(0))
+            self.bias.data = originalLayer.bias.data
         else:
             self.register_parameter("bias", None)
         self.input_transform = input_transform
