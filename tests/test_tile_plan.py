@@ -58,6 +58,12 @@ extern "C" int plans_missed(int n, int k, int lo, int hi) {
     return missed;
 }
 
+// Rows of the first launch of a call that runs as two, 0 if it runs as one.
+extern "C" int first_of_two(int m, int n, int k) {
+    const LinearPlan plan = linear_plan(m, n, k, n % 256 == 0, (size_t)12 << 20, 0);
+    return plan.parts == 2 ? plan.part[0].rows : 0;
+}
+
 // Rows lo..hi: in how many the launch that is taken is neither the rule's nor faster than it by its expected time.
 extern "C" int rule_left_for_nothing(int n, int k, int lo, int hi) {
     int bad = 0;
@@ -101,3 +107,10 @@ def test_the_search_rates_one_and_two_quartets(plans, n):
     for k in (128, 512, 1280, 2688, 4096, 7424, 10496, 14336):
         assert plans.plans_missed(n, k, 17, 1100) == 0, (n, k)
         assert plans.rule_left_for_nothing(n, k, 17, 1100) == 0, (n, k)
+
+
+@pytest.mark.parametrize("m,k,n,head", [(1100, 4096, 28672, 1024), (1100, 14336, 4096, 1024), (1057, 11008, 4096, 1024),
+                                        (1030, 11008, 4096, 1024), (1024, 4096, 18688, 768), (128, 4096, 28672, 0)])
+def test_calls_that_run_as_two_launches(plans, m, k, n, head):
+    """the sizes at which the GPU tests of two launches look at their results do run as two"""
+    assert plans.first_of_two(m, n, k) == head

@@ -319,6 +319,7 @@ static int fwht_vec_launch(const void* x, void* y, int64_t pieces, int block, fl
 // 16 to 128 bytes, so neighbouring tiles share cache lines: the tiles of one XCD (workgroups i, i + 8, i + 16, ...) are
 // neighbours, and run at the same time, so a line is fetched and written back once per second-level cache.
 // 4096 x 14336 fp16: 98 us, against 504 us for two transposed copies (230 each) and the row transform (44).
+// Three heights: the power-of-two output widths of the projections it rotates; others go through the copies.
 __device__ __forceinline__ int fwht_pad64(int idx) { return idx + ((idx >> 6) << 2); }
 
 template <typename T, int LOG2L>
@@ -489,11 +490,12 @@ __global__ __launch_bounds__(256) void fwht_composite_kernel(const T* __restrict
     }
 }
 
-// The same for P >= 128, at the memory rate: 16-byte loads with index bits 0..2 in registers, padded LDS passes of up
+// The same for P >= 128: 16-byte loads with index bits 0..2 in registers, padded LDS passes of up
 // to four bits, then the base matrix with its signs as constants, one addition per term (the mask bits tested at run
 // time are three instructions per term, 34 us of vector time at 1024 rows of 14336 against 12 us of memory
-// time), on pairs of neighbouring columns.  1024 rows of 14336 fp16: 23 us, against 65 us of fwht_composite_kernel;
-// 4096 rows: 84 against 230.  From BASE = 20 on two halves of the workgroup take half of the
+// time), on pairs of neighbouring columns.  1024 rows of 14336 fp16: 21 us, 12 of them memory time, against 64 us of
+// fwht_composite_kernel; 4096 rows: 80 against 230.  Two rows share a compute unit's LDS; the additions wait for the
+// loads of their own row.  From BASE = 20 on two halves of the workgroup take half of the
 // outputs each (a lane would otherwise hold the only use of its SIMD for BASE^2 dependent additions).
 // The terms are added in ascending order, starting from zero, as fwht_composite_kernel does: the same bits.
 template <int BASE>

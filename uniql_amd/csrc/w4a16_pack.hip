@@ -232,12 +232,13 @@ __global__ __launch_bounds__(256) void w4a16_cut_rows_kernel(const uint32_t* __r
 }
 
 // Keeps columns of a packed matrix, as they are: kept columns are up to five runs of `units` x (`kept` of every `full`
-// columns, from `base` on: the first `split`, and the others `skip` columns further on); columns behind them have code 0, those from n_scaled on scale 0; rows from k_real on get
-// code 0.  A column's four codes of a word are two of its bytes, so nothing is unpacked: a 16-byte piece of the output
+// columns, from `base` on: the first `split`, and the others `skip` columns further on); columns behind them have code 0,
+// those from n_scaled on scale 0; rows from k_real on get code 0.  A column's four codes of a word are two of its bytes,
+// so nothing is unpacked: a 16-byte piece of the output
 // takes eight 4-byte loads and a byte selection each, or, where its 64 columns are one source chunk (a kept prefix),
 // one load.  A workgroup resolves its chunk's 64 source columns once and keeps them for `per` groups of 128 rows.
 // Bound by memory and, for the small projections, by the launch (4096 x 14336 cut to 12160, 53 MB: 12.2 us = 4.3 TB/s,
-// 1024 columns: 5.4; the seven cuts of a decoder layer with their host calls 912 -> 86 us).
+// 1024 columns: 5.2).
 struct ColumnRuns {
     int count;
     int base[5], units[5], full[5], kept[5], split[5], skip[5];
