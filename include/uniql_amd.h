@@ -87,8 +87,8 @@ int uniql_clear(void* p, size_t bytes, void* stream);
  *              concurrently need separate buffers.  May be NULL when the size is 0.
  *   temp       device, uniql_w4a16_gemm_temp_bytes(m, n, k, had_block) bytes, contents
  *              irrelevant: rotated activations whenever the rotation is not fused, and
- *              the fp32 partial tiles of the tiled kernel when its plan splits K over
- *              workgroups; may be NULL when that size is 0.  Two calls that may run
+ *              the fp32 partial tiles of the tiled kernels and of the kernel for 9 to 64 rows
+ *              when their plan splits K over workgroups; may be NULL when that size is 0.  Two calls that may run
  *              concurrently need separate buffers.
  *   had_block  0: none.  Otherwise the activations are rotated first,
  *              A <- fp16(A . H_had_block * had_scale) on consecutive
@@ -138,7 +138,7 @@ int uniql_w4a16_gemm(const void* A, int64_t lda, const void* B, const void* S, v
  * streams, or graphs replayed concurrently) race and must use uniql_w4a16_gemm with separate
  * buffers instead.
  * Before a call is recorded into a graph, one call with the same m class (1, 2, 3..4, 5..8, 9..16,
- * more), flags and rotation must have run eagerly on that device: the first call per device
+ * 17..64, more), flags and rotation must have run eagerly on that device: the first call per device
  * resolves the array's address (hipGetSymbolAddress) and the first launch of a kernel that uses
  * more than 64 KiB of LDS sets a function attribute, neither of which may happen while a stream
  * is capturing.
@@ -191,9 +191,9 @@ size_t uniql_w4a16_linear_temp_bytes(int m, int n, int k, int k_in, int had_bloc
 
 /* Sizes of `accum` and `temp` for one call with these flags (the two functions above and
  * uniql_w4a16_gemm_accum_bytes answer for flags = 0; forced kernels or tuning fields can need
- * more).  `temp` holds the rotated or zero-padded copy of the activations and, when the tiled
- * kernel splits K over workgroups, one fp32 partial tile per (output tile, split); `accum` then
- * holds one arrival count per output tile.  No counterpart in the reference, whose wrapper
+ * more).  `temp` holds the rotated or zero-padded copy of the activations and, when a kernel other than
+ * the streaming one splits K over workgroups, one fp32 partial tile per (output tile, split); `accum` then
+ * holds the arrival counts of the output tiles.  No counterpart in the reference, whose wrapper
  * allocates its reduction buffer itself (csrc/linear/marlin_gemm_kernel.cuh:1018). */
 int uniql_w4a16_linear_workspace(int m, int n, int k, int k_in, int had_block, unsigned flags,
                                  size_t* accum_bytes, size_t* temp_bytes);

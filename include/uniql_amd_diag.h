@@ -27,7 +27,8 @@ enum {
        Tiled kernels: bits 8..15 number of K splits over workgroups, bits 16..19 row tiles of 32
        per workgroup (1 to 4: the 128-column kernel; 8: the 256 x 256 kernel for long prefill,
        which needs n % 256 == 0, k >= 256 and grouped scales and otherwise leaves the call to the
-       128-column kernel), bits 20..21 wave quartets per workgroup (1 or 2). */
+       128-column kernel; 9: the kernel for 9 to 64 rows, bits 8..15 its K-groups per wavefront),
+       bits 20..21 wave quartets per workgroup (1 or 2). */
 };
 
 /*

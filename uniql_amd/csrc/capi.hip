@@ -3,6 +3,7 @@
 #include <mutex>
 
 #include "common.hpp"
+#include "mid_plan.hpp"
 #include "tile_plan.hpp"
 #include "uniql_amd_diag.h"
 
@@ -19,6 +20,9 @@ int tile_launch(const void* A, int64_t lda, const void* B, const void* S, void* 
                 size_t accum_bytes, void* part, size_t part_bytes, int m, int n, int k, int groups, const TilePlan& plan,
                 hipStream_t stream);
 bool tile_shape_ok(int m, int n, int k, int64_t ldx, const TilePlan& plan);
+int mid_launch(const void* A, int64_t lda, int k_valid, const void* B, const void* S, void* D, const Epilogue& epi, void* accum,
+               void* part, int m, int n, int k, int groups, const MidPlan& plan, hipStream_t stream);
+bool mid_shape_ok(int m, int n, int k, int64_t lda);
 int pad_rows_launch(const void* A, int64_t lda, int k_in, void* dst, int k, int m, hipStream_t stream);
 int wide_launch(const void* A, int64_t lda, const void* B, const void* S, void* D, const Epilogue& epi, int m, int n,
                 int k, int groups, hipStream_t stream);
@@ -137,10 +141,36 @@ struct LinearNeeds {
     int had_mode;
     int64_t ld_kernel;   // row stride the product kernel will see
     LinearPlan plan;     // of the tiled kernels
+    MidPlan mid[2];      // the kernel for 9 to 64 rows, where it takes a launch of the plan (upw > 0)
     size_t accum_bytes;  // rounded to 256
     size_t act_bytes;    // copy of the activations at the start of temp (rounded to 256), or 0
     size_t part_bytes;   // the tiled kernel's partial tiles behind it, or 0
 };
+// The kernel for 9 to 64 rows (w4a16_mid.hip) for one launch of a call: upw = 0 where it does not take it.
+static const MidPlan kNoMid = {0, 0, 0, 0.0};
+
+// In place of the streaming kernel: from 9 rows on that kernel's one atomic per output element and K split costs more than
+// the exchange of partial tiles, except over few columns and a long K (11840 -> 1280 at 10 rows 8.3 us there, 10.1 here) and
+// where it does not split K at all (4096 -> 28672 at 9 to 12 rows 12.9 to 13.4 us there, 13.3 to 13.5 here).  4096 -> 4096 at 16 rows 8.5 -> 7.3 us, 4096 -> 6144 9.2 -> 7.7; of 1438 drawn calls of 9
+// to 16 rows 13 % on average.  A rotation stays with the streaming kernel, which applies it while it stages the rows.
+static MidPlan mid_for_few_rows(int m, int n, int k, int had_block, unsigned flags, size_t part_cap) {
+    if (m < kMidMinRows || m > kStreamMaxM || had_block != 0 || (flags & (UNIQL_F_FORCE_SKINNY | UNIQL_F_FORCE_TILED)) || (flags >> 8) != 0)
+        return kNoMid;
+    return n / 128 < 144 && (k <= 6144 || n >= 4096) ? mid_plan(m, n, k, 0, part_cap) : kNoMid;
+}
+
+// In place of a launch of the tiled kernels, where it is expected to be faster; padded: the tiled kernels would need a
+// zero-padded copy of the rows first (2 us).  Over a short K of fewer than 12 groups the tiled kernels' expected times are the
+// better ones from 33 rows on.  Drawn calls: 17 to 32 rows 1.26 x faster on average, 33 to 48 1.17, 49 to 64 1.03.
+static MidPlan mid_for_tiles(const RowPart& part, int n, int k, bool padded, unsigned flags, size_t part_cap) {
+    if (part.rows < kMidMinRows || part.rows > kMidMaxRows) return kNoMid;
+    if (((flags >> 16) & 0xfu) == 9) return mid_plan(part.rows, n, k, (int)((flags >> 8) & 0xffu), part_cap);  // asked for
+    if (part.rows <= kStreamMaxM || (part.rows > 32 && k < 12 * 128)) return kNoMid;
+    if ((flags & UNIQL_F_FORCE_TILED) || ((flags >> 8) & 0x3fffu) != 0) return kNoMid;
+    const MidPlan p = mid_plan(part.rows, n, k, 0, part_cap);
+    return p.upw > 0 && p.us < part.tile.us + (padded ? 2.0 : 0.0) ? p : kNoMid;
+}
+
 static LinearNeeds linear_needs(int m, int n, int k, int k_in, int64_t lda, int groups, int had_block, unsigned flags,
                                 size_t part_cap = kPartialCap) {
     LinearNeeds q;
@@ -152,27 +182,62 @@ static LinearNeeds linear_needs(int m, int n, int k, int k_in, int64_t lda, int 
     // (and zero-padded) into the temporary buffer, then rotated there in place
     q.pad_first = q.rotate_first ? (k_in != k || lda != k) : (k_in != k && !q.use_stream);
     q.ld_kernel = (q.rotate_first || q.pad_first) ? (int64_t)k : lda;
-    q.act_bytes = (q.rotate_first || q.pad_first) ? round256((size_t)m * k * sizeof(half_t)) : 0;
     q.plan.parts = 0;
+    q.mid[0] = q.mid[1] = kNoMid;
+    q.accum_bytes = q.part_bytes = 0;
     if (q.use_stream) {
-        q.accum_bytes = round256(stream_accum_bytes(m, n, k));
-        q.part_bytes = 0;
+        if (mid_shape_ok(m, n, k, lda)) q.mid[0] = mid_for_few_rows(m, n, k, had_block, flags, part_cap);
+        if (q.mid[0].upw > 0) {
+            q.use_stream = false;
+            q.plan.parts = 1;
+            q.plan.part[0] = RowPart{m, false, TilePlan{}};
+        } else {
+            q.accum_bytes = round256(stream_accum_bytes(m, n, k));
+        }
     } else {
         q.plan = linear_plan(m, n, k, wide_shape_ok(m, n, k, groups, q.ld_kernel), part_cap, tune);
-        q.accum_bytes = round256(plan_accum_bytes(q.plan, n));
-        q.part_bytes = plan_part_bytes(q.plan, n);
+        const bool one = q.plan.parts == 1;
+        for (int i = 0; i < q.plan.parts; ++i)
+            if (mid_shape_ok(q.plan.part[i].rows, n, k, q.rotate_first ? k : lda))
+                q.mid[i] = mid_for_tiles(q.plan.part[i], n, k, one && q.pad_first && !q.rotate_first, flags, part_cap);
+        if (one && q.mid[0].upw > 0 && !q.rotate_first) {  // that kernel guards its own loads
+            q.pad_first = false;
+            q.ld_kernel = lda;
+        }
     }
+    for (int i = 0; i < q.plan.parts; ++i) {
+        const RowPart& part = q.plan.part[i];
+        const bool mid = q.mid[i].upw > 0;
+        const size_t acc = round256(mid ? mid_accum_bytes(n, q.mid[i]) : part.wide ? 0 : tile_accum_bytes(part.rows, n, part.tile));
+        const size_t tmp = mid ? mid_part_bytes(part.rows, n, q.mid[i]) : part.wide ? 0 : tile_part_bytes(part.rows, n, part.tile);
+        q.accum_bytes = acc > q.accum_bytes ? acc : q.accum_bytes;
+        q.part_bytes = tmp > q.part_bytes ? tmp : q.part_bytes;
+    }
+    q.act_bytes = (q.rotate_first || q.pad_first) ? round256((size_t)m * k * sizeof(half_t)) : 0;
     return q;
 }
 
-// The most the tiled kernels may ask for, whether or not the call's scales and strides let the 256 x 256 kernel take part.
-static void tiled_workspace(int m, int n, int k, unsigned tune, size_t* accum, size_t* part) {
+// The most the kernels of a call may ask for, whichever of them its scales, strides and input width let take it.
+static void call_workspace(int m, int n, int k, int had_block, unsigned flags, size_t* accum, size_t* part) {
     *accum = *part = 0;
+    auto most = [&](int rows, const MidPlan& mid) {
+        if (mid.upw == 0) return;
+        const size_t a = mid_accum_bytes(n, mid), p = mid_part_bytes(rows, n, mid);
+        *accum = a > *accum ? a : *accum;
+        *part = p > *part ? p : *part;
+    };
+    if (takes_stream_kernel(m, flags)) {
+        *accum = stream_accum_bytes(m, n, k);
+        most(m, mid_for_few_rows(m, n, k, had_block, flags, kPartialCap));
+        return;
+    }
     for (int wide = 0; wide < 2; ++wide) {
-        const LinearPlan plan = linear_plan(m, n, k, wide != 0 && wide_shape_ok(m, n, k, k / 128, k), kPartialCap, tune);
+        const LinearPlan plan = linear_plan(m, n, k, wide != 0 && wide_shape_ok(m, n, k, k / 128, k), kPartialCap, flags >> 8);
         const size_t a = plan_accum_bytes(plan, n), p = plan_part_bytes(plan, n);
         *accum = a > *accum ? a : *accum;
         *part = p > *part ? p : *part;
+        for (int i = 0; i < plan.parts; ++i)
+            for (int padded = 0; padded < 2; ++padded) most(plan.part[i].rows, mid_for_tiles(plan.part[i], n, k, padded != 0, flags, kPartialCap));
     }
 }
 
@@ -187,8 +252,8 @@ int uniql_w4a16_linear_workspace(int m, int n, int k, int k_in, int had_block, u
     const size_t act = had_block != 0 && fused_rotation(m, k, k_in, had_block, use_stream, flags) == 0
                            ? round256((size_t)m * k * sizeof(half_t))
                            : activation_copy_bytes(m, k, k_in, had_block, use_stream, flags);
-    size_t accum = stream_accum_bytes(m, n, k), part = 0;
-    if (!use_stream) tiled_workspace(m, n, k, flags >> 8, &accum, &part);
+    size_t accum, part;
+    call_workspace(m, n, k, had_block, flags, &accum, &part);
     *accum_bytes = round256(accum);
     *temp_bytes = act + round256(part);
     return UNIQL_OK;
@@ -199,7 +264,7 @@ size_t uniql_w4a16_gemm_accum_bytes(int m, int n, int k) {
     // enough for either kernel with its own plan (forced tuning fields: uniql_w4a16_linear_workspace)
     const size_t a = stream_accum_bytes(m, n, k);
     size_t b, part;
-    tiled_workspace(m, n, k, 0, &b, &part);
+    call_workspace(m, n, k, 0, 0, &b, &part);
     return round256(a > b ? a : b);
 }
 
@@ -208,8 +273,8 @@ size_t uniql_w4a16_linear_temp_bytes(int m, int n, int k, int k_in, int had_bloc
     // the copy of the activations (as if the tiled kernel took the call: the larger case) and the
     // partial tiles of the tiled kernel's own plan
     const size_t act = (had_block != 0 || k_in != k) ? round256((size_t)m * k * sizeof(half_t)) : 0;
-    size_t accum = 0, part = 0;
-    if (!takes_stream_kernel(m, 0)) tiled_workspace(m, n, k, 0, &accum, &part);
+    size_t accum, part;
+    call_workspace(m, n, k, had_block, 0, &accum, &part);
     return act + round256(part);
 }
 
@@ -265,7 +330,7 @@ static int linear_impl(const void* A, int64_t lda, int k_in, const void* B, cons
     void* part = part_bytes ? reinterpret_cast<char*>(temp) + act_bytes : nullptr;
     // last check before the first kernel is enqueued: whether the tiled kernel can take the shape
     for (int i = 0; i < q.plan.parts; ++i)
-        if (!q.plan.part[i].wide && !tile_shape_ok(q.plan.part[i].rows, n, k, ld_kernel, q.plan.part[i].tile)) return UNIQL_E_SHAPE;
+        if (!q.plan.part[i].wide && q.mid[i].upw == 0 && !tile_shape_ok(q.plan.part[i].rows, n, k, ld_kernel, q.plan.part[i].tile)) return UNIQL_E_SHAPE;
     if (use_stream && !stream_shape_ok(k, ld_kernel)) return UNIQL_E_SHAPE;
     if (check_only) return UNIQL_OK;
     if (pad_first) {
@@ -300,7 +365,9 @@ static int linear_impl(const void* A, int64_t lda, int k_in, const void* B, cons
         const char* x = reinterpret_cast<const char*>(Ain) + (size_t)m0 * ld * sizeof(half_t);
         char* d = reinterpret_cast<char*>(D) + (size_t)m0 * (transpose ? 1 : ldd) * (out_f32 ? 4 : 2);
         epi.residual = residual ? reinterpret_cast<const half_t*>(residual) + (size_t)m0 * ldr : nullptr;
-        const int e = p.wide ? wide_launch(x, ld, B, S, d, epi, p.rows, n, k, groups, st)
+        const int e = q.mid[i].upw > 0
+                          ? mid_launch(x, ld, k_valid, B, S, d, epi, accum, part, p.rows, n, k, groups, q.mid[i], st)
+                      : p.wide ? wide_launch(x, ld, B, S, d, epi, p.rows, n, k, groups, st)
                                : tile_launch(x, ld, B, S, d, epi, accum, accum_bytes, part, part_bytes, p.rows, n, k, groups, p.tile, st);
         if (e != UNIQL_OK) return e;
         m0 += p.rows;
