@@ -1,0 +1,36 @@
+"""Composite widths: workgroups that take several rows one after the other, and rows that hold infinities or NaN."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+# widths of one, two, four and eight chunks of 128 values; more rows than the chip holds workgroups, an odd number of them
+@pytest.mark.parametrize("dim,base,rows", [(1536, 12, 3001), (3072, 12, 1401), (3584, 28, 1501), (5120, 40, 1157), (10240, 20, 781),
+                                           (14336, 28, 1103), (28672, 28, 523), (20480, 40, 517)])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
+def test_rows_behind_the_first(gpu, dim, base, rows, dtype):
+    """a row's result does not depend on how many rows the call has or which comes before it"""
+    from uniql_amd import ops
+    gen = torch.Generator(device=gpu).manual_seed(dim)
+    x = torch.randn((rows, dim), device=gpu, generator=gen).to(dtype)
+    y = ops.hadamard_composite(x, dim ** -0.5, base)
+    for first in (0, 250, rows - 200):
+        assert torch.equal(y[first:first + 200], ops.hadamard_composite(x[first:first + 200].clone(), dim ** -0.5, base))
+    # rows that are not on the 16-byte grid take the kernel that moves single values
+    odd = torch.empty(64 * dim + 1, dtype=dtype, device=gpu)[1:].view(64, dim)
+    odd.copy_(x[rows - 64:])
+    assert torch.equal(ops.hadamard_composite(odd, dim ** -0.5, base), y[rows - 64:])
+
+
+@pytest.mark.parametrize("dim,base", [(3584, 28), (5120, 40)])
+def test_infinities_and_nan_stay_in_their_row(gpu, dim, base):
+    from uniql_amd import ops
+    x = torch.randn((1200, dim), device=gpu, generator=torch.Generator(device=gpu).manual_seed(1)).half()
+    clean = ops.hadamard_composite(x, dim ** -0.5, base)
+    x[1, 3], x[600, 7], x[1199, dim - 1] = float("nan"), float("inf"), float("-inf")
+    y = ops.hadamard_composite(x, dim ** -0.5, base)
+    hit = torch.zeros(1200, dtype=torch.bool, device=gpu)
+    hit[[1, 600, 1199]] = True
+    assert torch.isnan(y[1]).all() and not torch.isfinite(y[600]).any() and not torch.isfinite(y[1199]).any()
+    assert torch.equal(y[~hit], clean[~hit])

@@ -1,6 +1,7 @@
 // Walsh-Hadamard transform of fp16 / bf16 / fp32 rows: y = T((x . H_block) * scale), H the
 // Sylvester (natural-order) matrix, applied to consecutive `block`-wide pieces.
 // Butterflies run in fp32, lowest index bit first, one rounding to T at the end.
+#include <algorithm>
 #include <atomic>
 
 #include "common.hpp"
@@ -18,6 +19,10 @@ template <>
 struct RowIo<half_t> {
     struct Raw { u32x4 a; };
     static __device__ __forceinline__ Raw load(const half_t* p) { return Raw{*reinterpret_cast<const u32x4*>(p)}; }
+    static __device__ __forceinline__ Raw load(__amdgpu_buffer_rsrc_t rsrc, unsigned bytes) {
+        return Raw{__builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rsrc, bytes, 0, 0))};
+    }
+    static __device__ __forceinline__ void settle(Raw& r) { asm volatile("" : "+v"(r.a)); }
     static __device__ __forceinline__ void unpack(const Raw& r, float (&f)[8]) {
 #pragma unroll
         for (int p = 0; p < 4; ++p) {
@@ -44,6 +49,10 @@ template <>
 struct RowIo<__bf16> {
     struct Raw { u32x4 a; };
     static __device__ __forceinline__ Raw load(const __bf16* p) { return Raw{*reinterpret_cast<const u32x4*>(p)}; }
+    static __device__ __forceinline__ Raw load(__amdgpu_buffer_rsrc_t rsrc, unsigned bytes) {
+        return Raw{__builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rsrc, bytes, 0, 0))};
+    }
+    static __device__ __forceinline__ void settle(Raw& r) { asm volatile("" : "+v"(r.a)); }
     static __device__ __forceinline__ void unpack(const Raw& r, float (&f)[8]) {
 #pragma unroll
         for (int p = 0; p < 4; ++p) {
@@ -71,6 +80,11 @@ struct RowIo<float> {
     static __device__ __forceinline__ Raw load(const float* p) {
         return Raw{*reinterpret_cast<const f4*>(p), *reinterpret_cast<const f4*>(p + 4)};
     }
+    static __device__ __forceinline__ Raw load(__amdgpu_buffer_rsrc_t rsrc, unsigned bytes) {
+        return Raw{__builtin_bit_cast(f4, __builtin_amdgcn_raw_buffer_load_b128(rsrc, bytes, 0, 0)),
+                   __builtin_bit_cast(f4, __builtin_amdgcn_raw_buffer_load_b128(rsrc, bytes + 16, 0, 0))};
+    }
+    static __device__ __forceinline__ void settle(Raw& r) { asm volatile("" : "+v"(r.a), "+v"(r.b)); }
     static __device__ __forceinline__ void unpack(const Raw& r, float (&f)[8]) {
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
@@ -490,14 +504,16 @@ __global__ __launch_bounds__(256) void fwht_composite_kernel(const T* __restrict
     }
 }
 
-// The same for P >= 128: 16-byte loads with index bits 0..2 in registers, padded LDS passes of up
-// to four bits, then the base matrix with its signs as constants, one addition per term (the mask bits tested at run
-// time are three instructions per term, 34 us of vector time at 1024 rows of 14336 against 12 us of memory
-// time), on pairs of neighbouring columns.  1024 rows of 14336 fp16: 21 us, 12 of them memory time, against 64 us of
-// fwht_composite_kernel; 4096 rows: 80 against 230.  Two rows share a compute unit's LDS; the additions wait for the
-// loads of their own row.  From BASE = 20 on two halves of the workgroup take half of the
-// outputs each (a lane would otherwise hold the only use of its SIMD for BASE^2 dependent additions).
-// The terms are added in ascending order, starting from zero, as fwht_composite_kernel does: the same bits.
+// The same for P >= 128.  A wave transforms blocks of 512 consecutive values (whole chunks, or a half or quarter of one) by
+// itself: 16-byte loads and index bits 0..2 in registers, bits 3..5 and 6..8 in two LDS passes without a workgroup barrier;
+// chunks of more than 512 values have one or two bits left for the workgroup.  Then the base matrix across the chunks with
+// its signs as constants, one addition per term, on pairs of neighbouring columns; the terms are added in ascending
+// order, starting from zero, as fwht_composite_kernel does: the same bits.
+// What bounds it: the additions, BASE for every value (a SIMD takes a plain fp32 addition in two clocks; the matrix unit's
+// fp32 forms, tried, hold the vector unit up for as long as the additions take), about as long as the memory time, and at
+// most two rows of 14336 in a compute unit's LDS.  So the workgroups stay, and request their next row before they
+// transform the current one.  fp16, against one row a workgroup with a barrier behind every pass: 1024 rows of 14336 20.9
+// -> 18.7 us, 4096 rows 72 -> 67; 1024 rows of 3584 8.3 -> 7.5, of 5120 (40 x 128) 13.6 -> 10.7, one row of 14336 6.9 -> 6.2.
 template <int BASE>
 struct BaseTable;
 template <> struct BaseTable<12> { static constexpr const uint64_t (&mask)[12] = kHadamard12; };
@@ -524,44 +540,116 @@ __device__ __forceinline__ void base_outputs(const float2 (&z)[BASE], T* yp, int
     }
 }
 
+// Barriers that order LDS alone: loads from and stores to memory stay in flight.
+__device__ __forceinline__ void lds_barrier() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+__device__ __forceinline__ void lds_wave_fence() {  // a wave's LDS operations complete in issue order
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
+}
+
+// Eight floats of padding per 64: the 64 lanes of either pass touch every bank once.
+__device__ __forceinline__ int fwht_pad8of64(int idx) { return idx + ((idx >> 6) << 3); }
+
 template <typename T, int BASE>
-__global__ __launch_bounds__(512) void fwht_composite_vec_kernel(const T* __restrict__ x, T* __restrict__ y, int P, int log2P,
-                                                                float scale) {
+__global__ __launch_bounds__(512, BASE == 40 ? 3 : 4) void fwht_composite_vec_kernel(const T* __restrict__ x, T* __restrict__ y, int rows, int P, int log2P,
+                                                                   float scale) {
     extern __shared__ __attribute__((aligned(16))) float fbuf[];
-    const int tid = threadIdx.x, nthreads = blockDim.x;
-    const int L = BASE * P, chunks = L >> 3;
-    const T* xp = x + (size_t)blockIdx.x * L;
-    T* yp = y + (size_t)blockIdx.x * L;
-    constexpr int kAhead = 4;  // chunks requested before the first is used
-    for (int c0 = tid; c0 < chunks; c0 += kAhead * nthreads) {
-        typename RowIo<T>::Raw v[kAhead];
+    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), W = blockDim.x >> 6;
+    const int L = BASE * P, blocks = L >> 9;  // BASE is a multiple of four, P of 128
+    constexpr int kAhead = sizeof(T) == 4 ? 2 : 4;  // blocks of a wave requested together
+    typename RowIo<T>::Raw v[kAhead];
+    // Always kAhead loads; blocks and rows that do not exist lie beyond the descriptor.
+    auto request = [&](int row, int first) __attribute__((always_inline)) {
+        const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(
+            const_cast<T*>(x + (size_t)(row < rows ? row : 0) * L), 0, row < rows ? (unsigned)(L * sizeof(T)) : 0u, 0x00020000);
 #pragma unroll
-        for (int i = 0; i < kAhead; ++i)
-            if (c0 + i * nthreads < chunks) v[i] = RowIo<T>::load(xp + 8 * (c0 + i * nthreads));
+        for (int i = 0; i < kAhead; ++i) v[i] = RowIo<T>::load(rsrc, (unsigned)((512 * (first + W * i) + 8 * lane) * sizeof(T)));
+    };
+    auto transform = [&](int first) __attribute__((always_inline)) {
 #pragma unroll
         for (int i = 0; i < kAhead; ++i) {
-            const int c = c0 + i * nthreads;
-            if (c >= chunks) break;
+            const int block = first + W * i;
+            if (block >= blocks) break;  // uniform
+            float* buf = fbuf + 576 * block;
             float f[8];
             RowIo<T>::unpack(v[i], f);
             wht8(f);
-            float* dst = fbuf + fwht_pad(8 * c);
-            *reinterpret_cast<f4*>(dst) = f4{f[0], f[1], f[2], f[3]};
-            *reinterpret_cast<f4*>(dst + 4) = f4{f[4], f[5], f[6], f[7]};
-        }
-    }
-    __syncthreads();
-    fwht_passes_from_bit3(fbuf, 1, 0, L, log2P, tid, nthreads);
-    constexpr int kHalves = BASE >= 20 ? 2 : 1;
-    const int pairs = P >> 1;  // a multiple of 64: a wave's lanes share the half
-    for (int item = tid; item < kHalves * pairs; item += nthreads) {
-        const int half = __builtin_amdgcn_readfirstlane(item >= pairs ? 1 : 0);
-        const int i = 2 * (item - half * pairs);
-        float2 z[BASE];
+            float* d0 = buf + fwht_pad8of64(8 * lane);
+            *reinterpret_cast<f4*>(d0) = f4{f[0], f[1], f[2], f[3]};
+            *reinterpret_cast<f4*>(d0 + 4) = f4{f[4], f[5], f[6], f[7]};
+            lds_wave_fence();
+            float* d1 = buf + 72 * (lane >> 3) + (lane & 7);
 #pragma unroll
-        for (int c = 0; c < BASE; ++c) z[c] = *reinterpret_cast<const float2*>(fbuf + fwht_pad(c * P + i));
-        if (half == 0) base_outputs<T, BASE, 0, BASE / kHalves>(z, yp + i, P, scale);
-        else base_outputs<T, BASE, BASE / kHalves, BASE>(z, yp + i, P, scale);
+            for (int e = 0; e < 8; ++e) f[e] = d1[8 * e];
+            wht8(f);
+#pragma unroll
+            for (int e = 0; e < 8; ++e) d1[8 * e] = f[e];
+            lds_wave_fence();
+            float* d2 = buf + lane;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) f[e] = d2[72 * e];
+#pragma unroll
+            for (int h = 1; h < 8; h <<= 1) {
+                if ((64 << (h >> 1)) >= P) break;  // bits 6, 7, 8 of the chunk, as far as it has them
+#pragma unroll
+                for (int e = 0; e < 8; ++e)
+                    if ((e & h) == 0) {
+                        const float p = f[e], q = f[e + h];
+                        f[e] = p + q;
+                        f[e + h] = p - q;
+                    }
+            }
+#pragma unroll
+            for (int e = 0; e < 8; ++e) d2[72 * e] = f[e];
+        }
+    };
+    // quarters of the outputs of 128 columns, in order, an equal share to every wave
+    const int tasks = P >> 5, t0 = w * tasks / W, t1 = (w + 1) * tasks / W;
+    int row = blockIdx.x;
+    request(row, w);
+    while (true) {
+        transform(w);
+        for (int first = w + W * kAhead; first < blocks; first += W * kAhead) {
+            request(row, first);
+            transform(first);
+        }
+        const int next = row + gridDim.x;
+        request(next, w);
+        lds_barrier();
+        for (int bit = 9; bit < log2P; ++bit) {
+#pragma unroll 4
+            for (int t = threadIdx.x; t < L >> 1; t += blockDim.x) {
+                const int at = ((t >> bit) << (bit + 1)) | (t & ((1 << bit) - 1));
+                float *p = fbuf + fwht_pad8of64(at), *q = p + (9 << (bit - 3));
+                const float a = *p, b = *q;
+                *p = a + b;
+                *q = a - b;
+            }
+            lds_barrier();
+        }
+        for (int set = t0 >> 2; 4 * set < t1; ++set) {
+            float2 z[BASE];
+            const float* src = fbuf + 144 * set + fwht_pad8of64(2 * lane);
+#pragma unroll
+            for (int c = 0; c < BASE; ++c) z[c] = *reinterpret_cast<const float2*>(src + c * (P + (P >> 3)));
+            // the next row has arrived by now; waited for behind the stores, it would be waited for with them
+#pragma unroll
+            for (int i = 0; i < kAhead; ++i) RowIo<T>::settle(v[i]);
+            T* yp = y + (size_t)row * L + 128 * set + 2 * lane;
+            auto mine = [&](int quarter) { return 4 * set + quarter >= t0 && 4 * set + quarter < t1; };  // uniform
+            if (mine(0)) base_outputs<T, BASE, 0, BASE / 4>(z, yp, P, scale);
+            if (mine(1)) base_outputs<T, BASE, BASE / 4, BASE / 2>(z, yp, P, scale);
+            if (mine(2)) base_outputs<T, BASE, BASE / 2, BASE * 3 / 4>(z, yp, P, scale);
+            if (mine(3)) base_outputs<T, BASE, BASE * 3 / 4, BASE>(z, yp, P, scale);
+        }
+        if (next >= rows) break;
+        row = next;
+        lds_barrier();  // the next row overwrites what other waves may still be reading
     }
 }
 
@@ -576,13 +664,17 @@ static int fwht_composite_go(const void* x, void* y, int64_t rows, int P, float 
     int log2P = 0;
     while ((1 << log2P) < P) ++log2P;
     const int L = BASE * P;
-    const size_t padded = (size_t)(L + (L >> 7) * 8) * sizeof(float);
-    if (P >= 128 && padded <= 160 * 1024 && rows_aligned(x, y)) {
+    const size_t image = (size_t)(L + (L >> 3)) * sizeof(float);
+    if (P >= 128 && image <= 160 * 1024 && rows_aligned(x, y)) {
         static std::atomic<unsigned long long> done{0};
-        if (!allow_lds(&fwht_composite_vec_kernel<T, BASE>, padded, done)) return UNIQL_E_LAUNCH;
-        const int threads = P >= 512 ? 512 : 256;
-        hipLaunchKernelGGL((fwht_composite_vec_kernel<T, BASE>), dim3((unsigned)rows), dim3(threads), padded, stream,
-                           reinterpret_cast<const T*>(x), reinterpret_cast<T*>(y), P, log2P, scale);
+        if (!allow_lds(&fwht_composite_vec_kernel<T, BASE>, image, done)) return UNIQL_E_LAUNCH;
+        // few waves where a row gives them little to do: several small workgroups instead (10240 = 40 x 256 at 4096 rows
+        // 56 us with four waves, 71 with eight)
+        const int waves = BASE == 12 ? (P == 128 ? 2 : P <= 512 ? 4 : 8) : P == 128 || (BASE == 40 && P == 256) ? 4 : 8;
+        // the workgroups that the chip holds at once: registers for sixteen waves a compute unit, LDS
+        const int64_t resident = 256 * std::min<int64_t>((BASE == 12 ? 20 : BASE == 40 ? 12 : 16) / waves, (int64_t)(160 * 1024 / image));
+        hipLaunchKernelGGL((fwht_composite_vec_kernel<T, BASE>), dim3((unsigned)std::min(rows, resident)), dim3(64 * waves), image, stream,
+                           reinterpret_cast<const T*>(x), reinterpret_cast<T*>(y), (int)rows, P, log2P, scale);
         return hipGetLastError() == hipSuccess ? UNIQL_OK : UNIQL_E_LAUNCH;
     }
     const size_t shmem = (size_t)L * sizeof(float);
