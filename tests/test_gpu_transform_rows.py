@@ -1,4 +1,5 @@
-"""Composite widths: workgroups that take several rows one after the other, and rows that hold infinities or NaN."""
+"""Transforms: workgroups that take several rows of a composite width one after the other, rows that hold infinities or NaN,
+and every tile width of the column transform."""
 import pytest
 import torch
 
@@ -34,3 +35,19 @@ def test_infinities_and_nan_stay_in_their_row(gpu, dim, base):
     hit[[1, 600, 1199]] = True
     assert torch.isnan(y[1]).all() and not torch.isfinite(y[600]).any() and not torch.isfinite(y[1199]).any()
     assert torch.equal(y[~hit], clean[~hit])
+
+
+# every tile width: four, eight and sixteen waves, at the edges of the rules that choose them; a last tile that is cut
+@pytest.mark.parametrize("rows,cols,dtype", [(1024, 4096, torch.float16), (1024, 8184, torch.float16), (1024, 8200, torch.bfloat16),
+                                             (2048, 4104, torch.float16), (4096, 4088, torch.float32), (4096, 4104, torch.float32),
+                                             (4096, 264, torch.float32), (2048, 8, torch.float32)])
+def test_column_tiles(gpu, rows, cols, dtype):
+    """bit for bit the row transform between two transposed copies; an infinity stays in its column"""
+    from uniql_amd import ops
+    x = torch.randn((rows, cols), device=gpu, generator=torch.Generator(device=gpu).manual_seed(cols)).to(dtype)
+    x[5, cols - 3] = float("inf")
+    y = ops.hadamard_columns(x, rows ** -0.5)
+    want = ops.hadamard_blockwise(x.t().contiguous(), rows ** -0.5, rows).t()
+    clean = torch.arange(cols, device=gpu) != cols - 3
+    assert torch.equal(y[:, clean], want[:, clean])
+    assert not torch.isfinite(y[:, cols - 3]).any()

@@ -40,6 +40,9 @@ struct RowIo<half_t> {
     static __device__ __forceinline__ void store2(half_t* p, float a, float b, float scale) {
         *reinterpret_cast<uint32_t*>(p) = pair(a, b, scale);
     }
+    static __device__ __forceinline__ void store4(half_t* p, f4 f, float scale) {
+        *reinterpret_cast<uint2*>(p) = make_uint2(pair(f[0], f[1], scale), pair(f[2], f[3], scale));
+    }
     static __device__ __forceinline__ void store8(half_t* p, const float (&f)[8], float scale) {
         *reinterpret_cast<u32x4*>(p) =
             u32x4{pair(f[0], f[1], scale), pair(f[2], f[3], scale), pair(f[4], f[5], scale), pair(f[6], f[7], scale)};
@@ -69,6 +72,9 @@ struct RowIo<__bf16> {
     static __device__ __forceinline__ void store2(__bf16* p, float a, float b, float scale) {
         *reinterpret_cast<uint32_t*>(p) = pair(a, b, scale);
     }
+    static __device__ __forceinline__ void store4(__bf16* p, f4 f, float scale) {
+        *reinterpret_cast<uint2*>(p) = make_uint2(pair(f[0], f[1], scale), pair(f[2], f[3], scale));
+    }
     static __device__ __forceinline__ void store8(__bf16* p, const float (&f)[8], float scale) {
         *reinterpret_cast<u32x4*>(p) =
             u32x4{pair(f[0], f[1], scale), pair(f[2], f[3], scale), pair(f[4], f[5], scale), pair(f[6], f[7], scale)};
@@ -95,6 +101,7 @@ struct RowIo<float> {
     static __device__ __forceinline__ void store2(float* p, float a, float b, float scale) {
         *reinterpret_cast<float2*>(p) = make_float2(a * scale, b * scale);
     }
+    static __device__ __forceinline__ void store4(float* p, f4 f, float scale) { *reinterpret_cast<f4*>(p) = f * scale; }
     static __device__ __forceinline__ void store8(float* p, const float (&f)[8], float scale) {
         *reinterpret_cast<f4*>(p) = f4{f[0] * scale, f[1] * scale, f[2] * scale, f[3] * scale};
         *reinterpret_cast<f4*>(p + 4) = f4{f[4] * scale, f[5] * scale, f[6] * scale, f[7] * scale};
@@ -322,124 +329,176 @@ static int fwht_vec_launch(const void* x, void* y, int64_t pieces, int block, fl
     return UNIQL_OK;
 }
 
+// Barriers that order LDS alone: loads from and stores to memory stay in flight.
+__device__ __forceinline__ void lds_barrier() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+__device__ __forceinline__ void lds_wave_fence() {  // a wave's LDS operations complete in issue order
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
+}
+
+// Eight floats of padding per 64: the 64 lanes of either pass touch every bank once.
+__device__ __forceinline__ int fwht_pad8of64(int idx) { return idx + ((idx >> 6) << 3); }
+
+// Index bits 3..5 of 512 values that lie eight to a lane, in an LDS pass: on entry f holds values 8 piece .. (bits 0..2 done,
+// every piece on one lane), behind it f[e] is value lane + 64 e.  buf: 576 floats of the wave's own.
+__device__ __forceinline__ void wht512_pass3(float* buf, int piece, int lane, float (&f)[8]) {
+    float* d0 = buf + fwht_pad8of64(8 * piece);
+    *reinterpret_cast<f4*>(d0) = f4{f[0], f[1], f[2], f[3]};
+    *reinterpret_cast<f4*>(d0 + 4) = f4{f[4], f[5], f[6], f[7]};
+    lds_wave_fence();
+    float* d1 = buf + 72 * (lane >> 3) + (lane & 7);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) f[e] = d1[8 * e];
+    wht8(f);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) d1[8 * e] = f[e];
+    lds_wave_fence();
+#pragma unroll
+    for (int e = 0; e < 8; ++e) f[e] = buf[lane + 72 * e];
+}
+// Bits 6.. of f[e] as far as a chunk of P values has them.
+__device__ __forceinline__ void wht512_upper(float (&f)[8], int P) {
+#pragma unroll
+    for (int b = 0; b < 3; ++b) {
+        if ((64 << b) >= P) break;
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+            if ((e & (1 << b)) == 0) {
+                const float p = f[e], q = f[e + (1 << b)];
+                f[e] = p + q;
+                f[e + (1 << b)] = p - q;
+            }
+    }
+}
+
 // ---- down the columns of a row-major matrix: y = T((H_L . x) * scale), L = 1024, 2048 or 4096 rows ------------
 // The output side of a weight rotation without the two transposed copies around the row transform.  A workgroup
-// takes 32768 / L neighbouring columns over all rows as one fp32 image in LDS (136 KB with its padding: four floats
-// per 64), so that a value is read and written once:
-//   load    a thread reads eight consecutive rows x eight columns (16 bytes of fp16 per row): index bits 0..2;
-//   middle  bits 3 .. n-5, one column of 2^(n-7) rows per task;
-//   final   the top four bits of two neighbouring columns, scaled, rounded and stored.
-// Same butterfly order as the row transform: the same values as transposing twice.  A row of a tile is only
-// 16 to 128 bytes, so neighbouring tiles share cache lines: the tiles of one XCD (workgroups i, i + 8, i + 16, ...) are
-// neighbours, and run at the same time, so a line is fetched and written back once per second-level cache.
-// 4096 x 14336 fp16: 98 us, against 504 us for two transposed copies (230 each) and the row transform (44).
+// takes 4096 WAVES / L neighbouring columns over all rows, 64 values a thread, and reads and writes a value once:
+//   load    a thread reads eight consecutive rows x eight columns (16 bytes of fp16 per row), neighbouring lanes the
+//           neighbouring columns of a row: index bits 0..2;
+//   wave    the next bits lie inside a wave: column by column through a few KB of LDS, no workgroup barrier;
+//   last    the remaining bits lie across the waves: half of the values at a time through LDS, scaled, rounded, stored.
+// Same butterfly order as the row transform: the same values as transposing twice.  Neighbouring tiles share cache lines: the
+// tiles of one XCD (workgroups i, i + 8, i + 16, ...) are neighbours, and run at the same time, so a line is fetched and
+// written back once per second-level cache.
+// What bounds it: the second-level cache's requests, one for every 16 to 64 bytes of a row that a tile is wide (4096 x 14336
+// fp16 as 8 columns a tile: 14.7 M of them, 55 us of the caches' request rate), and load, passes and store following each
+// other inside a workgroup; so tiles are wide, and
+// two workgroups share a compute unit where a tile has eight waves.  fp16, cold, against one workgroup of 136 KB and 4-byte
+// stores: 4096 x 14336 125 -> 101 us, 4096 x 4096 29 -> 25, 1024 x 14336 20.5 -> 17.1.
 // Three heights: the power-of-two output widths of the projections it rotates; others go through the copies.
-__device__ __forceinline__ int fwht_pad64(int idx) { return idx + ((idx >> 6) << 2); }
+template <int LOG2L, int WAVES>
+struct ColumnTile {
+    static constexpr int kColumns = (4096 * WAVES) >> LOG2L;
+    static constexpr int CB = (WAVES == 16 ? 4 : WAVES == 8 ? 3 : 2) + 9 - LOG2L;  // log2 of the chunks of eight columns
+    static constexpr int kRowsInWave = 512 >> CB;
+    // the last exchange, half of a wave's values: 64 << kRowBits rows x kHalfChunks chunks
+    static constexpr int kRowBits = CB < 2 ? 2 - CB : 0, kHalfChunks = CB < 2 ? 1 << CB : 4;
+    static constexpr int kStride = WAVES * 8 * kHalfChunks + 4;  // floats per row
+    static constexpr size_t kPasses = WAVES * 4 * 576 * sizeof(float), kLast = (size_t)(64 << kRowBits) * kStride * sizeof(float);
+    static constexpr size_t kBytes = kPasses > kLast ? kPasses : kLast;
+};
 
-template <typename T, int LOG2L>
-__global__ __launch_bounds__(512) void fwht_columns_kernel(const T* __restrict__ x, T* __restrict__ y, int cols, int tiles, float scale) {
+template <typename T, int LOG2L, int WAVES>
+__global__ __launch_bounds__(64 * WAVES, 4) void fwht_columns_kernel(const T* __restrict__ x, T* __restrict__ y, int cols, int tiles, float scale) {
     extern __shared__ __attribute__((aligned(16))) float fbuf[];
-    constexpr int L = 1 << LOG2L, CT = 32768 >> LOG2L, LOG2CT = 15 - LOG2L, CHUNKS = CT / 8;
-    const int tid = threadIdx.x;
+    using Tile = ColumnTile<LOG2L, WAVES>;
+    constexpr int CB = Tile::CB, RIW = Tile::kRowsInWave, RB = Tile::kRowBits, HC = Tile::kHalfChunks;
+    const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int per_xcd = (tiles + 7) >> 3;
     const int tile = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
     if (tile >= tiles) return;  // uniform
-    const int col0 = tile * CT;
+    const int col0 = tile * Tile::kColumns;
+    const int chunk = lane & ((1 << CB) - 1), rows8 = lane >> CB;
+    float f[8][8];  // [row, later what the wave's passes leave][column]
     {
-        const int chunk = tid & (CHUNKS - 1), row0 = (tid / CHUNKS) * 8;
-        const bool real = col0 + 8 * chunk < cols;  // cols is a multiple of eight: a chunk exists or it does not
         typename RowIo<T>::Raw raw[8];
-        if (real) {
+        // (cols is a multiple of eight: a chunk exists or it does not, and then stands in for the tile's first)
+        const int col = col0 + 8 * chunk < cols ? col0 + 8 * chunk : col0;
+        const T* src = x + (size_t)(RIW * w + 8 * rows8) * cols + col;
 #pragma unroll
-            for (int i = 0; i < 8; ++i) raw[i] = RowIo<T>::load(x + (size_t)(row0 + i) * cols + col0 + 8 * chunk);
-            float f[8][8];
+        for (int i = 0; i < 8; ++i) raw[i] = RowIo<T>::load(src + (size_t)i * cols);
 #pragma unroll
-            for (int i = 0; i < 8; ++i) RowIo<T>::unpack(raw[i], f[i]);
-#pragma unroll
-            for (int h = 1; h < 8; h <<= 1)
-#pragma unroll
-                for (int i = 0; i < 8; ++i)
-                    if ((i & h) == 0) {
-#pragma unroll
-                        for (int e = 0; e < 8; ++e) {
-                            const float p = f[i][e], q = f[i + h][e];
-                            f[i][e] = p + q;
-                            f[i + h][e] = p - q;
-                        }
-                    }
-#pragma unroll
-            for (int i = 0; i < 8; ++i) {
-                float* dst = fbuf + fwht_pad64((row0 + i) * CT + 8 * chunk);
-                *reinterpret_cast<f4*>(dst) = f4{f[i][0], f[i][1], f[i][2], f[i][3]};
-                *reinterpret_cast<f4*>(dst + 4) = f4{f[i][4], f[i][5], f[i][6], f[i][7]};
-            }
-        }
+        for (int i = 0; i < 8; ++i) RowIo<T>::unpack(raw[i], f[i]);
     }
-    __syncthreads();
-    {
-        constexpr int PB = LOG2L - 7, E = 1 << PB, LO = 3;
-        constexpr int LOWS = 8 * CT;  // (row bits 0..2, column): one run of consecutive floats
+    // A wave's values of column e of every chunk: chunk by chunk RIW rows, 512 in all.
+    float* own = fbuf + w * (4 * 576);
+    const int piece = (chunk << (6 - CB)) | rows8;
 #pragma unroll
-        for (int task = tid; task < 32768 / E; task += 512) {
-            const int low = task & (LOWS - 1), high = task / LOWS;  // high: row bits LO + PB ..
-            const int base = (high << (LO + PB + LOG2CT)) + low;
-            float v[E];
+    for (int e0 = 0; e0 < 8; e0 += 4) {
 #pragma unroll
-            for (int i = 0; i < E; ++i) v[i] = fbuf[fwht_pad64(base + (i << (LO + LOG2CT)))];
+        for (int e = e0; e < e0 + 4; ++e) {
+            float g[8];
 #pragma unroll
-            for (int h = 1; h < E; h <<= 1)
+            for (int i = 0; i < 8; ++i) g[i] = f[i][e];
+            wht8(g);
+            wht512_pass3(own + (e - e0) * 576, piece, lane, g);
+            wht512_upper(g, RIW);
 #pragma unroll
-                for (int i = 0; i < E; ++i)
-                    if ((i & h) == 0) {
-                        const float p = v[i], q = v[i + h];
-                        v[i] = p + q;
-                        v[i + h] = p - q;
-                    }
-#pragma unroll
-            for (int i = 0; i < E; ++i) fbuf[fwht_pad64(base + (i << (LO + LOG2CT)))] = v[i];
+            for (int i = 0; i < 8; ++i) f[i][e] = g[i];
         }
+        lds_wave_fence();
     }
-    __syncthreads();
-    {
-        constexpr int LO = LOG2L - 4;
+    // f[k][e]: value lane + 64 k.  The halves: rows with bit 6 clear and set, or, where k counts eight chunks, four of them each.
 #pragma unroll
-        for (int task = tid; task < 1024; task += 512) {
-            const int c = 2 * (task & (CT / 2 - 1)), row = task / (CT / 2);  // row bits 0 .. LO - 1
+    for (int half = 0; half < 2; ++half) {
+        lds_barrier();
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const float (&r)[8] = f[CB < 3 ? 2 * q + half : 4 * half + q];
+            float* dst = fbuf + (lane + 64 * (q & ((1 << RB) - 1))) * Tile::kStride + (w * HC + (q >> RB)) * 8;
+            *reinterpret_cast<f4*>(dst) = f4{r[0], r[1], r[2], r[3]};
+            *reinterpret_cast<f4*>(dst + 4) = f4{r[4], r[5], r[6], r[7]};
+        }
+        lds_barrier();
+        // an item: a row, four columns; 512 of them in a half (sixteen waves: the halves go to one half of the threads each)
+        for (int item = WAVES == 16 ? tid - 512 * half : tid; item >= 0 && item < 512; item += 64 * WAVES) {
+            const int quad = item & (2 * HC - 1), at = item / (2 * HC);
+            const int c = 4 * quad + (CB < 3 ? 0 : 32 * half);
             if (col0 + c >= cols) continue;
-            float a[16], b[16];
+            f4 v[WAVES];
 #pragma unroll
-            for (int i = 0; i < 16; ++i) {
-                const float2 v = *reinterpret_cast<const float2*>(fbuf + fwht_pad64(((i << LO) + row) * CT + c));
-                a[i] = v.x;
-                b[i] = v.y;
-            }
+            for (int r = 0; r < WAVES; ++r) v[r] = *reinterpret_cast<const f4*>(fbuf + at * Tile::kStride + r * 8 * HC + 4 * quad);
 #pragma unroll
-            for (int h = 1; h < 16; h <<= 1)
+            for (int h = 1; h < WAVES; h <<= 1)
 #pragma unroll
-                for (int i = 0; i < 16; ++i)
-                    if ((i & h) == 0) {
-                        const float p = a[i], q = a[i + h], r = b[i], t = b[i + h];
-                        a[i] = p + q;
-                        a[i + h] = p - q;
-                        b[i] = r + t;
-                        b[i + h] = r - t;
+                for (int r = 0; r < WAVES; ++r)
+                    if ((r & h) == 0) {
+                        const f4 p = v[r], q = v[r + h];
+                        v[r] = p + q;
+                        v[r + h] = p - q;
                     }
+            const int row = CB < 3 ? (at & 63) + 64 * half + 128 * (at >> 6) : at;
+            T* out = y + (size_t)row * cols + col0 + c;
 #pragma unroll
-            for (int i = 0; i < 16; ++i) RowIo<T>::store2(y + (size_t)((i << LO) + row) * cols + col0 + c, a[i], b[i], scale);
+            for (int r = 0; r < WAVES; ++r) RowIo<T>::store4(out + (size_t)(RIW * r) * cols, v[r], scale);
         }
     }
 }
 
-template <typename T, int LOG2L>
-static int fwht_columns_go(const void* x, void* y, int cols, float scale, hipStream_t stream) {
-    constexpr int CT = 32768 >> LOG2L;
-    constexpr size_t shmem = (32768 + 32768 / 16) * sizeof(float);
+template <typename T, int LOG2L, int WAVES>
+static int fwht_columns_tiles(const void* x, void* y, int cols, float scale, hipStream_t stream) {
+    using Tile = ColumnTile<LOG2L, WAVES>;
     static std::atomic<unsigned long long> done{0};
-    if (!allow_lds(&fwht_columns_kernel<T, LOG2L>, shmem, done)) return UNIQL_E_LAUNCH;
-    const int tiles = (cols + CT - 1) / CT;
-    hipLaunchKernelGGL((fwht_columns_kernel<T, LOG2L>), dim3((unsigned)((tiles + 7) / 8 * 8)), dim3(512), shmem, stream,
+    if (!allow_lds(&fwht_columns_kernel<T, LOG2L, WAVES>, Tile::kBytes, done)) return UNIQL_E_LAUNCH;
+    const int tiles = (cols + Tile::kColumns - 1) / Tile::kColumns;
+    hipLaunchKernelGGL((fwht_columns_kernel<T, LOG2L, WAVES>), dim3((unsigned)((tiles + 7) / 8 * 8)), dim3(64 * WAVES), Tile::kBytes, stream,
                        reinterpret_cast<const T*>(x), reinterpret_cast<T*>(y), cols, tiles, scale);
     return hipGetLastError() == hipSuccess ? UNIQL_OK : UNIQL_E_LAUNCH;
+}
+template <typename T, int LOG2L>
+static int fwht_columns_go(const void* x, void* y, int cols, float scale, hipStream_t stream) {
+    // The widest tiles of which every compute unit gets one: eight waves, two workgroups a compute unit; sixteen for fp32
+    // over 4096 rows, where eight columns are a full sector and only one workgroup's stores fit beside the other's loads
+    // (4096 x 14336: 150 us against 165; fp16 102 either way); four for few columns of 1024 rows (x 4096: 8.5 us against 9.3).
+    if (LOG2L == 12 && sizeof(T) == 4 && cols >= 256 * ColumnTile<LOG2L, 16>::kColumns) return fwht_columns_tiles<T, LOG2L, LOG2L == 12 && sizeof(T) == 4 ? 16 : 8>(x, y, cols, scale, stream);
+    if (LOG2L == 10 && cols < 256 * ColumnTile<LOG2L, 8>::kColumns) return fwht_columns_tiles<T, LOG2L, LOG2L == 10 ? 4 : 8>(x, y, cols, scale, stream);
+    return fwht_columns_tiles<T, LOG2L, 8>(x, y, cols, scale, stream);
 }
 template <typename T>
 static int fwht_columns_rows(const void* x, void* y, int rows, int cols, float scale, hipStream_t stream) {
@@ -540,21 +599,6 @@ __device__ __forceinline__ void base_outputs(const float2 (&z)[BASE], T* yp, int
     }
 }
 
-// Barriers that order LDS alone: loads from and stores to memory stay in flight.
-__device__ __forceinline__ void lds_barrier() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-    __builtin_amdgcn_s_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-}
-__device__ __forceinline__ void lds_wave_fence() {  // a wave's LDS operations complete in issue order
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
-}
-
-// Eight floats of padding per 64: the 64 lanes of either pass touch every bank once.
-__device__ __forceinline__ int fwht_pad8of64(int idx) { return idx + ((idx >> 6) << 3); }
-
 template <typename T, int BASE>
 __global__ __launch_bounds__(512, BASE == 40 ? 3 : 4) void fwht_composite_vec_kernel(const T* __restrict__ x, T* __restrict__ y, int rows, int P, int log2P,
                                                                    float scale) {
@@ -579,33 +623,10 @@ __global__ __launch_bounds__(512, BASE == 40 ? 3 : 4) void fwht_composite_vec_ke
             float f[8];
             RowIo<T>::unpack(v[i], f);
             wht8(f);
-            float* d0 = buf + fwht_pad8of64(8 * lane);
-            *reinterpret_cast<f4*>(d0) = f4{f[0], f[1], f[2], f[3]};
-            *reinterpret_cast<f4*>(d0 + 4) = f4{f[4], f[5], f[6], f[7]};
-            lds_wave_fence();
-            float* d1 = buf + 72 * (lane >> 3) + (lane & 7);
+            wht512_pass3(buf, lane, lane, f);
+            wht512_upper(f, P);
 #pragma unroll
-            for (int e = 0; e < 8; ++e) f[e] = d1[8 * e];
-            wht8(f);
-#pragma unroll
-            for (int e = 0; e < 8; ++e) d1[8 * e] = f[e];
-            lds_wave_fence();
-            float* d2 = buf + lane;
-#pragma unroll
-            for (int e = 0; e < 8; ++e) f[e] = d2[72 * e];
-#pragma unroll
-            for (int h = 1; h < 8; h <<= 1) {
-                if ((64 << (h >> 1)) >= P) break;  // bits 6, 7, 8 of the chunk, as far as it has them
-#pragma unroll
-                for (int e = 0; e < 8; ++e)
-                    if ((e & h) == 0) {
-                        const float p = f[e], q = f[e + h];
-                        f[e] = p + q;
-                        f[e + h] = p - q;
-                    }
-            }
-#pragma unroll
-            for (int e = 0; e < 8; ++e) d2[72 * e] = f[e];
+            for (int e = 0; e < 8; ++e) buf[lane + 72 * e] = f[e];
         }
     };
     // quarters of the outputs of 128 columns, in order, an equal share to every wave
