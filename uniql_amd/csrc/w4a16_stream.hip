@@ -246,7 +246,7 @@ void w4a16_stream_kernel(const StreamArgs a) {
         // zero: 2^-10 <= s < 2^-4.  The low pairs' products are summed apart (acc_low) and enter the
         // result times 16 at the end: a power of two, exact in fp32.  9 vector instructions per packed
         // word (a shift, four ANDs, four FMAs) instead of 13.  A lane checks its eight scales; if any
-        // lane of the wave finds one outside the range (or zero: padding columns, empty groups), the
+        // lane of the wave finds one outside the range, the
         // whole wave expands this unit the long way (mask-and-or into [1024, 1040), subtract, multiply:
         // exact for every scale), into the same accumulators.
         //
@@ -259,13 +259,28 @@ void w4a16_stream_kernel(const StreamArgs a) {
             const uint32_t t = scales[j] - 0x14001400u;
             out_of_range |= t | (t + 0x08000800u);
         }
-        const bool lane_ok = (out_of_range & 0xE000E000u) == 0;
-        if (__builtin_expect(__builtin_amdgcn_ballot_w64(!lane_ok) == 0ull, 1)) {
+        // Scales of zero (padding columns, empty groups) are taken out of that check when it fails: their
+        // weights come out as zeros once s 2^20 is one.  From 3 rows on, as the exit of padding strips (a pruned decoder
+        // layer at 8 rows 46.9 -> 45.8 us); with one or two rows the kernel waits for memory either way, and what the
+        // two add to its code costs a layer at one row 0.2 to 0.4 us of 37.7.
+        uint32_t not_zero[4] = {~0u, ~0u, ~0u, ~0u};
+        bool short_form = __builtin_amdgcn_ballot_w64((out_of_range & 0xE000E000u) != 0) == 0ull;
+        if (RC > 2 && __builtin_expect(!short_form, 0)) {
+            out_of_range = 0;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                not_zero[j] = ((((scales[j] & 0x7fff7fffu) + 0x7fff7fffu) >> 15) & 0x00010001u) * 0xffffu;
+                const uint32_t t = ((scales[j] & not_zero[j]) | (0x14001400u & ~not_zero[j])) - 0x14001400u;
+                out_of_range |= t | (t + 0x08000800u);
+            }
+            short_form = __builtin_amdgcn_ballot_w64((out_of_range & 0xE000E000u) != 0) == 0ull;
+        }
+        if (__builtin_expect(short_form, 1)) {
             h2 s20[4], c_high[4], c_low[4];
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
                 const h2 pr = bits_to_h2(scales[j]);
-                s20[j] = bits_to_h2(scales[j] + 0x50005000u);  // exponents + 20 (both are normal and stay in range)
+                s20[j] = bits_to_h2((scales[j] + 0x50005000u) & not_zero[j]);  // exponents + 20 (normal, and stay in range)
                 c_high[j] = pr * h2{(half_t)-8.0f, (half_t)-8.0f};
                 c_low[j] = pr * h2{(half_t)-0.5f, (half_t)-0.5f};
             }
@@ -341,6 +356,8 @@ void w4a16_stream_kernel(const StreamArgs a) {
     // the first group's loads leave before anything else is decided (a wave without groups asks
     // for the last group and ignores it)
     issue_loads(g_begin < a.G ? g_begin : a.G - 1, set_a);
+    // a strip of nothing but padding columns (the whole workgroup; behind the first loads, so that the entry stays one block)
+    if (EXT && RC > 2 && (a.epi.gated ? 64 : 128) * strip >= a.epi.n_store) return;
     if (a.per_column) {  // uniform, rare
         uint32_t t[4];
 #pragma unroll
