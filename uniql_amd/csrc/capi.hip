@@ -17,15 +17,15 @@ bool stream_shape_ok(int k, int64_t lda);
 int read_floor_launch(const void* B, const void* S, void* sink, int m, int n, int k, unsigned tune, hipStream_t stream);
 size_t read_floor_sink_bytes(int m, int n, int k, unsigned tune);
 int tile_launch(const void* A, int64_t lda, const void* B, const void* S, void* D, const Epilogue& epi, void* accum,
-                size_t accum_bytes, void* part, size_t part_bytes, int m, int n, int k, int groups, const TilePlan& plan,
-                hipStream_t stream);
-bool tile_shape_ok(int m, int n, int k, int64_t ldx, const TilePlan& plan);
+                size_t accum_bytes, void* part, size_t part_bytes, int m, int n, int k, int groups, int first, int columns,
+                const TilePlan& plan, hipStream_t stream);
+bool tile_shape_ok(int m, int n, int k, int64_t ldx, int columns, const TilePlan& plan);
 int mid_launch(const void* A, int64_t lda, int k_valid, const void* B, const void* S, void* D, const Epilogue& epi, void* accum,
                void* part, int m, int n, int k, int groups, const MidPlan& plan, hipStream_t stream);
 bool mid_shape_ok(int m, int n, int k, int64_t lda);
 int pad_rows_launch(const void* A, int64_t lda, int k_in, void* dst, int k, int m, hipStream_t stream);
 int wide_launch(const void* A, int64_t lda, const void* B, const void* S, void* D, const Epilogue& epi, int m, int n,
-                int k, int groups, hipStream_t stream);
+                int k, int groups, int first, int columns, hipStream_t stream);
 bool wide_shape_ok(int m, int n, int k, int groups, int64_t ldx);
 int dequant_launch(const void* B, const void* S, void* W, uint8_t* codes, int n, int k, int groups,
                    hipStream_t stream);
@@ -182,7 +182,7 @@ static LinearNeeds linear_needs(int m, int n, int k, int k_in, int64_t lda, int 
     // (and zero-padded) into the temporary buffer, then rotated there in place
     q.pad_first = q.rotate_first ? (k_in != k || lda != k) : (k_in != k && !q.use_stream);
     q.ld_kernel = (q.rotate_first || q.pad_first) ? (int64_t)k : lda;
-    q.plan.parts = 0;
+    q.plan.parts = q.plan.head_columns = 0;
     q.mid[0] = q.mid[1] = kNoMid;
     q.accum_bytes = q.part_bytes = 0;
     if (q.use_stream) {
@@ -195,10 +195,10 @@ static LinearNeeds linear_needs(int m, int n, int k, int k_in, int64_t lda, int 
             q.accum_bytes = round256(stream_accum_bytes(m, n, k));
         }
     } else {
-        q.plan = linear_plan(m, n, k, wide_shape_ok(m, n, k, groups, q.ld_kernel), part_cap, tune);
+        q.plan = call_plan(m, n, k, wide_shape_ok(m, n & ~255, k, groups, q.ld_kernel), part_cap, tune);
         const bool one = q.plan.parts == 1;
         for (int i = 0; i < q.plan.parts; ++i)
-            if (mid_shape_ok(q.plan.part[i].rows, n, k, q.rotate_first ? k : lda))
+            if (q.plan.head_columns == 0 && mid_shape_ok(q.plan.part[i].rows, n, k, q.rotate_first ? k : lda))
                 q.mid[i] = mid_for_tiles(q.plan.part[i], n, k, one && q.pad_first && !q.rotate_first, flags, part_cap);
         if (one && q.mid[0].upw > 0 && !q.rotate_first) {  // that kernel guards its own loads
             q.pad_first = false;
@@ -208,8 +208,9 @@ static LinearNeeds linear_needs(int m, int n, int k, int k_in, int64_t lda, int 
     for (int i = 0; i < q.plan.parts; ++i) {
         const RowPart& part = q.plan.part[i];
         const bool mid = q.mid[i].upw > 0;
-        const size_t acc = round256(mid ? mid_accum_bytes(n, q.mid[i]) : part.wide ? 0 : tile_accum_bytes(part.rows, n, part.tile));
-        const size_t tmp = mid ? mid_part_bytes(part.rows, n, q.mid[i]) : part.wide ? 0 : tile_part_bytes(part.rows, n, part.tile);
+        const int columns = part_columns(q.plan, i, n);
+        const size_t acc = round256(mid ? mid_accum_bytes(n, q.mid[i]) : part.wide ? 0 : tile_accum_bytes(part.rows, columns, part.tile));
+        const size_t tmp = mid ? mid_part_bytes(part.rows, n, q.mid[i]) : part.wide ? 0 : tile_part_bytes(part.rows, columns, part.tile);
         q.accum_bytes = acc > q.accum_bytes ? acc : q.accum_bytes;
         q.part_bytes = tmp > q.part_bytes ? tmp : q.part_bytes;
     }
@@ -232,7 +233,7 @@ static void call_workspace(int m, int n, int k, int had_block, unsigned flags, s
         return;
     }
     for (int wide = 0; wide < 2; ++wide) {
-        const LinearPlan plan = linear_plan(m, n, k, wide != 0 && wide_shape_ok(m, n, k, k / 128, k), kPartialCap, flags >> 8);
+        const LinearPlan plan = call_plan(m, n, k, wide != 0 && wide_shape_ok(m, n & ~255, k, k / 128, k), kPartialCap, flags >> 8);
         const size_t a = plan_accum_bytes(plan, n), p = plan_part_bytes(plan, n);
         *accum = a > *accum ? a : *accum;
         *part = p > *part ? p : *part;
@@ -330,7 +331,8 @@ static int linear_impl(const void* A, int64_t lda, int k_in, const void* B, cons
     void* part = part_bytes ? reinterpret_cast<char*>(temp) + act_bytes : nullptr;
     // last check before the first kernel is enqueued: whether the tiled kernel can take the shape
     for (int i = 0; i < q.plan.parts; ++i)
-        if (!q.plan.part[i].wide && q.mid[i].upw == 0 && !tile_shape_ok(q.plan.part[i].rows, n, k, ld_kernel, q.plan.part[i].tile)) return UNIQL_E_SHAPE;
+        if (!q.plan.part[i].wide && q.mid[i].upw == 0 && !tile_shape_ok(q.plan.part[i].rows, n, k, ld_kernel, part_columns(q.plan, i, n), q.plan.part[i].tile))
+            return UNIQL_E_SHAPE;
     if (use_stream && !stream_shape_ok(k, ld_kernel)) return UNIQL_E_SHAPE;
     if (check_only) return UNIQL_OK;
     if (pad_first) {
@@ -359,18 +361,20 @@ static int linear_impl(const void* A, int64_t lda, int k_in, const void* B, cons
     epi.vec_ok = (!transpose && ldd % 8 == 0 && aligned16(D)) ? 1 : 0;
     if (use_stream)
         return stream_launch(Ain, ld, k_valid, B, S, D, epi, accum, m, n, k, groups, had_mode, had_scale, tune, st);
-    int m0 = 0;
+    int m0 = 0, first = 0;
     for (int i = 0; i < q.plan.parts; ++i) {
+        const int columns = part_columns(q.plan, i, n);
         const RowPart& p = q.plan.part[i];
         const char* x = reinterpret_cast<const char*>(Ain) + (size_t)m0 * ld * sizeof(half_t);
         char* d = reinterpret_cast<char*>(D) + (size_t)m0 * (transpose ? 1 : ldd) * (out_f32 ? 4 : 2);
         epi.residual = residual ? reinterpret_cast<const half_t*>(residual) + (size_t)m0 * ldr : nullptr;
         const int e = q.mid[i].upw > 0
                           ? mid_launch(x, ld, k_valid, B, S, d, epi, accum, part, p.rows, n, k, groups, q.mid[i], st)
-                      : p.wide ? wide_launch(x, ld, B, S, d, epi, p.rows, n, k, groups, st)
-                               : tile_launch(x, ld, B, S, d, epi, accum, accum_bytes, part, part_bytes, p.rows, n, k, groups, p.tile, st);
+                      : p.wide ? wide_launch(x, ld, B, S, d, epi, p.rows, n, k, groups, first, columns, st)
+                               : tile_launch(x, ld, B, S, d, epi, accum, accum_bytes, part, part_bytes, p.rows, n, k, groups, first, columns, p.tile, st);
         if (e != UNIQL_OK) return e;
-        m0 += p.rows;
+        if (q.plan.head_columns == 0) m0 += p.rows;
+        else first += columns;
     }
     return UNIQL_OK;
 }

@@ -108,7 +108,7 @@ static inline TilePlan tile_plan(int m, int n, int k, int splits_override, int m
     return best;
 }
 
-// How the tiled kernels run the rows of a call: one launch, or two over consecutive rows.
+// How the tiled kernels run a call: one launch, or two over consecutive rows or columns.
 struct RowPart {
     int rows;
     bool wide;      // the 256 x 256 kernel; `tile` then only carries the expected time
@@ -117,7 +117,11 @@ struct RowPart {
 struct LinearPlan {
     int parts;
     RowPart part[2];
+    int head_columns;  // 0: two parts are consecutive rows; else all rows, the first of them over so many columns
 };
+static inline int part_columns(const LinearPlan& plan, int i, int n) {
+    return plan.head_columns == 0 ? n : (i == 0 ? plan.head_columns : n - plan.head_columns);
+}
 
 // The plan for m rows in one launch by the order of the tile heights alone.  In
 // units of the time one 128-row workgroup takes for its K loop when every compute unit has one: 128 rows 1 per started
@@ -185,6 +189,7 @@ static inline RowPart best_launch(int m, int n, int k, bool wide_ok, size_t part
 static inline LinearPlan linear_plan(int m, int n, int k, bool wide_ok, size_t part_cap, unsigned tune) {
     LinearPlan plan;
     plan.parts = 1;
+    plan.head_columns = 0;
     if ((tune & 0x3fffu) != 0) {
         const int rows = (int)((tune >> 8) & 0xfu);
         plan.part[0] = RowPart{m, rows == 8 && wide_ok,
@@ -208,10 +213,47 @@ static inline LinearPlan linear_plan(int m, int n, int k, bool wide_ok, size_t p
     }
     return plan;
 }
+
+// The same with the columns in two launches, where that is expected to be faster by a margin: first as many as fill whole
+// rounds of the 256 x 256 kernel or of 128-row tiles, then the rest on whatever suits it.  4096 -> 18688 at 1024 rows is 292
+// of the large tiles, 36 more than a round: 256 of them over 16384 columns and 96-row tiles over the other 2304 take 145 us
+// (768 rows of large tiles, then 256 rows of 64-row ones: 161).  Of 1100 drawn calls
+// of more than 64 rows 110 run so, 0.99 to 1.35 x as fast, 1.11 on average; with a margin of 3 % in place of 5 one in ten
+// of them was up to 2 % slower.  wide_ok: whether the 256 x 256 kernel can take the largest multiple of 256 columns;
+// n itself may be an odd number of strips (2048 -> 21376 at 2997 rows 326 -> 247).  Up to 64 rows the columns are one launch.
+static inline LinearPlan call_plan(int m, int n, int k, bool wide_ok, size_t part_cap, unsigned tune) {
+    LinearPlan plan = linear_plan(m, n, k, wide_ok && n % 256 == 0, part_cap, tune);
+    if ((tune & 0x3fffu) != 0 || m <= 64) return plan;
+    double us = plan.part[0].tile.us + (plan.parts == 2 ? plan.part[1].tile.us + 2.0 : 0.0);
+    const int wide_rows = (m + 255) / 256, tall_rows = (m + 127) / 128;
+    const int wide_columns = 256 * (int)((int64_t)wide_rows * (n / 256) / 256 * 256 / wide_rows);
+    const int tall_columns = 128 * (int)((int64_t)tall_rows * (n / 128) / 256 * 256 / tall_rows);
+    // One launch of large tiles whose last round is a third full and more ends sooner than expected (its workgroups
+    // start as the compute units become free, at a higher clock: 4096 -> 6144 at 4096 rows 189 us, 213 expected, 192 in two).
+    const int rest = (int)((int64_t)wide_rows * (n / 256) % 256);
+    const double gain = plan.parts == 1 && plan.part[0].wide && rest >= 96 ? 0.88 : 0.95;
+    const int columns[3] = {wide_ok ? wide_columns : 0, tall_columns, wide_ok && n % 256 != 0 ? n - 128 : 0};
+    for (int i = 0; i < 3; ++i) {
+        const int c = columns[i];
+        if (c <= 0 || c >= n) continue;
+        const RowPart head = best_launch(m, c, k, wide_ok && c % 256 == 0, part_cap);
+        if (head.tile.us + 2.0 >= us) continue;
+        const RowPart tail = best_launch(m, n - c, k, wide_ok && (n - c) % 256 == 0, part_cap);
+        const double both = head.tile.us + tail.tile.us + 2.0;
+        if (both < gain * us) {
+            us = both / gain;
+            plan.parts = 2;
+            plan.part[0] = head;
+            plan.part[1] = tail;
+            plan.head_columns = c;
+        }
+    }
+    return plan;
+}
 static inline size_t plan_accum_bytes(const LinearPlan& plan, int n) {
     size_t most = 0;
     for (int i = 0; i < plan.parts; ++i) {
-        const size_t b = plan.part[i].wide ? 0 : tile_accum_bytes(plan.part[i].rows, n, plan.part[i].tile);
+        const size_t b = plan.part[i].wide ? 0 : tile_accum_bytes(plan.part[i].rows, part_columns(plan, i, n), plan.part[i].tile);
         most = b > most ? b : most;
     }
     return most;
@@ -219,7 +261,7 @@ static inline size_t plan_accum_bytes(const LinearPlan& plan, int n) {
 static inline size_t plan_part_bytes(const LinearPlan& plan, int n) {
     size_t most = 0;
     for (int i = 0; i < plan.parts; ++i) {
-        const size_t b = plan.part[i].wide ? 0 : tile_part_bytes(plan.part[i].rows, n, plan.part[i].tile);
+        const size_t b = plan.part[i].wide ? 0 : tile_part_bytes(plan.part[i].rows, part_columns(plan, i, n), plan.part[i].tile);
         most = b > most ? b : most;
     }
     return most;

@@ -58,6 +58,8 @@ struct TileArgs {
     int gps;          // K groups per split
     int splits;
     int mblocks;      // ceil(M / (32 MT))
+    int strip0;       // first 128-column strip of the launch, and how many
+    int strips;
     Epilogue epi;
 };
 
@@ -144,9 +146,9 @@ __global__ __launch_bounds__(256 * KW, 1) void w4a16_tile_kernel(const TileArgs 
     const int dkq = lane >> 4;
 
     // tile coordinates: strips vary fastest so that neighbouring workgroups share X rows
-    const int nstrips = a.N >> 7;
+    const int nstrips = a.strips;
     int id = blockIdx.x;
-    const int strip = id % nstrips;
+    const int strip_of_launch = id % nstrips, strip = a.strip0 + strip_of_launch;
     id /= nstrips;
     const int mblock = id % a.mblocks;
     const int split = id / a.mblocks;
@@ -449,7 +451,7 @@ __global__ __launch_bounds__(256 * KW, 1) void w4a16_tile_kernel(const TileArgs 
     // A slot holds the tile as 512 MT units of (row, 8 columns); unit u of M tile mt (row u / 16,
     // columns 8 (u % 16)..) is the four words ((mt UPT + u / T) 4 + i) T + u % T, i = 0..3, with
     // T the workgroup's thread count: the thread that reduces a unit writes it, lane after lane.
-    const int tile = mblock * nstrips + strip;
+    const int tile = mblock * nstrips + strip_of_launch;
     constexpr int T = 256 * KW, UPT = 512 / T, kSlotWords = ROWS * 64;
     unsigned long long* part_tile =
         split_k ? reinterpret_cast<unsigned long long*>(a.part) + (size_t)tile * a.splits * kSlotWords : nullptr;
@@ -559,8 +561,8 @@ __global__ __launch_bounds__(256 * KW, 1) void w4a16_tile_kernel(const TileArgs 
 // Whether tile_launch can take the call: grid size, and the 32-bit offsets of the loads (128 rows of
 // ldx elements, 2 bytes each, and the packed weights must stay below 2^32 bytes).  Checked by the entry point
 // before anything is enqueued.
-bool tile_shape_ok(int m, int n, int k, int64_t ldx, const TilePlan& plan) {
-    const int64_t grid = (int64_t)(n / 128) * ceil_div_i(m, 32 * plan.mtiles) * plan.splits;
+bool tile_shape_ok(int m, int n, int k, int64_t ldx, int columns, const TilePlan& plan) {
+    const int64_t grid = (int64_t)(columns / 128) * ceil_div_i(m, 32 * plan.mtiles) * plan.splits;
     return grid <= 0x7fffffffLL && ldx < (1LL << 24) && (int64_t)k * n / 2 < (1LL << 32);
 }
 
@@ -589,11 +591,13 @@ static hipError_t tile_launch_ext(const TileArgs& a, bool ext, int grid, hipStre
     return ext ? tile_launch_one<MT, true, KW>(a, grid, stream) : tile_launch_one<MT, false, KW>(a, grid, stream);
 }
 
+// columns first .. first + columns - 1 of the layer's n
 int tile_launch(const void* A, int64_t lda, const void* B, const void* S, void* D, const Epilogue& epi, void* accum,
-                size_t accum_bytes, void* part, size_t part_bytes, int m, int n, int k, int groups, const TilePlan& plan,
-                hipStream_t stream) {
-    if (plan.splits > 1 && (!accum || accum_bytes < tile_accum_bytes(m, n, plan) || !part ||
-                            part_bytes < tile_part_bytes(m, n, plan)))
+                size_t accum_bytes, void* part, size_t part_bytes, int m, int n, int k, int groups, int first, int columns,
+                const TilePlan& plan, hipStream_t stream) {
+    if (first % 128 != 0 || first + columns > n) return UNIQL_E_SHAPE;
+    if (plan.splits > 1 && (!accum || accum_bytes < tile_accum_bytes(m, columns, plan) || !part ||
+                            part_bytes < tile_part_bytes(m, columns, plan)))
         return UNIQL_E_WORKSPACE;
     TileArgs a;
     a.part = reinterpret_cast<float*>(part);
@@ -611,8 +615,10 @@ int tile_launch(const void* A, int64_t lda, const void* B, const void* S, void* 
     a.gps = plan.gps;
     a.splits = plan.splits;
     a.mblocks = ceil_div_i(m, 32 * plan.mtiles);
+    a.strip0 = first / 128;
+    a.strips = columns / 128;
     a.epi = epi;
-    const int64_t grid = (int64_t)(n / 128) * a.mblocks * a.splits;
+    const int64_t grid = (int64_t)a.strips * a.mblocks * a.splits;
     if (grid > 0x7fffffffLL) return UNIQL_E_SHAPE;
     hipError_t e;
     const bool ext = epi.gated || epi.bias || epi.residual || epi.relu2 || epi.transpose || epi.n_store != n ||

@@ -73,6 +73,7 @@ struct WideArgs {
     int64_t ldx;
     int M, N, K;
     int mblocks;  // ceil(M / 256)
+    int first;    // first column of the launch (multiple of 128)
     Epilogue epi;
 };
 
@@ -118,7 +119,7 @@ __global__ __launch_bounds__(256, 1) void w4a16_wide_kernel(const WideArgs a) {
     // column block's codes are fetched from memory once
     const int mblock = blockIdx.x % a.mblocks;
     const int nblock = blockIdx.x / a.mblocks;
-    const int m0 = mblock * 256, n0 = nblock * 256;
+    const int m0 = mblock * 256, n0 = a.first + nblock * 256;
     const int ngroups = a.K >> 7;
     const int N4 = a.N >> 1;  // 16-byte pieces per packed row
 
@@ -501,9 +502,10 @@ static hipError_t wide_launch_one(const WideArgs& a, int grid, hipStream_t strea
     return hipGetLastError();
 }
 
+// columns first .. first + columns - 1 of the layer's n
 int wide_launch(const void* A, int64_t lda, const void* B, const void* S, void* D, const Epilogue& epi, int m, int n,
-                int k, int groups, hipStream_t stream) {
-    if (!wide_shape_ok(m, n, k, groups, lda)) return UNIQL_E_SHAPE;
+                int k, int groups, int first, int columns, hipStream_t stream) {
+    if (first % 128 != 0 || first + columns > n || !wide_shape_ok(m, columns, k, groups, lda) || (int64_t)k * n / 2 >= (1LL << 32)) return UNIQL_E_SHAPE;
     WideArgs a;
     a.B = reinterpret_cast<const u32x4*>(B);
     a.S = reinterpret_cast<const half_t*>(S);
@@ -514,8 +516,9 @@ int wide_launch(const void* A, int64_t lda, const void* B, const void* S, void* 
     a.N = n;
     a.K = k;
     a.mblocks = (m + 255) / 256;
+    a.first = first;
     a.epi = epi;
-    const int grid = (n / 256) * a.mblocks;
+    const int grid = (columns / 256) * a.mblocks;
     const hipError_t e = wide_launch_one(a, grid, stream);
     return e == hipSuccess ? UNIQL_OK : UNIQL_E_LAUNCH;
 }
