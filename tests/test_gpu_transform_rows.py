@@ -1,5 +1,5 @@
-"""Transforms: workgroups that take several rows of a composite width one after the other, rows that hold infinities or NaN,
-and every tile width of the column transform."""
+"""Transforms: workgroups that take several rows of a composite or power-of-two width one after the other, rows that hold
+infinities or NaN, and every tile width of the column transform."""
 import pytest
 import torch
 
@@ -22,6 +22,27 @@ def test_rows_behind_the_first(gpu, dim, base, rows, dtype):
     odd = torch.empty(64 * dim + 1, dtype=dtype, device=gpu)[1:].view(64, dim)
     odd.copy_(x[rows - 64:])
     assert torch.equal(ops.hadamard_composite(odd, dim ** -0.5, base), y[rows - 64:])
+
+
+# one to sixteen waves' worth of blocks; more rows than the chip holds workgroups, an odd number of them
+@pytest.mark.parametrize("dim,rows", [(1024, 4397), (2048, 2301), (4096, 2305), (8192, 1101), (16384, 577), (32768, 301)])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
+def test_power_of_two_rows(gpu, dim, rows, dtype):
+    """a row's result does not depend on how many rows the call has, which comes before it, or whether it
+    starts on the 16-byte grid; an infinity stays in its row"""
+    from uniql_amd import ops
+    gen = torch.Generator(device=gpu).manual_seed(dim)
+    x = torch.randn((rows, dim), device=gpu, generator=gen).to(dtype)
+    y = ops.hadamard_blockwise(x, dim ** -0.5, dim)
+    for first in (0, 250, rows - 50):
+        assert torch.equal(y[first:first + 50], ops.hadamard_blockwise(x[first:first + 50].clone(), dim ** -0.5, dim))
+    odd = torch.empty(40 * dim + 1, dtype=dtype, device=gpu)[1:].view(40, dim)
+    odd.copy_(x[rows - 40:])
+    assert torch.equal(ops.hadamard_blockwise(odd, dim ** -0.5, dim), y[rows - 40:])
+    x[rows - 2, dim - 1] = float("inf")
+    again = ops.hadamard_blockwise(x, dim ** -0.5, dim)
+    assert not torch.isfinite(again[rows - 2]).any()
+    assert torch.equal(again[:rows - 2], y[:rows - 2]) and torch.equal(again[rows - 1], y[rows - 1])
 
 
 @pytest.mark.parametrize("dim,base", [(3584, 28), (5120, 40)])

@@ -198,7 +198,7 @@ __global__ __launch_bounds__(256) void fwht_lds_kernel(const T* __restrict__ x, 
     }
 }
 
-// ---- power of two >= 256: vector loads, index bits 0..2 in registers, LDS passes of
+// ---- 256 and 512: vector loads, index bits 0..2 in registers, LDS passes of
 // up to four bits, vector stores ----------------------------------------------
 template <typename T>
 __global__ __launch_bounds__(256) void fwht_vec_kernel(const T* __restrict__ x, T* __restrict__ y, int L, int log2L, float scale) {
@@ -225,110 +225,6 @@ __global__ __launch_bounds__(256) void fwht_vec_kernel(const T* __restrict__ x, 
     }
 }
 
-// Long rows (L >= 4096): two LDS exchanges instead of one per four index bits.
-//   load    every thread takes L/8/T sixteen-byte chunks (consecutive lanes on consecutive chunks),
-//           transforms index bits 0..2 in registers and writes fp32 to LDS;
-//   middle  index bits 3 .. n-6 in passes of up to five bits (32 values per task in registers);
-//   final   the top five bits: a thread reads two neighbouring values at 32 strides of L/32,
-//           transforms, scales, rounds and stores a pair per stride: consecutive lanes store
-//           consecutive pairs, no trip back through LDS.
-// The stages run in ascending bit order like everywhere else, so the fp32 sums are associated
-// the same way and the result is the same bit for bit.  L / 64 threads per row.
-template <typename T>
-__global__ __launch_bounds__(512) void fwht_wide_kernel(const T* __restrict__ x, T* __restrict__ y, int L, int log2L, float scale) {
-    extern __shared__ __attribute__((aligned(16))) float fbuf[];
-    const int tid = threadIdx.x, nthreads = blockDim.x;
-    const T* xp = x + (size_t)blockIdx.x * L;
-    T* yp = y + (size_t)blockIdx.x * L;
-    constexpr int kChunksPerThread = 8;  // chunks / nthreads = (L / 8) / (L / 64)
-    typename RowIo<T>::Raw v[kChunksPerThread];
-#pragma unroll
-    for (int i = 0; i < kChunksPerThread; ++i) v[i] = RowIo<T>::load(xp + 8 * (tid + i * nthreads));
-#pragma unroll
-    for (int i = 0; i < kChunksPerThread; ++i) {
-        float f[8];
-        RowIo<T>::unpack(v[i], f);
-        wht8(f);
-        float* dst = fbuf + fwht_pad(8 * (tid + i * nthreads));
-        *reinterpret_cast<f4*>(dst) = f4{f[0], f[1], f[2], f[3]};
-        *reinterpret_cast<f4*>(dst + 4) = f4{f[4], f[5], f[6], f[7]};
-    }
-    __syncthreads();
-    // index bits 3 .. log2L - 6 (log2L = 12 .. 15), then the top five bits in the final phase
-    switch (log2L) {
-        case 12: fwht_pass_fixed<4, 3>(fbuf, L, tid, nthreads); __syncthreads(); break;
-        case 13: fwht_pass_fixed<5, 3>(fbuf, L, tid, nthreads); __syncthreads(); break;
-        case 14:
-            fwht_pass_fixed<5, 3>(fbuf, L, tid, nthreads);
-            __syncthreads();
-            fwht_pass_fixed<1, 8>(fbuf, L, tid, nthreads);
-            __syncthreads();
-            break;
-        case 15:
-            fwht_pass_fixed<5, 3>(fbuf, L, tid, nthreads);
-            __syncthreads();
-            fwht_pass_fixed<2, 8>(fbuf, L, tid, nthreads);
-            __syncthreads();
-            break;
-        default: break;
-    }
-    // final phase: values 2 tid, 2 tid + 1 at the 32 strides of L / 32
-    const int stride = L >> 5;
-    float a[32], b[32];
-#pragma unroll
-    for (int j = 0; j < 32; ++j) {
-        const float* src = fbuf + fwht_pad(2 * tid + j * stride);
-        a[j] = src[0];
-        b[j] = src[1];
-    }
-#pragma unroll
-    for (int h = 1; h < 32; h <<= 1) {
-#pragma unroll
-        for (int j = 0; j < 32; ++j) {
-            if ((j & h) == 0) {
-                const float p = a[j], q = a[j + h];
-                a[j] = p + q;
-                a[j + h] = p - q;
-                const float r = b[j], t = b[j + h];
-                b[j] = r + t;
-                b[j + h] = r - t;
-            }
-        }
-    }
-#pragma unroll
-    for (int j = 0; j < 32; ++j) RowIo<T>::store2(yp + 2 * tid + j * stride, a[j], b[j], scale);
-}
-
-// more than 64 KB of LDS: a property of (kernel, device), set on the first launch there
-template <typename K>
-static bool allow_lds(K kern, size_t bytes, std::atomic<unsigned long long>& done) {
-    if (bytes <= 64 * 1024) return true;
-    int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return false;
-    if ((done.load(std::memory_order_acquire) >> dev) & 1ull) return true;
-    if (hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024) != hipSuccess)
-        return false;
-    done.fetch_or(1ull << dev, std::memory_order_release);
-    return true;
-}
-
-template <typename T>
-static int fwht_vec_launch(const void* x, void* y, int64_t pieces, int block, float scale, hipStream_t stream) {
-    int log2L = 0;
-    while ((1 << log2L) < block) ++log2L;
-    const size_t shmem = (size_t)(block + (block >> 7) * 8) * sizeof(float);
-    if (block >= 4096) {
-        static std::atomic<unsigned long long> done{0};
-        if (!allow_lds(&fwht_wide_kernel<T>, shmem, done)) return UNIQL_E_LAUNCH;
-        hipLaunchKernelGGL(fwht_wide_kernel<T>, dim3((unsigned)pieces), dim3(block / 64), shmem, stream,
-                           reinterpret_cast<const T*>(x), reinterpret_cast<T*>(y), block, log2L, scale);
-        return UNIQL_OK;
-    }
-    hipLaunchKernelGGL(fwht_vec_kernel<T>, dim3((unsigned)pieces), dim3(block / 8), shmem, stream,
-                       reinterpret_cast<const T*>(x), reinterpret_cast<T*>(y), block, log2L, scale);
-    return UNIQL_OK;
-}
-
 // Barriers that order LDS alone: loads from and stores to memory stay in flight.
 __device__ __forceinline__ void lds_barrier() {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
@@ -344,22 +240,31 @@ __device__ __forceinline__ void lds_wave_fence() {  // a wave's LDS operations c
 // Eight floats of padding per 64: the 64 lanes of either pass touch every bank once.
 __device__ __forceinline__ int fwht_pad8of64(int idx) { return idx + ((idx >> 6) << 3); }
 
-// Index bits 3..5 of 512 values that lie eight to a lane, in an LDS pass: on entry f holds values 8 piece .. (bits 0..2 done,
-// every piece on one lane), behind it f[e] is value lane + 64 e.  buf: 576 floats of the wave's own.
-__device__ __forceinline__ void wht512_pass3(float* buf, int piece, int lane, float (&f)[8]) {
-    float* d0 = buf + fwht_pad8of64(8 * piece);
-    *reinterpret_cast<f4*>(d0) = f4{f[0], f[1], f[2], f[3]};
-    *reinterpret_cast<f4*>(d0 + 4) = f4{f[4], f[5], f[6], f[7]};
-    lds_wave_fence();
-    float* d1 = buf + 72 * (lane >> 3) + (lane & 7);
+// Index bits 3..5 of 512 values that lie eight to a lane, in an LDS pass of two fenced steps: on entry f holds values 8 piece ..
+// (bits 0..2 done, every piece on one lane), behind it f[e] is value lane + 64 e.  buf: 576 floats of the wave's own.
+__device__ __forceinline__ void wht512_put(float* buf, int piece, const float (&f)[8]) {
+    float* d = buf + fwht_pad8of64(8 * piece);
+    *reinterpret_cast<f4*>(d) = f4{f[0], f[1], f[2], f[3]};
+    *reinterpret_cast<f4*>(d + 4) = f4{f[4], f[5], f[6], f[7]};
+}
+__device__ __forceinline__ void wht512_middle(float* buf, int lane, float (&f)[8]) {
+    float* d = buf + 72 * (lane >> 3) + (lane & 7);
 #pragma unroll
-    for (int e = 0; e < 8; ++e) f[e] = d1[8 * e];
+    for (int e = 0; e < 8; ++e) f[e] = d[8 * e];
     wht8(f);
 #pragma unroll
-    for (int e = 0; e < 8; ++e) d1[8 * e] = f[e];
-    lds_wave_fence();
+    for (int e = 0; e < 8; ++e) d[8 * e] = f[e];
+}
+__device__ __forceinline__ void wht512_get(const float* buf, int lane, float (&f)[8]) {
 #pragma unroll
     for (int e = 0; e < 8; ++e) f[e] = buf[lane + 72 * e];
+}
+__device__ __forceinline__ void wht512_pass3(float* buf, int piece, int lane, float (&f)[8]) {
+    wht512_put(buf, piece, f);
+    lds_wave_fence();
+    wht512_middle(buf, lane, f);
+    lds_wave_fence();
+    wht512_get(buf, lane, f);
 }
 // Bits 6.. of f[e] as far as a chunk of P values has them.
 __device__ __forceinline__ void wht512_upper(float (&f)[8], int P) {
@@ -374,6 +279,152 @@ __device__ __forceinline__ void wht512_upper(float (&f)[8], int P) {
                 f[e + (1 << b)] = p - q;
             }
     }
+}
+
+// Long rows, 1024 to 32768 values.  A wave takes one, two or four neighbouring blocks of 512 values: 16-byte loads and index
+// bits 0..2 in registers, bits 3..5 and 6..8 in LDS passes of its own, bits 9 and 10 in registers again, no workgroup
+// barrier; then, behind one, the one to four bits that lie across the waves: a thread reads two or four neighbouring values at
+// the waves' strides, transforms, scales, rounds and stores them.  Bits in ascending order like everywhere else: the same
+// bits.  The workgroups stay and request their next row ahead of the last step.
+// What bounds it: memory (16384 rows of 4096: 5.9 TB/s), and for few rows the latency of load, passes and store.  fp16, cold,
+// against one workgroup a row with a workgroup barrier behind every pass: one row of 4096 4.6 -> 2.8 us, of 16384 7.7 -> 4.4;
+// 1024 rows of 1024 3.4 -> 3.2, of 4096 7.3 -> 5.9, of 8192 11.0 -> 9.7, of 16384 23.2 -> 16.5, of 32768 45 -> 31; 4096 rows
+// of 4096 18.4 -> 15.5, of 16384 72 -> 50.
+template <int LOG2L>
+struct RowShape {
+    static constexpr int kBlocks = LOG2L <= 11 ? 1 : LOG2L == 12 ? 2 : 4;               // of 512 values, a wave
+    static constexpr int kWaves = (1 << LOG2L) / (512 * kBlocks);
+    static constexpr size_t kBytes = (size_t)(1 << LOG2L) / 8 * 9 * sizeof(float);
+};
+
+template <typename T, int LOG2L>
+__global__ __launch_bounds__(64 * RowShape<LOG2L>::kWaves, 4) void fwht_rows_kernel(const T* __restrict__ x, T* __restrict__ y, int rows, float scale) {
+    extern __shared__ __attribute__((aligned(16))) float fbuf[];
+    constexpr int L = 1 << LOG2L, NB = RowShape<LOG2L>::kBlocks, W = RowShape<LOG2L>::kWaves, kSpan = 512 * NB;
+    constexpr int V = LOG2L == 11 || W == 16 ? 2 : 4;  // neighbouring values of a thread in the last step
+    typedef float fv __attribute__((ext_vector_type(V)));
+    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    typename RowIo<T>::Raw v[NB];
+    auto request = [&](int row) __attribute__((always_inline)) {  // a row that does not exist: beyond the descriptor
+        const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(
+            const_cast<T*>(x + (size_t)(row < rows ? row : 0) * L), 0, row < rows ? (unsigned)(L * sizeof(T)) : 0u, 0x00020000);
+#pragma unroll
+        for (int i = 0; i < NB; ++i) v[i] = RowIo<T>::load(rsrc, (unsigned)((kSpan * w + 512 * i + 8 * lane) * sizeof(T)));
+    };
+    float* const mine = fbuf + 576 * NB * w;
+    int row = blockIdx.x;
+    request(row);
+    while (true) {
+        float f[NB][8];
+#pragma unroll
+        for (int i = 0; i < NB; ++i) {
+            RowIo<T>::unpack(v[i], f[i]);
+            wht8(f[i]);
+            wht512_put(mine + 576 * i, lane, f[i]);
+        }
+        lds_wave_fence();
+#pragma unroll
+        for (int i = 0; i < NB; ++i) wht512_middle(mine + 576 * i, lane, f[i]);
+        lds_wave_fence();
+#pragma unroll
+        for (int i = 0; i < NB; ++i) {
+            wht512_get(mine + 576 * i, lane, f[i]);
+            wht512_upper(f[i], 512);
+        }
+#pragma unroll
+        for (int h = 1; h < NB; h <<= 1)
+#pragma unroll
+            for (int i = 0; i < NB; ++i)
+                if ((i & h) == 0)
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) {
+                        const float p = f[i][e], q = f[i + h][e];
+                        f[i][e] = p + q;
+                        f[i + h][e] = p - q;
+                    }
+#pragma unroll
+        for (int i = 0; i < NB; ++i)
+#pragma unroll
+            for (int e = 0; e < 8; ++e) mine[576 * i + lane + 72 * e] = f[i][e];
+        const int next = row + gridDim.x;
+        request(next);
+        lds_barrier();
+        T* const yp = y + (size_t)row * L;
+#pragma unroll
+        for (int t = 0; t < kSpan / (V * 64 * W); ++t) {
+            const int col = V * ((int)threadIdx.x + 64 * W * t);
+            fv g[W];
+#pragma unroll
+            for (int j = 0; j < W; ++j) g[j] = *reinterpret_cast<const fv*>(fbuf + 576 * NB * j + fwht_pad8of64(col));
+#pragma unroll
+            for (int h = 1; h < W; h <<= 1)
+#pragma unroll
+                for (int j = 0; j < W; ++j)
+                    if ((j & h) == 0) {
+                        const fv p = g[j], q = g[j + h];
+                        g[j] = p + q;
+                        g[j + h] = p - q;
+                    }
+            // the next row has arrived by now; waited for behind the stores, it would be waited for with them
+#pragma unroll
+            for (int i = 0; i < NB; ++i) RowIo<T>::settle(v[i]);
+#pragma unroll
+            for (int j = 0; j < W; ++j) {
+                if constexpr (V == 4) RowIo<T>::store4(yp + kSpan * j + col, g[j], scale);
+                else RowIo<T>::store2(yp + kSpan * j + col, g[j][0], g[j][1], scale);
+            }
+        }
+        if (next >= rows) break;
+        row = next;
+        lds_barrier();  // the next row overwrites what other waves may still be reading
+    }
+}
+
+// more than 64 KB of LDS: a property of (kernel, device), set on the first launch there
+template <typename K>
+static bool allow_lds(K kern, size_t bytes, std::atomic<unsigned long long>& done) {
+    if (bytes <= 64 * 1024) return true;
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return false;
+    if ((done.load(std::memory_order_acquire) >> dev) & 1ull) return true;
+    if (hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024) != hipSuccess)
+        return false;
+    done.fetch_or(1ull << dev, std::memory_order_release);
+    return true;
+}
+
+template <typename T, int LOG2L>
+static int fwht_rows_go(const void* x, void* y, int64_t rows, float scale, hipStream_t stream) {
+    using S = RowShape<LOG2L>;
+    static std::atomic<unsigned long long> done{0};
+    if (!allow_lds(&fwht_rows_kernel<T, LOG2L>, S::kBytes, done)) return UNIQL_E_LAUNCH;
+    // The workgroups that the chip holds at once, by registers.  fp32 rows of 4096 and more each get their own: memory is
+    // busy without the request ahead, and rows in launch order use it better (16384 rows of 8192: 199 us, 207 with
+    // workgroups that stay; fp16 102 either way).
+    const int64_t resident = 256 * ((LOG2L <= 12 && sizeof(T) == 2 ? 32 : 16) / S::kWaves);
+    const int64_t grid = sizeof(T) == 4 && LOG2L >= 12 ? rows : std::min(rows, resident);
+    hipLaunchKernelGGL((fwht_rows_kernel<T, LOG2L>), dim3((unsigned)grid), dim3(64 * S::kWaves), S::kBytes, stream,
+                       reinterpret_cast<const T*>(x), reinterpret_cast<T*>(y), (int)rows, scale);
+    return UNIQL_OK;
+}
+
+template <typename T>
+static int fwht_vec_launch(const void* x, void* y, int64_t pieces, int block, float scale, hipStream_t stream) {
+    int log2L = 0;
+    while ((1 << log2L) < block) ++log2L;
+    const size_t shmem = (size_t)(block + (block >> 7) * 8) * sizeof(float);
+    switch (log2L) {
+        case 10: return fwht_rows_go<T, 10>(x, y, pieces, scale, stream);
+        case 11: return fwht_rows_go<T, 11>(x, y, pieces, scale, stream);
+        case 12: return fwht_rows_go<T, 12>(x, y, pieces, scale, stream);
+        case 13: return fwht_rows_go<T, 13>(x, y, pieces, scale, stream);
+        case 14: return fwht_rows_go<T, 14>(x, y, pieces, scale, stream);
+        case 15: return fwht_rows_go<T, 15>(x, y, pieces, scale, stream);
+        default: break;
+    }
+    hipLaunchKernelGGL(fwht_vec_kernel<T>, dim3((unsigned)pieces), dim3(block / 8), shmem, stream,
+                       reinterpret_cast<const T*>(x), reinterpret_cast<T*>(y), block, log2L, scale);
+    return UNIQL_OK;
 }
 
 // ---- down the columns of a row-major matrix: y = T((H_L . x) * scale), L = 1024, 2048 or 4096 rows ------------
