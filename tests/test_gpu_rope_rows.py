@@ -1,0 +1,30 @@
+"""Rotary kernels at the edges of their rules: the kernel that gathers per pair up to 191 tokens, tables in LDS from 192 on,
+heads of one pair (quotients by division), one table row for all sequences."""
+import numpy as np
+import pytest
+import torch
+
+from oracle import uniql_oracle as O
+from tests.test_gpu_rope_embedding import pruned_indices
+from tests.test_oracle_fused_rope import rope_tables
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("b,hq,hk,s,d,D", [(1, 16, 2, 191, 96, 256), (1, 16, 2, 192, 96, 256), (2, 32, 32, 140, 64, 128),
+                                           (3, 6, 2, 100, 14, 32), (1, 28, 4, 300, 6, 128), (260, 4, 2, 1, 8, 16), (70, 8, 1, 1, 20, 32),
+                                           (1, 5, 5, 7, 2, 16), (1, 6, 3, 290, 2, 16), (3, 40, 8, 20, 108, 128), (1, 96, 3, 2, 250, 256)])
+@pytest.mark.parametrize("index_dtype", [torch.uint8, torch.int64, torch.int32])
+def test_rows_and_heads(gpu, b, hq, hk, s, d, D, index_dtype):
+    from uniql_amd import ops
+    rng = np.random.default_rng(b + s + d)
+    q = rng.standard_normal((b, s, hq, d)).astype(np.float16)
+    k = rng.standard_normal((b, s, hk, d)).astype(np.float16)
+    cos, sin, _ = rope_tables(s, D, batch=b if b == 2 else 1)
+    idx = pruned_indices(hk, d, D, seed=d)
+    want_q, want_k = O.rope_indices(q.transpose(0, 2, 1, 3), k.transpose(0, 2, 1, 3), cos, sin, idx)
+    qt, kt = torch.from_numpy(q).to(gpu), torch.from_numpy(k).to(gpu)
+    ops.rope_indices_(qt, kt, torch.from_numpy(cos).to(gpu), torch.from_numpy(sin).to(gpu),
+                      torch.from_numpy(idx).to(index_dtype).to(gpu))
+    assert np.array_equal(qt.cpu().numpy().view(np.uint16), want_q.transpose(0, 2, 1, 3).view(np.uint16))
+    assert np.array_equal(kt.cpu().numpy().view(np.uint16), want_k.transpose(0, 2, 1, 3).view(np.uint16))

@@ -23,7 +23,11 @@ struct RopeArgs {
     const void* indices;  // [n_kh][hd], index_bytes wide
     int64_t q_row_stride, k_row_stride, cos_row_stride;
     int seq_len, cos_batch, n_qh, n_kh, hd, index_bytes;
+    unsigned rows;
+    int per_head, group;                       // work items of a head, query heads of a key / value head
+    unsigned per_head_inverse, group_inverse;  // 2^32 / divisor, rounded up: quotients without a division
 };
+constexpr unsigned kRopeGridRows = 65535;
 
 __device__ __forceinline__ int load_index(const void* base, int index_bytes, int pos) {
     if (index_bytes == 1) return (int)reinterpret_cast<const uint8_t*>(base)[pos];
@@ -43,6 +47,18 @@ __device__ __forceinline__ void rotate_pair(half_t& lo, half_t& hi, half_t c_lo,
     hi = (half_t)((float)a_hi + (float)r_hi);
 }
 
+// Several column pairs at once in packed fp16 arithmetic.  An fp16 product or sum computed in fp32 and rounded to fp16 equals
+// the fp16 operation's own single rounding (fp32's 24 bits are at least 2 x 11 + 2), so these are the values of
+// rotate_pair bit for bit, at a fifth of its instructions: the conversions made the kernel for many tokens compute-bound.
+template <typename V>
+__device__ __forceinline__ void rotate_pairs(half_t* to_lo, half_t* to_hi, V lo, V hi, V c_lo, V s_lo, V c_hi, V s_hi) {
+#pragma clang fp contract(off)
+    const V a_lo = lo * c_lo, r_lo = (-hi) * s_lo;
+    const V a_hi = hi * c_hi, r_hi = lo * s_hi;
+    *reinterpret_cast<V*>(to_lo) = a_lo + r_lo;
+    *reinterpret_cast<V*>(to_hi) = a_hi + r_hi;
+}
+
 template <int VEC>
 struct HalfVec;  // VEC fp16 values moved with one access
 template <>
@@ -52,65 +68,85 @@ struct HalfVec<2> { typedef h2 type; };
 template <>
 struct HalfVec<1> { typedef half_t type; };
 
-// VEC columns per thread and half of the head: 8 (16-byte accesses), 2 or 1.  A block covers
-// 256 consecutive work items of one token, so the only divisions are 32-bit ones.
-template <int VEC>
+// the indices of VEC neighbouring columns, I bytes each (of eight the low word counts)
+template <int VEC, int I>
+__device__ __forceinline__ void load_indices(const void* base, int pos, int (&out)[VEC]) {
+    typedef uint32_t words4 __attribute__((ext_vector_type(4), aligned(8)));
+    typedef uint32_t words2 __attribute__((ext_vector_type(2), aligned(4)));
+    if constexpr (VEC == 2 && I == 8) {
+        const words4 v = *reinterpret_cast<const words4*>(reinterpret_cast<const uint64_t*>(base) + pos);
+        out[0] = (int)v[0];
+        out[1] = (int)v[2];
+    } else if constexpr (VEC == 2 && I == 4) {
+        const words2 v = *reinterpret_cast<const words2*>(reinterpret_cast<const uint32_t*>(base) + pos);
+        out[0] = (int)v[0];
+        out[1] = (int)v[1];
+    } else {
+#pragma unroll
+        for (int v = 0; v < VEC; ++v) out[v] = load_index(base, I, pos + v);
+    }
+}
+
+// Few tokens: VEC columns per thread and half of the head.  A block covers 256 consecutive work items of one token.
+// Bound by latency: kernel arguments, indices, table values and the store follow each other, and every instruction in
+// front of the first load is paid in full (four clocks each; a division is forty of them, a 64-bit one two hundred).
+// So no divisions, one round of
+// scalar loads, and a thread's indices in two loads: one token 2.6 -> 2.2 us, 48 tokens 2.75 -> 2.4 (heads of 128), 3.1 -> 2.8
+// (of 108).
+// DIVIDE: sizes for which the rounded inverses are not exact.
+template <int VEC, int I, bool DIVIDE>
 __global__ __launch_bounds__(256) void rope_indices_kernel(const RopeArgs a) {
     typedef typename HalfVec<VEC>::type vec_t;
-    const int half = a.hd >> 1;
-    const int per_head = half / VEC;
-    const int per_row = (a.n_qh + a.n_kh) * per_head;
-    const int blocks_per_row = (per_row + 255) >> 8;
-    const int64_t row = blockIdx.x / blocks_per_row;
-    const int t = (int)(blockIdx.x % blocks_per_row) * 256 + threadIdx.x;
-    if (t >= per_row) return;
-    const int head = t / per_head;
+    // the kernel arguments in one round of scalar loads
+    const int hd = a.hd, half = hd >> 1, n_qh = a.n_qh, n_kh = a.n_kh, per_head = a.per_head;
+    const unsigned per_head_inverse = a.per_head_inverse, group_inverse = a.group_inverse;
+    half_t *const q = a.q, *const k = a.k;
+    const half_t *const cos = a.cos, *const sin = a.sin;
+    const void* const indices = a.indices;
+    const unsigned rows = a.rows;
+    const int64_t q_stride = a.q_row_stride, k_stride = a.k_row_stride, cos_stride = a.cos_row_stride;
+    const unsigned seq_len = a.cos_batch == 1 && rows != (unsigned)a.seq_len ? (unsigned)a.seq_len : 0u;
+    asm volatile("" ::"s"(q), "s"(k), "s"(cos), "s"(sin), "s"(indices), "s"(per_head_inverse), "s"(group_inverse), "s"(q_stride),
+                 "s"(k_stride), "s"(cos_stride), "s"(seq_len));
+    const int t = (int)blockIdx.x * 256 + (int)threadIdx.x;
+    if (t >= (n_qh + n_kh) * per_head) return;
+    const int head = DIVIDE ? t / per_head : (int)__umulhi((unsigned)t, per_head_inverse);
     const int j = (t - head * per_head) * VEC;
-
-    const bool is_q = head < a.n_qh;
-    const int kv_head = is_q ? head / (a.n_qh / a.n_kh) : head - a.n_qh;
-    half_t* x = is_q ? a.q + row * a.q_row_stride + (int64_t)head * a.hd
-                     : a.k + row * a.k_row_stride + (int64_t)(head - a.n_qh) * a.hd;
-    const int64_t table_row = a.cos_batch == 1 ? row % a.seq_len : row;
-    const half_t* cos_row = a.cos + table_row * a.cos_row_stride;
-    const half_t* sin_row = a.sin + table_row * a.cos_row_stride;
-
-    vec_t lo_v = *reinterpret_cast<const vec_t*>(x + j), hi_v = *reinterpret_cast<const vec_t*>(x + half + j);
-    half_t lo[VEC], hi[VEC];
-    if constexpr (VEC == 1) {
-        lo[0] = lo_v;
-        hi[0] = hi_v;
-    } else {
+    const bool is_q = head < n_qh;
+    const int of_q = DIVIDE ? head / a.group : (a.group == 1 ? head : (int)__umulhi((unsigned)head, group_inverse));
+    const int kv_head = is_q ? of_q : head - n_qh;
+    int i_lo[VEC], i_hi[VEC];
+    load_indices<VEC, I>(indices, kv_head * hd + j, i_lo);
+    load_indices<VEC, I>(indices, kv_head * hd + half + j, i_hi);
+    for (unsigned row = blockIdx.y; row < rows; row += kRopeGridRows) {
+        half_t* x = is_q ? q + row * q_stride + (int64_t)head * hd : k + row * k_stride + (int64_t)(head - n_qh) * hd;
+        const int64_t table_row = seq_len == 1 ? 0 : (seq_len != 0 ? row % seq_len : row);
+        const half_t *cos_row = cos + table_row * cos_stride, *sin_row = sin + table_row * cos_stride;
+        const vec_t lo_v = *reinterpret_cast<const vec_t*>(x + j), hi_v = *reinterpret_cast<const vec_t*>(x + half + j);
+        if constexpr (VEC == 1) {
+            half_t lo = lo_v, hi = hi_v;
+            rotate_pair(lo, hi, cos_row[i_lo[0]], sin_row[i_lo[0]], cos_row[i_hi[0]], sin_row[i_hi[0]]);
+            x[j] = lo;
+            x[half + j] = hi;
+        } else {
+            vec_t c_lo, s_lo, c_hi, s_hi;
 #pragma unroll
-        for (int v = 0; v < VEC; ++v) {
-            lo[v] = lo_v[v];
-            hi[v] = hi_v[v];
+            for (int v = 0; v < VEC; ++v) {
+                c_lo[v] = cos_row[i_lo[v]];
+                s_lo[v] = sin_row[i_lo[v]];
+                c_hi[v] = cos_row[i_hi[v]];
+                s_hi[v] = sin_row[i_hi[v]];
+            }
+            rotate_pairs<vec_t>(x + j, x + half + j, lo_v, hi_v, c_lo, s_lo, c_hi, s_hi);
         }
     }
-#pragma unroll
-    for (int v = 0; v < VEC; ++v) {
-        const int i_lo = load_index(a.indices, a.index_bytes, kv_head * a.hd + j + v);
-        const int i_hi = load_index(a.indices, a.index_bytes, kv_head * a.hd + half + j + v);
-        rotate_pair(lo[v], hi[v], cos_row[i_lo], sin_row[i_lo], cos_row[i_hi], sin_row[i_hi]);
-    }
-    if constexpr (VEC == 1) {
-        lo_v = lo[0];
-        hi_v = hi[0];
-    } else {
-#pragma unroll
-        for (int v = 0; v < VEC; ++v) {
-            lo_v[v] = lo[v];
-            hi_v[v] = hi[v];
-        }
-    }
-    *reinterpret_cast<vec_t*>(x + j) = lo_v;
-    *reinterpret_cast<vec_t*>(x + half + j) = hi_v;
 }
 
 // Many tokens: one workgroup per token builds the token's gathered (cos, sin) pairs once per
 // key/value head in LDS (n_kv_heads x head_dim entries of 4 bytes) and every query head of the
 // group reads them from there, instead of every element gathering from the tables in memory.
-template <int VEC>
+// DIVIDE as above; without the divisions 1024 tokens of heads of 108 take 6.0 us instead of 7.05, 333 4.55 instead of 5.2.
+template <int VEC, bool DIVIDE>
 __global__ __launch_bounds__(256) void rope_indices_lds_kernel(const RopeArgs a, int cos_dim) {
     typedef typename HalfVec<VEC>::type vec_t;
     extern __shared__ __attribute__((aligned(16))) uint32_t rope_lds[];
@@ -119,8 +155,8 @@ __global__ __launch_bounds__(256) void rope_indices_lds_kernel(const RopeArgs a,
     uint16_t* tab_cos = reinterpret_cast<uint16_t*>(rope_lds + ((cos_dim + 3) & ~3));
     uint16_t* tab_sin = tab_cos + a.n_kh * a.hd;
     const int tid = threadIdx.x;
-    const int64_t row = blockIdx.x;
-    const int64_t table_row = a.cos_batch == 1 ? row % a.seq_len : row;
+    const unsigned row = blockIdx.x;
+    const int64_t table_row = a.cos_batch == 1 && a.rows != (unsigned)a.seq_len ? row % (unsigned)a.seq_len : row;
     const uint16_t* cos_row = reinterpret_cast<const uint16_t*>(a.cos + table_row * a.cos_row_stride);
     const uint16_t* sin_row = reinterpret_cast<const uint16_t*>(a.sin + table_row * a.cos_row_stride);
     // Everything the token needs from memory is requested before the first barrier: the (cos, sin)
@@ -139,10 +175,10 @@ __global__ __launch_bounds__(256) void rope_indices_lds_kernel(const RopeArgs a,
         idx_ahead[i] = e < entries ? load_index(a.indices, a.index_bytes, e) : 0;
     }
     auto item = [&](int t, half_t*& x, int& kv_head, int& j) __attribute__((always_inline)) {
-        const int head = t / per_head;
+        const int head = DIVIDE ? t / per_head : (int)__umulhi((unsigned)t, a.per_head_inverse);
         j = (t - head * per_head) * VEC;
         const bool is_q = head < a.n_qh;
-        kv_head = is_q ? head / (a.n_qh / a.n_kh) : head - a.n_qh;
+        kv_head = is_q ? (DIVIDE ? head / a.group : (a.group == 1 ? head : (int)__umulhi((unsigned)head, a.group_inverse))) : head - a.n_qh;
         x = is_q ? a.q + row * a.q_row_stride + (int64_t)head * a.hd
                  : a.k + row * a.k_row_stride + (int64_t)(head - a.n_qh) * a.hd;
     };
@@ -183,18 +219,9 @@ __global__ __launch_bounds__(256) void rope_indices_lds_kernel(const RopeArgs a,
     auto rotate_item = [&](half_t* x, int kv_head, int j, vec_t lo_v, vec_t hi_v) __attribute__((always_inline)) {
         const int e0 = kv_head * a.hd + j;
         if constexpr (VEC > 1) {
-            // All of the item's column pairs at once in packed fp16 arithmetic.  An fp16 product or sum
-            // computed in fp32 and rounded to fp16 equals the fp16 operation's own single rounding
-            // (fp32's 24 bits are at least 2 x 11 + 2), so these are the values of rotate_pair bit for
-            // bit, at a fifth of its instructions: the conversions made this kernel compute-bound.
-#pragma clang fp contract(off)
-            const vec_t c_lo = *reinterpret_cast<const vec_t*>(tab_cos + e0), s_lo = *reinterpret_cast<const vec_t*>(tab_sin + e0);
-            const vec_t c_hi = *reinterpret_cast<const vec_t*>(tab_cos + e0 + half);
-            const vec_t s_hi = *reinterpret_cast<const vec_t*>(tab_sin + e0 + half);
-            const vec_t a_lo = lo_v * c_lo, r_lo = (-hi_v) * s_lo;
-            const vec_t a_hi = hi_v * c_hi, r_hi = lo_v * s_hi;
-            *reinterpret_cast<vec_t*>(x + j) = a_lo + r_lo;
-            *reinterpret_cast<vec_t*>(x + half + j) = a_hi + r_hi;
+            rotate_pairs<vec_t>(x + j, x + half + j, lo_v, hi_v, *reinterpret_cast<const vec_t*>(tab_cos + e0),
+                                *reinterpret_cast<const vec_t*>(tab_sin + e0), *reinterpret_cast<const vec_t*>(tab_cos + e0 + half),
+                                *reinterpret_cast<const vec_t*>(tab_sin + e0 + half));
         } else {
             half_t lo = lo_v, hi = hi_v;
             rotate_pair(lo, hi, __builtin_bit_cast(half_t, tab_cos[e0]), __builtin_bit_cast(half_t, tab_sin[e0]),
@@ -213,6 +240,24 @@ __global__ __launch_bounds__(256) void rope_indices_lds_kernel(const RopeArgs a,
         const vec_t lo_v = *reinterpret_cast<const vec_t*>(x + j), hi_v = *reinterpret_cast<const vec_t*>(x + half + j);
         rotate_item(x, kv_head, j, lo_v, hi_v);
     }
+}
+
+template <int VEC, int I>
+static void rope_indices_bytes(const RopeArgs& a, bool divide, dim3 grid, hipStream_t stream) {
+    if (divide) hipLaunchKernelGGL((rope_indices_kernel<VEC, I, true>), grid, dim3(256), 0, stream, a);
+    else hipLaunchKernelGGL((rope_indices_kernel<VEC, I, false>), grid, dim3(256), 0, stream, a);
+}
+template <int VEC>
+static void rope_indices_go(const RopeArgs& a, bool divide, dim3 grid, hipStream_t stream) {
+    if (a.index_bytes == 1) rope_indices_bytes<VEC, 1>(a, divide, grid, stream);
+    else if (a.index_bytes == 4) rope_indices_bytes<VEC, 4>(a, divide, grid, stream);
+    else rope_indices_bytes<VEC, 8>(a, divide, grid, stream);
+}
+
+template <int VEC>
+static void rope_tables_go(const RopeArgs& a, bool divide, int cos_dim, size_t lds_bytes, hipStream_t stream) {
+    if (divide) hipLaunchKernelGGL((rope_indices_lds_kernel<VEC, true>), dim3(a.rows), dim3(256), lds_bytes, stream, a, cos_dim);
+    else hipLaunchKernelGGL((rope_indices_lds_kernel<VEC, false>), dim3(a.rows), dim3(256), lds_bytes, stream, a, cos_dim);
 }
 
 int rope_indices_launch(void* q, int64_t q_row_stride, void* k, int64_t k_row_stride, const void* cos, const void* sin,
@@ -240,29 +285,33 @@ int rope_indices_launch(void* q, int64_t q_row_stride, void* k, int64_t k_row_st
     int vec = 1;
     if (half % 8 == 0 && q_row_stride % 8 == 0 && k_row_stride % 8 == 0 && (bases & 15u) == 0) vec = 8;
     else if (half % 2 == 0 && q_row_stride % 2 == 0 && k_row_stride % 2 == 0 && (bases & 3u) == 0) vec = 2;
-    // enough tokens to fill the chip with one workgroup each, and tables that fit LDS
+    // From 192 tokens on a workgroup each builds the token's tables in LDS (where they fit), below that every pair gathers its
+    // own values, two columns at a time: more threads in flight hide the dependent index -> table loads better than wide
+    // accesses do (32 + 8 heads of 108: 128 tokens 3.4 us against 4.0, 192 4.0 either way, 256 4.35 against 4.15, 512 6.2
+    // against 4.8).
     const size_t lds_bytes = ((size_t)((cos_dim + 3) & ~3) + (size_t)n_kh * hd) * 4;
-    if (rows >= 64 && lds_bytes <= 32 * 1024 && rows <= 0x7fffffffLL) {
-        if (vec == 8)
-            hipLaunchKernelGGL(rope_indices_lds_kernel<8>, dim3((unsigned)rows), dim3(256), lds_bytes, stream, a, cos_dim);
-        else if (vec == 2)
-            hipLaunchKernelGGL(rope_indices_lds_kernel<2>, dim3((unsigned)rows), dim3(256), lds_bytes, stream, a, cos_dim);
-        else
-            hipLaunchKernelGGL(rope_indices_lds_kernel<1>, dim3((unsigned)rows), dim3(256), lds_bytes, stream, a, cos_dim);
-        return hipGetLastError() == hipSuccess ? UNIQL_OK : UNIQL_E_LAUNCH;
+    const bool tables = rows >= 192 && lds_bytes <= 32 * 1024 && rows <= 0x7fffffffLL;
+    if (!tables && vec == 8) vec = 2;
+    a.per_head = half / vec;
+    a.group = n_qh / n_kh;
+    const int64_t per_row = (int64_t)(n_qh + n_kh) * a.per_head, blocks = (per_row + 255) / 256;
+    if (!tables && (per_row > 0x7fffff00LL || rows * blocks > 0x7fffffffLL)) return UNIQL_E_SHAPE;
+    a.rows = (unsigned)rows;
+    // floor(t / d) = floor(t inverse / 2^32) while t times the inverse's rounding, less than d, stays below 2^32
+    auto exact = [](int64_t dividends, int64_t divisor) { return dividends * divisor < (1LL << 32); };
+    auto inverse = [](int divisor) { return (unsigned)(((1ULL << 32) + divisor - 1) / divisor); };
+    const bool divide = a.per_head == 1 || !exact(256 * blocks, a.per_head) || !exact(n_qh + n_kh, a.group);
+    a.per_head_inverse = divide ? 0u : inverse(a.per_head);
+    a.group_inverse = divide || a.group == 1 ? 0u : inverse(a.group);
+    if (tables) {
+        if (vec == 8) rope_tables_go<8>(a, divide, cos_dim, lds_bytes, stream);
+        else if (vec == 2) rope_tables_go<2>(a, divide, cos_dim, lds_bytes, stream);
+        else rope_tables_go<1>(a, divide, cos_dim, lds_bytes, stream);
+    } else {
+        const dim3 grid((unsigned)blocks, rows < (int64_t)kRopeGridRows ? (unsigned)rows : kRopeGridRows);
+        if (vec == 2) rope_indices_go<2>(a, divide, grid, stream);
+        else rope_indices_go<1>(a, divide, grid, stream);
     }
-    // few tokens: the direct gather, narrow accesses (more threads in flight hide the dependent
-    // index -> table loads better than wide accesses do)
-    if (vec == 8) vec = 2;
-    const int per_row = (n_qh + n_kh) * (half / vec);
-    const int64_t blocks = rows * ((per_row + 255) / 256);
-    if (blocks > 0x7fffffffLL) return UNIQL_E_SHAPE;
-    if (vec == 8)
-        hipLaunchKernelGGL(rope_indices_kernel<8>, dim3((unsigned)blocks), dim3(256), 0, stream, a);
-    else if (vec == 2)
-        hipLaunchKernelGGL(rope_indices_kernel<2>, dim3((unsigned)blocks), dim3(256), 0, stream, a);
-    else
-        hipLaunchKernelGGL(rope_indices_kernel<1>, dim3((unsigned)blocks), dim3(256), 0, stream, a);
     return hipGetLastError() == hipSuccess ? UNIQL_OK : UNIQL_E_LAUNCH;
 }
 
