@@ -150,13 +150,18 @@ struct LinearNeeds {
 static const MidPlan kNoMid = {0, 0, 0, 0.0};
 
 // In place of the streaming kernel: from 9 rows on that kernel's one atomic per output element and K split costs more than
-// the exchange of partial tiles, except over few columns and a long K (11840 -> 1280 at 10 rows 8.3 us there, 10.1 here) and
-// where it does not split K at all (4096 -> 28672 at 9 to 12 rows 12.9 to 13.4 us there, 13.3 to 13.5 here).  4096 -> 4096 at 16 rows 8.5 -> 7.3 us, 4096 -> 6144 9.2 -> 7.7; of 1438 drawn calls of 9
-// to 16 rows 13 % on average.  A rotation stays with the streaming kernel, which applies it while it stages the rows.
+// the exchange of partial tiles, except where it does not split K at all (4096 -> 28672 at 9 to 12 rows 12.9 to 13.4 us there,
+// 13.3 to 13.5 here), and over a longer K, where this one's units follow each other in a wave: above 2048 it takes narrow
+// layers from 12 rows on (4096 -> 512 at 10 rows 6.65 us there, 6.7 here, at 12 7.1 and 6.8; 4096 -> 4096 at 9 rows 7.75 and
+// 7.0), above 4096 calls from 13 rows on (6144 -> 512 at 9 rows 6.65 and 7.45, 14336 -> 4096 11.25 and 11.5; at 16 rows 8.25 and
+// 7.45, 12.7 and 11.75), but few columns and a long K not at all (11840 -> 1280 at 10 rows 8.3 us there, 10.1 here).
+// 4096 -> 4096 at 16 rows 8.5 -> 7.3 us, 4096 -> 6144 9.2 -> 7.7.  A rotation stays with the streaming kernel,
+// which applies it while it stages the rows.
 static MidPlan mid_for_few_rows(int m, int n, int k, int had_block, unsigned flags, size_t part_cap) {
     if (m < kMidMinRows || m > kStreamMaxM || had_block != 0 || (flags & (UNIQL_F_FORCE_SKINNY | UNIQL_F_FORCE_TILED)) || (flags >> 8) != 0)
         return kNoMid;
-    return n / 128 < 144 && (k <= 6144 || n >= 4096) ? mid_plan(m, n, k, 0, part_cap) : kNoMid;
+    const bool faster = k > 4096 ? m >= 13 && (k <= 6144 || n >= 4096) : k <= 2048 || m >= 12 || n >= 4096;
+    return n / 128 < 144 && faster ? mid_plan(m, n, k, 0, part_cap) : kNoMid;
 }
 
 // In place of a launch of the tiled kernels, where it is expected to be faster; padded: the tiled kernels would need a
