@@ -97,7 +97,8 @@ const char* uniql_status_string(int code) {
 // rows up to this many take the weight-streaming kernel, more take the tiled one
 static constexpr int kStreamMaxM = 16;
 
-// which kernel takes a call
+// Which kernels a call goes to: the streaming kernel, or (see mid_for_few_rows) the one for 9 to 64 rows in its place, or those of
+// the plan below.
 static bool takes_stream_kernel(int m, unsigned flags) {
     bool use_stream = m <= kStreamMaxM;
     if (flags & UNIQL_F_FORCE_SKINNY) use_stream = true;

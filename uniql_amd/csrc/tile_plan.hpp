@@ -1,4 +1,4 @@
-// How the tiled kernels run the rows of a call: pure host functions of the sizes, plain C++.  A plan is made
+// How the tiled kernels run a call: pure host functions of the sizes, plain C++.  A plan is made
 // once per call and handed as it is to the argument checks, the scratch sizes and the launch.
 #pragma once
 

@@ -1,4 +1,4 @@
-// Tiled W4A16 kernel for M > 16 (prefill): D[M,N] = X[M,K] . dequant(B)[K,N].
+// Tiled W4A16 kernel for prompts (more than 64 rows, and fewer where the kernels for them are not faster): D[M,N] = X[M,K] . dequant(B)[K,N].
 //
 // A workgroup of four wavefronts owns a (32 MT) x 128 output tile (MT = 1 to 4) and a
 // range of 128-wide K groups.  The four waves split K: of the eight packed rows (16 K
