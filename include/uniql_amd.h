@@ -88,7 +88,9 @@ int uniql_clear(void* p, size_t bytes, void* stream);
  *   temp       device, uniql_w4a16_gemm_temp_bytes(m, n, k, had_block) bytes, contents
  *              irrelevant: rotated activations whenever the rotation is not fused, and
  *              the fp32 partial tiles of the tiled kernels and of the kernel for 9 to 64 rows
- *              when their plan splits K over workgroups; may be NULL when that size is 0.  Two calls that may run
+ *              when their plan splits K over workgroups; may be NULL when that size is 0.  (A buffer that
+ *              is too small for the latter, or for two launches over columns, is enough wherever it is for
+ *              the other kernels: up to 16 rows without a rotation none is needed.)  Two calls that may run
  *              concurrently need separate buffers.
  *   had_block  0: none.  Otherwise the activations are rotated first,
  *              A <- fp16(A . H_had_block * had_scale) on consecutive
@@ -99,7 +101,7 @@ int uniql_clear(void* p, size_t bytes, void* stream);
  *              (<= 32768, dividing k), and every rotation for larger m, runs the
  *              transform kernel into `temp` first.  Same values either way.
  *   k % 128 == 0, n % 128 == 0 (the module pads n to 256).
- *   Calls of more than 128 rows may run as two launches over consecutive rows (on the same stream,
+ *   Calls of more than 64 rows may run as two launches over consecutive rows or columns (on the same stream,
  *   sharing accum and temp); the kernels are chosen from m, n, k.
  *
  * Partial sums that meet in the streaming kernel's `accum` words are rounded to multiples of

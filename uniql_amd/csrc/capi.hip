@@ -177,8 +177,10 @@ static MidPlan mid_for_tiles(const RowPart& part, int n, int k, bool padded, uns
     return p.upw > 0 && p.us < part.tile.us + (padded ? 2.0 : 0.0) ? p : kNoMid;
 }
 
+// basic: neither the kernel for 9 to 64 rows nor columns in two launches, for callers whose scratch memory is enough for the
+// other kernels only (none at all up to 16 rows, or sized by a library in front of those).
 static LinearNeeds linear_needs(int m, int n, int k, int k_in, int64_t lda, int groups, int had_block, unsigned flags,
-                                size_t part_cap = kPartialCap) {
+                                size_t part_cap = kPartialCap, bool basic = false) {
     LinearNeeds q;
     const unsigned tune = flags >> 8;
     q.use_stream = takes_stream_kernel(m, flags);
@@ -192,7 +194,7 @@ static LinearNeeds linear_needs(int m, int n, int k, int k_in, int64_t lda, int 
     q.mid[0] = q.mid[1] = kNoMid;
     q.accum_bytes = q.part_bytes = 0;
     if (q.use_stream) {
-        if (mid_shape_ok(m, n, k, lda)) q.mid[0] = mid_for_few_rows(m, n, k, had_block, flags, part_cap);
+        if (!basic && mid_shape_ok(m, n, k, lda)) q.mid[0] = mid_for_few_rows(m, n, k, had_block, flags, part_cap);
         if (q.mid[0].upw > 0) {
             q.use_stream = false;
             q.plan.parts = 1;
@@ -201,10 +203,11 @@ static LinearNeeds linear_needs(int m, int n, int k, int k_in, int64_t lda, int 
             q.accum_bytes = round256(stream_accum_bytes(m, n, k));
         }
     } else {
-        q.plan = call_plan(m, n, k, wide_shape_ok(m, n & ~255, k, groups, q.ld_kernel), part_cap, tune);
+        q.plan = basic ? linear_plan(m, n, k, wide_shape_ok(m, n, k, groups, q.ld_kernel), part_cap, tune)
+                       : call_plan(m, n, k, wide_shape_ok(m, n & ~255, k, groups, q.ld_kernel), part_cap, tune);
         const bool one = q.plan.parts == 1;
         for (int i = 0; i < q.plan.parts; ++i)
-            if (q.plan.head_columns == 0 && mid_shape_ok(q.plan.part[i].rows, n, k, q.rotate_first ? k : lda))
+            if (!basic && q.plan.head_columns == 0 && mid_shape_ok(q.plan.part[i].rows, n, k, q.rotate_first ? k : lda))
                 q.mid[i] = mid_for_tiles(q.plan.part[i], n, k, one && q.pad_first && !q.rotate_first, flags, part_cap);
         if (one && q.mid[0].upw > 0 && !q.rotate_first) {  // that kernel guards its own loads
             q.pad_first = false;
@@ -322,18 +325,22 @@ static int linear_impl(const void* A, int64_t lda, int k_in, const void* B, cons
     if ((accum && !aligned16(accum)) || (temp && !aligned16(temp))) return UNIQL_E_ALIGN;
     hipStream_t st = reinterpret_cast<hipStream_t>(stream);
     const unsigned tune = flags >> 8;  // tuning fields, see the header
-    const LinearNeeds q = linear_needs(m, n, k, k_in, lda, groups, had_block, flags, part_cap);
+    LinearNeeds q = linear_needs(m, n, k, k_in, lda, groups, had_block, flags, part_cap);
+    auto enough = [&]() {
+        return (q.accum_bytes == 0 || (accum && accum_bytes >= q.accum_bytes)) &&
+               (q.act_bytes + q.part_bytes == 0 || (temp && temp_bytes >= q.act_bytes + q.part_bytes));
+    };
+    if (!enough() && ((flags >> 16) & 0xfu) != 9)
+        q = linear_needs(m, n, k, k_in, lda, groups, had_block, flags, part_cap, true);
     const bool use_stream = q.use_stream, rotate_first = q.rotate_first, pad_first = q.pad_first;
     const int had_mode = q.had_mode;
     const int64_t ld_kernel = q.ld_kernel;
     const void* Ain = A;
     int64_t ld = lda;
     int k_valid = k_in;
-    const size_t need_accum = q.accum_bytes;
-    if (need_accum > 0 && (!accum || accum_bytes < need_accum)) return UNIQL_E_WORKSPACE;
-    // temp: the copy of the activations, then the tiled kernel's partial tiles when it splits K
+    if (!enough()) return UNIQL_E_WORKSPACE;
+    // temp: the copy of the activations, then the partial tiles of a kernel that splits K
     const size_t act_bytes = q.act_bytes, part_bytes = q.part_bytes;
-    if (act_bytes + part_bytes > 0 && (!temp || temp_bytes < act_bytes + part_bytes)) return UNIQL_E_WORKSPACE;
     void* part = part_bytes ? reinterpret_cast<char*>(temp) + act_bytes : nullptr;
     // last check before the first kernel is enqueued: whether the tiled kernel can take the shape
     for (int i = 0; i < q.plan.parts; ++i)
