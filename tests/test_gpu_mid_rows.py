@@ -110,6 +110,28 @@ def test_nan_and_infinite_sums_cross_the_split(gpu, m):
     assert (y[rest].double() - ref[rest]).abs().max() < 2e-4
 
 
+@pytest.mark.parametrize("m", [16, 30, 48, 64])
+def test_infinite_values_meet_scales_of_the_long_expansion(gpu, m):
+    """a group whose scales are beyond the short expansion's range: an infinite value times its weights is infinite, not NaN"""
+    from uniql_amd import ops
+    k, n = 1536, 128
+    gen, b, s = _layer(gpu, k, n, 6)
+    s[0, 9], s[5] = 0.5, 0.25
+    x = torch.randn((m, k), device=gpu, generator=gen).half()
+    x[2, 7], x[3, 5 * 128 + 70], x[m - 1, 11 * 128] = float("inf"), float("-inf"), float("inf")
+    w = ops.w4a16_dequant(b, s, n, k)
+    for scale, weight in ((s, w), (s[5:6].clone(), ops.w4a16_dequant(b, s[5:6].clone(), n, k))):
+        y = ops.w4a16_gemm_ex(x, b, scale, workspace_for(n, gpu), m, n, k, out_f32=True, flags=_flags(2))
+        ref = x.double() @ weight.double()
+        assert torch.isinf(ref[2]).any() and torch.isinf(ref[3]).any()
+        assert torch.equal(torch.isnan(y), torch.isnan(ref))
+        assert torch.equal(torch.where(torch.isinf(y), y, 0.0).double(), torch.where(torch.isinf(ref), ref, 0.0))
+        finite = torch.isfinite(ref)
+        # fp32 sums of 1536 products, |x w| < 5 x 4: far less than 1536 2^-24 times their absolute sum
+        bound = 1536 * 2.0 ** -24 * (torch.nan_to_num(x.double(), posinf=0.0, neginf=0.0).abs() @ weight.double().abs())
+        assert torch.all(((y.double() - ref).abs() <= bound + 1e-6)[finite])
+
+
 def test_calls_take_it_and_replay(gpu):
     """the calls that the library hands to it by itself, recorded once and replayed between eager calls that share
     nothing with the graph but the stream's buffers; every replay and every eager repeat gives the same bits"""

@@ -199,7 +199,7 @@ __global__ __launch_bounds__(64 * WAVES, WAVES / 4) void w4a16_mid_kernel(const 
     // One unit against the staged rows.  A code left where it is, everything else masked away, is the fp16 number
     // c 2^-20; with S = s 2^20, fma(c 2^-20, S, -8 s) = fp16_rn((c - 8) s), the reference's weight, for every scale
     // whose S is finite: |s| < 2^-4, zeros and subnormals included.  A unit with a larger scale is left out (its
-    // scales count as zeros) and done behind the others.
+    // scales and its X count as zeros, since an infinite X times zero would be NaN) and done behind the others.
     bool left_out = false;
     auto too_large = [&](const u32x4& scales) __attribute__((always_inline)) {
         uint32_t large = 0;
@@ -211,6 +211,14 @@ __global__ __launch_bounds__(64 * WAVES, WAVES / 4) void w4a16_mid_kernel(const 
         const u32x4 scales = a.per_column ? sc_fixed : unit.sc;
         const bool large = too_large(scales);
         left_out |= large;
+        if (__builtin_expect(large, 0)) {  // uniform
+#pragma unroll
+            for (int i = 0; i < XQ; ++i) {
+#pragma unroll
+                for (int p = 0; p < 4; ++p) xwrite[4 * i * kMidXStride + 4 * p] = 0u;
+            }
+            fence();
+        }
         h2 s20[4], m8[4];
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
