@@ -178,6 +178,27 @@ def test_cut_rows(gpu, n, n_real, pad, k, units, full, kept, per_column):
         ops.w4a16_cut_rows(w, s, n, k, 2, k, 100, n_real, pad_out=pad)
 
 
+# even runs an even distance apart, whose rows are expanded two at a time: single pairs, runs that overlap or follow each other,
+# runs off the words' and groups' grids, one long run
+@pytest.mark.parametrize("k,units,full,kept", [(1024, 255, 4, 2), (512, 100, 2, 4), (2048, 93, 22, 10), (4096, 32, 128, 108),
+                                               (4096, 1, 0, 4094), (640, 5, 128, 128)])
+@pytest.mark.parametrize("n,n_real,pad", [(256, 200, 56), (128, 128, 0)])
+def test_cut_rows_in_pairs(gpu, k, units, full, kept, n, n_real, pad):
+    """the same bits for scales on the 16-byte grid, off it, and as quantising the gathered dequantised rows, groups of zeros,
+    subnormal and large scales among them"""
+    from uniql_amd import ops
+    (w, s), _, _ = _packed_layer(gpu, k, n, torch.Generator().manual_seed(k + kept))
+    s = s.clone()
+    s[0, 3:70], s[1, ::2], s[2, 5], s[3, 9] = 0.0, 6e-8, 300.0, -0.01
+    rows = torch.tensor([u * full + i for u in range(units) for i in range(kept)], device=gpu)
+    want = ops.w4a16_quantize(ops.w4a16_dequant(w, s, n, k)[rows][:, :n_real].t().contiguous(), None, pad_out=pad)
+    off = torch.empty(s.numel() + 1, dtype=s.dtype, device=gpu)[1:].view_as(s)
+    off.copy_(s)
+    for scales in (s, off):
+        got = ops.w4a16_cut_rows(w, scales, n, k, units, full, kept, n_real, pad_out=pad)
+        assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
+
+
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("dim", [128, 256, 4096, 32768, 20 * 128, 28 * 512])
 def test_transform_of_rows_off_the_16_byte_grid(gpu, dtype, dim):

@@ -178,22 +178,52 @@ __global__ __launch_bounds__(256) void w4a16_quantize_kernel(const half_t* __res
 }
 
 // Keeps rows of a packed matrix that no longer line up with the groups, and quantises them again: what dequantising, gathering
-// the rows, transposing and the kernel above give, without the fp16 matrix and its two copies (4096 x 4096, 32 heads of 128
-// cut to 108 rows: 14.3 us).  Kept row i is row (i / kept) full + i % kept.  One workgroup takes 64 columns x one group of the
-// OUTPUT: 1024 tasks of one kept row x eight columns (one 16-byte piece holds them; neighbouring rows read the same
+// the rows, transposing and the kernel above give, without the fp16 matrix and its two copies.  Kept row i is row
+// (i / kept) full + i % kept.  One workgroup takes 64 columns x one group of the
+// OUTPUT: tasks of kept rows x eight columns (one 16-byte piece holds them; neighbouring rows read the same
 // pieces, from the first-level cache) expand into LDS, from where every thread takes its 2 x 16 values.
+// Bound by vector instructions.  PAIRED: runs of an even number of rows, an even distance apart, so that kept rows 2 p and 2 p + 1
+// are the two halves of the same words: a task is two rows, expanded in packed arithmetic (the same values: code - 8 is
+// exact, one rounding), and the division by `kept` is a product with its rounded inverse.
+// Out of cache, one row a task -> this: 4096 x 4096, 32 heads of 128 cut to 108 rows, 13.0 -> 10.2 us; 8192 x 4096, 128 of 64
+// to 48, 19.4 -> 15.3; 14336 x 4096, one run of 14000, 39.5 -> 29.7.
 constexpr int kCutLdsRow = 136;  // fp16 values per column in LDS: 128 + 8, 16-byte reads of eight columns on different banks
 
+template <bool PAIRED>
 __global__ __launch_bounds__(256) void w4a16_cut_rows_kernel(const uint32_t* __restrict__ Bin, const half_t* __restrict__ Sin,
                                                             half_t* __restrict__ S, uint32_t* __restrict__ B, int n, int k_kept,
-                                                            int full, int kept, int per_column, int vec_ok, int n_real,
-                                                            int n_pad, int groups) {
+                                                            int full, int kept, unsigned kept_inverse, int per_column, int vec_ok,
+                                                            int n_real, int n_pad, int groups) {
     __shared__ __attribute__((aligned(16))) uint32_t words[8 * kPackLdsRow];
     __shared__ __attribute__((aligned(16))) half_t scales[64];
     __shared__ __attribute__((aligned(16))) half_t values[64 * kCutLdsRow];
     const int g = blockIdx.x % groups, chunk = blockIdx.x / groups;
     const int tid = threadIdx.x, c8 = tid & 7;
-    if (64 * chunk < n_real) {  // n_real <= n: the chunk exists in the source
+    if (PAIRED && 64 * chunk < n_real) {  // n_real <= n: the chunk exists in the source
+        NibbleMagic magic;
+        magic.init();
+        u32x4 q4[2];
+        h8 s[2];
+        int down[2];
+#pragma unroll
+        for (int t = 0; t < 2; ++t) {
+            const int i = 128 * g + 64 * t + 2 * (tid >> 3), at = i < k_kept ? i : k_kept - 2;
+            const int unit = (int)__umulhi((unsigned)at, kept_inverse), k = unit * full + (at - unit * kept);
+            q4[t] = *reinterpret_cast<const u32x4*>(Bin + (size_t)(k >> 4) * 2 * n + 128 * (size_t)chunk + 16 * c8 + 4 * ((k >> 1) & 3));
+            s[t] = *reinterpret_cast<const h8*>(Sin + (size_t)(k >> 7) * n + 64 * chunk + 8 * c8);
+            down[t] = 4 * ((k >> 3) & 1);
+        }
+#pragma unroll
+        for (int t = 0; t < 2; ++t) {
+            const int row = 64 * t + 2 * (tid >> 3);
+            const bool real = 128 * g + row < k_kept;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {  // column 8 e + c8
+                const h2 v = magic.pair_low((q4[t][e >> 1] >> down[t]) >> (8 * (e & 1))) * h2{s[t][e], s[t][e]};
+                *reinterpret_cast<uint32_t*>(values + (8 * e + c8) * kCutLdsRow + row) = real ? h2_to_bits(v) : 0u;
+            }
+        }
+    } else if (64 * chunk < n_real) {
 #pragma unroll
         for (int t = 0; t < 4; ++t) {
             const int row = 32 * t + (tid >> 3), i = 128 * g + row;
@@ -382,10 +412,17 @@ int cut_rows_launch(const void* B, const void* S, int n, int groups_in, int unit
     const int k_kept = units * kept, groups = (k_kept + 127) / 128;
     const int64_t grid = (int64_t)groups * (n_pad / 64);
     if (grid > 0x7fffffffLL) return UNIQL_E_SHAPE;
-    hipLaunchKernelGGL(w4a16_cut_rows_kernel, dim3((unsigned)grid), dim3(256), 0, stream, reinterpret_cast<const uint32_t*>(B),
-                       reinterpret_cast<const half_t*>(S), reinterpret_cast<half_t*>(S_out), reinterpret_cast<uint32_t*>(B_out),
-                       n, k_kept, full, kept, groups_in == 1 ? 1 : 0, (reinterpret_cast<uintptr_t>(S) & 15u) == 0 ? 1 : 0,
-                       n_real, n_pad, groups);
+    const bool vec_ok = (reinterpret_cast<uintptr_t>(S) & 15u) == 0;
+    // floor(i / kept) = floor(i inverse / 2^32) while i times the inverse's rounding, less than kept, stays below 2^32
+    const bool paired = kept % 2 == 0 && full % 2 == 0 && groups_in != 1 && vec_ok && (int64_t)k_kept * kept < (1LL << 32);
+    const unsigned inverse = paired ? (unsigned)(((1ULL << 32) + kept - 1) / kept) : 0u;
+    auto go = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3((unsigned)grid), dim3(256), 0, stream, reinterpret_cast<const uint32_t*>(B),
+                           reinterpret_cast<const half_t*>(S), reinterpret_cast<half_t*>(S_out), reinterpret_cast<uint32_t*>(B_out),
+                           n, k_kept, full, kept, inverse, groups_in == 1 ? 1 : 0, vec_ok ? 1 : 0, n_real, n_pad, groups);
+    };
+    if (paired) go(w4a16_cut_rows_kernel<true>);
+    else go(w4a16_cut_rows_kernel<false>);
     return hipGetLastError() == hipSuccess ? UNIQL_OK : UNIQL_E_LAUNCH;
 }
 
