@@ -178,6 +178,20 @@ def test_cut_rows(gpu, n, n_real, pad, k, units, full, kept, per_column):
         ops.w4a16_cut_rows(w, s, n, k, 2, k, 100, n_real, pad_out=pad)
 
 
+# a run of single columns (whose inverse does not fit 32 bits), pairs, odd lengths, a prefix, padding columns inside a chunk
+@pytest.mark.parametrize("runs", [[(0, 100, 5, 1, 1, 0)], [(3, 90, 4, 2, 1, 1)], [(0, 7, 71, 67, 30, 4), (500, 1, 12, 11, 11, 0)], [(64, 1, 448, 448, 448, 0)]])
+def test_cut_columns_quotients(gpu, runs):
+    from uniql_amd import ops
+    k, n = 384, 512
+    (w, s), codes, scales = _packed_layer(gpu, k, n, torch.Generator().manual_seed(9))
+    cols = torch.tensor([base + u * full + i + (skip if i >= split else 0) for base, units, full, kept, split, skip in runs
+                         for u in range(units) for i in range(kept)], device=gpu)
+    pad = -len(cols) % 256
+    want = ops.w4a16_pack(codes[:, cols], scales[:, cols], pad_out=pad)
+    got = ops.w4a16_cut_columns(w, s, n, k, runs, pad_out=pad)
+    assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
+
+
 # even runs an even distance apart, whose rows are expanded two at a time: single pairs, runs that overlap or follow each other,
 # runs off the words' and groups' grids, one long run
 @pytest.mark.parametrize("k,units,full,kept", [(1024, 255, 4, 2), (512, 100, 2, 4), (2048, 93, 22, 10), (4096, 32, 128, 108),

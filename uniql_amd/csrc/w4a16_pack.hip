@@ -267,14 +267,19 @@ __global__ __launch_bounds__(256) void w4a16_cut_rows_kernel(const uint32_t* __r
 // so nothing is unpacked: a 16-byte piece of the output
 // takes eight 4-byte loads and a byte selection each, or, where its 64 columns are one source chunk (a kept prefix),
 // one load.  A workgroup resolves its chunk's 64 source columns once and keeps them for `per` groups of 128 rows.
-// Bound by memory and, for the small projections, by the launch (4096 x 14336 cut to 12160, 53 MB: 12.2 us = 4.3 TB/s,
-// 1024 columns: 5.2).
+// Bound by memory and, for the small projections, by the launch; so the eight loads are all in flight together (columns
+// without a source load, too, and are masked: skipped loads had been waited for one by one), quotients are products with
+// rounded inverses, and registers stay within 64 for eight waves a SIMD (with 75 the kept prefix took 15 us).  Out of cache,
+// before and now: 4096 x 14336 cut to 12160 (53 MB) 13.4 -> 12.8 us, 112 heads of 128 to 108 22.6 -> 17.0; 4096 x 18688 of
+// two runs of 64 to 48 25.8 -> 18.6; 4096 x 4096 to 3456 8.3 -> 7.5; 1024 columns 4.9 -> 4.3.  Requesting the next group's words
+// ahead: 19.2, 24.6, 28.8, 10.3 (registers).
 struct ColumnRuns {
     int count;
     int base[5], units[5], full[5], kept[5], split[5], skip[5];
+    unsigned inverse[5];  // 2^32 / kept, rounded up, where that gives the exact quotients; else 0
 };
 
-__global__ __launch_bounds__(256) void w4a16_cut_columns_kernel(const uint32_t* __restrict__ Bin, const half_t* __restrict__ Sin,
+__global__ __launch_bounds__(256, 8) void w4a16_cut_columns_kernel(const uint32_t* __restrict__ Bin, const half_t* __restrict__ Sin,
                                                                uint32_t* __restrict__ B, half_t* __restrict__ S, int n,
                                                                int groups, int k_real, ColumnRuns runs, int n_scaled, int n_pad,
                                                                int per) {
@@ -290,8 +295,9 @@ __global__ __launch_bounds__(256) void w4a16_cut_columns_kernel(const uint32_t* 
             if (s < runs.count && col < 0) {
                 const int len = runs.units[s] * runs.kept[s];
                 if (i < len) {
-                    const int at = i % runs.kept[s];
-                    col = runs.base[s] + (i / runs.kept[s]) * runs.full[s] + at + (at >= runs.split[s] ? runs.skip[s] : 0);
+                    const int unit = runs.inverse[s] ? (int)__umulhi((unsigned)i, runs.inverse[s]) : i / runs.kept[s];
+                    const int at = i - unit * runs.kept[s];
+                    col = runs.base[s] + unit * runs.full[s] + at + (at >= runs.split[s] ? runs.skip[s] : 0);
                 }
                 i -= len;
             }
@@ -305,28 +311,38 @@ __global__ __launch_bounds__(256) void w4a16_cut_columns_kernel(const uint32_t* 
     __syncthreads();
     const int piece = tid & 31, row = tid >> 5, c8 = piece >> 2, kq = piece & 3;
     const int from = whole_chunk;
-    int word[8], shift[8];       // columns 8 e + c8: word of a packed row and bits to go down; -1: none
+    // columns 8 e + c8: word of a packed row, bits to go down, and what of it counts (nothing where there is no source
+    // column: every load is made, since one that is skipped waits for those in front of it)
+    unsigned word[8];
+    int shift[8], counts = 0;  // counts: bit e
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
-        const int col = source[8 * e + c8];
-        word[e] = col < 0 ? -1 : 128 * (col >> 6) + 16 * (col & 7) + 4 * kq + ((col & 63) >> 4);
-        shift[e] = 8 * ((col >> 3) & 1);
+        const int col = source[8 * e + c8], real = col < 0 ? 0 : col;
+        word[e] = 128 * (real >> 6) + 16 * (real & 7) + 4 * kq + ((real & 63) >> 4);
+        shift[e] = 8 * ((real >> 3) & 1);
+        counts |= col < 0 ? 0 : 1 << e;
     }
-    int scale_from = -1;
+    int scale_from = 0;
+    bool scaled = false;
     if (tid < 64) {  // the scale at position tid of a chunk belongs to column (tid / 8) + 8 (tid % 8)
         const int at = 8 * (tid & 7) + (tid >> 3), col = source[at];
-        if (col >= 0 && 64 * chunk + at < n_scaled) scale_from = (int)group_scale_pos(col);
+        scaled = col >= 0 && 64 * chunk + at < n_scaled;
+        scale_from = scaled ? (int)group_scale_pos(col) : 0;
     }
     const int g1 = g0 + per < groups ? g0 + per : groups;
     for (int g = g0; g < g1; ++g) {
         const uint32_t* src = Bin + (size_t)(8 * g + row) * 2 * n;
+        half_t sv = (half_t)0.0f;
+        if (tid < 64) sv = Sin[(size_t)g * n + scale_from];
         u32x4 v;
         if (from >= 0) {
             v = *reinterpret_cast<const u32x4*>(src + 128 * (size_t)from + 4 * piece);
         } else {
             uint32_t q[8];
 #pragma unroll
-            for (int e = 0; e < 8; ++e) q[e] = word[e] >= 0 ? (src[word[e]] >> shift[e]) & 0x00ff00ffu : 0u;
+            for (int e = 0; e < 8; ++e) q[e] = src[word[e]];
+#pragma unroll
+            for (int e = 0; e < 8; ++e) q[e] = (q[e] >> shift[e]) & 0x00ff00ffu & (uint32_t)__builtin_amdgcn_sbfe(counts, e, 1);
 #pragma unroll
             for (int j = 0; j < 4; ++j) v[j] = q[2 * j] | (q[2 * j + 1] << 8);
         }
@@ -338,7 +354,7 @@ __global__ __launch_bounds__(256) void w4a16_cut_columns_kernel(const uint32_t* 
             for (int j = 0; j < 4; ++j) v[j] &= mask;
         }
         *reinterpret_cast<u32x4*>(B + (size_t)(8 * g + row) * 2 * n_pad + 128 * (size_t)chunk + 4 * piece) = v;
-        if (tid < 64) S[(size_t)g * n_pad + 64 * (size_t)chunk + tid] = scale_from >= 0 ? Sin[(size_t)g * n + scale_from] : (half_t)0.0f;
+        if (tid < 64) S[(size_t)g * n_pad + 64 * (size_t)chunk + tid] = scaled ? sv : (half_t)0.0f;
     }
 }
 
@@ -437,6 +453,8 @@ int cut_columns_launch(const void* B, const void* S, int n, int k, int k_real, c
         r.kept[i] = runs[6 * i + 3];
         r.split[i] = runs[6 * i + 4];
         r.skip[i] = runs[6 * i + 5];
+        const int64_t kept = r.kept[i];
+        r.inverse[i] = kept > 1 && r.units[i] * kept * kept < (1LL << 32) ? (unsigned)(((1LL << 32) + kept - 1) / kept) : 0u;
     }
     const int groups = k / 128;
     const int64_t tiles = (int64_t)groups * (n_pad / 64);
