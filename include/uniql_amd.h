@@ -109,8 +109,11 @@ int uniql_clear(void* p, size_t bytes, void* stream);
  * gives an infinite fp16 result; with UNIQL_F_OUT_F32 the clamp itself is visible).  A NaN
  * partial sum makes the result NaN, as without a K split.  The one difference from a launch
  * that does not split K: +inf and -inf that meet from DIFFERENT workgroups cancel to a finite
- * value instead of NaN.  Either kernel's result is the same from run to run: integer additions
- * in the first, partial tiles added in split order in the second.
+ * value instead of NaN.  The kernel for 9 to 64 rows and the tiled kernels exchange fp32 partial
+ * tiles and add them in a fixed order, the former up to 16 rows in 64 bits: no clamp, and
+ * infinities of both signs give NaN.  Every kernel's result is the same from run to run, and the
+ * kernel that takes a call by itself is, in front of the fp16 rounding, as close to the exact sum
+ * as the streaming kernel (up to 16 rows) or the 128-column kernel (up to 64) would be.
  */
 size_t uniql_w4a16_gemm_accum_bytes(int m, int n, int k);
 size_t uniql_w4a16_gemm_temp_bytes(int m, int n, int k, int had_block);

@@ -8,7 +8,7 @@ from tests.helpers import check_layer_output_torch, make_linear_problem, referen
 
 pytestmark = pytest.mark.gpu
 
-F_FORCE_TILED, MID = 1 << 2, 9 << 16
+F_FORCE_SKINNY, F_FORCE_TILED, MID = 1 << 1, 1 << 2, 9 << 16
 
 
 def _flags(groups_per_wave):
@@ -130,6 +130,28 @@ def test_infinite_values_meet_scales_of_the_long_expansion(gpu, m):
         # fp32 sums of 1536 products, |x w| < 5 x 4: far less than 1536 2^-24 times their absolute sum
         bound = 1536 * 2.0 ** -24 * (torch.nan_to_num(x.double(), posinf=0.0, neginf=0.0).abs() @ weight.double().abs())
         assert torch.all(((y.double() - ref).abs() <= bound + 1e-6)[finite])
+
+
+# sizes of this kernel: one and several groups a wave, K split into 2 to 9 and not at all, each row class; the last two where its
+# fastest plan would add longer chains than the tiled kernel's
+@pytest.mark.parametrize("m,k,n", [(15, 4480, 512), (12, 1920, 1024), (16, 8192, 4096), (13, 512, 13056), (29, 4864, 7168), (23, 12800, 1536),
+                                   (17, 3328, 8704), (40, 4096, 28672), (48, 4096, 4096), (35, 12288, 1280), (40, 9216, 3072), (56, 6784, 2048), (53, 6400, 256), (56, 8192, 512)])
+def test_sums_are_as_exact_as_the_other_kernels(gpu, m, k, n):
+    """distance from float64 in front of the fp16 rounding against that of the kernel which took such calls before: the
+    streaming kernel, whose partial sums meet as integers, up to 16 rows, the tiled kernel above.  Both round fp32
+    sums of the same exact products; with a few thousand outputs the two distances are known to about 1 %."""
+    from uniql_amd import ops
+    gen, b, s = _layer(gpu, k, n, 77)
+    x = torch.randn((m, k), device=gpu, generator=gen)
+    x[:, torch.randint(0, k, (max(1, k // 512),), device=gpu, generator=gen)] *= 16.0   # a few much larger channels
+    x = x.half()
+    ref = x.double() @ ops.w4a16_dequant(b, s, n, k).double()
+    ws = workspace_for(n, gpu)
+
+    def distance(flags):
+        return float((ops.w4a16_gemm_ex(x, b, s, ws, m, n, k, out_f32=True, flags=flags).double() - ref).norm() / ref.norm())
+
+    assert distance(0) <= 1.03 * distance(F_FORCE_SKINNY if m <= 16 else F_FORCE_TILED)
 
 
 def test_calls_take_it_and_replay(gpu):

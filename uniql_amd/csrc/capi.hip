@@ -167,13 +167,15 @@ static MidPlan mid_for_few_rows(int m, int n, int k, int had_block, unsigned fla
 
 // In place of a launch of the tiled kernels, where it is expected to be faster; padded: the tiled kernels would need a
 // zero-padded copy of the rows first (2 us).  Over a short K of fewer than 12 groups the tiled kernels' expected times are the
-// better ones from 33 rows on.  Drawn calls: 17 to 32 rows 1.26 x faster on average, 33 to 48 1.17, 49 to 64 1.03.
+// better ones from 33 rows on.  Plans that add longer chains of products than the tiled kernel's own are left out: a sum
+// is no less exact here than there (8192 -> 512 at 56 rows with two groups a wave: 1.1 x the distance from float64).
+// Drawn calls: 17 to 32 rows 1.26 x faster on average, 33 to 48 1.17, 49 to 64 1.03.
 static MidPlan mid_for_tiles(const RowPart& part, int n, int k, bool padded, unsigned flags, size_t part_cap) {
     if (part.rows < kMidMinRows || part.rows > kMidMaxRows) return kNoMid;
     if (((flags >> 16) & 0xfu) == 9) return mid_plan(part.rows, n, k, (int)((flags >> 8) & 0xffu), part_cap);  // asked for
     if (part.rows <= kStreamMaxM || (part.rows > 32 && k < 12 * 128)) return kNoMid;
     if ((flags & UNIQL_F_FORCE_TILED) || ((flags >> 8) & 0x3fffu) != 0) return kNoMid;
-    const MidPlan p = mid_plan(part.rows, n, k, 0, part_cap);
+    const MidPlan p = mid_plan(part.rows, n, k, 0, part_cap, tile_chain(part.tile));
     return p.upw > 0 && p.us < part.tile.us + (padded ? 2.0 : 0.0) ? p : kNoMid;
 }
 

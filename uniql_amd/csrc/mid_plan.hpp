@@ -17,6 +17,17 @@ struct MidPlan {
 
 static inline int mid_row_tiles(int m) { return m <= 16 ? 1 : m <= 32 ? 2 : m <= 48 ? 3 : 4; }  // of 16 rows
 
+// Accumulators of a wave: the products of the low and of the high codes apart (SETS = 2) wherever the registers hold both
+// and a wave has more than one unit or nothing to lose: with 33 to 48 rows and one unit a wave the second set costs 0.7 us
+// of 9.4 (its zeros, its moves to vector registers), with 49 to 64 rows it does not fit.
+static inline int mid_sets(int m, int upw) {
+    const int tiles = mid_row_tiles(m);
+    return tiles <= 2 || (tiles == 3 && upw > 1) ? 2 : 1;
+}
+// The K values whose products enter one accumulator one after another: what a sum's error grows with (the matrix unit
+// rounds each of its additions; the waves' and workgroups' sums meet in a few levels).
+static inline int mid_chain(int m, int upw) { return 128 * upw / mid_sets(m, upw); }
+
 // What a plan that splits K over workgroups needs: an arrival count per strip and wave in `accum` (zero on entry and
 // exit), the partial tiles in units of four rows, a whole number per wave, in a scratch area whose contents do not matter.
 static inline size_t mid_accum_bytes(int n, const MidPlan& p) { return p.splits <= 1 ? 0 : (size_t)(n / 128) * p.waves * sizeof(unsigned long long); }
@@ -47,11 +58,14 @@ static inline double mid_us(int m, int64_t wgs, int upw, int splits) {
 
 // Eight waves, two a SIMD, up to 32 rows (4096 -> 4096 at 17 rows 8.2 us against 8.8 with four), four from 33 rows on
 // (4096 -> 4096 at 48 rows 10.1 against 10.5: eight have no registers there to load a unit ahead).
-static inline MidPlan mid_plan(int m, int n, int k, int upw_override, size_t part_cap) {
+// longest_chain: plans whose sums take an eighth more than so many K values one after another do not count (0: all do).
+// The eighth: at equal chains the sums are 2 to 4 % closer here, since the waves' and workgroups' sums meet in pairs.
+static inline MidPlan mid_plan(int m, int n, int k, int upw_override, size_t part_cap, int longest_chain = 0) {
     const int G = k / 128, waves = m <= 32 ? 8 : 4, longest = (G + waves - 1) / waves;
     MidPlan best = {0, 0, 0, 1e30};
     for (int upw = 1; upw <= longest; ++upw) {
         if (upw_override > 0 && upw != (upw_override < longest ? upw_override : longest)) continue;
+        if (longest_chain > 0 && 8 * mid_chain(m, upw) > 9 * longest_chain) continue;
         MidPlan p = {upw, waves, (G + waves * upw - 1) / (waves * upw), 0.0};
         p.us = mid_us(m, (int64_t)(n / 128) * p.splits, upw, p.splits);
         if (mid_part_bytes(m, n, p) <= part_cap && p.us < best.us) best = p;

@@ -18,6 +18,10 @@ struct TilePlan {
     double us;     // expected time
 };
 
+// The K values whose products enter one accumulator one after another: a wave takes 32 of a group's 128, a quartet its
+// share of the groups.
+static inline int tile_chain(const TilePlan& plan) { return 32 * ceil_div_i(plan.gps, plan.quartets); }
+
 // What a plan that splits K over workgroups needs: one arrival count per output tile in `accum` (zero on entry,
 // zero again on exit) and one fp32 partial tile per (tile, split) in a scratch area whose contents do not matter.
 static inline size_t tile_accum_bytes(int m, int n, const TilePlan& plan) {

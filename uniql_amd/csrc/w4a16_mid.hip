@@ -10,16 +10,24 @@
 // What bounds it: vector instructions.  A SIMD takes one shift, packed multiply-add or MFMA issue every four clocks from
 // however many waves (an MFMA occupies two issue slots, its other clocks pass under them; 2 clocks only for plain AND / fp32
 // adds), so a unit of 392 of them and 32 MQ MFMAs is 2080 clocks at 32 rows, 2340 at 48, beside 14 clocks for a load and
-// 12 for an LDS access that another wave has to fill: hence two waves a SIMD up to 32 rows (168 registers), one with
-// the next unit's loads spread over the current one above (272 to 340).  A 32x32x16 form (half the MFMAs) was no faster:
+// 12 for an LDS access that another wave has to fill: hence two waves a SIMD up to 32 rows (226 registers), one with
+// the next unit's loads spread over the current one above (360 to 448).  A 32x32x16 form (half the MFMAs) was no faster:
 // it multiplies 64 rows where there are 33 to 48, at a lower clock.
-//   us, weights out of cache:          17 rows        32 rows        48 rows        64 rows
-//   4096 ->  6144 (tiled -> this)   10.9 ->  8.5   10.9 ->  9.0   12.6 -> 10.5   12.9 -> 12.2
-//   4096 ->  4096                   10.2 ->  8.2   10.2 ->  8.6   10.7 -> 10.2   10.7 -> 11.5
-//   4096 -> 28672                   18.7 -> 16.9   19.1 -> 17.1   24.6 -> 22.3   25.5 -> 26.1
-//  14336 ->  4096                   16.1 -> 13.8   16.8 -> 14.7   19.4 -> 16.4   20.2 -> 18.9
-// and at 16 rows, against the streaming kernel, 9.2 -> 7.7, 8.5 -> 7.3, 14.5 -> 13.7, 12.7 -> 11.8.
+//   us, weights out of cache:          17 rows        32 rows        48 rows
+//   4096 ->  6144 (tiled -> this)   10.7 ->  7.7   11.0 ->  8.3   12.6 -> 10.6
+//   4096 ->  4096                    9.9 ->  7.4   10.1 ->  7.8   10.6 -> 10.2
+//   4096 -> 28672                   20.0 -> 16.6   20.8 -> 17.5   27.1 -> 21.6
+//  14336 ->  4096                   16.5 -> 11.8   17.2 -> 13.0   19.7 -> 16.3
+// and at 16 rows, against the streaming kernel, 9.0 -> 7.1, 8.5 -> 6.8, the third no faster, 12.8 -> 10.7; 64 rows over
+// 4096 -> 512 9.6 -> 9.2.
+//
+// How exact its sums are: the distance from float64 in front of the fp16 rounding is 0.81 to 1.00 x the streaming
+// kernel's at 9 to 16 rows, 0.60 to 1.03 x the tiled kernel's above (216 drawn calls, 0.87 on average).  It grows with the
+// number of products that enter one accumulator one after another, hence two sets of accumulators (SETS, mid_sets) and
+// mid_plan's longest_chain, and sums of waves and workgroups in pairs, up to 16 rows in 64 bits: the streaming kernel adds its
+// workgroups' sums as integers.  With one set and the sums added in a row it was up to 1.39 x.
 #include <atomic>
+#include <type_traits>
 
 #include "common.hpp"
 #include "mid_plan.hpp"
@@ -49,13 +57,41 @@ struct MidArgs {
 constexpr int kMidNonTemporal = 2;   // cache policy bit nt
 constexpr int kMidDeviceScope = 16;  // cache policy bit sc1: as relaxed device-scope loads and stores compile to
 
+// How sums from several waves and workgroups are added.  In pairs of pairs: a term goes through as few roundings as there
+// are levels.
+struct TreeSums {
+    typedef f4 Total;
+    template <int N>
+    static __device__ __forceinline__ void add(f4& total, f4 (&v)[N]) {
+#pragma unroll
+        for (int h = 1; h < N; h <<= 1)
+#pragma unroll
+            for (int i = 0; i + h < N; i += 2 * h) v[i] += v[i + h];
+        total += v[0];
+    }
+    static __device__ __forceinline__ f4 rounded(f4 total) { return total; }
+};
+// In 64 bits, one rounding at the end.
+struct DoubleSums {
+    typedef double Total __attribute__((ext_vector_type(4)));
+    template <int N>
+    static __device__ __forceinline__ void add(Total& total, const f4 (&v)[N]) {
+#pragma unroll
+        for (int j = 0; j < N; ++j)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) total[i] += (double)v[j][i];
+    }
+    static __device__ __forceinline__ f4 rounded(Total total) { return f4{(float)total[0], (float)total[1], (float)total[2], (float)total[3]}; }
+};
+
 template <int MQ, int WAVES>
 struct MidLds {
     static constexpr size_t kBytes = (size_t)WAVES * 16 * MQ * kMidRedStride * 4;  // an area per wave
 };
 
-// MQ: 16-row tiles (M <= 16 MQ).  EXT: the call uses something beyond the plain product, as in w4a16_stream.hip.
-template <int MQ, int WAVES, bool EXT>
+// MQ: 16-row tiles (M <= 16 MQ).  SETS: the products of the low and of the high code pairs go to accumulators of their own (2)
+// or to the same ones.  EXT: the call uses something beyond the plain product, as in w4a16_stream.hip.
+template <int MQ, int WAVES, int SETS, bool EXT>
 __global__ __launch_bounds__(64 * WAVES, WAVES / 4) void w4a16_mid_kernel(const MidArgs a) {
     extern __shared__ __attribute__((aligned(16))) uint32_t lds[];
     constexpr int MR = 16 * MQ, XQ = 4 * MQ;
@@ -79,15 +115,9 @@ __global__ __launch_bounds__(64 * WAVES, WAVES / 4) void w4a16_mid_kernel(const 
     const u32x4* strip_w = a.B + (size_t)strip * 64;
     const half_t* strip_s = a.S + (size_t)strip * 128;
 
-    // acc[mq][jb][v]: row 16 mq + slot, column slot 4 kq + v of column block jb
-    // (the zeros are hidden from the compiler: it takes a sum that starts as a constant apart into scalars, which then
-    // wander between accumulator and vector registers all through the loop)
-    f4 acc[MQ][8], zeros = f4{0.f, 0.f, 0.f, 0.f};
-    asm volatile("" : "+v"(zeros));
-#pragma unroll
-    for (int mq = 0; mq < MQ; ++mq)
-#pragma unroll
-        for (int jb = 0; jb < 8; ++jb) acc[mq][jb] = zeros;
+    // acc[set][mq][jb][v]: row 16 mq + slot, column slot 4 kq + v of column block jb
+    typedef typename std::conditional<MQ == 1, DoubleSums, TreeSums>::type Sums;
+    f4 acc[SETS][MQ][8];
 
     // this wave's area: the staged rows of X, at the end its partial tile
     uint32_t* area = lds + (size_t)w * (MR * kMidRedStride);
@@ -181,9 +211,9 @@ __global__ __launch_bounds__(64 * WAVES, WAVES / 4) void w4a16_mid_kernel(const 
             prefetch(b);
             if (b < 15) expand(b + 1, nl, nh);
 #pragma unroll
-            for (int mq = 0; mq < MQ; ++mq) acc[mq][jb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(bl, xl[mq], acc[mq][jb], 0, 0, 0);
+            for (int mq = 0; mq < MQ; ++mq) acc[0][mq][jb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(bl, xl[mq], acc[0][mq][jb], 0, 0, 0);
 #pragma unroll
-            for (int mq = 0; mq < MQ; ++mq) acc[mq][jb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(bh, xh[mq], acc[mq][jb], 0, 0, 0);
+            for (int mq = 0; mq < MQ; ++mq) acc[SETS - 1][mq][jb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(bh, xh[mq], acc[SETS - 1][mq][jb], 0, 0, 0);
 #pragma unroll
             for (int i = 0; i < 2 * MQ; ++i) {
                 __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);                                 // one MFMA,
@@ -246,8 +276,30 @@ __global__ __launch_bounds__(64 * WAVES, WAVES / 4) void w4a16_mid_kernel(const 
         }, [](int) {});
     };
 
-    if (g_begin < g_end) {
+    // ---- the waves' partial tiles meet in LDS ---------------------------------------------
+    auto red_of = [&](int tile) __attribute__((always_inline)) { return reinterpret_cast<float*>(lds) + tile * (MR * kMidRedStride); };
+    auto put = [&](auto&& value) __attribute__((always_inline)) {
+        float* red = red_of(w) + slot * kMidRedStride + 64 * (kq >> 1) + 4 * (kq & 1);
+#pragma unroll
+        for (int mq = 0; mq < MQ; ++mq)
+#pragma unroll
+            for (int jb = 0; jb < 8; ++jb)
+                *reinterpret_cast<f4*>(red + 16 * mq * kMidRedStride + 16 * (jb >> 1) + 8 * (jb & 1)) = value(mq, jb);
+    };
+    if (g_begin >= g_end) {
+        put([](int, int) { return f4{0.f, 0.f, 0.f, 0.f}; });
+    } else {
         load_unit(g_begin);
+        // Zeros while the first unit is on its way.  (They are hidden from the compiler: it takes a sum that starts as a
+        // constant apart into scalars, which then wander between accumulator and vector registers all through the loop.)
+        f4 zeros = f4{0.f, 0.f, 0.f, 0.f};
+        asm volatile("" : "+v"(zeros));
+#pragma unroll
+        for (int set = 0; set < SETS; ++set)
+#pragma unroll
+            for (int mq = 0; mq < MQ; ++mq)
+#pragma unroll
+                for (int jb = 0; jb < 8; ++jb) acc[set][mq][jb] = zeros;
         if (a.per_column) {  // uniform, rare
             uint32_t t[4];
 #pragma unroll
@@ -296,17 +348,7 @@ __global__ __launch_bounds__(64 * WAVES, WAVES / 4) void w4a16_mid_kernel(const 
                 process_any();
             }
         }
-    }
-
-    // ---- the waves' partial tiles meet in LDS ---------------------------------------------
-    auto red_of = [&](int tile) __attribute__((always_inline)) { return reinterpret_cast<float*>(lds) + tile * (MR * kMidRedStride); };
-    {
-        float* red = red_of(w) + slot * kMidRedStride + 64 * (kq >> 1) + 4 * (kq & 1);
-#pragma unroll
-        for (int mq = 0; mq < MQ; ++mq)
-#pragma unroll
-            for (int jb = 0; jb < 8; ++jb)
-                *reinterpret_cast<f4*>(red + 16 * mq * kMidRedStride + 16 * (jb >> 1) + 8 * (jb & 1)) = acc[mq][jb];
+        put([&](int mq, int jb) { return SETS == 2 ? acc[0][mq][jb] + acc[SETS - 1][mq][jb] : acc[0][mq][jb]; });
     }
     __syncthreads();
     // four rows are a unit; wave w finishes units w, w + WAVES ..: lane l row l / 16, columns 8 (l % 16) ..
@@ -317,18 +359,22 @@ __global__ __launch_bounds__(64 * WAVES, WAVES / 4) void w4a16_mid_kernel(const 
     for (int t = 0; t < UT; ++t) {
         const int u = w + t * WAVES < XQ ? w + t * WAVES : w;
         const float* src = red_of(0) + (4 * u + kq) * kMidRedStride + 8 * slot;
-        lo[t] = *reinterpret_cast<const f4*>(src);
-        hi[t] = *reinterpret_cast<const f4*>(src + 4);
+        f4 l[WAVES], h[WAVES];
 #pragma unroll
-        for (int ww = 1; ww < WAVES; ++ww) {
-            lo[t] += *reinterpret_cast<const f4*>(src + ww * MR * kMidRedStride);
-            hi[t] += *reinterpret_cast<const f4*>(src + ww * MR * kMidRedStride + 4);
+        for (int ww = 0; ww < WAVES; ++ww) {
+            l[ww] = *reinterpret_cast<const f4*>(src + ww * MR * kMidRedStride);
+            h[ww] = *reinterpret_cast<const f4*>(src + ww * MR * kMidRedStride + 4);
         }
+        typename Sums::Total sum_lo{}, sum_hi{};
+        Sums::add(sum_lo, l);
+        Sums::add(sum_hi, h);
+        lo[t] = Sums::rounded(sum_lo);
+        hi[t] = Sums::rounded(sum_hi);
     }
     if (a.splits > 1) {  // uniform
         // K split over workgroups.  Every wave exchanges its own quarter of the rows: it writes its sums to the
         // quarter's slot, waits until the memory side has acknowledged them and counts itself in; the wave that
-        // completes the count adds the slots in split order.  The accesses and what they rely on are those of the
+        // completes the count adds the slots, in an order that does not depend on it.  The accesses and what they rely on are those of the
         // 128-column kernel's exchange (w4a16_tile.hip); no workgroup barrier, since nobody else's stores matter.
         constexpr int kSlotBytes = WAVES * UT * 2048;
         char* tile = reinterpret_cast<char*>(a.part) + (size_t)strip * a.splits * kSlotBytes;
@@ -349,27 +395,36 @@ __global__ __launch_bounds__(64 * WAVES, WAVES / 4) void w4a16_mid_kernel(const 
         if (arrived != a.splits - 1) return;
         asm volatile("" ::: "memory");
         if (lane == 0) __hip_atomic_store(count, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        // Slots are requested up to eight together; those that do not exist lie beyond the descriptor and read as zeros.
+        typename Sums::Total total_lo[UT], total_hi[UT];
 #pragma unroll
-        for (int t = 0; t < UT; ++t) lo[t] = hi[t] = f4{0.f, 0.f, 0.f, 0.f};
-        constexpr int kBatch = UT <= 3 ? 8 : 4;  // splits requested together
-        for (int s0 = 0; s0 < a.splits; s0 += kBatch) {
-            u32x4 v[kBatch][2 * UT];
+        for (int t = 0; t < UT; ++t) total_lo[t] = total_hi[t] = typename Sums::Total{};
+        auto gather = [&](int first, auto batch) __attribute__((always_inline)) {
+            constexpr int N = decltype(batch)::value;
+            const __amdgpu_buffer_rsrc_t slots = __builtin_amdgcn_make_buffer_rsrc(
+                tile + (size_t)first * kSlotBytes, 0, (unsigned)((a.splits - first) * kSlotBytes), 0x00020000);
+            f4 v[2 * UT][N];
 #pragma unroll
-            for (int b = 0; b < kBatch; ++b) {
-                const int s = s0 + b < a.splits ? s0 + b : a.splits - 1;
+            for (int b = 0; b < N; ++b)
 #pragma unroll
                 for (int t = 0; t < 2 * UT; ++t)
-                    v[b][t] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rsrc, mine + 1024u * t, (uint32_t)(s * kSlotBytes), kMidDeviceScope));
-            }
+                    v[t][b] = __builtin_bit_cast(f4, __builtin_amdgcn_raw_buffer_load_b128(slots, mine + (uint32_t)(b * kSlotBytes) + 1024u * t, 0, kMidDeviceScope));
 #pragma unroll
-            for (int b = 0; b < kBatch; ++b) {
-                if (s0 + b >= a.splits) break;  // uniform
-#pragma unroll
-                for (int t = 0; t < UT; ++t) {
-                    lo[t] += __builtin_bit_cast(f4, v[b][2 * t]);
-                    hi[t] += __builtin_bit_cast(f4, v[b][2 * t + 1]);
-                }
+            for (int t = 0; t < UT; ++t) {
+                Sums::add(total_lo[t], v[2 * t]);
+                Sums::add(total_hi[t], v[2 * t + 1]);
             }
+        };
+        for (int first = 0; first < a.splits; first += 8) {
+            const int rest = a.splits - first;  // uniform
+            if (rest > 4) gather(first, std::integral_constant<int, 8>{});
+            else if (rest > 2) gather(first, std::integral_constant<int, 4>{});
+            else gather(first, std::integral_constant<int, 2>{});
+        }
+#pragma unroll
+        for (int t = 0; t < UT; ++t) {
+            lo[t] = Sums::rounded(total_lo[t]);
+            hi[t] = Sums::rounded(total_hi[t]);
         }
     }
 #pragma unroll
@@ -409,28 +464,28 @@ __global__ __launch_bounds__(64 * WAVES, WAVES / 4) void w4a16_mid_kernel(const 
 // ---------------------------------------------------------------------------------
 // More than 64 KiB of LDS is a property of (kernel, device): set for all of them on the first launch on a device, so that a
 // later launch that is recorded into a graph sets nothing.
-template <int MQ, int WAVES>
+template <int MQ, int WAVES, int SETS>
 static bool mid_allow_lds() {
     const int bytes = (int)MidLds<MQ, WAVES>::kBytes;
-    return hipFuncSetAttribute(reinterpret_cast<const void*>(&w4a16_mid_kernel<MQ, WAVES, false>), hipFuncAttributeMaxDynamicSharedMemorySize, bytes) == hipSuccess &&
-           hipFuncSetAttribute(reinterpret_cast<const void*>(&w4a16_mid_kernel<MQ, WAVES, true>), hipFuncAttributeMaxDynamicSharedMemorySize, bytes) == hipSuccess;
+    return hipFuncSetAttribute(reinterpret_cast<const void*>(&w4a16_mid_kernel<MQ, WAVES, SETS, false>), hipFuncAttributeMaxDynamicSharedMemorySize, bytes) == hipSuccess &&
+           hipFuncSetAttribute(reinterpret_cast<const void*>(&w4a16_mid_kernel<MQ, WAVES, SETS, true>), hipFuncAttributeMaxDynamicSharedMemorySize, bytes) == hipSuccess;
 }
 static bool mid_prepare_device() {
     static std::atomic<unsigned long long> done{0};
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return false;
     if ((done.load(std::memory_order_acquire) >> dev) & 1ull) return true;
-    if (!mid_allow_lds<1, 8>() || !mid_allow_lds<2, 8>() || !mid_allow_lds<3, 4>() || !mid_allow_lds<4, 4>()) return false;
+    if (!mid_allow_lds<1, 8, 2>() || !mid_allow_lds<2, 8, 2>() || !mid_allow_lds<3, 4, 1>() || !mid_allow_lds<3, 4, 2>() || !mid_allow_lds<4, 4, 1>()) return false;
     done.fetch_or(1ull << dev, std::memory_order_release);
     return true;
 }
 
-template <int MQ, int WAVES>
+template <int MQ, int WAVES, int SETS>
 static hipError_t mid_launch_rows(const MidArgs& a, bool ext, hipStream_t stream) {
     const dim3 grid(a.N / 128, a.splits), block(64 * WAVES);
     constexpr size_t shmem = MidLds<MQ, WAVES>::kBytes;
-    if (ext) hipLaunchKernelGGL((w4a16_mid_kernel<MQ, WAVES, true>), grid, block, shmem, stream, a);
-    else hipLaunchKernelGGL((w4a16_mid_kernel<MQ, WAVES, false>), grid, block, shmem, stream, a);
+    if (ext) hipLaunchKernelGGL((w4a16_mid_kernel<MQ, WAVES, SETS, true>), grid, block, shmem, stream, a);
+    else hipLaunchKernelGGL((w4a16_mid_kernel<MQ, WAVES, SETS, false>), grid, block, shmem, stream, a);
     return hipGetLastError();
 }
 
@@ -465,10 +520,10 @@ int mid_launch(const void* A, int64_t lda, int k_valid, const void* B, const voi
     if (!mid_prepare_device()) return UNIQL_E_LAUNCH;
     hipError_t e;
     switch (mid_row_tiles(m)) {
-        case 1: e = mid_launch_rows<1, 8>(a, ext, stream); break;
-        case 2: e = mid_launch_rows<2, 8>(a, ext, stream); break;
-        case 3: e = mid_launch_rows<3, 4>(a, ext, stream); break;
-        default: e = mid_launch_rows<4, 4>(a, ext, stream); break;
+        case 1: e = mid_launch_rows<1, 8, 2>(a, ext, stream); break;
+        case 2: e = mid_launch_rows<2, 8, 2>(a, ext, stream); break;
+        case 3: e = mid_sets(m, plan.upw) == 2 ? mid_launch_rows<3, 4, 2>(a, ext, stream) : mid_launch_rows<3, 4, 1>(a, ext, stream); break;
+        default: e = mid_launch_rows<4, 4, 1>(a, ext, stream); break;
     }
     return e == hipSuccess ? UNIQL_OK : UNIQL_E_LAUNCH;
 }
