@@ -15,6 +15,15 @@ struct MidPlan {
     double us;   // expected time
 };
 
+// A lane offset behind every descriptor of this kernel, also where the bounds check adds or subtracts a scalar offset.
+constexpr uint32_t kMidNoLoad = 0x80000000u;
+// Bytes of X from column 128 g of its first row to the end of its last row; none for a unit that does not exist.
+constexpr uint32_t mid_x_records(uint32_t x_bytes, int g, bool real) {
+    return real && x_bytes > 256u * (uint32_t)g ? x_bytes - 256u * (uint32_t)g : 0u;
+}
+// Bytes of a group's eight packed rows over all columns.
+constexpr int64_t mid_group_bytes(int n) { return 64 * (int64_t)n; }
+
 static inline int mid_row_tiles(int m) { return m <= 16 ? 1 : m <= 32 ? 2 : m <= 48 ? 3 : 4; }  // of 16 rows
 
 // Accumulators of a wave: the products of the low and of the high codes apart (SETS = 2) wherever the registers hold both

@@ -135,14 +135,17 @@ __global__ __launch_bounds__(64 * WAVES, WAVES / 4) void w4a16_mid_kernel(const 
     u32x4 xv[XQ];
     // A load brings four rows; rows and columns of X that do not exist lie beyond the descriptor and read as zeros.
     const uint32_t x_lane = (uint32_t)kq * (uint32_t)a.ldx * 2u + 16u * (uint32_t)slot, x_step = 8u * (uint32_t)a.ldx;
-    // What a unit needs from memory.  Every load goes through a descriptor that covers what exists of its group, nothing
-    // for the group behind a wave's last one, so that all units run the same loop body.
+    // What a unit needs from memory.  Every load goes through a descriptor that covers what exists of its group, and none
+    // of them brings anything for the group behind a wave's last one, so that all units run the same loop body: X and the
+    // scales by a descriptor of no bytes at scalar offset zero, the packed rows, which have scalar offsets, by a lane offset
+    // behind a descriptor of full size.  So no load leaves its descriptor, however the bounds check counts a scalar offset.
     const uint32_t packed_row_bytes = 16u * (uint32_t)N4;
-    auto x_of = [&](bool real) __attribute__((always_inline)) {
-        return __builtin_amdgcn_make_buffer_rsrc(const_cast<half_t*>(a.X), 0, real ? a.x_bytes : 0u, 0x00020000);
+    auto x_of = [&](int g, bool real) __attribute__((always_inline)) {
+        return __builtin_amdgcn_make_buffer_rsrc(const_cast<half_t*>(a.X) + (size_t)128 * g, 0,
+                                                 __builtin_amdgcn_readfirstlane(mid_x_records(a.x_bytes, g, real)), 0x00020000);
     };
-    auto w_of = [&](int g, bool real) __attribute__((always_inline)) {
-        return __builtin_amdgcn_make_buffer_rsrc(const_cast<u32x4*>(strip_w + (size_t)(8 * g) * N4), 0, real ? 8u * packed_row_bytes : 0u, 0x00020000);
+    auto w_of = [&](int g) __attribute__((always_inline)) {
+        return __builtin_amdgcn_make_buffer_rsrc(const_cast<u32x4*>(strip_w + (size_t)(8 * g) * N4), 0, (unsigned)mid_group_bytes(a.N), 0x00020000);
     };
     auto s_of = [&](int g, bool real) __attribute__((always_inline)) {
         return __builtin_amdgcn_make_buffer_rsrc(const_cast<half_t*>(strip_s + (size_t)(a.per_column ? 0 : g) * a.N), 0, real ? 256u : 0u, 0x00020000);
@@ -150,21 +153,21 @@ __global__ __launch_bounds__(64 * WAVES, WAVES / 4) void w4a16_mid_kernel(const 
     auto load_x = [&](__amdgpu_buffer_rsrc_t rsrc, int g, int i) __attribute__((always_inline)) {
         const bool real = !EXT || 128 * g + 8 * slot < a.k_valid;
         const uint32_t off = x_lane + (uint32_t)i * x_step;
-        xv[i] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rsrc, real ? off : 0x80000000u, 256u * (uint32_t)g, 0));
+        xv[i] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rsrc, real ? off : kMidNoLoad, 0, 0));
     };
-    auto load_row = [&](__amdgpu_buffer_rsrc_t rsrc, int row) __attribute__((always_inline)) {
-        unit.wq[row] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rsrc, 16u * piece_off, (uint32_t)row * packed_row_bytes, kMidNonTemporal));
+    auto load_row = [&](__amdgpu_buffer_rsrc_t rsrc, int row, bool real) __attribute__((always_inline)) {
+        unit.wq[row] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rsrc, real ? 16u * piece_off : kMidNoLoad, (uint32_t)row * packed_row_bytes, kMidNonTemporal));
     };
     auto load_scales = [&](__amdgpu_buffer_rsrc_t rsrc) __attribute__((always_inline)) {
         unit.sc = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rsrc, 2u * scale_off, 0, 0));
     };
     auto load_unit = [&](int g) __attribute__((always_inline)) {
-        const auto xr = x_of(true), wr = w_of(g, true);
+        const auto xr = x_of(g, true), wr = w_of(g);
 #pragma unroll
         for (int i = 0; i < XQ; ++i) load_x(xr, g, i);
         load_scales(s_of(g, true));
 #pragma unroll
-        for (int row = 0; row < 8; ++row) load_row(wr, row);
+        for (int row = 0; row < 8; ++row) load_row(wr, row, true);
         __builtin_amdgcn_sched_barrier(0);
     };
     auto fence = [&]() __attribute__((always_inline)) {
@@ -327,16 +330,16 @@ __global__ __launch_bounds__(64 * WAVES, WAVES / 4) void w4a16_mid_kernel(const 
             for (int g = g_begin; g < g_end; ++g) {
                 stage();
                 const bool more = g + 1 < g_end;
-                const auto xr = x_of(more), wr = w_of(g + 1, more), sr = s_of(g + 1, more);
+                const auto xr = x_of(g + 1, more), wr = w_of(g + 1), sr = s_of(g + 1, more);
                 process([&](int b) __attribute__((always_inline)) {
 #pragma unroll
                     for (int i = 2 * b; i < 2 * b + 2; ++i)
                         if (i < XQ) load_x(xr, g + 1, i);
                     if (b == 8) load_scales(sr);
-                    if (b >= 9 && b < 13) load_row(wr, b - 9);
+                    if (b >= 9 && b < 13) load_row(wr, b - 9, more);
                 });
 #pragma unroll
-                for (int row = 4; row < 8; ++row) load_row(wr, row);
+                for (int row = 4; row < 8; ++row) load_row(wr, row, more);
                 __builtin_amdgcn_sched_barrier(0);
             }
         }
@@ -489,10 +492,11 @@ static hipError_t mid_launch_rows(const MidArgs& a, bool ext, hipStream_t stream
     return hipGetLastError();
 }
 
-// Rows, and the 32-bit offsets of the loads: row strides and packed weights as far as the tiled kernels take them.
+// Rows, and the 32-bit offsets of the loads: row strides and packed weights as far as the tiled kernels take them, and
+// descriptors of X and of a group's packed rows that end in front of kMidNoLoad.
 bool mid_shape_ok(int m, int n, int k, int64_t lda) {
     return m >= kMidMinRows && m <= kMidMaxRows && lda < (1LL << 24) && ((int64_t)(m - 1) * lda + k) * 2 < (1LL << 31) &&
-           (int64_t)k * n / 2 < (1LL << 32);
+           (int64_t)k * n / 2 < (1LL << 32) && mid_group_bytes(n) <= (int64_t)kMidNoLoad;
 }
 
 int mid_launch(const void* A, int64_t lda, int k_valid, const void* B, const void* S, void* D, const Epilogue& epi, void* accum,
