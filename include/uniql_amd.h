@@ -142,11 +142,10 @@ int uniql_w4a16_gemm(const void* A, int64_t lda, const void* B, const void* S, v
  * Every call on a GPU shares that GPU's array: calls that may overlap on one GPU (different
  * streams, or graphs replayed concurrently) race and must use uniql_w4a16_gemm with separate
  * buffers instead.
- * Before a call is recorded into a graph, one call with the same m class (1, 2, 3..4, 5..8, 9..16,
- * 17..64, more), flags and rotation must have run eagerly on that device: the first call per device
- * resolves the array's address (hipGetSymbolAddress) and the first launch of a kernel that uses
- * more than 64 KiB of LDS sets a function attribute, neither of which may happen while a stream
- * is capturing.
+ * Before a call is recorded into a graph, one call of this function, of any sizes and flags, must have run
+ * eagerly on that device: the first one resolves the array's address (hipGetSymbolAddress) and lets every
+ * kernel of these calls use more than 64 KiB of LDS (a function attribute), neither of which may happen while
+ * a stream is capturing.  (The other product calls set the attributes on their first call on a device, too.)
  */
 size_t uniql_w4a16_gemm_static_limit(int which);
 int uniql_w4a16_gemm_static(const void* A, int64_t lda, const void* B, const void* S, void* D,

@@ -1,5 +1,6 @@
 // extern "C" surface: argument checks and dispatch.  Nothing here allocates,
 // synchronises or throws.
+#include <atomic>
 #include <mutex>
 
 #include "common.hpp"
@@ -49,6 +50,11 @@ int cut_columns_launch(const void* B, const void* S, int n, int k, int k_real, c
                        void* B_out, void* S_out, int n_pad, hipStream_t stream);
 int cut_rows_launch(const void* B, const void* S, int n, int groups_in, int units, int full, int kept, int n_real, void* B_out,
                     void* S_out, int n_pad, hipStream_t stream);
+bool stream_allow_lds();
+bool mid_allow_lds();
+bool tile_allow_lds();
+bool wide_allow_lds();
+bool fwht_allow_lds();
 }  // namespace uniql
 
 using namespace uniql;
@@ -56,6 +62,19 @@ using namespace uniql;
 static inline bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 static inline bool is_pow2(int v) { return v > 0 && (v & (v - 1)) == 0; }
 static inline size_t round256(size_t v) { return (v + 255) & ~(size_t)255; }
+
+// More than 64 KiB of LDS is a property of (kernel, device) that may not be set while a stream is capturing, and which kernel
+// a layer call launches follows from all of its sizes: so the first call on a device sets it for every kernel of these calls.
+static bool prepare_device() {
+    static std::atomic<unsigned long long> done{0};
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess) return false;
+    const unsigned long long bit = dev < 64 ? 1ull << dev : 0ull;  // further devices: set again on every call
+    if (done.load(std::memory_order_acquire) & bit) return true;
+    if (!stream_allow_lds() || !mid_allow_lds() || !tile_allow_lds() || !wide_allow_lds() || !fwht_allow_lds()) return false;
+    done.fetch_or(bit, std::memory_order_release);
+    return true;
+}
 
 static int check_linear_shape(int m, int n, int k, int groups) {
     if (m < 0 || n <= 0 || k <= 0) return UNIQL_E_SHAPE;
@@ -350,6 +369,7 @@ static int linear_impl(const void* A, int64_t lda, int k_in, const void* B, cons
             return UNIQL_E_SHAPE;
     if (use_stream && !stream_shape_ok(k, ld_kernel)) return UNIQL_E_SHAPE;
     if (check_only) return UNIQL_OK;
+    if (!prepare_device()) return UNIQL_E_LAUNCH;
     if (pad_first) {
         const int e = pad_rows_launch(A, lda, k_in, temp, k, m, st);
         if (e != UNIQL_OK) return e;

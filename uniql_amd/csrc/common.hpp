@@ -16,6 +16,14 @@ typedef float f4 __attribute__((ext_vector_type(4)));
 typedef float f16 __attribute__((ext_vector_type(16)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
+// Lets a kernel be launched with more than 64 KiB of LDS on the current device.  Not while a stream is capturing: the kernels
+// of a layer call are all prepared on the first call on a device (prepare_device in capi.hip).
+template <typename K>
+static bool allow_lds(K kern, size_t bytes) {
+    return bytes <= 64 * 1024 || hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                                     (int)bytes) == hipSuccess;
+}
+
 constexpr int kGroup = 128;      // quantisation group along K
 constexpr int kTileK = 16;       // K rows covered by one packed weight row
 constexpr int kChunkN = 64;      // columns covered by 512 contiguous bytes of a packed row

@@ -380,24 +380,31 @@ __global__ __launch_bounds__(64 * RowShape<LOG2L>::kWaves, 4) void fwht_rows_ker
     }
 }
 
-// more than 64 KB of LDS: a property of (kernel, device), set on the first launch there
+// more than 64 KiB of LDS, for calls that launch one kernel: set on its first launch on a device
 template <typename K>
 static bool allow_lds(K kern, size_t bytes, std::atomic<unsigned long long>& done) {
     if (bytes <= 64 * 1024) return true;
     int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return false;
-    if ((done.load(std::memory_order_acquire) >> dev) & 1ull) return true;
-    if (hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024) != hipSuccess)
-        return false;
-    done.fetch_or(1ull << dev, std::memory_order_release);
+    if (hipGetDevice(&dev) != hipSuccess) return false;
+    const unsigned long long bit = dev < 64 ? 1ull << dev : 0ull;
+    if (done.load(std::memory_order_acquire) & bit) return true;
+    if (!allow_lds(kern, 160 * 1024)) return false;
+    done.fetch_or(bit, std::memory_order_release);
     return true;
 }
 
 template <typename T, int LOG2L>
+static bool fwht_rows_allow_lds() {
+    static std::atomic<unsigned long long> done{0};
+    return allow_lds(&fwht_rows_kernel<T, LOG2L>, RowShape<LOG2L>::kBytes, done);
+}
+// the rotations in front of a layer's product
+bool fwht_allow_lds() { return fwht_rows_allow_lds<half_t, 14>() && fwht_rows_allow_lds<half_t, 15>(); }
+
+template <typename T, int LOG2L>
 static int fwht_rows_go(const void* x, void* y, int64_t rows, float scale, hipStream_t stream) {
     using S = RowShape<LOG2L>;
-    static std::atomic<unsigned long long> done{0};
-    if (!allow_lds(&fwht_rows_kernel<T, LOG2L>, S::kBytes, done)) return UNIQL_E_LAUNCH;
+    if (!fwht_rows_allow_lds<T, LOG2L>()) return UNIQL_E_LAUNCH;
     // The workgroups that the chip holds at once, by registers.  fp32 rows of 4096 and more each get their own: memory is
     // busy without the request ahead, and rows in launch order use it better (16384 rows of 8192: 199 us, 207 with
     // workgroups that stay; fp16 102 either way).

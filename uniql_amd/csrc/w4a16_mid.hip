@@ -26,7 +26,6 @@
 // number of products that enter one accumulator one after another, hence two sets of accumulators (SETS, mid_sets) and
 // mid_plan's longest_chain, and sums of waves and workgroups in pairs, up to 16 rows in 64 bits: the streaming kernel adds its
 // workgroups' sums as integers.  With one set and the sums added in a row it was up to 1.39 x.
-#include <atomic>
 #include <type_traits>
 
 #include "common.hpp"
@@ -465,22 +464,14 @@ __global__ __launch_bounds__(64 * WAVES, WAVES / 4) void w4a16_mid_kernel(const 
 // ---------------------------------------------------------------------------------
 // host side
 // ---------------------------------------------------------------------------------
-// More than 64 KiB of LDS is a property of (kernel, device): set for all of them on the first launch on a device, so that a
-// later launch that is recorded into a graph sets nothing.
 template <int MQ, int WAVES, int SETS>
-static bool mid_allow_lds() {
-    const int bytes = (int)MidLds<MQ, WAVES>::kBytes;
-    return hipFuncSetAttribute(reinterpret_cast<const void*>(&w4a16_mid_kernel<MQ, WAVES, SETS, false>), hipFuncAttributeMaxDynamicSharedMemorySize, bytes) == hipSuccess &&
-           hipFuncSetAttribute(reinterpret_cast<const void*>(&w4a16_mid_kernel<MQ, WAVES, SETS, true>), hipFuncAttributeMaxDynamicSharedMemorySize, bytes) == hipSuccess;
+static bool mid_allow_lds_rows() {
+    return allow_lds(&w4a16_mid_kernel<MQ, WAVES, SETS, false>, MidLds<MQ, WAVES>::kBytes) &&
+           allow_lds(&w4a16_mid_kernel<MQ, WAVES, SETS, true>, MidLds<MQ, WAVES>::kBytes);
 }
-static bool mid_prepare_device() {
-    static std::atomic<unsigned long long> done{0};
-    int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return false;
-    if ((done.load(std::memory_order_acquire) >> dev) & 1ull) return true;
-    if (!mid_allow_lds<1, 8, 2>() || !mid_allow_lds<2, 8, 2>() || !mid_allow_lds<3, 4, 1>() || !mid_allow_lds<3, 4, 2>() || !mid_allow_lds<4, 4, 1>()) return false;
-    done.fetch_or(1ull << dev, std::memory_order_release);
-    return true;
+bool mid_allow_lds() {
+    return mid_allow_lds_rows<1, 8, 2>() && mid_allow_lds_rows<2, 8, 2>() && mid_allow_lds_rows<3, 4, 1>() &&
+           mid_allow_lds_rows<3, 4, 2>() && mid_allow_lds_rows<4, 4, 1>();
 }
 
 template <int MQ, int WAVES, int SETS>
@@ -521,7 +512,6 @@ int mid_launch(const void* A, int64_t lda, int k_valid, const void* B, const voi
     a.epi = epi;
     const bool ext = epi.gated || epi.bias || epi.residual || epi.relu2 || epi.transpose || epi.n_store != n ||
                      epi.ldd != n || k_valid != k || !epi.vec_ok;
-    if (!mid_prepare_device()) return UNIQL_E_LAUNCH;
     hipError_t e;
     switch (mid_row_tiles(m)) {
         case 1: e = mid_launch_rows<1, 8, 2>(a, ext, stream); break;

@@ -41,8 +41,6 @@
 // looks at the returned old word: whoever sees count == splits - 1 was last, owns the
 // total (old + own), stores the output and writes the word back to zero.  Integer adds
 // commute, so the result does not depend on arrival order, and nobody waits for anyone.
-#include <atomic>
-
 #include "common.hpp"
 #include "fwht_device.hpp"
 
@@ -569,19 +567,23 @@ static hipError_t launch_one(StreamArgs a, hipStream_t stream) {
         shmem += (size_t)a.M * (a.K + (a.K >> 5)) * 4;
     }
     auto kern = &w4a16_stream_kernel<RC, HAD, WAVES, EXT>;
-    if (shmem > 64 * 1024) {
-        static std::atomic<unsigned long long> attribute_set{0};  // a bit per device, once per instantiation
-        int dev = 0;
-        if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return hipErrorInvalidDevice;
-        if (!((attribute_set.load(std::memory_order_acquire) >> dev) & 1ull)) {
-            const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
-                                                     hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
-            if (e != hipSuccess) return e;
-            attribute_set.fetch_or(1ull << dev, std::memory_order_release);
-        }
-    }
     hipLaunchKernelGGL(kern, dim3(a.N / 128, a.splits), dim3(64 * WAVES), shmem, stream, a);
     return hipGetLastError();
+}
+
+// The forms whose LDS may exceed 64 KiB: whole rows rotated inside the kernel (the rows' images), sixteen rows with eight waves
+// (staging and exchange areas).
+template <int RC, int HAD, int WAVES>
+static bool stream_allow_lds_one() {
+    return allow_lds(&w4a16_stream_kernel<RC, HAD, WAVES, false>, 160 * 1024) && allow_lds(&w4a16_stream_kernel<RC, HAD, WAVES, true>, 160 * 1024);
+}
+template <int RC>
+static bool stream_allow_lds_rows() {
+    return stream_allow_lds_one<RC, 2, 4>() && stream_allow_lds_one<RC, 2, 8>();
+}
+bool stream_allow_lds() {
+    return stream_allow_lds_rows<1>() && stream_allow_lds_rows<2>() && stream_allow_lds_rows<4>() && stream_allow_lds_rows<8>() &&
+           stream_allow_lds_rows<16>() && stream_allow_lds_one<16, 0, 8>() && stream_allow_lds_one<16, 1, 8>();
 }
 
 template <int RC, int HAD>

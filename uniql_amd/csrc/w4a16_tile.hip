@@ -33,8 +33,6 @@
 //
 // When K is also split over workgroups every workgroup writes its fp32 partial tile to a scratch
 // area and the last one to arrive (one arrival count per tile) adds them in split order.
-#include <atomic>
-
 #include "common.hpp"
 #include "tile_plan.hpp"
 
@@ -570,18 +568,6 @@ template <int MT, bool EXT, int KW>
 static hipError_t tile_launch_one(const TileArgs& a, int grid, hipStream_t stream) {
     const size_t shmem = TileLds<MT, KW>::kBytes;
     auto kern = &w4a16_tile_kernel<MT, EXT, KW>;
-    if (shmem > 64 * 1024) {
-        // the attribute is a property of (instantiation, device): set it on the first launch there
-        static std::atomic<unsigned long long> done{0};
-        int dev = 0;
-        if (hipGetDevice(&dev) != hipSuccess) return hipErrorInvalidDevice;
-        if (dev < 0 || dev >= 64 || !((done.load(std::memory_order_relaxed) >> dev) & 1ull)) {
-            hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
-                                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)shmem);
-            if (e != hipSuccess) return e;
-            if (dev >= 0 && dev < 64) done.fetch_or(1ull << dev, std::memory_order_relaxed);
-        }
-    }
     hipLaunchKernelGGL(kern, dim3(grid), dim3(256 * KW), shmem, stream, a);
     return hipGetLastError();
 }
@@ -589,6 +575,15 @@ static hipError_t tile_launch_one(const TileArgs& a, int grid, hipStream_t strea
 template <int MT, int KW>
 static hipError_t tile_launch_ext(const TileArgs& a, bool ext, int grid, hipStream_t stream) {
     return ext ? tile_launch_one<MT, true, KW>(a, grid, stream) : tile_launch_one<MT, false, KW>(a, grid, stream);
+}
+
+template <int MT, int KW>
+static bool tile_allow_lds_one() {
+    return allow_lds(&w4a16_tile_kernel<MT, false, KW>, TileLds<MT, KW>::kBytes) && allow_lds(&w4a16_tile_kernel<MT, true, KW>, TileLds<MT, KW>::kBytes);
+}
+bool tile_allow_lds() {
+    return tile_allow_lds_one<1, 1>() && tile_allow_lds_one<1, 2>() && tile_allow_lds_one<2, 1>() && tile_allow_lds_one<2, 2>() &&
+           tile_allow_lds_one<3, 1>() && tile_allow_lds_one<4, 1>();
 }
 
 // columns first .. first + columns - 1 of the layer's n

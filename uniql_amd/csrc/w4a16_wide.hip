@@ -42,7 +42,6 @@
 // what the code is written for (about 4.6 per MFMA).  vmcnt is counted by hand: nothing but the
 // loop's own loads uses the counter, and their number and order per iteration are fixed.  The
 // last group runs a copy of the loop body that requests nothing but the last upper rows.
-#include <atomic>
 
 #include "common.hpp"
 
@@ -487,17 +486,10 @@ bool wide_shape_ok(int m, int n, int k, int groups, int64_t ldx) {
            (int64_t)(n / 256) * ((m + 255) / 256) <= 0x7fffffffLL;
 }
 
+bool wide_allow_lds() { return allow_lds(&w4a16_wide_kernel, kWideLdsBytes); }
+
 static hipError_t wide_launch_one(const WideArgs& a, int grid, hipStream_t stream) {
     auto kern = &w4a16_wide_kernel;
-    static std::atomic<unsigned long long> done{0};  // the attribute is set once per device
-    int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess) return hipErrorInvalidDevice;
-    if (dev < 0 || dev >= 64 || !((done.load(std::memory_order_relaxed) >> dev) & 1ull)) {
-        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                           kWideLdsBytes);
-        if (e != hipSuccess) return e;
-        if (dev >= 0 && dev < 64) done.fetch_or(1ull << dev, std::memory_order_relaxed);
-    }
     hipLaunchKernelGGL(kern, dim3(grid), dim3(256), kWideLdsBytes, stream, a);
     return hipGetLastError();
 }
