@@ -80,7 +80,9 @@ int uniql_clear(void* p, size_t bytes, void* stream);
  *              and all zero again when the kernels have finished: the words through
  *              which workgroups that share output columns combine their partial sums
  *              (streaming kernel: a 64-bit sum|count word per output element of up to
- *              16 rows; tiled kernel: an arrival count per output tile).  Replaces the
+ *              16 rows; tiled kernel: an arrival count per output tile).  As many as any plan
+ *              for m, n, k needs; uniql_w4a16_linear_workspace tells what one call needs, nothing
+ *              where it does not split K.  Replaces the
  *              reference's per-call fp16 `C` buffer and its locks
  *              (marlin_gemm_kernel.cuh:515-570,1018).  A caller clears it once and
  *              reuses it for every call on the same stream; two calls that may run
@@ -132,7 +134,7 @@ int uniql_w4a16_gemm(const void* A, int64_t lda, const void* B, const void* S, v
  * Same arguments and results as uniql_w4a16_gemm without `accum` and `temp`: both come from a
  * 16 MiB array inside the library's device image (one copy per GPU, held until the process ends):
  * uniql_w4a16_gemm_static_limit(0) bytes of exchange words (4 MiB: the streaming kernel's 16-row
- * slab up to n = 32768) and uniql_w4a16_gemm_static_limit(1) bytes of temporary area (12 MiB:
+ * slab up to n = 32768; a wider call of so many rows is refused also where its plan exchanges nothing) and uniql_w4a16_gemm_static_limit(1) bytes of temporary area (12 MiB:
  * rotated activations, the tiled kernel's partial tiles).  A call whose plan needs more of either
  * returns UNIQL_E_STATIC_LIMIT and launches nothing (the needs are those of the kernel that takes
  * the call: at most what uniql_w4a16_linear_workspace reports, nothing at all for a long prefill

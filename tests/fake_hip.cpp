@@ -10,7 +10,7 @@ struct Dim3 {
     uint32_t x, y, z;
 };
 static std::set<const void*> large;  // kernels that may use more than 64 KiB
-static int attributes, launches, refused;
+static int attributes, launches, refused, grid_y;
 static thread_local Dim3 config_grid, config_block;
 static thread_local size_t config_lds;
 static thread_local void* config_stream;
@@ -27,8 +27,9 @@ int hipFuncSetAttribute(const void* kernel, int, int) {
     large.insert(kernel);
     return 0;
 }
-int hipLaunchKernel(const void* kernel, Dim3, Dim3, void**, size_t lds, void*) {
+int hipLaunchKernel(const void* kernel, Dim3 grid, Dim3, void**, size_t lds, void*) {
     ++launches;
+    grid_y = (int)grid.y;
     refused += lds > 64 * 1024 && large.count(kernel) == 0;
     return 0;
 }
@@ -42,5 +43,6 @@ int __hipPopCallConfiguration(Dim3* grid, Dim3* block, size_t* lds, void** strea
 }
 int fake_attributes() { return attributes; }
 int fake_launches() { return launches; }
+int fake_grid_y() { return grid_y; }  // of the last launch
 int fake_refused() { return refused; }  // launches with more LDS than their kernel was allowed
 }

@@ -1,6 +1,7 @@
-"""What a layer call asks of the HIP runtime beside launches, on a recorder in the runtime's place (tests/fake_hip.cpp, no
-GPU): function attributes are set on the first call on a device, for every kernel that a later call may launch, so
-that a call recorded into a graph sets none."""
+"""What a layer call asks of the HIP runtime beside launches and of its caller, on a recorder in the runtime's place
+(tests/fake_hip.cpp, no GPU).  Function attributes are set on the first call on a device, for every kernel that a later call may
+launch, so that a call recorded into a graph sets none; exchange words, which a graph may have to clear on every replay, are
+asked for where workgroups share output columns and nowhere else."""
 import os
 import shutil
 import subprocess
@@ -12,7 +13,7 @@ from uniql_amd.build import LIB_PATH
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 
-CALLS = r"""
+SETUP = r"""
 import ctypes, itertools, sys
 hip = ctypes.CDLL(sys.argv[1], mode=ctypes.RTLD_GLOBAL)
 lib = ctypes.CDLL(sys.argv[2])
@@ -34,7 +35,11 @@ def call(m, k, n, had=0, flags=0, k_in=None, static=False, n_out=None):
                                       fake, acc.value, fake, tmp.value, m, n, k, k // 128, had, 1.0, flags, None)
     assert code == (-7 if code == -7 and static else 0), (m, k, n, had, flags, code)
     assert code != 0 or hip.fake_launches() > before
+    return None if static else acc.value
 
+"""
+
+CALLS = SETUP + r"""
 first = eval(sys.argv[3])
 call(*first[0], **first[1])
 once = hip.fake_attributes()
@@ -72,4 +77,28 @@ def recorder(tmp_path_factory):
                                    "((1, 512, 256), dict(static=True))"])
 def test_the_first_call_prepares_every_later_one(recorder, first):
     run = subprocess.run([sys.executable, "-c", CALLS, recorder, LIB_PATH, first], capture_output=True, text=True, timeout=300)
+    assert run.returncode == 0, run.stderr[-2000:]
+
+
+WORDS = SETUP + r"""
+skinny = 1 << 1
+for k, n in itertools.product((256, 512, 640, 2048, 2176, 4096, 8192, 8320, 14336), (128, 1024, 4096, 18304, 18432, 24320, 28672)):
+    for m in (1, 2, 3, 4, 7, 8, 9, 12, 16, 20, 35):
+        for tune in (0, 1, 3, 8 << 8, 4 << 8 | 2, 8 << 8 | 32):   # groups a wave, waves a workgroup
+            words = call(m, k, n, flags=skinny | tune << 8)
+            split = hip.fake_grid_y() > 1   # of the last slab of 16 rows
+            slabs = [16] * (m // 16) + ([m % 16] if m % 16 else [])
+            if len(slabs) == 1:
+                assert words == (m * n * 8 if split else 0), (m, k, n, tune, words)
+            else:
+                assert words in (0, slabs[-1] * n * 8, 16 * n * 8) and (words > 0 or not split)
+                lone = [call(rows, k, n, flags=skinny | tune << 8) for rows in slabs]
+                assert words == max(lone)
+for m in range(1, 9):
+    assert call(m, 4096, 28672) == 0 and call(m, 4096, 24320) == 0
+"""
+
+
+def test_words_are_asked_for_where_k_is_split(recorder):
+    run = subprocess.run([sys.executable, "-c", WORDS, recorder, LIB_PATH], capture_output=True, text=True, timeout=300)
     assert run.returncode == 0, run.stderr[-2000:]

@@ -68,3 +68,24 @@ def test_larger_requests_than_a_share_are_cleared_in_the_graph(gpu, monkeypatch)
         assert torch.equal(y, want)
     assert ops._accum_reserve[gpu.index][1] == 0
     ops.reset_accumulators()
+
+
+@pytest.mark.parametrize("m", [1, 8, 12, 16])
+def test_a_call_that_exchanges_nothing_takes_no_words(gpu, monkeypatch, m):
+    """a workgroup per strip over all of K: neither words of the reserve nor a clearing kernel in the graph"""
+    from uniql_amd import ops
+    lib = ops._capi.load()
+    monkeypatch.setattr(lib, "uniql_clear", lambda *a: pytest.fail("a clear in the graph"))
+    call = _call(m, 4096, 28672, 14, gpu)
+    ops.reset_accumulators()
+    want = call().clone()
+    assert not ops._accum_cache
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        y = call()
+    assert not ops._accum_in_capture
+    for _ in range(3):
+        y.fill_(float("nan"))
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(y, want)

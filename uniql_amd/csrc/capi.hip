@@ -13,7 +13,8 @@ int stream_launch(const void* A, int64_t lda, int k_valid, const void* B, const 
                   const Epilogue& epi, void* accum, int m, int n, int k, int groups, int had_mode, float had_scale,
                   unsigned tune, hipStream_t stream);
 bool stream_rotates_rows(int m, int k);
-size_t stream_accum_bytes(int m, int n, int k);
+size_t stream_accum_bytes(int m, int n, int k, unsigned tune);
+size_t stream_accum_bound(int m, int n, int k);
 bool stream_shape_ok(int k, int64_t lda);
 int read_floor_launch(const void* B, const void* S, void* sink, int m, int n, int k, unsigned tune, hipStream_t stream);
 size_t read_floor_sink_bytes(int m, int n, int k, unsigned tune);
@@ -221,7 +222,7 @@ static LinearNeeds linear_needs(int m, int n, int k, int k_in, int64_t lda, int 
             q.plan.parts = 1;
             q.plan.part[0] = RowPart{m, false, TilePlan{}};
         } else {
-            q.accum_bytes = round256(stream_accum_bytes(m, n, k));
+            q.accum_bytes = round256(stream_accum_bytes(m, n, k, tune));
         }
     } else {
         q.plan = basic ? linear_plan(m, n, k, wide_shape_ok(m, n, k, groups, q.ld_kernel), part_cap, tune)
@@ -258,7 +259,7 @@ static void call_workspace(int m, int n, int k, int had_block, unsigned flags, s
         *part = p > *part ? p : *part;
     };
     if (takes_stream_kernel(m, flags)) {
-        *accum = stream_accum_bytes(m, n, k);
+        *accum = stream_accum_bytes(m, n, k, flags >> 8);
         most(m, mid_for_few_rows(m, n, k, had_block, flags, kPartialCap));
         return;
     }
@@ -293,7 +294,7 @@ int uniql_w4a16_linear_workspace(int m, int n, int k, int k_in, int had_block, u
 size_t uniql_w4a16_gemm_accum_bytes(int m, int n, int k) {
     if (m <= 0 || n <= 0 || k <= 0 || n % 128 != 0 || k % 128 != 0) return 0;
     // enough for either kernel with its own plan (forced tuning fields: uniql_w4a16_linear_workspace)
-    const size_t a = stream_accum_bytes(m, n, k);
+    const size_t a = stream_accum_bound(m, n, k);
     size_t b, part;
     call_workspace(m, n, k, 0, 0, &b, &part);
     return round256(a > b ? a : b);
@@ -486,7 +487,9 @@ int uniql_w4a16_gemm_static(const void* A, int64_t lda, const void* B, const voi
         q = linear_needs(m, n, k, k, lda, groups, had_block, flags, part_cap);
     }
     const size_t need_accum = q.accum_bytes, need_temp = q.act_bytes + round256(q.part_bytes);
-    if (need_accum > kStaticAccumBytes || need_temp > kStaticTempBytes) return UNIQL_E_STATIC_LIMIT;
+    // (up to 16 rows the words of a K split have to fit, whether or not this call's plan makes one)
+    const size_t words = takes_stream_kernel(m, flags) ? round256(stream_accum_bound(m, n, k)) : need_accum;
+    if (words > kStaticAccumBytes || need_accum > kStaticAccumBytes || need_temp > kStaticTempBytes) return UNIQL_E_STATIC_LIMIT;
     if (!A || !B || !S || !D) return UNIQL_E_NULL;
     unsigned char* base = static_scratch();
     if (!base) return UNIQL_E_LAUNCH;

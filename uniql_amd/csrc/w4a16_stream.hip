@@ -547,13 +547,21 @@ static StreamPlan stream_plan(int m, int n, int k, int upw_override, int waves_o
     return p;
 }
 
-size_t stream_accum_bytes(int m, int n, int k) {
-    // one 64-bit word per output element of a 16-row slab, whenever some plan splits K
-    const int G = k / 128;
-    if (G <= 4) return 0;
-    const int mrows = m < 16 ? m : 16;
-    return (size_t)mrows * n * sizeof(unsigned long long);
+// tune: as stream_launch
+static StreamPlan stream_plan_tuned(int m, int n, int k, unsigned tune) {
+    int waves = (int)((tune >> 8) & 0x1fu);
+    if (waves != 4 && waves != 8) waves = 0;
+    return stream_plan(m, n, k, (int)(tune & 0xffu), waves);
 }
+
+// Exchange words of an m-row call: one 64-bit word per output element of a 16-row slab, if the plan of any of its slabs splits K.
+size_t stream_accum_bytes(int m, int n, int k, unsigned tune) {
+    auto words = [&](int rows) { return rows > 0 && stream_plan_tuned(rows, n, k, tune).splits > 1 ? (size_t)rows * n : 0; };
+    const size_t full = words(m >= 16 ? 16 : 0), last = words(m % 16);
+    return (full > last ? full : last) * sizeof(unsigned long long);
+}
+// As many as any plan asks for.
+size_t stream_accum_bound(int m, int n, int k) { return k / 128 <= 4 ? 0 : (size_t)(m < 16 ? m : 16) * n * sizeof(unsigned long long); }
 
 template <int RC, int HAD, int WAVES, bool EXT>
 static hipError_t launch_one(StreamArgs a, hipStream_t stream) {
@@ -639,12 +647,10 @@ int stream_launch(const void* A, int64_t lda, int k_valid, const void* B, const 
     a.fwht_lds = 0;
     a.log2K = 0;
     while ((1 << a.log2K) < k) ++a.log2K;
-    int waves_override = (int)((tune >> 8) & 0x1fu);
-    if (waves_override != 4 && waves_override != 8) waves_override = 0;
     const size_t out_elt = epi.out_f32 ? 4 : 2;
     for (int m0 = 0; m0 < m; m0 += 16) {
         const int mm = (m - m0) < 16 ? (m - m0) : 16;
-        const StreamPlan plan = stream_plan(mm, n, k, (int)(tune & 0xffu), waves_override);
+        const StreamPlan plan = stream_plan_tuned(mm, n, k, tune);
         a.upw = plan.upw;
         a.splits = plan.splits;
         a.M = mm;
@@ -720,9 +726,7 @@ static void read_floor_depth(int depth, dim3 grid, hipStream_t stream, const u32
 // tune: as stream_launch (bits 0..7 groups per wave, bits 8..12 waves per workgroup), plus bits
 // 13..15 the number of units a wave requests before it consumes the first (0 = 1)
 int read_floor_launch(const void* B, const void* S, void* sink, int m, int n, int k, unsigned tune, hipStream_t stream) {
-    int waves_override = (int)((tune >> 8) & 0x1fu);
-    if (waves_override != 4 && waves_override != 8) waves_override = 0;
-    const StreamPlan plan = stream_plan(m < 16 ? m : 16, n, k, (int)(tune & 0xffu), waves_override);
+    const StreamPlan plan = stream_plan_tuned(m < 16 ? m : 16, n, k, tune);
     const int depth = (int)((tune >> 13) & 7u);
     const dim3 grid(n / 128, plan.splits);
     if (plan.waves == 8)
@@ -735,9 +739,7 @@ int read_floor_launch(const void* B, const void* S, void* sink, int m, int n, in
 }
 
 size_t read_floor_sink_bytes(int m, int n, int k, unsigned tune) {
-    int waves_override = (int)((tune >> 8) & 0x1fu);
-    if (waves_override != 4 && waves_override != 8) waves_override = 0;
-    const StreamPlan plan = stream_plan(m < 16 ? m : 16, n, k, (int)(tune & 0xffu), waves_override);
+    const StreamPlan plan = stream_plan_tuned(m < 16 ? m : 16, n, k, tune);
     return (size_t)(n / 128) * plan.splits * plan.waves * sizeof(uint32_t);
 }
 
