@@ -120,10 +120,12 @@ def _fill_reserve(device: torch.device) -> None:
             return
         try:
             words = torch.zeros(_RESERVE_WORDS, dtype=torch.int64, device=device)
-        except torch.cuda.OutOfMemoryError:
+            # once per device: a graph may replay on any stream, so the zeros are waited for here
+            torch.cuda.current_stream(device).synchronize()
+        except RuntimeError:
+            # No memory, or an allocation or a wait that is refused while another thread captures: the call that
+            # brought us here has its own buffer and needs none of this.  The next new buffer tries again.
             return
-        # once per device: a graph may replay on any stream, so the zeros are waited for here
-        torch.cuda.current_stream(device).synchronize()
         _accum_reserve[device.index] = [words, 0]
 
 
