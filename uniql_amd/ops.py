@@ -69,8 +69,13 @@ _accum_in_capture: dict = {}
 # words from here records no zero fill: 1.8 to 4.6 us and a gap between kernels on each replay
 # (decoder layer of one token 42.3 -> 37.6 us, of 8 tokens 53.2 -> 46.8, of 48 tokens 73.6 -> 67.1).  It is filled beside
 # the device's first eager buffer.  32 MB, in shares of at most 2 MB (16 rows of 16384 columns):
-# captures that find no room, or ask for more, get a buffer and a zero fill of their own.
+# captures that find no room, or ask for more, get a buffer and a zero fill of their own.  A share is
+# never handed out twice, since nothing tells when a graph is destroyed: a captured layer of 1 / 8 / 16 rows
+# (4096 -> 6144 the widest that splits K) takes 0.05 / 0.4 / 0.8 MB, so there are some 40 to 600 of them.
 _accum_reserve: dict = {}
+# Reserves of before reset_accumulators(), [words, how many of them captures have taken]: graphs that were captured from
+# them may be replayed by mistake, and must then find words that are theirs.  What no capture took serves on.
+_accum_reserve_old: dict = {}
 _RESERVE_WORDS = 1 << 22
 _RESERVE_SHARE = 1 << 18
 _reserve_lock = threading.Lock()
@@ -118,6 +123,10 @@ def _fill_reserve(device: torch.device) -> None:
     with _reserve_lock:
         if device.index in _accum_reserve:
             return
+        words, taken = _accum_reserve_old.get(device.index, [[torch.empty(0), 0]])[-1]
+        if words.numel() - taken >= max(_RESERVE_WORDS // 2, 1):   # zeros, waited for when they were made
+            _accum_reserve[device.index] = [words[taken:taken + _RESERVE_WORDS], 0]
+            return
         try:
             words = torch.zeros(_RESERVE_WORDS, dtype=torch.int64, device=device)
             # once per device: a graph may replay on any stream, so the zeros are waited for here
@@ -135,7 +144,7 @@ def _from_reserve(device: torch.device, nbytes: int) -> torch.Tensor | None:
     words = (nbytes + 255) // 256 * 32
     with _reserve_lock:
         reserve = _accum_reserve.get(device.index)
-        if reserve is None or words > _RESERVE_SHARE or reserve[1] + words > _RESERVE_WORDS:
+        if reserve is None or words > _RESERVE_SHARE or reserve[1] + words > reserve[0].numel():
             return None
         begin = reserve[1]
         reserve[1] = begin + words
@@ -150,6 +159,8 @@ def reset_accumulators() -> None:
     _accum_retired.clear()
     _accum_in_capture.clear()
     with _reserve_lock:
+        for device, reserve in _accum_reserve.items():
+            _accum_reserve_old.setdefault(device, []).append(reserve)
         _accum_reserve.clear()
 
 
