@@ -134,7 +134,7 @@ def test_infinite_values_meet_scales_of_the_long_expansion(gpu, m):
 
 # sizes of this kernel: one and several groups a wave, K split into 2 to 9 and not at all, each row class; the last two where its
 # fastest plan would add longer chains than the tiled kernel's
-@pytest.mark.parametrize("m,k,n", [(15, 4480, 512), (12, 1920, 1024), (16, 8192, 4096), (13, 512, 13056), (29, 4864, 7168), (23, 12800, 1536),
+@pytest.mark.parametrize("m,k,n", [(15, 4480, 512), (12, 1920, 1024), (16, 8192, 4096), (13, 512, 13056), (9, 14336, 4096), (10, 6144, 512), (29, 4864, 7168), (23, 12800, 1536),
                                    (17, 3328, 8704), (40, 4096, 28672), (48, 4096, 4096), (35, 12288, 1280), (40, 9216, 3072), (56, 6784, 2048), (53, 6400, 256), (56, 8192, 512)])
 def test_sums_are_as_exact_as_the_other_kernels(gpu, m, k, n):
     """distance from float64 in front of the fp16 rounding against that of the kernel which took such calls before: the

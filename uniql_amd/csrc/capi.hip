@@ -171,18 +171,16 @@ struct LinearNeeds {
 static const MidPlan kNoMid = {0, 0, 0, 0.0};
 
 // In place of the streaming kernel: from 9 rows on that kernel's one atomic per output element and K split costs more than
-// the exchange of partial tiles, except where it does not split K at all (4096 -> 28672 at 9 to 12 rows 12.9 to 13.4 us there,
-// 13.3 to 13.5 here), and over a longer K, where this one's units follow each other in a wave: above 2048 it takes narrow
-// layers from 12 rows on (4096 -> 512 at 10 rows 6.65 us there, 6.7 here, at 12 7.1 and 6.8; 4096 -> 4096 at 9 rows 7.75 and
-// 7.0), above 4096 calls from 13 rows on (6144 -> 512 at 9 rows 6.65 and 7.45, 14336 -> 4096 11.25 and 11.5; at 16 rows 8.25 and
-// 7.45, 12.7 and 11.75), but few columns and a long K not at all (11840 -> 1280 at 10 rows 8.3 us there, 10.1 here).
-// 4096 -> 4096 at 16 rows 8.5 -> 7.3 us, 4096 -> 6144 9.2 -> 7.7.  A rotation stays with the streaming kernel,
-// which applies it while it stages the rows.
+// the exchange of partial tiles, and its single row tile does not use what the second wave of a SIMD hides.  us at 9 / 16 rows,
+// there and here: 1024 -> 4096 0.69 / 0.56 x; 4096 -> 512 6.4 / 6.6 and 6.3 / 6.2; 4096 -> 4096 7.5 / 8.5 and 6.5 / 6.8; 14336 -> 4096
+// 10.7 / 12.2 and 10.0 / 10.3.  Not for few columns over a long K, where more than eight partial tiles meet (9984 -> 2560 8.0 / 9.0 and
+// 8.7 / 9.1, 11904 -> 512 1.22 / 1.03 x; 8192 -> 2560 0.90 / 0.84 x, 11904 -> 3072 9.75 / 10.8 and 8.9 / 9.2), and not from 144
+// strips on, where the streaming kernel mostly splits nothing (4096 -> 28672 within 3 %, 4096 -> 128256 46.0 / 48.6 and 48.7 /
+// 52.0).  Rows that are rotated stay with the streaming kernel, which rotates blocks of 128 and short rows while it stages them.
 static MidPlan mid_for_few_rows(int m, int n, int k, int had_block, unsigned flags, size_t part_cap) {
     if (m < kMidMinRows || m > kStreamMaxM || had_block != 0 || (flags & (UNIQL_F_FORCE_SKINNY | UNIQL_F_FORCE_TILED)) || (flags >> 8) != 0)
         return kNoMid;
-    const bool faster = k > 4096 ? m >= 13 && (k <= 6144 || n >= 4096) : k <= 2048 || m >= 12 || n >= 4096;
-    return n / 128 < 144 && faster ? mid_plan(m, n, k, 0, part_cap) : kNoMid;
+    return n / 128 < 144 && (k <= 8192 || n >= 3072) ? mid_plan(m, n, k, 0, part_cap) : kNoMid;
 }
 
 // In place of a launch of the tiled kernels, where it is expected to be faster; padded: the tiled kernels would need a

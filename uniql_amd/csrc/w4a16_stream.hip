@@ -70,8 +70,8 @@ struct StreamArgs {
 };
 
 // One launch covers up to 16 rows of X (the rows of one MFMA tile); more rows run as further
-// launches over the same weights, which only the forcing flag asks for: from 9 rows on other
-// kernels are faster, wherever it splits K.  RC: row class, an upper bound of M
+// launches over the same weights, which only the forcing flag asks for: from 17 rows on other
+// kernels are faster, from 9 rows on mostly (mid_for_few_rows in capi.hip).  RC: row class, an upper bound of M
 // (1, 2, 4, 8, 16): it fixes NV, how many of the four output rows of a lane's accumulator
 // quad are real, and XQ, how many quads of activation rows are loaded and staged.  WAVES:
 // wavefronts per workgroup (4 or 8); with 8 a workgroup can cover all of K for shapes with
