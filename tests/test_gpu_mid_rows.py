@@ -17,7 +17,10 @@ def _flags(groups_per_wave):
 
 # a 16-row tile's edges; one group, fewer groups than waves, K split with a short last workgroup and one unit, many splits
 @pytest.mark.parametrize("m,k,n,upw", [(9, 128, 128, 1), (16, 1152, 256, 1), (17, 640, 128, 1), (31, 2176, 256, 2), (32, 1024, 384, 1),
-                                       (33, 512, 256, 1), (48, 1664, 128, 2), (49, 384, 256, 1), (64, 2560, 128, 1), (64, 640, 256, 3)])
+                                       (33, 512, 256, 1), (48, 1664, 128, 2), (49, 384, 256, 1), (64, 2560, 128, 1), (64, 640, 256, 3),
+                                       # 3, 4, 9 and 19 partial tiles: the last wave asks for them by two, four and eight
+                                       (9, 3200, 128, 1), (16, 9216, 128, 1), (30, 3072, 128, 1), (40, 4608, 128, 1), (50, 1536, 128, 1),
+                                       (64, 9600, 128, 1)])
 def test_every_row_tile_and_split(gpu, m, k, n, upw):
     from uniql_amd import ops
     p = make_linear_problem(m, k, n, seed=m + k + n)
@@ -134,8 +137,9 @@ def test_infinite_values_meet_scales_of_the_long_expansion(gpu, m):
 
 # sizes of this kernel: one and several groups a wave, K split into 2 to 9 and not at all, each row class; the last two where its
 # fastest plan would add longer chains than the tiled kernel's
-@pytest.mark.parametrize("m,k,n", [(15, 4480, 512), (12, 1920, 1024), (16, 8192, 4096), (13, 512, 13056), (9, 14336, 4096), (10, 6144, 512), (29, 4864, 7168), (23, 12800, 1536),
-                                   (17, 3328, 8704), (40, 4096, 28672), (48, 4096, 4096), (35, 12288, 1280), (40, 9216, 3072), (56, 6784, 2048), (53, 6400, 256), (56, 8192, 512)])
+@pytest.mark.parametrize("m,k,n", [(15, 4480, 512), (12, 1920, 1024), (16, 8192, 4096), (13, 512, 13056), (9, 14336, 4096), (10, 6144, 512),
+                                   (29, 4864, 7168), (23, 12800, 1536), (17, 3328, 8704), (40, 4096, 28672), (48, 4096, 4096), (35, 12288, 1280), (40, 9216, 3072),
+                                   (56, 6784, 2048), (53, 6400, 256), (56, 8192, 512)])
 def test_sums_are_as_exact_as_the_other_kernels(gpu, m, k, n):
     """distance from float64 in front of the fp16 rounding against that of the kernel which took such calls before: the
     streaming kernel, whose partial sums meet as integers, up to 16 rows, the tiled kernel above.  Both round fp32
