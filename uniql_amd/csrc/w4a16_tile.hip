@@ -33,6 +33,8 @@
 //
 // When K is also split over workgroups every workgroup writes its fp32 partial tile to a scratch
 // area and the last one to arrive (one arrival count per tile) adds them in split order.
+#include <type_traits>
+
 #include "common.hpp"
 #include "tile_plan.hpp"
 
@@ -41,6 +43,7 @@ namespace uniql {
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 
 constexpr int kRing = 3;
+constexpr int kDeviceScope = 16;  // cache policy bit sc1: as relaxed device-scope loads and stores compile to
 
 struct TileArgs {
     const u32x4* B;
@@ -72,34 +75,6 @@ __device__ __forceinline__ void buffer_to_lds16(__amdgpu_buffer_rsrc_t rsrc, uin
 
 // s_waitcnt vmcnt(n) with the other counters left alone (gfx9 encoding)
 #define UNIQL_WAIT_VMCNT(n) __builtin_amdgcn_s_waitcnt(((n) & 15) | (((n) >> 4) << 14) | 0x0F70)
-
-// Eight fp32 partial sums to / from a workgroup's slot of the split-K scratch area: relaxed
-// device-scope accesses (write-through stores, loads that do not trust a stale cache line), so
-// workgroups on different XCDs exchange them without flushing or invalidating a whole L2.  The
-// four 8-byte words of a unit lie `stride` words apart: word i of all threads of the workgroup is
-// one contiguous run, so every store instruction writes whole cache lines.
-__device__ __forceinline__ unsigned long long pack_floats(float a, float b) {
-    return (unsigned long long)__float_as_uint(a) | ((unsigned long long)__float_as_uint(b) << 32);
-}
-__device__ __forceinline__ void store_partial(unsigned long long* d, int stride, f4 lo, f4 hi) {
-    __hip_atomic_store(d, pack_floats(lo[0], lo[1]), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    __hip_atomic_store(d + stride, pack_floats(lo[2], lo[3]), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    __hip_atomic_store(d + 2 * stride, pack_floats(hi[0], hi[1]), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    __hip_atomic_store(d + 3 * stride, pack_floats(hi[2], hi[3]), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-__device__ __forceinline__ void add_partial(const unsigned long long* p, int stride, f4& lo, f4& hi) {
-    unsigned long long w[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) w[i] = __hip_atomic_load(p + i * stride, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    lo[0] += __uint_as_float((uint32_t)w[0]);
-    lo[1] += __uint_as_float((uint32_t)(w[0] >> 32));
-    lo[2] += __uint_as_float((uint32_t)w[1]);
-    lo[3] += __uint_as_float((uint32_t)(w[1] >> 32));
-    hi[0] += __uint_as_float((uint32_t)w[2]);
-    hi[1] += __uint_as_float((uint32_t)(w[2] >> 32));
-    hi[2] += __uint_as_float((uint32_t)w[3]);
-    hi[3] += __uint_as_float((uint32_t)(w[3] >> 32));
-}
 
 template <int MT, int KW = 1>
 struct TileLds {
@@ -444,17 +419,16 @@ __global__ __launch_bounds__(256 * KW, 1) void w4a16_tile_kernel(const TileArgs 
     };
 
     // K split over workgroups: every workgroup writes its 32 MT x 128 partial tile (fp32) to its
-    // slot of the scratch area, then counts itself in the tile's word; whoever completes the count
-    // adds the slots in split order (so the sum does not depend on who came last) and stores.
-    // A slot holds the tile as 512 MT units of (row, 8 columns); unit u of M tile mt (row u / 16,
-    // columns 8 (u % 16)..) is the four words ((mt UPT + u / T) 4 + i) T + u % T, i = 0..3, with
-    // T the workgroup's thread count: the thread that reduces a unit writes it, lane after lane.
+    // slot of the scratch area, and the last one to arrive adds the slots in split order (so the sum does not
+    // depend on who came last) and stores.  A slot holds the tile as units of (row, 8 columns), a thread's t-th unit of M tile
+    // mt as the 16-byte words ((mt UPT + t) 2 + i) T + tid, i = 0, 1, with T the workgroup's thread count: a store
+    // instruction of a wave writes whole cache lines, and a wave adds up the units that waves of its number wrote.
     const int tile = mblock * nstrips + strip_of_launch;
-    constexpr int T = 256 * KW, UPT = 512 / T, kSlotWords = ROWS * 64;
-    unsigned long long* part_tile =
-        split_k ? reinterpret_cast<unsigned long long*>(a.part) + (size_t)tile * a.splits * kSlotWords : nullptr;
-    unsigned long long* part_mine = split_k ? part_tile + (size_t)split * kSlotWords : nullptr;
-    auto unit_word = [&](int mt, int unit) { return ((mt * UPT + unit / T) * 4) * T + unit % T; };
+    constexpr int T = 256 * KW, UPT = 512 / T, kSlotBytes = ROWS * 512;
+    char* part_tile = split_k ? reinterpret_cast<char*>(a.part) + (size_t)tile * a.splits * kSlotBytes : nullptr;
+    // (The slot is the descriptor's base and not a scalar offset: with a scalar offset in a register the compiler puts no wait
+    // state between a 16-byte store and the next instruction, and one that overwrites the stored registers changed what was stored.)
+    const __amdgpu_buffer_rsrc_t part_rsrc = __builtin_amdgcn_make_buffer_rsrc(part_tile + (size_t)split * kSlotBytes, 0, split_k ? (unsigned)kSlotBytes : 0u, kRsrcFlags);
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) {
         if (m0 + mt * 32 < a.M) {  // uniform
@@ -485,7 +459,11 @@ __global__ __launch_bounds__(256 * KW, 1) void w4a16_tile_kernel(const TileArgs 
                     hi += *reinterpret_cast<const f4*>(src + ww * 32 * kRedStride + 4);
                 }
                 if (split_k) {
-                    if (m < a.M) store_partial(part_mine + unit_word(mt, unit), T, lo, hi);  // (1) rows that exist only
+                    const uint32_t at = 16u * (uint32_t)tid + 32u * T * (uint32_t)(mt * UPT + unit / T);
+                    if (m < a.M) {  // (1) rows that exist only
+                        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, lo), part_rsrc, at, 0, kDeviceScope);
+                        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, hi), part_rsrc, at + 16u * T, 0, kDeviceScope);
+                    }
                 } else if (!gated) {
                     if (m < a.M) emit(m, c0, lo, hi);
                 } else {
@@ -504,7 +482,7 @@ __global__ __launch_bounds__(256 * KW, 1) void w4a16_tile_kernel(const TileArgs 
 
     // ---- the split-K exchange: message passing with relaxed device-scope operations only -------
     // What it relies on, step by step (the numbers are used again at the lines they govern):
-    //  (1) store_partial: relaxed agent-scope stores.  On gfx950 these are write-through (sc1)
+    //  (1) the partial sums' stores: relaxed agent-scope stores.  On gfx950 these are write-through (sc1)
     //      stores that bypass the XCD's own L2, so a workgroup on another XCD can see them.
     //  (2) s_waitcnt vmcnt(0): the counter is decremented when such a store has been ACKNOWLEDGED
     //      by the memory side, i.e. is visible to every XCD.  A workgroup barrier alone does not
@@ -514,7 +492,7 @@ __global__ __launch_bounds__(256 * KW, 1) void w4a16_tile_kernel(const TileArgs 
     //  (4) thread 0's relaxed agent-scope fetch_add on the tile's arrival count; nothing may move
     //      it in front of (3) (the barrier is a compiler and hardware ordering point for it).
     //  (5) the workgroup that completes the count reads the slots with relaxed agent-scope loads
-    //      (add_partial; sc1: they do not hit a stale line of the local L2).
+    //      (sc1: they do not hit a stale line of the local L2).
     // The language's memory model would ask for a release at (4) and an acquire before (5); at
     // agent scope those compile to a write-back and an invalidate of the whole L2, measured at two
     // to three times the K loop the split saves.  (2), which the ISA documents for vmcnt, stands in
@@ -529,30 +507,71 @@ __global__ __launch_bounds__(256 * KW, 1) void w4a16_tile_kernel(const TileArgs 
     }
     __syncthreads();
     if (*last_flag == 0) return;  // uniform
-    const int units = gated ? 256 : 512;
+    if (tid == 0) __hip_atomic_store(a.accum + tile, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    // The slots of a batch are requested together, and an M tile's while the one in front of it is added up: one round trip
+    // in place of one for every unit and split.  us of a launch, mean of 8 heights of prompt over 9 layers, against those: 96-row
+    // tiles 3.4 less with 3 splits, 9.0 with 8; 128-row tiles 4.3 and 10.4; 64-row tiles 2.1 and 6.0; 32-row tiles 0.8 and 2.8; with
+    // two quartets 0.7 to 3.3.  (A count per wave in place of the workgroup's costs more than it saves: atomics on one cache line go
+    // one by one, two quartets with 4 splits were 3.6 us slower.)  Slots and M tiles that do not exist lie beyond the descriptor and read as zeros.
+    // Where several workgroups share a compute unit (one quartet, 32- and 64-row tiles) the batches are as small as its registers.
+    constexpr int kAhead = KW == 1 && MT <= 2 ? 0 : 1, kBatch = KW == 2 ? 8 : MT <= 2 ? 2 : 4;
+    f4 total[MT][2 * UPT];
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+        for (int u = 0; u < 2 * UPT; ++u) total[mt][u] = f4{0.f, 0.f, 0.f, 0.f};
+    auto gather = [&](int first, auto batch) __attribute__((always_inline)) {
+        constexpr int N = decltype(batch)::value;
+        f4 v[kAhead + 1][N][2 * UPT];
+        const unsigned slots_bytes = (unsigned)((a.splits - first) * kSlotBytes);
+        auto request = [&](int mt) __attribute__((always_inline)) {
+            const __amdgpu_buffer_rsrc_t slots = __builtin_amdgcn_make_buffer_rsrc(part_tile + (size_t)first * kSlotBytes, 0,
+                                                                                   m0 + mt * 32 < a.M ? slots_bytes : 0u, kRsrcFlags);
+#pragma unroll
+            for (int b = 0; b < N; ++b)
+#pragma unroll
+                for (int u = 0; u < 2 * UPT; ++u)
+                    v[mt & kAhead][b][u] = __builtin_bit_cast(f4, __builtin_amdgcn_raw_buffer_load_b128(
+                        slots, 16u * (uint32_t)tid + (uint32_t)(b * kSlotBytes + 16 * T * (2 * UPT * mt + u)), 0, kDeviceScope));  // (5)
+        };
+        if (kAhead) request(0);
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt) {
+            if (mt + kAhead < MT) request(mt + kAhead);
+#pragma unroll
+            for (int b = 0; b < N; ++b)
+#pragma unroll
+                for (int u = 0; u < 2 * UPT; ++u) total[mt][u] += v[mt & kAhead][b][u];
+            if (!kAhead) __builtin_amdgcn_sched_barrier(0);
+        }
+    };
+    for (int first = 0; first < a.splits; first += kBatch) {
+        const int rest = a.splits - first;  // uniform
+        if (kBatch == 8 && rest > 4) gather(first, std::integral_constant<int, kBatch>{});
+        else if (kBatch >= 4 && rest > 2) gather(first, std::integral_constant<int, kBatch >= 4 ? 4 : 2>{});
+        else gather(first, std::integral_constant<int, 2>{});
+    }
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) {
         if (m0 + mt * 32 >= a.M) break;  // uniform
-        for (int unit = tid; unit < units; unit += 256 * KW) {
-            const int row = gated ? unit >> 3 : unit >> 4;
-            const int c0 = gated ? (unit & 7) * 8 : (unit & 15) * 8;
-            const int m = m0 + mt * 32 + row;
-            if (m >= a.M) continue;
-            // the unit's number in the writers' enumeration (16 units per row); a gated pair's up
-            // half is 8 units on
-            const int wunit = row * 16 + (c0 >> 3);
-            const unsigned long long* src = part_tile + unit_word(mt, wunit);
-            const unsigned long long* usrc = part_tile + unit_word(mt, wunit + 8);
-            f4 lo = f4{0.f, 0.f, 0.f, 0.f}, hi = lo, ulo = lo, uhi = lo;
-            for (int sp = 0; sp < a.splits; ++sp) {
-                add_partial(src + (size_t)sp * kSlotWords, T, lo, hi);  // (5)
-                if (gated) add_partial(usrc + (size_t)sp * kSlotWords, T, ulo, uhi);
+#pragma unroll
+        for (int t = 0; t < UPT; ++t) {
+            const int unit = tid + t * T, slot = unit & 15, m = m0 + mt * 32 + (unit >> 4);
+            const f4 lo = total[mt][2 * t], hi = total[mt][2 * t + 1];
+            if (gated) {
+                // the up value of gate columns 8 slot .. (slot < 8) is eight lanes on
+                f4 ulo, uhi;
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    ulo[i] = __shfl_down(lo[i], 8, kWave);
+                    uhi[i] = __shfl_down(hi[i], 8, kWave);
+                }
+                if (m < a.M && slot < 8) store_eight_gated(a.epi, a.D, m, 64 * strip + 8 * slot, lo, hi, ulo, uhi);
+            } else if (m < a.M) {
+                emit(m, 8 * slot, lo, hi);
             }
-            if (!gated) emit(m, c0, lo, hi);
-            else store_eight_gated(a.epi, a.D, m, 64 * strip + c0, lo, hi, ulo, uhi);
         }
     }
-    if (tid == 0) __hip_atomic_store(a.accum + tile, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 // ---------------------------------------------------------------------------------
