@@ -394,6 +394,7 @@ static int linear_impl(const void* A, int64_t lda, int k_in, const void* B, cons
     epi.transpose = transpose ? 1 : 0;
     epi.relu2 = epilogue == UNIQL_EPI_RELU2 ? 1 : 0;
     epi.vec_ok = (!transpose && ldd % 8 == 0 && aligned16(D)) ? 1 : 0;
+    epi.residual_vec = residual && epi.vec_ok && !out_f32 && aligned16(residual) && ldr % 8 == 0 && ldr < (1 << 22) ? 1 : 0;
     if (use_stream)
         return stream_launch(Ain, ld, k_valid, B, S, D, epi, accum, m, n, k, groups, had_mode, had_scale, tune, st);
     int m0 = 0, first = 0;

@@ -106,6 +106,8 @@ struct Epilogue {
     int transpose;       // 1: D is [n_store][ldd] with the row index running along the inner axis
                          //    (the reference's output_transpose, "sequence length last")
     int relu2;           // 1: the stored value is relu(y)^2 of the rounded (and biased) product y
+    int residual_vec;    // the residual may be requested ahead in 16-byte pieces (residual_rows): vec_ok, fp16 output, its own
+                         //    alignment and row stride, 256 rows of it below 2^31 bytes
 
     __device__ __forceinline__ size_t offset(int m, int n) const {
         return transpose ? (size_t)n * ldd + m : (size_t)m * ldd + n;
@@ -161,110 +163,145 @@ __device__ __forceinline__ void finish_store_gated(const Epilogue& e, void* D, i
     }
 }
 
-// Eight consecutive fp16 values from p: one 16-byte load where the address allows it.
-__device__ __forceinline__ void load_eight(const half_t* p, bool aligned16, float (&out)[8]) {
-    if (aligned16) {
+// Eight consecutive fp16 values from p, the first `left` of which exist: one 16-byte load where the address allows it.
+__device__ __forceinline__ void load_eight(const half_t* p, bool aligned16, int left, float (&out)[8]) {
+    if (aligned16 && left >= 8) {
         const h8 v = *reinterpret_cast<const h8*>(p);
 #pragma unroll
         for (int i = 0; i < 8; ++i) out[i] = (float)v[i];
     } else {
+        asm volatile("" : "+v"(left));
 #pragma unroll
-        for (int i = 0; i < 8; ++i) out[i] = (float)p[i];
+        for (int i = 0; i < 8; ++i) out[i] = (float)p[i < left ? i : left - 1];
     }
+}
+// Eight consecutive outputs of row m from column n0 on, the first `left` of which exist.
+__device__ __forceinline__ void store_halves(const Epilogue& e, void* D, int m, int n0, int left, const half_t (&r)[8]) {
+    if (e.vec_ok && left >= 8) {
+        *reinterpret_cast<h8*>(reinterpret_cast<half_t*>(D) + (size_t)m * e.ldd + n0) = h8{r[0], r[1], r[2], r[3], r[4], r[5], r[6], r[7]};
+        return;
+    }
+    asm volatile("" : "+v"(left));  // eight masks for all units of a tile, kept in scalar registers, would be most of those
+    half_t* d = reinterpret_cast<half_t*>(D) + e.offset(m, n0);
+    const int64_t step = e.transpose ? e.ldd : 1;
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+        if (i < left) d[i * step] = r[i];
+}
+// the next of eight values to the front
+__device__ __forceinline__ void shift_down(f4& lo, f4& hi) {
+    lo = f4{lo[1], lo[2], lo[3], hi[0]};
+    hi = f4{hi[1], hi[2], hi[3], hi[3]};
+}
+
+// The residual of up to 256 rows from row m0 on and of the columns from n0 on, for loads in front of the loop that stores:
+// a unit that first loads its residual waits for one round trip after another.  Rows and columns that do not exist read as
+// zeros or as another column; a unit that holds one of those loads its residual itself (store_eight).
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t residual_rows(const Epilogue& e, int m0, int M, int n0) {
+    const int64_t rows = M - m0 < 256 ? M - m0 : 256, columns = e.n_store - n0 < 128 ? e.n_store - n0 : 128;
+    const unsigned bytes = e.residual_vec && rows > 0 && columns > 0 ? (unsigned)(((rows - 1) * e.ldr + columns) * 2) : 0u;
+    const half_t* from = e.residual_vec ? e.residual + (int64_t)m0 * e.ldr + n0 : nullptr;
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<half_t*>(from), 0, bytes, 0x00020000);
+}
+__device__ __forceinline__ u32x4 residual_load(const Epilogue& e, __amdgpu_buffer_rsrc_t rows, int row, int column) {
+    return __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rows, 2u * ((uint32_t)row * (uint32_t)e.ldr + (uint32_t)column), 0, 0));
 }
 
 // Eight consecutive outputs of row m starting at column n0 (a multiple of 8): one 16-byte
 // store where the output's layout allows it, element stores otherwise.  Bias and residual come as
-// 16-byte loads where they are aligned; the roundings are those of finish_half / finish_half_gated.
-__device__ __forceinline__ void store_eight(const Epilogue& e, void* D, int m, int n0, f4 lo, f4 hi) {
-    if (e.vec_ok && n0 + 8 <= e.n_store) {
-        const size_t o = (size_t)m * e.ldd + n0;
-        if (e.out_f32 && !e.bias && !e.residual && !e.relu2) {
-            float* d = reinterpret_cast<float*>(D) + o;
+// 16-byte loads where they are aligned, the residual from `ahead` where it was requested in advance; the roundings are those of
+// finish_half / finish_half_gated.  Short on purpose: it is instantiated for every unit of a tile, and with eight copies of
+// finish_store in it the 128-column kernels were 1.8 x as long, their scalar registers spilled, and odd widths waited for a
+// bias or residual element by element.
+template <bool AHEAD = false>
+__device__ __forceinline__ void store_eight(const Epilogue& e, void* D, int m, int n0, f4 lo, f4 hi, u32x4 ahead = u32x4{0u, 0u, 0u, 0u}) {
+    const int left = e.n_store - n0;
+    if (left <= 0) return;
+    if (e.out_f32) {
+        if (e.vec_ok && left >= 8 && !e.bias && !e.residual && !e.relu2) {
+            float* d = reinterpret_cast<float*>(D) + (size_t)m * e.ldd + n0;
             *reinterpret_cast<f4*>(d) = lo;
             *reinterpret_cast<f4*>(d + 4) = hi;
             return;
         }
-        if (!e.out_f32 && !e.bias && !e.residual && !e.relu2) {
-            const h2 r0 = h2{(half_t)lo[0], (half_t)lo[1]}, r1 = h2{(half_t)lo[2], (half_t)lo[3]};
-            const h2 r2 = h2{(half_t)hi[0], (half_t)hi[1]}, r3 = h2{(half_t)hi[2], (half_t)hi[3]};
-            *reinterpret_cast<u32x4*>(reinterpret_cast<half_t*>(D) + o) =
-                u32x4{h2_to_bits(r0), h2_to_bits(r1), h2_to_bits(r2), h2_to_bits(r3)};
-            return;
+#pragma clang loop unroll(disable)
+        for (int i = 0; i < 8; ++i) {
+            finish_store(e, D, m, n0 + i, lo[0]);
+            shift_down(lo, hi);
         }
-        if (!e.out_f32) {
-            half_t r[8];
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                r[i] = (half_t)lo[i];
-                r[4 + i] = (half_t)hi[i];
-            }
-            if (e.bias) {
-                float b[8];
-                load_eight(e.bias + n0, (reinterpret_cast<uintptr_t>(e.bias) & 15u) == 0, b);
-#pragma unroll
-                for (int i = 0; i < 8; ++i) r[i] = (half_t)((float)r[i] + b[i]);
-            }
-            if (e.relu2) {
-#pragma unroll
-                for (int i = 0; i < 8; ++i) {
-                    const float p = (float)r[i] > 0.f ? (float)r[i] : 0.f;
-                    r[i] = (half_t)(p * p);
-                }
-            }
-            if (e.residual) {
-                float q[8];
-                load_eight(e.residual + (size_t)m * e.ldr + n0,
-                           (reinterpret_cast<uintptr_t>(e.residual) & 15u) == 0 && (e.ldr & 7) == 0, q);
-#pragma unroll
-                for (int i = 0; i < 8; ++i) r[i] = (half_t)(q[i] + (float)r[i]);
-            }
-            *reinterpret_cast<h8*>(reinterpret_cast<half_t*>(D) + o) = h8{r[0], r[1], r[2], r[3], r[4], r[5], r[6], r[7]};
-            return;
-        }
+        return;
     }
+    half_t r[8];
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-        finish_store(e, D, m, n0 + i, lo[i]);
-        finish_store(e, D, m, n0 + 4 + i, hi[i]);
+        r[i] = (half_t)lo[i];
+        r[4 + i] = (half_t)hi[i];
     }
+    if (e.bias) {
+        float b[8];
+        load_eight(e.bias + n0, (reinterpret_cast<uintptr_t>(e.bias) & 15u) == 0, left, b);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) r[i] = (half_t)((float)r[i] + b[i]);
+    }
+    if (e.relu2) {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            const float p = (float)r[i] > 0.f ? (float)r[i] : 0.f;
+            r[i] = (half_t)(p * p);
+        }
+    }
+    if (e.residual) {
+        float q[8];
+        if (AHEAD && e.residual_vec && left >= 8) {
+            const h8 v = __builtin_bit_cast(h8, ahead);
+#pragma unroll
+            for (int i = 0; i < 8; ++i) q[i] = (float)v[i];
+        } else {
+            load_eight(e.residual + (size_t)m * e.ldr + n0, (reinterpret_cast<uintptr_t>(e.residual) & 15u) == 0 && (e.ldr & 7) == 0, left, q);
+        }
+#pragma unroll
+        for (int i = 0; i < 8; ++i) r[i] = (half_t)(q[i] + (float)r[i]);
+    }
+    store_halves(e, D, m, n0, left, r);
 }
 __device__ __forceinline__ void store_eight_gated(const Epilogue& e, void* D, int m, int n0, f4 glo, f4 ghi, f4 ulo,
                                                   f4 uhi) {
-    if (e.vec_ok && !e.out_f32 && n0 + 8 <= e.n_store) {
-        half_t r[8], g16[8], u16[8];
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            g16[i] = (half_t)glo[i];
-            g16[4 + i] = (half_t)ghi[i];
-            u16[i] = (half_t)ulo[i];
-            u16[4 + i] = (half_t)uhi[i];
-        }
-        if (e.bias) {
-            float bg[8], bu[8];
-            const bool al = (reinterpret_cast<uintptr_t>(e.bias) & 15u) == 0;
-            load_eight(e.bias + n0, al, bg);
-            load_eight(e.bias + e.n_store + n0, al && (e.n_store & 7) == 0, bu);
-#pragma unroll
-            for (int i = 0; i < 8; ++i) {
-                g16[i] = (half_t)((float)g16[i] + bg[i]);
-                u16[i] = (half_t)((float)u16[i] + bu[i]);
-            }
-        }
-#pragma unroll
+    const int left = e.n_store - n0;
+    if (left <= 0) return;
+    if (e.out_f32) {
+#pragma clang loop unroll(disable)
         for (int i = 0; i < 8; ++i) {
-            const half_t a16 = (half_t)silu_f32((float)g16[i]);
-            r[i] = (half_t)((float)a16 * (float)u16[i]);
+            finish_store_gated(e, D, m, n0 + i, glo[0], ulo[0]);
+            shift_down(glo, ghi);
+            shift_down(ulo, uhi);
         }
-        *reinterpret_cast<h8*>(reinterpret_cast<half_t*>(D) + (size_t)m * e.ldd + n0) =
-            h8{r[0], r[1], r[2], r[3], r[4], r[5], r[6], r[7]};
         return;
     }
+    half_t r[8], g16[8], u16[8];
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-        finish_store_gated(e, D, m, n0 + i, glo[i], ulo[i]);
-        finish_store_gated(e, D, m, n0 + 4 + i, ghi[i], uhi[i]);
+        g16[i] = (half_t)glo[i];
+        g16[4 + i] = (half_t)ghi[i];
+        u16[i] = (half_t)ulo[i];
+        u16[4 + i] = (half_t)uhi[i];
     }
+    if (e.bias) {
+        float bg[8], bu[8];
+        const bool al = (reinterpret_cast<uintptr_t>(e.bias) & 15u) == 0;
+        load_eight(e.bias + n0, al, left, bg);
+        load_eight(e.bias + e.n_store + n0, al && (e.n_store & 7) == 0, left, bu);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            g16[i] = (half_t)((float)g16[i] + bg[i]);
+            u16[i] = (half_t)((float)u16[i] + bu[i]);
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+        const half_t a16 = (half_t)silu_f32((float)g16[i]);
+        r[i] = (half_t)((float)a16 * (float)u16[i]);
+    }
+    store_halves(e, D, m, n0, left, r);
 }
 
 // ---- exchange of partial sums between workgroups that split K ------------------------

@@ -356,6 +356,16 @@ __global__ __launch_bounds__(64 * WAVES, WAVES / 4) void w4a16_mid_kernel(const 
     // four rows are a unit; wave w finishes units w, w + WAVES ..: lane l row l / 16, columns 8 (l % 16) ..
     constexpr int UT = (XQ + WAVES - 1) / WAVES;
     if (4 * w >= a.M) return;
+    // the residual of the wave's units, requested in front of the sums
+    u32x4 ahead[UT];
+    auto request_residual = [&]() __attribute__((always_inline)) {
+        if constexpr (EXT) {
+            const __amdgpu_buffer_rsrc_t rows = residual_rows(a.epi, 0, a.M, 128 * strip);
+#pragma unroll
+            for (int t = 0; t < UT; ++t) ahead[t] = residual_load(a.epi, rows, 4 * (w + t * WAVES) + kq, 8 * slot);
+        }
+    };
+    if (a.splits == 1) request_residual();
     f4 lo[UT], hi[UT];
 #pragma unroll
     for (int t = 0; t < UT; ++t) {
@@ -397,6 +407,7 @@ __global__ __launch_bounds__(64 * WAVES, WAVES / 4) void w4a16_mid_kernel(const 
         if (arrived != a.splits - 1) return;
         asm volatile("" ::: "memory");
         if (lane == 0) __hip_atomic_store(count, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        request_residual();
         // Slots are requested up to eight together; those that do not exist lie beyond the descriptor and read as zeros.
         typename Sums::Total total_lo[UT], total_hi[UT];
 #pragma unroll
@@ -443,7 +454,7 @@ __global__ __launch_bounds__(64 * WAVES, WAVES / 4) void w4a16_mid_kernel(const 
                 }
                 if (m < a.M && slot < 8) store_eight_gated(a.epi, a.D, m, 64 * strip + 8 * slot, lo[t], hi[t], ulo, uhi);
             } else if (m < a.M) {
-                store_eight(a.epi, a.D, m, 128 * strip + 8 * slot, lo[t], hi[t]);
+                store_eight<true>(a.epi, a.D, m, 128 * strip + 8 * slot, lo[t], hi[t], ahead[t]);
             }
         } else if (m < a.M) {
             const size_t o = (size_t)m * a.N + 128 * strip + 8 * slot;

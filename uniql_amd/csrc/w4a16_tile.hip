@@ -88,13 +88,14 @@ struct TileLds {
     static constexpr size_t kBytes = kRingBytes > kRedBytes ? kRingBytes : kRedBytes;
 };
 
-// EXT: the call uses something beyond the plain product (output cut or strided, bias, gated
-// pairs); the plain instantiation leaves that code out of the epilogue.
+// EXT: 0 the plain product; 1 the call uses something beyond it (output cut or strided, bias, residual, squared ReLU); 2 gated
+// pairs.  An instantiation leaves the others' code out of its epilogue: with both in one, its conditions are more than the
+// scalar registers hold (4096 -> 24320 gated at 192 rows: 57.8 us apart, 59.3 in one).
 // KW: quartets of waves per workgroup (1 or 2).  With two, the quartets take alternate K groups of
 // the same tile (each with its own LDS ring): two waves per SIMD cover each other's LDS and
 // expansion latencies, which is what small M tiles (little matrix work per group) lack when the
 // grid only gives a compute unit one workgroup.
-template <int MT, bool EXT, int KW>
+template <int MT, int EXT, int KW>
 __global__ __launch_bounds__(256 * KW, 1) void w4a16_tile_kernel(const TileArgs a) {
     extern __shared__ __attribute__((aligned(16))) uint32_t lds_all[];
     using L = TileLds<MT, KW>;
@@ -397,12 +398,12 @@ __global__ __launch_bounds__(256 * KW, 1) void w4a16_tile_kernel(const TileArgs 
     float* red = reinterpret_cast<float*>(lds_all);  // [4 KW waves][32 rows][132]
     constexpr int NW = 4 * KW;
     const bool split_k = a.splits > 1;
-    const bool gated = EXT && a.epi.gated != 0;  // uniform
+    constexpr bool gated = EXT == 2;
 
     // one finished unit: eight consecutive columns c0.. of output row m
-    auto emit = [&](int m, int c0, f4 lo, f4 hi) {
-        if constexpr (EXT) {
-            store_eight(a.epi, a.D, m, 128 * strip + c0, lo, hi);
+    auto emit = [&](int m, int c0, f4 lo, f4 hi, u32x4 ahead) {
+        if constexpr (EXT == 1) {
+            store_eight<true>(a.epi, a.D, m, 128 * strip + c0, lo, hi, ahead);
         } else {
             const size_t o = (size_t)m * a.N + 128 * strip + c0;
             if (a.epi.out_f32) {
@@ -428,6 +429,19 @@ __global__ __launch_bounds__(256 * KW, 1) void w4a16_tile_kernel(const TileArgs 
     char* part_tile = split_k ? reinterpret_cast<char*>(a.part) + (size_t)tile * a.splits * kSlotBytes : nullptr;
     // (The slot is the descriptor's base and not a scalar offset: with a scalar offset in a register the compiler puts no wait
     // state between a 16-byte store and the next instruction, and one that overwrites the stored registers changed what was stored.)
+    // The residual of a thread's units, requested in front of the exchange between the waves or of the slots' reading: a
+    // round trip in all, not one for every unit.
+    u32x4 ahead[MT][UPT];
+    auto request_residual = [&]() __attribute__((always_inline)) {
+        if constexpr (EXT == 1) {
+            const __amdgpu_buffer_rsrc_t rows = residual_rows(a.epi, m0, a.M, 128 * strip);
+#pragma unroll
+            for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+                for (int t = 0; t < UPT; ++t) ahead[mt][t] = residual_load(a.epi, rows, 32 * mt + ((tid + t * T) >> 4), 8 * (tid & 15));
+        }
+    };
+    if (!split_k) request_residual();
     const __amdgpu_buffer_rsrc_t part_rsrc = __builtin_amdgcn_make_buffer_rsrc(part_tile + (size_t)split * kSlotBytes, 0, split_k ? (unsigned)kSlotBytes : 0u, kRsrcFlags);
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) {
@@ -447,7 +461,10 @@ __global__ __launch_bounds__(256 * KW, 1) void w4a16_tile_kernel(const TileArgs 
             // c0 and c0 + 64 of the strip); else 512 units, two per thread
             const bool pairs_now = gated && !split_k;
             const int units = pairs_now ? 256 : 512;
-            for (int unit = tid; unit < units; unit += 256 * KW) {
+#pragma unroll
+            for (int t = 0; t < UPT; ++t) {
+                const int unit = tid + t * T;
+                if (unit >= units) break;  // uniform
                 const int row = pairs_now ? unit >> 3 : unit >> 4;
                 const int c0 = pairs_now ? (unit & 7) * 8 : (unit & 15) * 8;
                 const int m = m0 + mt * 32 + row;
@@ -459,13 +476,13 @@ __global__ __launch_bounds__(256 * KW, 1) void w4a16_tile_kernel(const TileArgs 
                     hi += *reinterpret_cast<const f4*>(src + ww * 32 * kRedStride + 4);
                 }
                 if (split_k) {
-                    const uint32_t at = 16u * (uint32_t)tid + 32u * T * (uint32_t)(mt * UPT + unit / T);
+                    const uint32_t at = 16u * (uint32_t)tid + 32u * T * (uint32_t)(mt * UPT + t);
                     if (m < a.M) {  // (1) rows that exist only
                         __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, lo), part_rsrc, at, 0, kDeviceScope);
                         __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, hi), part_rsrc, at + 16u * T, 0, kDeviceScope);
                     }
                 } else if (!gated) {
-                    if (m < a.M) emit(m, c0, lo, hi);
+                    if (m < a.M) emit(m, c0, lo, hi, ahead[mt][t]);
                 } else {
                     f4 ulo = *reinterpret_cast<const f4*>(src + 64), uhi = *reinterpret_cast<const f4*>(src + 68);
 #pragma unroll
@@ -508,6 +525,7 @@ __global__ __launch_bounds__(256 * KW, 1) void w4a16_tile_kernel(const TileArgs 
     __syncthreads();
     if (*last_flag == 0) return;  // uniform
     if (tid == 0) __hip_atomic_store(a.accum + tile, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    request_residual();
     // The slots of a batch are requested together, and an M tile's while the one in front of it is added up: one round trip
     // in place of one for every unit and split.  us of a launch, mean of 8 heights of prompt over 9 layers, against those: 96-row
     // tiles 3.4 less with 3 splits, 9.0 with 8; 128-row tiles 4.3 and 10.4; 64-row tiles 2.1 and 6.0; 32-row tiles 0.8 and 2.8; with
@@ -568,7 +586,7 @@ __global__ __launch_bounds__(256 * KW, 1) void w4a16_tile_kernel(const TileArgs 
                 }
                 if (m < a.M && slot < 8) store_eight_gated(a.epi, a.D, m, 64 * strip + 8 * slot, lo, hi, ulo, uhi);
             } else if (m < a.M) {
-                emit(m, 8 * slot, lo, hi);
+                emit(m, 8 * slot, lo, hi, ahead[mt][t]);
             }
         }
     }
@@ -583,7 +601,7 @@ bool tile_shape_ok(int m, int n, int k, int64_t ldx, int columns, const TilePlan
     return grid <= 0x7fffffffLL && ldx < (1LL << 24) && (int64_t)k * n / 2 < (1LL << 32);
 }
 
-template <int MT, bool EXT, int KW>
+template <int MT, int EXT, int KW>
 static hipError_t tile_launch_one(const TileArgs& a, int grid, hipStream_t stream) {
     const size_t shmem = TileLds<MT, KW>::kBytes;
     auto kern = &w4a16_tile_kernel<MT, EXT, KW>;
@@ -593,12 +611,14 @@ static hipError_t tile_launch_one(const TileArgs& a, int grid, hipStream_t strea
 
 template <int MT, int KW>
 static hipError_t tile_launch_ext(const TileArgs& a, bool ext, int grid, hipStream_t stream) {
-    return ext ? tile_launch_one<MT, true, KW>(a, grid, stream) : tile_launch_one<MT, false, KW>(a, grid, stream);
+    if (a.epi.gated) return tile_launch_one<MT, 2, KW>(a, grid, stream);
+    return ext ? tile_launch_one<MT, 1, KW>(a, grid, stream) : tile_launch_one<MT, 0, KW>(a, grid, stream);
 }
 
 template <int MT, int KW>
 static bool tile_allow_lds_one() {
-    return allow_lds(&w4a16_tile_kernel<MT, false, KW>, TileLds<MT, KW>::kBytes) && allow_lds(&w4a16_tile_kernel<MT, true, KW>, TileLds<MT, KW>::kBytes);
+    constexpr size_t bytes = TileLds<MT, KW>::kBytes;
+    return allow_lds(&w4a16_tile_kernel<MT, 0, KW>, bytes) && allow_lds(&w4a16_tile_kernel<MT, 1, KW>, bytes) && allow_lds(&w4a16_tile_kernel<MT, 2, KW>, bytes);
 }
 bool tile_allow_lds() {
     return tile_allow_lds_one<1, 1>() && tile_allow_lds_one<1, 2>() && tile_allow_lds_one<2, 1>() && tile_allow_lds_one<2, 2>() &&
@@ -635,7 +655,7 @@ int tile_launch(const void* A, int64_t lda, const void* B, const void* S, void* 
     const int64_t grid = (int64_t)a.strips * a.mblocks * a.splits;
     if (grid > 0x7fffffffLL) return UNIQL_E_SHAPE;
     hipError_t e;
-    const bool ext = epi.gated || epi.bias || epi.residual || epi.relu2 || epi.transpose || epi.n_store != n ||
+    const bool ext = epi.bias || epi.residual || epi.relu2 || epi.transpose || epi.n_store != n ||
                      epi.ldd != n || !epi.vec_ok;
     if (plan.mtiles == 1)
         e = plan.quartets == 2 ? tile_launch_ext<1, 2>(a, ext, (int)grid, stream) : tile_launch_ext<1, 1>(a, ext, (int)grid, stream);
