@@ -228,3 +228,21 @@ def test_transform_of_rows_off_the_16_byte_grid(gpu, dtype, dim):
             go(x)
         return
     assert torch.equal(go(x), go(x.clone()))
+
+
+@pytest.mark.parametrize("where", ["cpu", "cuda"])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
+def test_scales_of_a_quantised_weight_stay_on_the_device(gpu, where, dtype):
+    """the same layer wherever the scales are, and no wait for the device where they are beside the weight"""
+    from uniql_amd import layout
+    from uniql_amd.quantize.quant_linear_layers import W4A16B16O16Linear
+    lin = torch.nn.Linear(384, 200, bias=False, device=gpu, dtype=torch.float16)
+    lin.apply_gptq, lin.bits, lin.group_size = True, 4, 128
+    lin.group_scale = (0.006 + 0.004 * torch.rand((3, 200), generator=torch.Generator().manual_seed(3))).to(dtype).to(where)
+    torch.cuda.set_sync_debug_mode("error" if where == "cuda" else "default")
+    try:
+        q = W4A16B16O16Linear.from_fp16(lin)
+    finally:
+        torch.cuda.set_sync_debug_mode("default")
+    _, packed, scale = layout.quantize_and_pack(lin.weight.detach().cpu().t().contiguous(), 128, lin.group_scale.half().cpu(), pad_out=56)
+    assert torch.equal(q.weight.cpu(), packed) and torch.equal(q.scale.cpu(), scale)

@@ -106,7 +106,7 @@ _host_lock = threading.Lock()
 
 
 def host():
-    """The native binding of the calls a token is made of (lib/_host.so), bound to the loaded library."""
+    """The native binding of the calls a token is made of and of those that produce and cut a model (lib/_host.so), bound to the loaded library."""
     global _host
     if _host is not None:
         return _host
@@ -121,6 +121,7 @@ def host():
             spec.loader.exec_module(module)
             module.bind(*(ctypes.cast(fn, ctypes.c_void_p).value
                           for fn in (lib.uniql_w4a16_linear, lib.uniql_w4a16_linear_workspace, lib.uniql_w4_embedding_lookup,
-                                     lib.uniql_fwht, lib.uniql_fwht_composite, lib.uniql_status_string)))
+                                     lib.uniql_fwht, lib.uniql_fwht_composite, lib.uniql_fwht_columns, lib.uniql_w4a16_quantize,
+                                     lib.uniql_w4a16_cut_columns, lib.uniql_w4a16_cut_rows, lib.uniql_status_string)))
             _host = module
     return _host

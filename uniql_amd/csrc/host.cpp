@@ -1,9 +1,11 @@
-// The host side of the calls that a token is made of - layer, embedding lookup, rotation - between torch and the C
-// ABI, in one native step per call: argument checks, the output's allocation and the launch.
+// The host side of the calls that a token is made of - layer, embedding lookup, rotation - and of those that producing and
+// loading a model is made of - quantising, rotating down the columns, cutting - between torch and the C ABI, in one native
+// step per call: argument checks, the output's allocation and the launch.
 //
 // Bound by what it costs to get a launch out: at one token the kernels take 4-5 us, and the same checks in Python with
 // a ctypes call of 26 arguments took 14.2 us per W4A16B16O16Linear call, 10.9 per embedding lookup and 9.6 per
-// rotation.  The checks, their messages and the order in which they are made are those of uniql_amd.ops, which
+// rotation; the seven cuts of a pruned decoder layer, 53 us of kernels, took 77 (54 now), quantising
+// 14336 x 4096 39 (35 now; the kernel: 29).  The checks, their messages and the order in which they are made are those of uniql_amd.ops, which
 // validates a layer's own tensors once (prepare_linear) and hands the functions' addresses over (bind).
 // Nothing of a call is kept: no address of an input, no check, no output.  A layer's sizes -> scratch sizes map belongs to
 // the layer's handle and is a pure function of its key.  The interpreter lock is given up for the whole call - copies of
@@ -28,14 +30,23 @@ decltype(&uniql_w4a16_linear_workspace) p_workspace = nullptr;
 decltype(&uniql_w4_embedding_lookup) p_embedding = nullptr;
 decltype(&uniql_fwht) p_fwht = nullptr;
 decltype(&uniql_fwht_composite) p_composite = nullptr;
+decltype(&uniql_fwht_columns) p_fwht_columns = nullptr;
+decltype(&uniql_w4a16_quantize) p_quantize = nullptr;
+decltype(&uniql_w4a16_cut_columns) p_cut_columns = nullptr;
+decltype(&uniql_w4a16_cut_rows) p_cut_rows = nullptr;
 decltype(&uniql_status_string) p_status = nullptr;
 
-void bind(uintptr_t linear, uintptr_t workspace, uintptr_t embedding, uintptr_t fwht, uintptr_t composite, uintptr_t status) {
+void bind(uintptr_t linear, uintptr_t workspace, uintptr_t embedding, uintptr_t fwht, uintptr_t composite, uintptr_t fwht_columns,
+          uintptr_t quantize, uintptr_t cut_columns, uintptr_t cut_rows, uintptr_t status) {
     p_linear = reinterpret_cast<decltype(p_linear)>(linear);
     p_workspace = reinterpret_cast<decltype(p_workspace)>(workspace);
     p_embedding = reinterpret_cast<decltype(p_embedding)>(embedding);
     p_fwht = reinterpret_cast<decltype(p_fwht)>(fwht);
     p_composite = reinterpret_cast<decltype(p_composite)>(composite);
+    p_fwht_columns = reinterpret_cast<decltype(p_fwht_columns)>(fwht_columns);
+    p_quantize = reinterpret_cast<decltype(p_quantize)>(quantize);
+    p_cut_columns = reinterpret_cast<decltype(p_cut_columns)>(cut_columns);
+    p_cut_rows = reinterpret_cast<decltype(p_cut_rows)>(cut_rows);
     p_status = reinterpret_cast<decltype(p_status)>(status);
 }
 
@@ -182,6 +193,8 @@ Tensor embedding(const Tensor& ids_in, const Tensor& weight, const Tensor& scale
     return y;
 }
 
+int value_type(at::ScalarType t) { return t == at::kHalf ? UNIQL_DT_F16 : (t == at::kBFloat16 ? UNIQL_DT_BF16 : UNIQL_DT_F32); }
+
 // base 0: blocks of `block` values; else the composite transform of width base * 2^k.  New tensor.
 Tensor hadamard(const Tensor& x_in, int64_t block, int base, double scale, uintptr_t stream) {
     const py::gil_scoped_release release;
@@ -190,7 +203,7 @@ Tensor hadamard(const Tensor& x_in, int64_t block, int base, double scale, uintp
     const at::ScalarType t = x_in.scalar_type();
     if (t != at::kHalf && t != at::kBFloat16 && t != at::kFloat)
         fail("hadamard transform supports float16 / bfloat16 / float32, got " + std::string(c10::toString(t)));
-    const int type = t == at::kHalf ? UNIQL_DT_F16 : (t == at::kBFloat16 ? UNIQL_DT_BF16 : UNIQL_DT_F32);
+    const int type = value_type(t);
     const Tensor x = x_in.contiguous();
     const int64_t dim = x.size(-1), rows = dim ? x.numel() / dim : 0;
     if (dim > 0x7fffffff || block > 0x7fffffff) fail("the last axis is too wide");
@@ -201,6 +214,95 @@ Tensor hadamard(const Tensor& x_in, int64_t block, int base, double scale, uintp
                                : p_composite(x.data_ptr(), y.data_ptr(), rows, (int)dim, base, (float)scale, type, st);
     check(code, base == 0 ? "uniql_fwht" : "uniql_fwht_composite");
     return y;
+}
+
+// Down the columns of x [rows, cols]; nothing where the kernel does not take the matrix.  New tensor.
+std::optional<Tensor> hadamard_columns(const Tensor& x, double scale, uintptr_t stream) {
+    const py::gil_scoped_release release;
+    const at::NoGradGuard no_grad;
+    require_gpu(x, "x");
+    const at::ScalarType t = x.scalar_type();
+    if (x.dim() != 2 || (t != at::kHalf && t != at::kBFloat16 && t != at::kFloat) || !x.is_contiguous()) return std::nullopt;
+    const int64_t rows = x.size(0), cols = x.size(1);
+    if ((rows != 1024 && rows != 2048 && rows != 4096) || cols == 0 || cols % 8 || reinterpret_cast<uintptr_t>(x.data_ptr()) % 16)
+        return std::nullopt;
+    if (cols > 0x7fffffff) fail("the last axis is too wide");
+    const c10::DeviceGuard guard(x.device());
+    Tensor y = at::empty_like(x);
+    check(p_fwht_columns(x.data_ptr(), y.data_ptr(), (int)rows, (int)cols, (float)scale, value_type(t), reinterpret_cast<void*>(stream)),
+          "uniql_fwht_columns");
+    return y;
+}
+
+// weight [out, in] and, of weights that are quantised already, their scales [k_pad / 128, out] -> packed and permuted.  New tensors.
+std::pair<Tensor, Tensor> new_packed(int64_t k, int64_t n, const Tensor& like) {
+    return {new_output({k / 16, 2 * n}, at::kInt, like), new_output({k / 128, n}, at::kHalf, like)};
+}
+std::pair<Tensor, Tensor> quantize(const Tensor& weight, const std::optional<Tensor>& given, int64_t pad_out, uintptr_t stream) {
+    const py::gil_scoped_release release;
+    const at::NoGradGuard no_grad;
+    require_gpu(weight, "weight");
+    if (weight.scalar_type() != at::kHalf || weight.dim() != 2 || weight.stride(1) != 1)
+        fail("weight must be float16 [out_features, in_features] with unit inner stride");
+    const int64_t n = weight.size(0), k = weight.size(1), k_pad = (k + 127) / 128 * 128, n_pad = n + pad_out;
+    if (given) {
+        require_gpu(*given, "given_scale");
+        if (given->scalar_type() != at::kHalf || given->dim() != 2 || given->size(0) != k_pad / 128 || given->size(1) != n ||
+            !given->is_contiguous())
+            fail("given_scale must be contiguous float16 [k_pad/128, out_features]");
+    }
+    if (n > 0x7fffffff || n_pad < 0 || n_pad > 0x7fffffff || k_pad > 0x7fffffff) fail("weight is larger than a call can take");
+    const c10::DeviceGuard guard(weight.device());
+    auto out = new_packed(k_pad, n_pad, weight);
+    check(p_quantize(weight.data_ptr(), weight.stride(0), given ? given->data_ptr() : nullptr, out.first.data_ptr(), out.second.data_ptr(),
+                     (int)n, (int)k, (int)n_pad, (int)k_pad, reinterpret_cast<void*>(stream)),
+          "uniql_w4a16_quantize");
+    return out;
+}
+
+// A packed group-128 matrix [k / 16, 2 n] with its scales [groups, n].
+void require_packed(const Tensor& B, const Tensor& s, int64_t n, int64_t k) {
+    require_gpu(B, "B");
+    require_gpu(s, "s");
+    if (B.scalar_type() != at::kInt || s.scalar_type() != at::kHalf || !B.is_contiguous() || !s.is_contiguous())
+        fail("B must be contiguous int32 and s contiguous float16");
+    if (k < 0 || B.dim() != 2 || B.size(0) != k / 16 || B.size(1) != 2 * n || s.dim() != 2 || s.size(1) != n)
+        fail("B / s shapes do not match size_k, size_n");
+}
+
+// runs: six values each.  New tensors.
+std::pair<Tensor, Tensor> cut_columns(const Tensor& B, const Tensor& s, int n, int k, const std::vector<int>& runs,
+                                      std::optional<int> k_real, std::optional<int> n_scaled, int64_t pad_out, uintptr_t stream) {
+    const py::gil_scoped_release release;
+    const at::NoGradGuard no_grad;
+    require_packed(B, s, n, k);
+    if (s.size(0) != k / 128) fail("scales must be [k/128, n]");
+    if (runs.size() % 6) fail("runs must have six values each");
+    int64_t n_pad = pad_out;
+    for (size_t i = 0; i < runs.size(); i += 6) n_pad += (int64_t)runs[i + 1] * runs[i + 3];
+    if (n_pad < 0 || n_pad > 0x7fffffff) fail("the kept width is not one that a call can take");
+    const c10::DeviceGuard guard(B.device());
+    auto out = new_packed(k, n_pad, B);
+    check(p_cut_columns(B.data_ptr(), s.data_ptr(), n, k, k_real.value_or(k), runs.data(), (int)(runs.size() / 6),
+                        n_scaled.value_or((int)n_pad), out.first.data_ptr(), out.second.data_ptr(), (int)n_pad,
+                        reinterpret_cast<void*>(stream)),
+          "uniql_w4a16_cut_columns");
+    return out;
+}
+
+std::pair<Tensor, Tensor> cut_rows(const Tensor& B, const Tensor& s, int n, int k, int units, int full, int kept, int n_real,
+                                   int64_t pad_out, uintptr_t stream) {
+    const py::gil_scoped_release release;
+    const at::NoGradGuard no_grad;
+    require_packed(B, s, n, k);
+    const int64_t k_pad = ((int64_t)units * kept + 127) / 128 * 128, n_pad = n_real + pad_out;
+    if (k_pad < 0 || n_pad < 0 || n_pad > 0x7fffffff) fail("the kept sizes are not ones that a call can take");
+    const c10::DeviceGuard guard(B.device());
+    auto out = new_packed(k_pad, n_pad, B);
+    check(p_cut_rows(B.data_ptr(), s.data_ptr(), n, k, (int)s.size(0), units, full, kept, n_real, out.first.data_ptr(),
+                     out.second.data_ptr(), (int)n_pad, reinterpret_cast<void*>(stream)),
+          "uniql_w4a16_cut_rows");
+    return out;
 }
 
 }  // namespace
@@ -229,4 +331,8 @@ PYBIND11_MODULE(_host, module) {
     module.def("bind", &bind);
     module.def("embedding", &embedding);
     module.def("hadamard", &hadamard);
+    module.def("hadamard_columns", &hadamard_columns);
+    module.def("quantize", &quantize);
+    module.def("cut_columns", &cut_columns);
+    module.def("cut_rows", &cut_rows);
 }

@@ -423,28 +423,7 @@ def w4a16_quantize(weight: torch.Tensor, given_scale: torch.Tensor | None = None
     GPU) into (packed int32 [k_pad/16, 2 n_pad], permuted scale fp16 [k_pad/128, n_pad]), with the
     host arithmetic of the reference's from_fp16 / w4a16_quantize bit for bit.  given_scale:
     natural-order [k_pad/128, out_features] scales of already fake-quantised weights (GPTQ)."""
-    _require_gpu(weight, "weight")
-    if weight.dtype != torch.float16 or weight.dim() != 2 or weight.stride(1) != 1:
-        raise RuntimeError("weight must be float16 [out_features, in_features] with unit inner stride")
-    out_features, in_features = weight.shape
-    k_pad = (in_features + 127) // 128 * 128
-    n_pad = out_features + pad_out
-    dev = weight.device
-    if given_scale is not None:
-        _require_gpu(given_scale, "given_scale")
-        if given_scale.dtype != torch.float16 or tuple(given_scale.shape) != (k_pad // 128, out_features) \
-                or not given_scale.is_contiguous():
-            raise RuntimeError("given_scale must be contiguous float16 [k_pad/128, out_features]")
-    lib = _capi.load()
-    with _device_guard(dev):
-        B = torch.empty((k_pad // 16, 2 * n_pad), dtype=torch.int32, device=dev)
-        S = torch.empty((k_pad // 128, n_pad), dtype=torch.float16, device=dev)
-        code = lib.uniql_w4a16_quantize(weight.data_ptr(), weight.stride(0),
-                                        given_scale.data_ptr() if given_scale is not None else None,
-                                        B.data_ptr(), S.data_ptr(), out_features, in_features, n_pad, k_pad,
-                                        _stream_ptr(dev))
-    _capi.check(code, "uniql_w4a16_quantize")
-    return B, S
+    return _capi.host().quantize(weight, given_scale, pad_out, _stream_of(weight, "weight"))
 
 
 def w4a16_pack(codes: torch.Tensor, scales: torch.Tensor, pad_out: int = 0):
@@ -480,52 +459,20 @@ def w4a16_unpack(B: torch.Tensor, s: torch.Tensor, size_n: int, size_k: int):
     return codes, s[:, pos].contiguous()
 
 
-def _require_packed(B: torch.Tensor, s: torch.Tensor, size_n: int, size_k: int) -> None:
-    _require_gpu(B, "B")
-    _require_gpu(s, "s")
-    if B.dtype != torch.int32 or s.dtype != torch.float16 or not (B.is_contiguous() and s.is_contiguous()):
-        raise RuntimeError("B must be contiguous int32 and s contiguous float16")
-    if tuple(B.shape) != (size_k // 16, 2 * size_n) or s.dim() != 2 or s.shape[1] != size_n:
-        raise RuntimeError("B / s shapes do not match size_k, size_n")
-
-
 def w4a16_cut_columns(B: torch.Tensor, s: torch.Tensor, size_n: int, size_k: int, runs, k_real: int | None = None,
                       n_scaled: int | None = None, pad_out: int = 0):
     """Keeps columns of a packed group-128 matrix: w4a16_pack of the kept columns of w4a16_unpack, straight from packed to
     packed.  runs: up to five (base, units, full, kept, split, skip), each `kept` of every `full` columns from `base` on, `units`
     times: the first `split`, and the others `skip` columns further on.  Rows from k_real on get code 0; kept columns from n_scaled on get scale 0; pad_out padding columns follow."""
-    _require_packed(B, s, size_n, size_k)
-    if s.shape[0] != size_k // 128:
-        raise RuntimeError("scales must be [k/128, n]")
-    n_pad = sum(run[1] * run[3] for run in runs) + pad_out
     flat = [int(v) for run in runs for v in run]
-    lib = _capi.load()
-    dev = B.device
-    with _device_guard(dev):
-        B_out = torch.empty((size_k // 16, 2 * n_pad), dtype=torch.int32, device=dev)
-        S_out = torch.empty((size_k // 128, n_pad), dtype=torch.float16, device=dev)
-        code = lib.uniql_w4a16_cut_columns(B.data_ptr(), s.data_ptr(), size_n, size_k, size_k if k_real is None else k_real,
-                                           (ctypes.c_int * len(flat))(*flat), len(runs), n_pad if n_scaled is None else n_scaled,
-                                           B_out.data_ptr(), S_out.data_ptr(), n_pad, _stream_ptr(dev))
-    _capi.check(code, "uniql_w4a16_cut_columns")
-    return B_out, S_out
+    return _capi.host().cut_columns(B, s, size_n, size_k, flat, k_real, n_scaled, pad_out, _stream_of(B, "B"))
 
 
 def w4a16_cut_rows(B: torch.Tensor, s: torch.Tensor, size_n: int, size_k: int, units: int, full: int, kept: int, n_real: int,
                    pad_out: int = 0):
     """Keeps the first `kept` of every `full` rows, `units` times, of a packed matrix's first n_real columns and quantises them
     in their new groups: w4a16_quantize of the kept rows of w4a16_dequant, in one kernel."""
-    _require_packed(B, s, size_n, size_k)
-    k_pad, n_pad = (units * kept + 127) // 128 * 128, n_real + pad_out
-    lib = _capi.load()
-    dev = B.device
-    with _device_guard(dev):
-        B_out = torch.empty((k_pad // 16, 2 * n_pad), dtype=torch.int32, device=dev)
-        S_out = torch.empty((k_pad // 128, n_pad), dtype=torch.float16, device=dev)
-        code = lib.uniql_w4a16_cut_rows(B.data_ptr(), s.data_ptr(), size_n, size_k, s.shape[0], units, full, kept, n_real,
-                                        B_out.data_ptr(), S_out.data_ptr(), n_pad, _stream_ptr(dev))
-    _capi.check(code, "uniql_w4a16_cut_rows")
-    return B_out, S_out
+    return _capi.host().cut_rows(B, s, size_n, size_k, units, full, kept, n_real, pad_out, _stream_of(B, "B"))
 
 
 def w4a16_embedding_lookup(input: torch.Tensor, weight: torch.Tensor, scale: torch.Tensor) -> torch.Tensor:
@@ -614,25 +561,10 @@ def hadamard_composite(x: torch.Tensor, scale: float, base: int) -> torch.Tensor
     return _capi.host().hadamard(x, x.shape[-1], base, scale, _stream_of(x, "x"))
 
 
-_COLUMN_ROWS = (1024, 2048, 4096)   # heights uniql_fwht_columns takes
-
-
 def hadamard_columns(x: torch.Tensor, scale: float) -> torch.Tensor | None:
     """(H_rows . x) * scale for a contiguous matrix x [rows, cols]: fast_hadamard_transform(x.t(), scale).t() without
     the transposed copies, a new contiguous tensor; None where the kernel does not take the shape."""
-    _require_gpu(x, "x")
-    dtypes = {torch.float16: _capi.DT_F16, torch.bfloat16: _capi.DT_BF16, torch.float32: _capi.DT_F32}
-    if x.dim() != 2 or x.dtype not in dtypes or not x.is_contiguous() or x.shape[0] not in _COLUMN_ROWS or x.shape[1] == 0 \
-            or x.shape[1] % 8 or x.data_ptr() % 16:
-        return None
-    lib = _capi.load()
-    dev = x.device
-    with _device_guard(dev):
-        y = torch.empty_like(x)
-        code = lib.uniql_fwht_columns(x.data_ptr(), y.data_ptr(), x.shape[0], x.shape[1], float(scale), dtypes[x.dtype],
-                                      _stream_ptr(dev))
-    _capi.check(code, "uniql_fwht_columns")
-    return y
+    return _capi.host().hadamard_columns(x, scale, _stream_of(x, "x"))
 
 
 class UnpinnedHadamardWarning(UserWarning):

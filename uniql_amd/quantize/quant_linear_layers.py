@@ -63,7 +63,7 @@ class W4A16B16O16Linear(nn.Module):
             if originalLayer.bits != 4:
                 raise AssertionError("Only support 4-bit quantization")
             group_size = originalLayer.group_size
-            given_scale = originalLayer.group_scale.to(torch.float16).cpu()
+            given_scale = originalLayer.group_scale.to(torch.float16)
         if group_size not in (-1, 128):
             raise ValueError("Only groupsize -1 and 128 are supported.")
         W = originalLayer.weight
@@ -79,6 +79,7 @@ class W4A16B16O16Linear(nn.Module):
                 q.bias = nn.Parameter(originalLayer.bias.data.clone())
             return q
         w_t = W.detach().cpu().to(torch.float16).t().contiguous()      # [Din, Dout]
+        given_scale = None if given_scale is None else given_scale.cpu()
         w_ref, packed, scale = layout.quantize_and_pack(w_t, group_size, given_scale, pad_out=q.pad_out)
         q.size_k, q.size_n = w_ref.shape
         q.pad_in = q.size_k - w_t.shape[0]
