@@ -624,13 +624,16 @@ __global__ __launch_bounds__(256) void fwht_composite_kernel(const T* __restrict
 // The same for P >= 128.  A wave transforms blocks of 512 consecutive values (whole chunks, or a half or quarter of one) by
 // itself: 16-byte loads and index bits 0..2 in registers, bits 3..5 and 6..8 in two LDS passes without a workgroup barrier;
 // chunks of more than 512 values have one or two bits left for the workgroup.  Then the base matrix across the chunks with
-// its signs as constants, one addition per term, on pairs of neighbouring columns; the terms are added in ascending
-// order, starting from zero, as fwht_composite_kernel does: the same bits.
-// What bounds it: the additions, BASE for every value (a SIMD takes a plain fp32 addition in two clocks; the matrix unit's
-// fp32 forms, tried, hold the vector unit up for as long as the additions take), about as long as the memory time, and at
-// most two rows of 14336 in a compute unit's LDS.  So the workgroups stay, and request their next row before they
-// transform the current one.  fp16, against one row a workgroup with a barrier behind every pass: 1024 rows of 14336 20.9
-// -> 18.7 us, 4096 rows 72 -> 67; 1024 rows of 3584 8.3 -> 7.5, of 5120 (40 x 128) 13.6 -> 10.7, one row of 14336 6.9 -> 6.2.
+// its signs as constants, on pairs of neighbouring columns; the terms are added in ascending order, starting from zero, as
+// fwht_composite_kernel does: the same bits.  Outputs whose first signs agree share the sums of those terms: with the outputs
+// in the order of their signs, quarter by quarter, 639 additions a column in place of 784 (28), 1134 of 1600 (40), 333 of 400
+// (20), 112 of 144 (12).
+// What bounds it: the additions (a SIMD takes one of a wave in 2.4 clocks; the matrix unit's fp32 forms, tried, hold the
+// vector unit up for as long as the additions take) and eight passes of the row through LDS, each about as long as the memory
+// time, and at most two rows of 14336 in a compute unit's LDS to overlap them.  So the workgroups stay, and request their next
+// row before they transform the current one.  fp16, one row a workgroup with a barrier behind every pass -> workgroups that
+// stay -> shared sums: 1024 rows of 14336 20.9 -> 18.7 -> 18.2 us, 4096 rows 72 -> 66.3 -> 63.9; 4096 rows of 5120 (40 x 128)
+// 30.7 -> 26.3 by the shared sums, of fp32 34.8 -> 32.6; one row of 14336 6.9 -> 6.2.
 template <int BASE>
 struct BaseTable;
 template <> struct BaseTable<12> { static constexpr const uint64_t (&mask)[12] = kHadamard12; };
@@ -638,22 +641,42 @@ template <> struct BaseTable<20> { static constexpr const uint64_t (&mask)[20] =
 template <> struct BaseTable<28> { static constexpr const uint64_t (&mask)[28] = kHadamard28; };
 template <> struct BaseTable<40> { static constexpr const uint64_t (&mask)[40] = kHadamard40; };
 
-template <int BASE, int C, int CP>
-__device__ __forceinline__ void base_terms(const float2 (&z)[BASE], float& a, float& b) {
-    if constexpr (CP < BASE) {
-        constexpr bool minus = (BaseTable<BASE>::mask[C] >> CP) & 1ull;
-        a = minus ? a - z[CP].x : a + z[CP].x;
-        b = minus ? b - z[CP].y : b + z[CP].y;
-        base_terms<BASE, C, CP + 1>(z, a, b);
+// The outputs ordered by the signs of their terms, the first term's first: those whose sums begin alike are neighbours.
+template <int BASE>
+struct BaseOrder {
+    int output[BASE];
+    constexpr BaseOrder() : output() {
+        for (int i = 0; i < BASE; ++i) {
+            int at = i;
+            for (; at > 0 && before(i, output[at - 1]); --at) output[at] = output[at - 1];
+            output[at] = i;
+        }
     }
-}
-template <typename T, int BASE, int C, int END>
-__device__ __forceinline__ void base_outputs(const float2 (&z)[BASE], T* yp, int P, float scale) {
-    if constexpr (C < END) {
-        float a = 0.f, b = 0.f;
-        base_terms<BASE, C, 0>(z, a, b);
-        RowIo<T>::store2(yp + C * P, a, b, scale);
-        base_outputs<T, BASE, C + 1, END>(z, yp, P, scale);
+    static constexpr bool minus(int c, int term) { return (BaseTable<BASE>::mask[c] >> term) & 1ull; }
+    static constexpr bool before(int a, int b) {
+        for (int t = 0; t < BASE; ++t)
+            if (minus(a, t) != minus(b, t)) return minus(b, t);
+        return false;
+    }
+    // of outputs lo .. hi - 1 in this order, which agree in the terms in front of `term`: the first that subtracts it
+    constexpr int split(int lo, int hi, int term) const {
+        while (lo < hi && !minus(output[lo], term)) ++lo;
+        return lo;
+    }
+};
+template <int BASE>
+inline constexpr BaseOrder<BASE> kBaseOrder{};
+
+// Outputs LO .. HI - 1 of that order, which agree in their first TERM terms: a, b are the sums of those.
+template <typename T, int BASE, int LO, int HI, int TERM = 0>
+__device__ __forceinline__ void base_outputs(const float2 (&z)[BASE], T* yp, int P, float scale, float a = 0.f, float b = 0.f) {
+    if constexpr (TERM == BASE) {
+        static_assert(HI - LO == 1);
+        RowIo<T>::store2(yp + kBaseOrder<BASE>.output[LO] * P, a, b, scale);
+    } else {
+        constexpr int mid = kBaseOrder<BASE>.split(LO, HI, TERM);
+        if constexpr (LO < mid) base_outputs<T, BASE, LO, mid, TERM + 1>(z, yp, P, scale, a + z[TERM].x, b + z[TERM].y);
+        if constexpr (mid < HI) base_outputs<T, BASE, mid, HI, TERM + 1>(z, yp, P, scale, a - z[TERM].x, b - z[TERM].y);
     }
 }
 
