@@ -41,6 +41,11 @@ static inline size_t tile_part_bytes(int m, int n, const TilePlan& plan) {
 // is off is mostly the epilogue, which a plan must not depend on (a layer's sum is the same with and without a residual):
 // adding one costs the tall tiles 4 to 8 us a round.  Of another 6250 calls the plan with the smallest time here took 1.003 x
 // the best plan's time on average.
+// The exchange of 64- (one quartet), 96- and 128-row tiles since its slots are read in batches: of 300 drawn calls of 65 to 700
+// rows whose plan that changed (96-row tiles with 2 to 7 splits in place of shorter ones, mostly) 282 are faster, by 12 % on
+// average (14336 -> 6144 at 84 rows 35.6 -> 27.9 us, 12160 -> 4096 at 66 27.2 -> 21.4, 4096 -> 11264 at 96 20.8 -> 19.3), and 8
+// slower by more than 4 %.  Kept above what is measured (1 us for two splits, 2 for eight) for 64-row tiles, so that one quartet
+// does not replace two, whose sums are half as long chains, and as it was for 32-row tiles, up to 64 rows the other kernel's rivals.
 struct LaunchFit {
     double full, full_g;        // a whole round: constant, per K group
     double split, split_each;   // the exchange between K splits (partial tiles' stores, count, the last one's reading of all of them)
@@ -56,10 +61,10 @@ static const LaunchFit kLaunchFits[7] = {
     {8.65, 1.351, 0.537, 0.77, 4.03, 4, {{5.34, 0.814, 0.391, 0.355, 0.404}, {5.78, 1.127, 0.581, 0.639, 0.715},
      {6.82, 1.054, 1.019, 1.032, 1.138}, {8.86, 1.117, 1.304, 1.379, 1.453}}},  // 32 rows, one quartet
     {5.29, 0.35, 0.763, 0.547, 5.46, 1, {{5.46, 1.0, 0.279, 0.282, 0.339}}},  // 32 rows, two quartets
-    {5.59, 1.001, 1.509, 1.112, 5.58, 2, {{6.82, 0.989, 0.447, 0.452, 0.577}, {7.16, 1.085, 0.8, 0.938, 1.074}}},  // 64 rows, one quartet
+    {5.59, 1.001, 1.6, 0.85, 5.58, 2, {{6.82, 0.989, 0.447, 0.452, 0.577}, {7.16, 1.085, 0.8, 0.938, 1.074}}},  // 64 rows, one quartet
     {7.46, 0.521, 0.852, 0.935, 7.15, 1, {{7.15, 1.0, 0.365, 0.381, 0.498}}},  // 64 rows, two quartets
-    {6.97, 0.74, 2.88, 1.858, 4.67, 1, {{6.35, 1.083, 0.478, 0.604, 0.743}}},  // 96 rows
-    {5.98, 0.95, 1.877, 2.68, 7.49, 1, {{8.94, 1.043, 0.493, 0.692, 0.9}}},  // 128 rows
+    {6.97, 0.74, 2.3, 0.79, 4.67, 1, {{6.35, 1.083, 0.478, 0.604, 0.743}}},  // 96 rows
+    {5.98, 0.95, 1.877, 1.2, 7.49, 1, {{8.94, 1.043, 0.493, 0.692, 0.9}}},  // 128 rows
     {7.65, 3.39, 0.0, 0.0, 4.41, 1, {{13.28, 1.095, 2.15, 2.64, 3.29}}},  // 256 x 256
 };
 static inline double launch_us(const LaunchFit& f, int64_t wgs, int g, int splits) {
