@@ -61,7 +61,10 @@ def test_infinities_and_nan_stay_in_their_row(gpu, dim, base):
 # every tile width: four, eight and sixteen waves, at the edges of the rules that choose them; a last tile that is cut
 @pytest.mark.parametrize("rows,cols,dtype", [(1024, 4096, torch.float16), (1024, 8184, torch.float16), (1024, 8200, torch.bfloat16),
                                              (2048, 4104, torch.float16), (4096, 4088, torch.float32), (4096, 4104, torch.float32),
-                                             (4096, 264, torch.float32), (2048, 8, torch.float32)])
+                                             (4096, 264, torch.float32), (2048, 8, torch.float32),
+                                             (4096, 2552, torch.float16), (4096, 2560, torch.float16), (4096, 2568, torch.bfloat16),
+                                             (4096, 4352, torch.float16), (4096, 4360, torch.float16), (4096, 6152, torch.bfloat16),
+                                             (4096, 8200, torch.float16)])
 def test_column_tiles(gpu, rows, cols, dtype):
     """bit for bit the row transform between two transposed copies; an infinity stays in its column"""
     from uniql_amd import ops

@@ -539,6 +539,125 @@ __global__ __launch_bounds__(64 * WAVES, 4) void fwht_columns_kernel(const T* __
     }
 }
 
+// The same over 4096 rows for 16-bit values, two chunks of eight columns a workgroup, one after the other.  Eight columns are
+// 16 bytes of a row, and the caches' requests for those were what bound the tiles above; here neighbouring lanes read and
+// write neighbouring chunks of a row, 32 bytes a request, and swap halves: a wave then holds one chunk of its 512 rows in
+// fp32, as above, and the other as it was read, later the first one's results, rounded.  That is all the registers of two
+// workgroups a compute unit, hence the empty asm statements (values packed, and columns finished, where they are written) and
+// the scheduling barriers: without them 40 to 70 registers spill.
+// What bounds it now: load, passes and stores follow each other in all workgroups at once.  fp16, cold, us with eight columns and
+// with sixteen: 4096 x 4096 35.7 -> 28.9, x 8192 82.4 -> 54.8, x 11008 98 -> 64, x 14336 103.5 -> 82.0.
+__device__ __forceinline__ void swap_neighbours(bool odd, uint32_t& a, uint32_t& b) {  // an even lane's b for the next lane's a
+    const uint32_t mine = odd ? a : b;
+    const uint32_t other = (uint32_t)__builtin_amdgcn_mov_dpp((int)mine, 0xB1, 0xF, 0xF, true);  // lane ^ 1
+    a = odd ? other : a;
+    b = odd ? b : other;
+}
+
+template <typename T>
+__global__ __launch_bounds__(512, 4) void fwht_column_pairs_kernel(const T* __restrict__ x, T* __restrict__ y, int cols, int tiles, float scale) {
+    extern __shared__ __attribute__((aligned(16))) float fbuf[];
+    using Tile = ColumnTile<12, 8>;
+    constexpr int kFlight = 2;  // columns of a wave in LDS together
+    const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int per_xcd = (tiles + 7) >> 3;
+    const int tile = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
+    if (tile >= tiles) return;  // uniform
+    const int col0 = tile * 16;
+    const bool odd = lane & 1, second = col0 + 8 < cols;  // cols is a multiple of eight
+    u32x4 chunk[2][8];  // [.. of eight columns][row 8 lane + ..]
+    {
+        const char* src = reinterpret_cast<const char*>(x + (size_t)(512 * w) * cols + col0);
+        const uint32_t mine = 16u * ((uint32_t)(lane & ~1) * (uint32_t)cols + (odd && second ? 1u : 0u));  // bytes
+#pragma unroll
+        for (int i = 0; i < 16; ++i) chunk[i >> 3][i & 7] = *reinterpret_cast<const u32x4*>(src + (size_t)i * cols * sizeof(T) + mine);
+    }
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            uint32_t a = chunk[0][i][j], b = chunk[1][i][j];
+            swap_neighbours(odd, a, b);
+            chunk[0][i][j] = a;
+            chunk[1][i][j] = b;
+        }
+    __builtin_amdgcn_sched_barrier(0);
+    float* own = fbuf + w * (kFlight * 576);
+    const int quad = tid & 1, at = tid >> 1;
+    const uint32_t out = quad == 1 && !second ? 0xfffffff0u : 2u * (((uint32_t)(at & 63) + 128 * (uint32_t)(at >> 6)) * (uint32_t)cols + 8 * (uint32_t)quad);  // bytes
+    uint32_t kept[2][8][2];  // the first chunk's results: [half][wave]
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {
+        float f[8][8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            asm volatile("" : "+v"(chunk[c][i]));
+            RowIo<T>::unpack(typename RowIo<T>::Raw{chunk[c][i]}, f[i]);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        if (c == 1) lds_barrier();  // others may still be reading the first chunk's last half
+#pragma unroll
+        for (int e0 = 0; e0 < 8; e0 += kFlight) {
+#pragma unroll
+            for (int e = e0; e < e0 + kFlight; ++e) {
+                float g[8];
+#pragma unroll
+                for (int i = 0; i < 8; ++i) g[i] = f[i][e];
+                wht8(g);
+                wht512_pass3(own + (e - e0) * 576, lane, lane, g);
+                wht512_upper(g, 512);
+#pragma unroll
+                for (int i = 0; i < 8; ++i) f[i][e] = g[i];
+                asm volatile("" : "+v"(f[0][e]), "+v"(f[1][e]), "+v"(f[2][e]), "+v"(f[3][e]), "+v"(f[4][e]), "+v"(f[5][e]), "+v"(f[6][e]), "+v"(f[7][e]));
+            }
+            lds_wave_fence();
+            __builtin_amdgcn_sched_barrier(0);
+        }
+#pragma unroll
+        for (int half = 0; half < 2; ++half) {
+            __builtin_amdgcn_sched_barrier(0);
+            lds_barrier();
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const float (&r)[8] = f[2 * q + half];
+                float* dst = fbuf + (lane + 64 * q) * Tile::kStride + w * 8;
+                *reinterpret_cast<f4*>(dst) = f4{r[0], r[1], r[2], r[3]};
+                *reinterpret_cast<f4*>(dst + 4) = f4{r[4], r[5], r[6], r[7]};
+            }
+            lds_barrier();
+            f4 v[8];
+#pragma unroll
+            for (int r = 0; r < 8; ++r) v[r] = *reinterpret_cast<const f4*>(fbuf + at * Tile::kStride + r * 8 + 4 * quad);
+#pragma unroll
+            for (int h = 1; h < 8; h <<= 1)
+#pragma unroll
+                for (int r = 0; r < 8; ++r)
+                    if ((r & h) == 0) {
+                        const f4 p = v[r], q = v[r + h];
+                        v[r] = p + q;
+                        v[r + h] = p - q;
+                    }
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int r = 0; r < 8; ++r) {
+                uint32_t lo = RowIo<T>::pair(v[r][0], v[r][1], scale), hi = RowIo<T>::pair(v[r][2], v[r][3], scale);
+                if (c == 0) {
+                    asm volatile("" : "+v"(lo), "+v"(hi));  // in 32 registers
+                    kept[half][r][0] = lo;
+                    kept[half][r][1] = hi;
+                } else {
+                    // an even thread has columns 0 .. 3 of both chunks, the next one 4 .. 7
+                    swap_neighbours(odd, kept[half][r][0], lo);
+                    swap_neighbours(odd, kept[half][r][1], hi);
+                    const __amdgpu_buffer_rsrc_t rows = __builtin_amdgcn_make_buffer_rsrc(y + (size_t)(512 * r + 64 * half) * cols + col0, 0, 0x7fffffff, 0x00020000);
+                    __builtin_amdgcn_raw_buffer_store_b128(u32x4{kept[half][r][0], kept[half][r][1], lo, hi}, rows, out, 0, 0);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+    }
+}
+
 template <typename T, int LOG2L, int WAVES>
 static int fwht_columns_tiles(const void* x, void* y, int cols, float scale, hipStream_t stream) {
     using Tile = ColumnTile<LOG2L, WAVES>;
@@ -549,9 +668,24 @@ static int fwht_columns_tiles(const void* x, void* y, int cols, float scale, hip
                        reinterpret_cast<const T*>(x), reinterpret_cast<T*>(y), cols, tiles, scale);
     return hipGetLastError() == hipSuccess ? UNIQL_OK : UNIQL_E_LAUNCH;
 }
+template <typename T>
+static int fwht_column_pairs(const void* x, void* y, int cols, float scale, hipStream_t stream) {
+    static std::atomic<unsigned long long> done{0};
+    constexpr size_t bytes = ColumnTile<12, 8>::kBytes;
+    if (!allow_lds(&fwht_column_pairs_kernel<T>, bytes, done)) return UNIQL_E_LAUNCH;
+    const int tiles = (cols + 15) / 16;
+    hipLaunchKernelGGL(fwht_column_pairs_kernel<T>, dim3((unsigned)((tiles + 7) / 8 * 8)), dim3(512), bytes, stream,
+                       reinterpret_cast<const T*>(x), reinterpret_cast<T*>(y), cols, tiles, scale);
+    return hipGetLastError() == hipSuccess ? UNIQL_OK : UNIQL_E_LAUNCH;
+}
 template <typename T, int LOG2L>
 static int fwht_columns_go(const void* x, void* y, int cols, float scale, hipStream_t stream) {
-    // The widest tiles of which every compute unit gets one: eight waves, two workgroups a compute unit; sixteen for fp32
+    if constexpr (LOG2L == 12 && sizeof(T) == 2)
+        if (cols >= 2560 && cols < (1 << 21) && !(cols > 4352 && cols <= 6144)) return fwht_column_pairs<T>(x, y, cols, scale, stream);
+    // 16-bit values of 4096 rows in tiles of sixteen columns from 2560 columns on, where they keep more than half of the compute
+    // units busy (2048: 22 us, 18.4 with eight columns; 2560: 27.5 and 28.2), and not from 4353 to 6144, where a few compute
+    // units get a second one (5120: 48 us and 42.7).
+    // Else the widest tiles of which every compute unit gets one: eight waves, two workgroups a compute unit; sixteen for fp32
     // over 4096 rows, where eight columns are a full sector and only one workgroup's stores fit beside the other's loads
     // (4096 x 14336: 150 us against 165; fp16 102 either way); four for few columns of 1024 rows (x 4096: 8.5 us against 9.3).
     if (LOG2L == 12 && sizeof(T) == 4 && cols >= 256 * ColumnTile<LOG2L, 16>::kColumns) return fwht_columns_tiles<T, LOG2L, LOG2L == 12 && sizeof(T) == 4 ? 16 : 8>(x, y, cols, scale, stream);
