@@ -106,6 +106,25 @@ def test_embedding_quantize_bit_exact(gpu, v, d):
     assert np.array_equal(packed.cpu().numpy(), np.asarray(o_packed))
 
 
+@pytest.mark.parametrize("d", [8, 512, 520, 2048, 2056, 4096, 4104, 5120, 5128, 8184, 8192])
+def test_embedding_quantize_rows_in_registers(gpu, d):
+    """the same bits as the rows inside a wider table, which takes the kernel that divides: every magnitude, subnormal scales,
+    rows with infinities and NaN"""
+    from uniql_amd import ops
+    g = torch.Generator(device=gpu).manual_seed(d)
+    rows = 403
+    w = torch.randn((rows, d), device=gpu, generator=g) * torch.exp2(torch.rand((rows, 1), device=gpu, generator=g) * 38 - 23)
+    w = w.clamp(-65504, 65504).half()
+    w[7, d // 2], w[11, 0], w[13, d - 1] = float("inf"), float("nan"), float("-inf")
+    w[17], w[19] = 0, 65504.0
+    wide = torch.zeros((rows, 8200), dtype=torch.float16, device=gpu)
+    wide[:, :d] = w
+    packed, scales = ops.w4_embedding_quantize(w)
+    want, want_scales = ops.w4_embedding_quantize(wide)
+    assert torch.equal(packed, want[:, :d // 8])
+    assert torch.equal(scales.view(torch.int16), want_scales.view(torch.int16))
+
+
 def test_embedding_quantize_hand_computed_ties(gpu):
     """The device quantiser on the rows whose codes are worked out by hand in
     tests/test_oracle_golden.py::test_embedding_quantize_rounding_ties_by_hand (fp16 rounding of
