@@ -1,0 +1,57 @@
+"""Inputs with fewer columns than the packed weights have rows: the kernels for more than 64 rows read such rows as they are.  The
+same bits as behind a zero-padded copy, whatever follows a row in memory."""
+import pytest
+import torch
+
+from tests.helpers import make_linear_problem, to_gpu, workspace_for
+
+pytestmark = pytest.mark.gpu
+F_TILED = 4
+# every tile height, one and two quartets, with and without a K split, and the 256 x 256 kernel
+PLANS = [(s << 8) | (mt << 16) | (kw << 20) for mt, kw in ((1, 1), (1, 2), (2, 1), (2, 2), (3, 1), (4, 1)) for s in (1, 2)] + [8 << 16]
+
+
+@pytest.mark.parametrize("plan", PLANS)
+@pytest.mark.parametrize("groups,missing", [(2, 8), (2, 120), (3, 64), (4, 72), (6, 56), (12, 16), (14, 104)])
+def test_short_rows(gpu, plan, groups, missing):
+    from uniql_amd import ops
+    m, k, n = 300, 128 * groups, 256
+    k_in = k - missing
+    p = make_linear_problem(m, k, n, seed=groups + missing)
+    x, b, s = to_gpu(p, gpu)
+    ws = workspace_for(n, gpu)
+    flags = F_TILED | plan
+    x = x[:, :k_in].contiguous()           # a row is followed by the next one
+    x[7, :8], x[m - 1, :8] = float("inf"), float("nan")
+    padded = torch.zeros((m, k), dtype=x.dtype, device=gpu)
+    padded[:, :k_in] = x
+    apart = torch.full((m * (k_in + 24),), float("nan"), dtype=x.dtype, device=gpu)[:(m - 1) * (k_in + 24) + k_in]
+    apart = apart.as_strided((m, k_in), (k_in + 24, 1))   # or by something else, and the last one ends the buffer
+    apart.copy_(x)
+    want = ops.w4a16_linear(padded, b, s, ws, n, k, flags=flags)
+    clean = torch.ones(m, dtype=torch.bool, device=gpu)
+    clean[[7, m - 1]] = False
+    assert torch.isfinite(want[clean]).all() and not torch.isfinite(want[~clean]).any()
+    for rows in (x, apart):
+        got = ops.w4a16_linear(rows, b, s, ws, n, k, flags=flags)
+        assert torch.equal(got[clean], want[clean])
+        assert not torch.isfinite(got[~clean]).any()
+
+
+@pytest.mark.parametrize("m", [65, 129, 333, 1100])
+def test_short_rows_on_the_plan_of_the_call(gpu, m):
+    """rows and columns in two launches, bias, residual and gated pairs among them"""
+    from uniql_amd import ops
+    for k_in, n, kw in ((1992, 4096, dict(residual=True)), (2048 - 120, 2816, dict(bias=True)), (2040, 1536, dict(silu_mul=True))):
+        k = 2048
+        p = make_linear_problem(m, k, n, seed=m + k_in)
+        x, b, s = to_gpu(p, gpu)
+        ws = workspace_for(n, gpu)
+        x = x[:, :k_in].contiguous()
+        padded = torch.zeros((m, k), dtype=x.dtype, device=gpu)
+        padded[:, :k_in] = x
+        if "residual" in kw:
+            kw = dict(residual=torch.randn((m, n), device=gpu, generator=torch.Generator(device=gpu).manual_seed(m)).half())
+        if "bias" in kw:
+            kw = dict(bias=torch.randn(n, device=gpu, generator=torch.Generator(device=gpu).manual_seed(m)).half())
+        assert torch.equal(ops.w4a16_linear(x, b, s, ws, n, k, **kw), ops.w4a16_linear(padded, b, s, ws, n, k, **kw))

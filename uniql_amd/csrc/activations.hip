@@ -1,7 +1,7 @@
-// Activation preparation for the tiled kernel: rows whose width is not a multiple of the
-// quantisation group are copied into a zero-padded buffer (the module's F.pad,
-// quantize/quant_linear_layers.py:96-98).  The streaming kernel pads while loading and does
-// not need this.
+// Activation preparation in front of a rotation that is a launch of its own: rows whose width is not a multiple of the
+// quantisation group, or that are strided, are copied into a dense zero-padded buffer (the module's F.pad,
+// quantize/quant_linear_layers.py:96-98).  The product kernels read short rows as they are; only rows 2^24 elements and
+// more apart are copied for the tiled ones, whose offsets have 32 bits.
 #include "common.hpp"
 
 namespace uniql {

@@ -18,7 +18,7 @@ size_t stream_accum_bound(int m, int n, int k);
 bool stream_shape_ok(int k, int64_t lda);
 int read_floor_launch(const void* B, const void* S, void* sink, int m, int n, int k, unsigned tune, hipStream_t stream);
 size_t read_floor_sink_bytes(int m, int n, int k, unsigned tune);
-int tile_launch(const void* A, int64_t lda, const void* B, const void* S, void* D, const Epilogue& epi, void* accum,
+int tile_launch(const void* A, int64_t lda, int k_valid, const void* B, const void* S, void* D, const Epilogue& epi, void* accum,
                 size_t accum_bytes, void* part, size_t part_bytes, int m, int n, int k, int groups, int first, int columns,
                 const TilePlan& plan, hipStream_t stream);
 bool tile_shape_ok(int m, int n, int k, int64_t ldx, int columns, const TilePlan& plan);
@@ -26,7 +26,7 @@ int mid_launch(const void* A, int64_t lda, int k_valid, const void* B, const voi
                void* part, int m, int n, int k, int groups, const MidPlan& plan, hipStream_t stream);
 bool mid_shape_ok(int m, int n, int k, int64_t lda);
 int pad_rows_launch(const void* A, int64_t lda, int k_in, void* dst, int k, int m, hipStream_t stream);
-int wide_launch(const void* A, int64_t lda, const void* B, const void* S, void* D, const Epilogue& epi, int m, int n,
+int wide_launch(const void* A, int64_t lda, int k_valid, const void* B, const void* S, void* D, const Epilogue& epi, int m, int n,
                 int k, int groups, int first, int columns, hipStream_t stream);
 bool wide_shape_ok(int m, int n, int k, int groups, int64_t ldx);
 int dequant_launch(const void* B, const void* S, void* W, uint8_t* codes, int n, int k, int groups,
@@ -137,9 +137,9 @@ static int fused_rotation(int m, int k, int k_in, int had_block, bool use_stream
     return (had_block == k && k_in == k && stream_rotates_rows(m, k)) ? 2 : 0;
 }
 
-// bytes of the rotated or zero-padded copy of the activations at the start of `temp`: every
-// rotation that is not fused into the streaming kernel, and padding whenever the
-// kernel cannot guard its own loads (tiled kernel) or a rotation comes first
+// bytes of the rotated or zero-padded copy of the activations at the start of `temp`, at most: every
+// rotation that is not fused into the streaming kernel, and padding in front of a rotation or where
+// the rows are too far apart for the tiled kernels to read short ones as they are (the stride is not known here)
 static size_t activation_copy_bytes(int m, int k, int k_in, int had_block, bool use_stream, unsigned flags) {
     const bool rotate_first = had_block != 0 && fused_rotation(m, k, k_in, had_block, use_stream, flags) == 0;
     const bool pad_first = k_in != k && (rotate_first || !use_stream);
@@ -184,8 +184,8 @@ static MidPlan mid_for_few_rows(int m, int n, int k, int had_block, unsigned fla
     return n / 128 < 144 && (k <= 8192 || n >= 3072) ? mid_plan(m, n, k, 0, part_cap) : kNoMid;
 }
 
-// In place of a launch of the tiled kernels, where it is expected to be faster; padded: the tiled kernels would need a
-// zero-padded copy of the rows first (2 us).  Over a short K of fewer than 12 groups the tiled kernels' expected times are the
+// In place of a launch of the tiled kernels, where it is expected to be faster; padded: the tiled kernels need a
+// zero-padded copy of the rows first (2 us; rows too far apart for them).  Over a short K of fewer than 12 groups the tiled kernels' expected times are the
 // better ones from 33 rows on.  Plans that add longer chains of products than the tiled kernel's own are left out: a sum
 // is no less exact here than there (8192 -> 512 at 56 rows with two groups a wave: 1.1 x the distance from float64).
 // Drawn calls: 17 to 32 rows 1.26 x faster on average, 33 to 48 1.17, 49 to 64 1.03.
@@ -208,8 +208,9 @@ static LinearNeeds linear_needs(int m, int n, int k, int k_in, int64_t lda, int 
     q.had_mode = fused_rotation(m, k, k_in, had_block, q.use_stream, flags);
     q.rotate_first = had_block != 0 && q.had_mode == 0;
     // the transform kernel reads dense rows of k values: a strided or short input is first copied
-    // (and zero-padded) into the temporary buffer, then rotated there in place
-    q.pad_first = q.rotate_first ? (k_in != k || lda != k) : (k_in != k && !q.use_stream);
+    // (and zero-padded) into the temporary buffer, then rotated there in place; rows too far apart for the tiled kernels'
+    // 32-bit offsets are copied as well where they are short
+    q.pad_first = q.rotate_first ? (k_in != k || lda != k) : (k_in != k && !q.use_stream && lda >= (1LL << 24));
     q.ld_kernel = (q.rotate_first || q.pad_first) ? (int64_t)k : lda;
     q.plan.parts = q.plan.head_columns = 0;
     q.mid[0] = q.mid[1] = kNoMid;
@@ -382,6 +383,7 @@ static int linear_impl(const void* A, int64_t lda, int k_in, const void* B, cons
         if (e != UNIQL_OK) return e;
         Ain = temp;
         ld = k;
+        k_valid = k;
     }
     Epilogue epi;
     epi.bias = reinterpret_cast<const half_t*>(bias);
@@ -406,8 +408,8 @@ static int linear_impl(const void* A, int64_t lda, int k_in, const void* B, cons
         epi.residual = residual ? reinterpret_cast<const half_t*>(residual) + (size_t)m0 * ldr : nullptr;
         const int e = q.mid[i].upw > 0
                           ? mid_launch(x, ld, k_valid, B, S, d, epi, accum, part, p.rows, n, k, groups, q.mid[i], st)
-                      : p.wide ? wide_launch(x, ld, B, S, d, epi, p.rows, n, k, groups, first, columns, st)
-                               : tile_launch(x, ld, B, S, d, epi, accum, accum_bytes, part, part_bytes, p.rows, n, k, groups, first, columns, p.tile, st);
+                      : p.wide ? wide_launch(x, ld, k_valid, B, S, d, epi, p.rows, n, k, groups, first, columns, st)
+                               : tile_launch(x, ld, k_valid, B, S, d, epi, accum, accum_bytes, part, part_bytes, p.rows, n, k, groups, first, columns, p.tile, st);
         if (e != UNIQL_OK) return e;
         if (q.plan.head_columns == 0) m0 += p.rows;
         else first += columns;

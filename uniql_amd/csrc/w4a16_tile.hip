@@ -62,6 +62,7 @@ struct TileArgs {
     int strip0;       // first 128-column strip of the launch, and how many
     int strips;
     Epilogue epi;
+    int k_valid;  // columns of X that exist (a multiple of eight, in the last K group); the rest of K counts as zeros
 };
 
 typedef const __attribute__((address_space(1))) void* gptr_t;
@@ -95,7 +96,12 @@ struct TileLds {
 // the same tile (each with its own LDS ring): two waves per SIMD cover each other's LDS and
 // expansion latencies, which is what small M tiles (little matrix work per group) lack when the
 // grid only gives a compute unit one workgroup.
-template <int MT, int EXT, int KW>
+// CUT: X has fewer columns than K.  The iterations that request or multiply the last group then take descriptors that end where X
+// does, and cut the columns that do not exist out of its operands.  (Kernels of their own: longer code costs the short launches
+// of everybody else 1 to 3 %.)  A zero-padded copy of the rows in front of the kernel, which this replaces, took 2.5 to 5 us at 65 to 128
+// rows and more with their number; a decoder layer of 128 rows with heads of
+// 114 and an MLP width of 8104 86.5 -> 82.9 us, of 640 with 90 and 9000 256 -> 250.
+template <int MT, int EXT, int KW, bool CUT>
 __global__ __launch_bounds__(256 * KW, 1) void w4a16_tile_kernel(const TileArgs a) {
     extern __shared__ __attribute__((aligned(16))) uint32_t lds_all[];
     using L = TileLds<MT, KW>;
@@ -192,15 +198,23 @@ __global__ __launch_bounds__(256 * KW, 1) void w4a16_tile_kernel(const TileArgs 
     // instruction goes into an address (the host keeps the packed weights below 4 GiB).
     constexpr int kRsrcFlags = 0x00020000;  // raw buffer, 32-bit data format
     const __amdgpu_buffer_rsrc_t x_rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<half_t*>(x_tile), 0, 0xffffffffu, kRsrcFlags);
+    // X around the last group (`ends`): the group's columns up to the end of the tile's last row.  What a row lacks of that
+    // group is read from the next row, or is beyond the descriptor, and is cut out of the operands (cut_xa).
+    const int x_rows = a.M - m0 < ROWS ? a.M - m0 : ROWS;
+    const uint32_t x_bytes = 2u * ((uint32_t)(x_rows - 1) * (uint32_t)a.ldx + (uint32_t)a.k_valid);
     const __amdgpu_buffer_rsrc_t w_rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<u32x4*>(strip_w), 0, 0xffffffffu, kRsrcFlags);
     const __amdgpu_buffer_rsrc_t s_rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<half_t*>(strip_s), 0, 0xffffffffu, kRsrcFlags);
     const uint32_t piece_bytes = 16u * piece_off, scale_lane_bytes = 16u * (uint32_t)dslot;
     const uint32_t packed_row_bytes = 16u * (uint32_t)N4, scale_row_bytes = 2u * (uint32_t)scale_row_stride;
-    auto issue_piece = [&](int g, int ring, int idx) __attribute__((always_inline)) {
+    auto issue_piece = [&](int g, int ring, int idx, bool ends) __attribute__((always_inline)) {
         uint32_t* stage = lds + ring * L::kStageDwords;
         if (idx < kXOps) {
             uint32_t* xbuf = stage + (kXOps * 4 * w) * 64;  // this wave's X rows
-            buffer_to_lds16(x_rsrc, xbuf + idx * 256, xsrc[idx], 256u * (uint32_t)g);
+            if (ends)
+                buffer_to_lds16(__builtin_amdgcn_make_buffer_rsrc(const_cast<half_t*>(x_tile + 128 * (size_t)g), 0, x_bytes - 256u * (uint32_t)g, kRsrcFlags),
+                                xbuf + idx * 256, xsrc[idx], 0);
+            else
+                buffer_to_lds16(x_rsrc, xbuf + idx * 256, xsrc[idx], 256u * (uint32_t)g);
         } else if (idx < kXOps + 2) {
             uint32_t* bbuf = stage + L::kXDwords + w * 512 + (idx - kXOps) * 256;
             buffer_to_lds16(w_rsrc, bbuf, piece_bytes, (uint32_t)(8 * g + 4 * (idx - kXOps)) * packed_row_bytes);
@@ -213,9 +227,10 @@ __global__ __launch_bounds__(256 * KW, 1) void w4a16_tile_kernel(const TileArgs 
             buffer_to_lds16(s_rsrc, sbuf, scale_lane_bytes, (uint32_t)g * scale_row_bytes);
         }
     };
-    auto issue_stage = [&](int g, int ring) __attribute__((always_inline)) {
+    auto issue_pieces = [&](int g, int ring, int count, bool ends) __attribute__((always_inline)) {
 #pragma unroll
-        for (int idx = 0; idx < kStageOps; ++idx) issue_piece(g, ring, idx);
+        for (int idx = 0; idx < kStageOps; ++idx)
+            if (idx < count) issue_piece(g, ring, idx, ends);
     };
 
     // LDS read offsets (dwords).  X: row s of an M tile, packed row w + 4 t -> segments
@@ -257,6 +272,16 @@ __global__ __launch_bounds__(256 * KW, 1) void w4a16_tile_kernel(const TileArgs 
             xa[mt] = h8{d0.x, d0.y, d1.x, d1.y, d2.x, d2.y, d3.x, d3.y};
         }
     };
+    // The operands of packed row w + 4 t in the last group: its K values 8 (2 (w + 4 t) + x) .. are the registers 2 x, 2 x + 1.
+    const int last_octets = (a.k_valid - 128 * (a.G - 1)) >> 3;
+    auto cut_xa = [&](h8 (&xa)[MT], int t) __attribute__((always_inline)) {
+        const uint32_t lo = 2 * (w + 4 * t) < last_octets ? ~0u : 0u, hi = 2 * (w + 4 * t) + 1 < last_octets ? ~0u : 0u;
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt) {
+            const u32x4 v = __builtin_bit_cast(u32x4, xa[mt]);
+            xa[mt] = __builtin_bit_cast(h8, u32x4{v[0] & lo, v[1] & lo, v[2] & hi, v[3] & hi});
+        }
+    };
     // One quarter (two of the eight values) of B operand `block` = 4 t + 2 jo + blk of a stage.
     // K order of the operand: 4h, 4h+1 | 4h+2, 4h+3 | 4h+8, 4h+9 | 4h+10, 4h+11, i.e. quarter
     // q = 0, 1: low-nibble form of pieces kq = 2h, 2h+1; q = 2, 3: high-nibble form.
@@ -280,7 +305,7 @@ __global__ __launch_bounds__(256 * KW, 1) void w4a16_tile_kernel(const TileArgs 
     // path, or they stall at issue and the matrix pipe starves) and the LDS reads the caller
     // assigns to the slot.  A scheduling barrier closes every slot: with one wave
     // per SIMD nothing else fills the matrix pipe's shadow, so the order is fixed by hand.
-    auto half_stage = [&](int t, h8 (&xa)[MT], h8& bw, int dma_first, int dma_count, int next_g, int next_ring, auto&& lds_reads) __attribute__((always_inline)) {
+    auto half_stage = [&](int t, h8 (&xa)[MT], h8& bw, int dma_first, int dma_count, int next_g, int next_ring, bool ends, auto&& lds_reads) __attribute__((always_inline)) {
         constexpr int kDmaStride = MT == 1 ? 1 : 2;  // slots between two LDS-DMA loads
 #pragma unroll
         for (int op = 0; op < 4; ++op) {
@@ -300,7 +325,7 @@ __global__ __launch_bounds__(256 * KW, 1) void w4a16_tile_kernel(const TileArgs 
                     e[q] = bits_to_h2(bits);
                 }
                 if (slot_i % kDmaStride == 0 && slot_i / kDmaStride < dma_count)
-                    issue_piece(next_g, next_ring, dma_first + slot_i / kDmaStride);
+                    issue_piece(next_g, next_ring, dma_first + slot_i / kDmaStride, ends);
                 lds_reads(slot_i);
                 if (MT >= 3) {
                     // inside the slot: the first two operations of the quarter, the MFMA, the rest;
@@ -343,28 +368,34 @@ __global__ __launch_bounds__(256 * KW, 1) void w4a16_tile_kernel(const TileArgs 
         xa[mt] = h8{d0.x, d0.y, d1.x, d1.y, d2.x, d2.y, d3.x, d3.y};
     };
     const int g_last = g_end - 1;
+    const bool short_end = CUT && g_end == a.G;  // uniform: the workgroup's last group has fewer than 128 columns of X
+    const int cut_at = short_end && g_begin + KW * (ngroups - 1) == a.G - 1 ? ngroups - 1 : -1;  // the iteration with that group
     h8 bw;
     if (ngroups > 0) {
-        issue_stage(g_begin, 0);
-        issue_stage(ngroups > 1 ? g_begin + KW : g_last, 1);
-#pragma unroll
-        for (int idx = 0; idx < kDmaA; ++idx) issue_piece(group_or_last(g_begin + 2 * KW), 2, idx);
+        auto first_stages = [&](bool ends) __attribute__((always_inline)) {
+            issue_pieces(g_begin, 0, kStageOps, ends);
+            issue_pieces(ngroups > 1 ? g_begin + KW : g_last, 1, kStageOps, ends);
+            issue_pieces(group_or_last(g_begin + 2 * KW), 2, kDmaA, ends);
+        };
+        first_stages(CUT);
         UNIQL_WAIT_VMCNT(kStageOps + kDmaA);
         __builtin_amdgcn_s_barrier();
         read_words(0, 0);
         read_xa(xa0, 0, 0);
+        if (CUT && cut_at == 0) cut_xa(xa0, 0);
         bw = expand(0, 0);
     }
-    // one iteration; called with a literal `slot` the ring addresses are constants
-    auto iteration = [&](int it, int slot) __attribute__((always_inline)) {
+    // one iteration; called with a literal `slot` the ring addresses are constants; `ends`: it may request or multiply the last group
+    auto iteration = [&](int it, int slot, bool ends) __attribute__((always_inline)) {
         const int slot_next = slot + 1 == kRing ? 0 : slot + 1;
         const int slot_prev = slot == 0 ? kRing - 1 : slot - 1;   // holds stage it+2
-        half_stage(0, xa0, bw, kDmaA, kDmaB, group_or_last(g_begin + KW * (it + 2)), slot_prev, [&](int i) __attribute__((always_inline)) {
+        half_stage(0, xa0, bw, kDmaA, kDmaB, group_or_last(g_begin + KW * (it + 2)), slot_prev, ends, [&](int i) __attribute__((always_inline)) {
             if (i < MT) read_xa_one(xa1, slot, 1, i);
         });
         UNIQL_WAIT_VMCNT(kStageOps);   // stage it+1 has landed; only stage it+2's loads are outstanding
         __builtin_amdgcn_s_barrier();
-        half_stage(1, xa1, bw, 0, kDmaA, group_or_last(g_begin + KW * (it + 3)), slot, [&](int i) __attribute__((always_inline)) {
+        if (ends && it == cut_at) cut_xa(xa1, 1);
+        half_stage(1, xa1, bw, 0, kDmaA, group_or_last(g_begin + KW * (it + 3)), slot, ends, [&](int i) __attribute__((always_inline)) {
             if (i == 0) read_words(1, slot_next);
             if (i >= 1 && i <= MT) read_xa_one(xa0, slot_next, 0, i - 1);
         });
@@ -374,15 +405,21 @@ __global__ __launch_bounds__(256 * KW, 1) void w4a16_tile_kernel(const TileArgs 
             pw[0][t][1] = pw[1][t][1];
         }
         scv[0] = scv[1];
+        if (ends && it + 1 == cut_at) cut_xa(xa0, 0);
     };
     // three iterations at a time walk the ring once: every LDS address in them is a constant
     int it = 0;
-    for (; it + kRing <= ngroups; it += kRing) {
-        iteration(it, 0);
-        iteration(it + 1, 1);
-        iteration(it + 2, 2);
+    const int plain = short_end ? ngroups - 4 : ngroups;  // from here on the last group may be requested
+    for (; it + kRing <= plain; it += kRing) {
+        iteration(it, 0, false);
+        iteration(it + 1, 1, false);
+        iteration(it + 2, 2, false);
     }
-    for (int slot = 0; it < ngroups; ++it, ++slot) iteration(it, slot);
+    if constexpr (CUT) {
+        for (int slot = 0; it < ngroups; ++it, slot = slot + 1 == kRing ? 0 : slot + 1) iteration(it, slot, true);
+    } else {
+        for (int slot = 0; it < ngroups; ++it, ++slot) iteration(it, slot, false);
+    }
     UNIQL_WAIT_VMCNT(0);
     __syncthreads();
 
@@ -601,32 +638,45 @@ bool tile_shape_ok(int m, int n, int k, int64_t ldx, int columns, const TilePlan
     return grid <= 0x7fffffffLL && ldx < (1LL << 24) && (int64_t)k * n / 2 < (1LL << 32);
 }
 
-template <int MT, int EXT, int KW>
+template <int MT, int EXT, int KW, bool CUT>
 static hipError_t tile_launch_one(const TileArgs& a, int grid, hipStream_t stream) {
     const size_t shmem = TileLds<MT, KW>::kBytes;
-    auto kern = &w4a16_tile_kernel<MT, EXT, KW>;
+    auto kern = &w4a16_tile_kernel<MT, EXT, KW, CUT>;
     hipLaunchKernelGGL(kern, dim3(grid), dim3(256 * KW), shmem, stream, a);
     return hipGetLastError();
 }
 
-template <int MT, int KW>
+template <int MT, int KW, bool CUT>
 static hipError_t tile_launch_ext(const TileArgs& a, bool ext, int grid, hipStream_t stream) {
-    if (a.epi.gated) return tile_launch_one<MT, 2, KW>(a, grid, stream);
-    return ext ? tile_launch_one<MT, 1, KW>(a, grid, stream) : tile_launch_one<MT, 0, KW>(a, grid, stream);
+    if (a.epi.gated) return tile_launch_one<MT, 2, KW, CUT>(a, grid, stream);
+    if constexpr (CUT) return tile_launch_one<MT, 1, KW, true>(a, grid, stream);
+    else return ext ? tile_launch_one<MT, 1, KW, false>(a, grid, stream) : tile_launch_one<MT, 0, KW, false>(a, grid, stream);
+}
+template <bool CUT>
+static hipError_t tile_launch_plan(const TileArgs& a, const TilePlan& plan, bool ext, int grid, hipStream_t stream) {
+    if (plan.mtiles == 1)
+        return plan.quartets == 2 ? tile_launch_ext<1, 2, CUT>(a, ext, grid, stream) : tile_launch_ext<1, 1, CUT>(a, ext, grid, stream);
+    if (plan.mtiles == 2)
+        return plan.quartets == 2 ? tile_launch_ext<2, 2, CUT>(a, ext, grid, stream) : tile_launch_ext<2, 1, CUT>(a, ext, grid, stream);
+    if (plan.mtiles == 3) return tile_launch_ext<3, 1, CUT>(a, ext, grid, stream);
+    return tile_launch_ext<4, 1, CUT>(a, ext, grid, stream);
 }
 
-template <int MT, int KW>
+template <int MT, int KW, bool CUT>
 static bool tile_allow_lds_one() {
     constexpr size_t bytes = TileLds<MT, KW>::kBytes;
-    return allow_lds(&w4a16_tile_kernel<MT, 0, KW>, bytes) && allow_lds(&w4a16_tile_kernel<MT, 1, KW>, bytes) && allow_lds(&w4a16_tile_kernel<MT, 2, KW>, bytes);
+    return (CUT || allow_lds(&w4a16_tile_kernel<MT, 0, KW, false>, bytes)) && allow_lds(&w4a16_tile_kernel<MT, 1, KW, CUT>, bytes) &&
+           allow_lds(&w4a16_tile_kernel<MT, 2, KW, CUT>, bytes);
 }
-bool tile_allow_lds() {
-    return tile_allow_lds_one<1, 1>() && tile_allow_lds_one<1, 2>() && tile_allow_lds_one<2, 1>() && tile_allow_lds_one<2, 2>() &&
-           tile_allow_lds_one<3, 1>() && tile_allow_lds_one<4, 1>();
+template <bool CUT>
+static bool tile_allow_lds_all() {
+    return tile_allow_lds_one<1, 1, CUT>() && tile_allow_lds_one<1, 2, CUT>() && tile_allow_lds_one<2, 1, CUT>() && tile_allow_lds_one<2, 2, CUT>() &&
+           tile_allow_lds_one<3, 1, CUT>() && tile_allow_lds_one<4, 1, CUT>();
 }
+bool tile_allow_lds() { return tile_allow_lds_all<false>() && tile_allow_lds_all<true>(); }
 
-// columns first .. first + columns - 1 of the layer's n
-int tile_launch(const void* A, int64_t lda, const void* B, const void* S, void* D, const Epilogue& epi, void* accum,
+// columns first .. first + columns - 1 of the layer's n; k_valid: columns of A that exist
+int tile_launch(const void* A, int64_t lda, int k_valid, const void* B, const void* S, void* D, const Epilogue& epi, void* accum,
                 size_t accum_bytes, void* part, size_t part_bytes, int m, int n, int k, int groups, int first, int columns,
                 const TilePlan& plan, hipStream_t stream) {
     if (first % 128 != 0 || first + columns > n) return UNIQL_E_SHAPE;
@@ -641,6 +691,7 @@ int tile_launch(const void* A, int64_t lda, const void* B, const void* S, void* 
     a.D = D;
     a.accum = reinterpret_cast<unsigned long long*>(accum);
     a.ldx = lda;
+    a.k_valid = k_valid;
     a.M = m;
     a.N = n;
     a.K = k;
@@ -654,17 +705,9 @@ int tile_launch(const void* A, int64_t lda, const void* B, const void* S, void* 
     a.epi = epi;
     const int64_t grid = (int64_t)a.strips * a.mblocks * a.splits;
     if (grid > 0x7fffffffLL) return UNIQL_E_SHAPE;
-    hipError_t e;
     const bool ext = epi.bias || epi.residual || epi.relu2 || epi.transpose || epi.n_store != n ||
                      epi.ldd != n || !epi.vec_ok;
-    if (plan.mtiles == 1)
-        e = plan.quartets == 2 ? tile_launch_ext<1, 2>(a, ext, (int)grid, stream) : tile_launch_ext<1, 1>(a, ext, (int)grid, stream);
-    else if (plan.mtiles == 2)
-        e = plan.quartets == 2 ? tile_launch_ext<2, 2>(a, ext, (int)grid, stream) : tile_launch_ext<2, 1>(a, ext, (int)grid, stream);
-    else if (plan.mtiles == 3)
-        e = tile_launch_ext<3, 1>(a, ext, (int)grid, stream);
-    else
-        e = tile_launch_ext<4, 1>(a, ext, (int)grid, stream);
+    const hipError_t e = a.k_valid < a.K ? tile_launch_plan<true>(a, plan, ext, (int)grid, stream) : tile_launch_plan<false>(a, plan, ext, (int)grid, stream);
     return e == hipSuccess ? UNIQL_OK : UNIQL_E_LAUNCH;
 }
 

@@ -73,6 +73,7 @@ struct WideArgs {
     int M, N, K;
     int mblocks;  // ceil(M / 256)
     int first;    // first column of the launch (multiple of 128)
+    int k_valid;  // columns of X that exist (a multiple of eight, in the last K group); the rest of K counts as zeros
     Epilogue epi;
 };
 
@@ -105,6 +106,11 @@ struct WideInt {
     static constexpr int value = V;
 };
 
+// CUT: X has fewer columns than K.  The group in front of the last one, which requests the last one's X, is then a copy of the
+// loop body of its own, with descriptors that end where X does (a descriptor that changes in the loop costs it 6 %), and the
+// last group cuts the columns that do not exist out of its operands.  A zero-padded copy of the rows in front of the kernel, which
+// this replaces, took 2 % of a layer (4000 rows, heads of 90, an MLP width of 9000: 1173 -> 1152 us).
+template <bool CUT>
 __global__ __launch_bounds__(256, 1) void w4a16_wide_kernel(const WideArgs a) {
     extern __shared__ __attribute__((aligned(16))) uint32_t lds[];
     char* const ldsb = reinterpret_cast<char*>(lds);
@@ -158,6 +164,15 @@ __global__ __launch_bounds__(256, 1) void w4a16_wide_kernel(const WideArgs a) {
     auto load_x = [&](int slot, int i) __attribute__((always_inline)) {
         __builtin_amdgcn_raw_ptr_buffer_load_lds(x_rsrc, (wide_lptr_t)(ldsb + kWideXBase + slot * kWideXBytes + i * 1024 + wave_x),
                                                  16, xsrc[i], x_next, 0, 0);
+    };
+    // The last group's pairs (2 ngroups - 2 + pair): from the pair's columns to the end of the tile's last row.  What a row lacks
+    // of them is read from the next row, or is beyond the descriptor.
+    auto load_last_x = [&](int slot, int i, int pair) __attribute__((always_inline)) {
+        const int rows = a.M - m0 < 256 ? a.M - m0 : 256;
+        const uint32_t bytes = 2u * ((uint32_t)(rows - 1) * (uint32_t)a.ldx + (uint32_t)a.k_valid), from = 128u * (uint32_t)(2 * ngroups - 2 + pair);
+        const __amdgpu_buffer_rsrc_t rest = __builtin_amdgcn_make_buffer_rsrc(
+            const_cast<half_t*>(a.X + (size_t)m0 * a.ldx) + from / 2, 0, bytes > from ? bytes - from : 0u, kRsrcFlags);
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(rest, (wide_lptr_t)(ldsb + kWideXBase + slot * kWideXBytes + i * 1024 + wave_x), 16, xsrc[i], 0, 0, 0);
     };
     auto load_c = [&](int slot) __attribute__((always_inline)) {
         __builtin_amdgcn_raw_ptr_buffer_load_lds(c_rsrc, (wide_lptr_t)(ldsb + kWideCBase + slot * kWideCBytes + wave_kib), 16,
@@ -258,6 +273,16 @@ __global__ __launch_bounds__(256, 1) void w4a16_wide_kernel(const WideArgs a) {
         }
     };
 
+    // Of the last group's block J: K eighth 4 J + 2 s + h of the group.
+    auto cut_operands = [&](int set, int first_octet) __attribute__((always_inline)) {
+        const uint32_t keep = 8 * (first_octet + h) + 128 * (ngroups - 1) < a.k_valid ? ~0u : 0u;
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+            const u32x4 v = __builtin_bit_cast(u32x4, xa[set][t]);
+            xa[set][t] = __builtin_bit_cast(h8, u32x4{v[0] & keep, v[1] & keep, v[2] & keep, v[3] & keep});
+        }
+    };
+
     // ---- prologue: the loads the iterations before the first would have issued, block 0 expanded ---
     int s_issue_bytes = 0;  // scales ring slot (as a byte offset) of the next group to request
     int s_fetch_bytes = 0;  //                                      of the next group to fetch
@@ -319,9 +344,10 @@ __global__ __launch_bounds__(256, 1) void w4a16_wide_kernel(const WideArgs a) {
     // are written with (loops over kXRowLoads, one load_c per iteration, load_s in iteration 0),
     // so a load added there changes the wait here; the static_assert states the table the
     // pipeline was validated with.
+    // tailc: 1 the last group, 2 the one in front of it where X is cut
     auto iteration = [&](auto jc, auto tailc) __attribute__((always_inline)) {
         constexpr int J = decltype(jc)::value;
-        constexpr bool kTail = decltype(tailc)::value != 0;
+        constexpr bool kTail = decltype(tailc)::value == 1, kBeforeTail = decltype(tailc)::value == 2;
         constexpr int kVm = kTail && J != 0 ? 0 : wide_vmcnt_at_barrier(J);
         static_assert(wide_vmcnt_at_barrier(0) == 14 && wide_vmcnt_at_barrier(1) == 2 && wide_vmcnt_at_barrier(2) == 15 &&
                           wide_vmcnt_at_barrier(3) == 1,
@@ -329,6 +355,7 @@ __global__ __launch_bounds__(256, 1) void w4a16_wide_kernel(const WideArgs a) {
         constexpr int wbuf = J & 1, wbuf_next = (J + 1) & 1;
         // first half: K values 0..15 of block kb with operand set 0.  Meanwhile the second
         // half's operands are read and block kb+1 is expanded into the other weight buffer.
+        if constexpr (CUT && kTail) cut_operands(0, 4 * J);
 #pragma unroll
         for (int i = 0; i < 16; ++i) {
             const int nt = i >> 2, mt = i & 3;
@@ -345,7 +372,10 @@ __global__ __launch_bounds__(256, 1) void w4a16_wide_kernel(const WideArgs a) {
             if ((J & 1) == 0 && (!kTail || J == 0)) {
 #pragma unroll
                 for (int q = 0; q < kWideXRowLoads; ++q)
-                    if (i == 8 + 2 * q) load_x(((J + 2) >> 1) & 1, kWideXRowLoads + q);
+                    if (i == 8 + 2 * q) {
+                        if constexpr (CUT && (kTail || (kBeforeTail && J == 2))) load_last_x(((J + 2) >> 1) & 1, kWideXRowLoads + q, kTail ? 1 : 0);
+                        else load_x(((J + 2) >> 1) & 1, kWideXRowLoads + q);
+                    }
                 if (i == 15) x_next += 128;
             }
             __builtin_amdgcn_sched_barrier(0);
@@ -354,6 +384,7 @@ __global__ __launch_bounds__(256, 1) void w4a16_wide_kernel(const WideArgs a) {
         // weights of block kb+1 are written and everybody has read what the loads issued behind
         // the barrier will overwrite.  Then: the next block's first operands, the words of block
         // kb+2 (and, where that block starts a group, the group's scales), this iteration's loads.
+        if constexpr (CUT && kTail) cut_operands(1, 4 * J + 2);
 #pragma unroll
         for (int i = 0; i < 16; ++i) {
             const int nt = i >> 2, mt = i & 3;
@@ -382,7 +413,10 @@ __global__ __launch_bounds__(256, 1) void w4a16_wide_kernel(const WideArgs a) {
                 if ((J & 1) == 1) {  // the lower rows of the pair after next, into the slot this barrier has freed
 #pragma unroll
                     for (int q = 0; q < kWideXRowLoads; ++q)
-                        if (i == 6 + 2 * q) load_x(((J + 3) >> 1) & 1, q);
+                        if (i == 6 + 2 * q) {
+                            if constexpr (kBeforeTail) load_last_x(((J + 3) >> 1) & 1, q, J >> 1);
+                            else load_x(((J + 3) >> 1) & 1, q);
+                        }
                 }
                 if (i == 14) load_c((J + 1) & 3);
                 if (i == 15) c_next += c_step;
@@ -393,16 +427,18 @@ __global__ __launch_bounds__(256, 1) void w4a16_wide_kernel(const WideArgs a) {
 
     // groups 0 .. ngroups-2 request what lies four and five blocks ahead (the scales two groups
     // ahead: the last such request asks for the last group again); the last group requests nothing
-    for (int g = 0; g < ngroups - 1; ++g) {
-        iteration(WideInt<0>{}, WideInt<0>{});
+    auto body = [&](int g, auto kind) __attribute__((always_inline)) {
+        iteration(WideInt<0>{}, kind);
         if (g + 3 < ngroups) s_next += s_group_bytes;
-        iteration(WideInt<1>{}, WideInt<0>{});
+        iteration(WideInt<1>{}, kind);
         // block kb + 5 of the last two iterations before the last group does not exist: they ask
         // for the last block again (into a slot nobody reads any more)
         if (g + 2 == ngroups) c_step = 0;
-        iteration(WideInt<2>{}, WideInt<0>{});
-        iteration(WideInt<3>{}, WideInt<0>{});
-    }
+        iteration(WideInt<2>{}, kind);
+        iteration(WideInt<3>{}, kind);
+    };
+    for (int g = 0; g < ngroups - (CUT ? 2 : 1); ++g) body(g, WideInt<0>{});
+    if constexpr (CUT) body(ngroups - 2, WideInt<2>{});
     iteration(WideInt<0>{}, WideInt<1>{});
     iteration(WideInt<1>{}, WideInt<1>{});
     iteration(WideInt<2>{}, WideInt<1>{});
@@ -519,16 +555,16 @@ bool wide_shape_ok(int m, int n, int k, int groups, int64_t ldx) {
            (int64_t)(n / 256) * ((m + 255) / 256) <= 0x7fffffffLL;
 }
 
-bool wide_allow_lds() { return allow_lds(&w4a16_wide_kernel, kWideLdsBytes); }
+bool wide_allow_lds() { return allow_lds(&w4a16_wide_kernel<false>, kWideLdsBytes) && allow_lds(&w4a16_wide_kernel<true>, kWideLdsBytes); }
 
 static hipError_t wide_launch_one(const WideArgs& a, int grid, hipStream_t stream) {
-    auto kern = &w4a16_wide_kernel;
+    auto kern = a.k_valid < a.K ? &w4a16_wide_kernel<true> : &w4a16_wide_kernel<false>;
     hipLaunchKernelGGL(kern, dim3(grid), dim3(256), kWideLdsBytes, stream, a);
     return hipGetLastError();
 }
 
-// columns first .. first + columns - 1 of the layer's n
-int wide_launch(const void* A, int64_t lda, const void* B, const void* S, void* D, const Epilogue& epi, int m, int n,
+// columns first .. first + columns - 1 of the layer's n; k_valid: columns of A that exist
+int wide_launch(const void* A, int64_t lda, int k_valid, const void* B, const void* S, void* D, const Epilogue& epi, int m, int n,
                 int k, int groups, int first, int columns, hipStream_t stream) {
     if (first % 128 != 0 || first + columns > n || !wide_shape_ok(m, columns, k, groups, lda) || (int64_t)k * n / 2 >= (1LL << 32)) return UNIQL_E_SHAPE;
     WideArgs a;
@@ -537,6 +573,7 @@ int wide_launch(const void* A, int64_t lda, const void* B, const void* S, void* 
     a.X = reinterpret_cast<const half_t*>(A);
     a.D = D;
     a.ldx = lda;
+    a.k_valid = k_valid;
     a.M = m;
     a.N = n;
     a.K = k;
