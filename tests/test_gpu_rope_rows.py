@@ -1,5 +1,5 @@
-"""Rotary kernels at the edges of their rules: the kernel that gathers per pair up to 191 tokens, tables in LDS from 192 on,
-heads of one pair (quotients by division), one table row for all sequences."""
+"""Rotary kernels at the edges of their rules: the kernel that gathers per pair up to 191 tokens, tables in LDS from 128 or 192 on,
+a token's heads in one workgroup or in several, heads of one pair (quotients by division), one table row for all sequences."""
 import numpy as np
 import pytest
 import torch
@@ -13,7 +13,10 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("b,hq,hk,s,d,D", [(1, 16, 2, 191, 96, 256), (1, 16, 2, 192, 96, 256), (2, 32, 32, 140, 64, 128),
                                            (3, 6, 2, 100, 14, 32), (1, 28, 4, 300, 6, 128), (260, 4, 2, 1, 8, 16), (70, 8, 1, 1, 20, 32),
-                                           (1, 5, 5, 7, 2, 16), (1, 6, 3, 290, 2, 16), (3, 40, 8, 20, 108, 128), (1, 96, 3, 2, 250, 256)])
+                                           (1, 5, 5, 7, 2, 16), (1, 6, 3, 290, 2, 16), (3, 40, 8, 20, 108, 128), (1, 96, 3, 2, 250, 256),
+                                           (1, 32, 32, 127, 108, 128), (1, 32, 32, 128, 108, 128), (2, 64, 64, 97, 90, 128),
+                                           (1, 48, 12, 333, 112, 128), (1, 24, 24, 200, 128, 128), (1, 8, 1, 1024, 64, 64),
+                                           (1, 8, 4, 1025, 20, 32), (1, 40, 4, 1024, 16, 32), (1, 14, 14, 130, 6, 16)])
 @pytest.mark.parametrize("index_dtype", [torch.uint8, torch.int64, torch.int32])
 def test_rows_and_heads(gpu, b, hq, hk, s, d, D, index_dtype):
     from uniql_amd import ops

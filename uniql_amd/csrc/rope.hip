@@ -25,6 +25,7 @@ struct RopeArgs {
     int seq_len, cos_batch, n_qh, n_kh, hd, index_bytes;
     unsigned rows;
     int per_head, group;                       // work items of a head, query heads of a key / value head
+    int kh;                                    // key / value heads of a workgroup
     unsigned per_head_inverse, group_inverse;  // 2^32 / divisor, rounded up: quotients without a division
 };
 constexpr unsigned kRopeGridRows = 65535;
@@ -142,9 +143,12 @@ __global__ __launch_bounds__(256) void rope_indices_kernel(const RopeArgs a) {
     }
 }
 
-// Many tokens: one workgroup per token builds the token's gathered (cos, sin) pairs once per
-// key/value head in LDS (n_kv_heads x head_dim entries of 4 bytes) and every query head of the
+// Many tokens: a workgroup builds a token's gathered (cos, sin) pairs once per
+// key/value head in LDS (kh x head_dim entries of 4 bytes) and every query head of the
 // group reads them from there, instead of every element gathering from the tables in memory.
+// The phases of a workgroup wait for each other, so a token's heads are shared out to several (see the launch): 32 + 32 heads of
+// 128, one workgroup a token -> four: 333 tokens 7.6 -> 4.8 us, 1024 12.2 -> 9.0, 4096 30.0 -> 23.8; 32 + 8, two: 333 3.9 -> 3.6,
+// of 126 6.7 -> 5.3.
 // DIVIDE as above; without the divisions 1024 tokens of heads of 108 take 6.0 us instead of 7.05, 333 4.55 instead of 5.2.
 template <int VEC, bool DIVIDE>
 __global__ __launch_bounds__(256) void rope_indices_lds_kernel(const RopeArgs a, int cos_dim) {
@@ -153,9 +157,10 @@ __global__ __launch_bounds__(256) void rope_indices_lds_kernel(const RopeArgs a,
     uint16_t* trow = reinterpret_cast<uint16_t*>(rope_lds);  // the token's cos row, then its sin row
     // gathered tables: entry (kv head, column) of the cosines, then the same of the sines, as fp16
     uint16_t* tab_cos = reinterpret_cast<uint16_t*>(rope_lds + ((cos_dim + 3) & ~3));
-    uint16_t* tab_sin = tab_cos + a.n_kh * a.hd;
+    uint16_t* tab_sin = tab_cos + a.kh * a.hd;
     const int tid = threadIdx.x;
     const unsigned row = blockIdx.x;
+    const int first_kv = (int)blockIdx.y * a.kh, qh = a.kh * a.group;
     const int64_t table_row = a.cos_batch == 1 && a.rows != (unsigned)a.seq_len ? row % (unsigned)a.seq_len : row;
     const uint16_t* cos_row = reinterpret_cast<const uint16_t*>(a.cos + table_row * a.cos_row_stride);
     const uint16_t* sin_row = reinterpret_cast<const uint16_t*>(a.sin + table_row * a.cos_row_stride);
@@ -163,24 +168,24 @@ __global__ __launch_bounds__(256) void rope_indices_lds_kernel(const RopeArgs a,
     // row, the thread's first four index entries and its first two work items' q / k values are three
     // independent loads, and issued one behind a barrier behind the other they would cost three
     // memory round trips in a launch that lasts little longer than that.
-    const int entries = a.n_kh * a.hd;
+    const int entries = a.kh * a.hd, first_entry = first_kv * a.hd;
     const int half = a.hd >> 1;
     const int per_head = half / VEC;
-    const int per_row = (a.n_qh + a.n_kh) * per_head;
+    const int per_row = (qh + a.kh) * per_head;
     constexpr int kIdxAhead = 4;
     int idx_ahead[kIdxAhead];
 #pragma unroll
     for (int i = 0; i < kIdxAhead; ++i) {
         const int e = tid + 256 * i;
-        idx_ahead[i] = e < entries ? load_index(a.indices, a.index_bytes, e) : 0;
+        idx_ahead[i] = e < entries ? load_index(a.indices, a.index_bytes, first_entry + e) : 0;
     }
     auto item = [&](int t, half_t*& x, int& kv_head, int& j) __attribute__((always_inline)) {
         const int head = DIVIDE ? t / per_head : (int)__umulhi((unsigned)t, a.per_head_inverse);
         j = (t - head * per_head) * VEC;
-        const bool is_q = head < a.n_qh;
-        kv_head = is_q ? (DIVIDE ? head / a.group : (a.group == 1 ? head : (int)__umulhi((unsigned)head, a.group_inverse))) : head - a.n_qh;
-        x = is_q ? a.q + row * a.q_row_stride + (int64_t)head * a.hd
-                 : a.k + row * a.k_row_stride + (int64_t)(head - a.n_qh) * a.hd;
+        const bool is_q = head < qh;
+        kv_head = is_q ? (DIVIDE ? head / a.group : (a.group == 1 ? head : (int)__umulhi((unsigned)head, a.group_inverse))) : head - qh;
+        x = is_q ? a.q + row * a.q_row_stride + (int64_t)(first_kv * a.group + head) * a.hd
+                 : a.k + row * a.k_row_stride + (int64_t)(first_kv + head - qh) * a.hd;
     };
     constexpr int kItemsAhead = 2;  // 32 + 8 heads of 128 are 320 work items of eight column pairs: two per thread at most
     half_t* x0[kItemsAhead];
@@ -211,7 +216,7 @@ __global__ __launch_bounds__(256) void rope_indices_lds_kernel(const RopeArgs a,
         }
     }
     for (int e = tid + 256 * kIdxAhead; e < entries; e += 256) {
-        const int i = load_index(a.indices, a.index_bytes, e);
+        const int i = load_index(a.indices, a.index_bytes, first_entry + e);
         tab_cos[e] = trow[i];
         tab_sin[e] = trow[cos_dim + i];
     }
@@ -256,8 +261,9 @@ static void rope_indices_go(const RopeArgs& a, bool divide, dim3 grid, hipStream
 
 template <int VEC>
 static void rope_tables_go(const RopeArgs& a, bool divide, int cos_dim, size_t lds_bytes, hipStream_t stream) {
-    if (divide) hipLaunchKernelGGL((rope_indices_lds_kernel<VEC, true>), dim3(a.rows), dim3(256), lds_bytes, stream, a, cos_dim);
-    else hipLaunchKernelGGL((rope_indices_lds_kernel<VEC, false>), dim3(a.rows), dim3(256), lds_bytes, stream, a, cos_dim);
+    const dim3 grid(a.rows, (unsigned)(a.n_kh / a.kh));
+    if (divide) hipLaunchKernelGGL((rope_indices_lds_kernel<VEC, true>), grid, dim3(256), lds_bytes, stream, a, cos_dim);
+    else hipLaunchKernelGGL((rope_indices_lds_kernel<VEC, false>), grid, dim3(256), lds_bytes, stream, a, cos_dim);
 }
 
 int rope_indices_launch(void* q, int64_t q_row_stride, void* k, int64_t k_row_stride, const void* cos, const void* sin,
@@ -285,15 +291,20 @@ int rope_indices_launch(void* q, int64_t q_row_stride, void* k, int64_t k_row_st
     int vec = 1;
     if (half % 8 == 0 && q_row_stride % 8 == 0 && k_row_stride % 8 == 0 && (bases & 15u) == 0) vec = 8;
     else if (half % 2 == 0 && q_row_stride % 2 == 0 && k_row_stride % 2 == 0 && (bases & 3u) == 0) vec = 2;
-    // From 192 tokens on a workgroup each builds the token's tables in LDS (where they fit), below that every pair gathers its
+    // From 128 tokens on workgroups build a token's tables in LDS (where they fit), below that every pair gathers its
     // own values, two columns at a time: more threads in flight hide the dependent index -> table loads better than wide
-    // accesses do (32 + 8 heads of 108: 128 tokens 3.4 us against 4.0, 192 4.0 either way, 256 4.35 against 4.15, 512 6.2
-    // against 4.8).
-    const size_t lds_bytes = ((size_t)((cos_dim + 3) & ~3) + (size_t)n_kh * hd) * 4;
-    const bool tables = rows >= 192 && lds_bytes <= 32 * 1024 && rows <= 0x7fffffffLL;
+    // accesses do (32 + 8 heads of 108: 96 tokens 3.15 us against 3.1, 128 3.4 against 3.1, 192 4.1 against 3.3; of 126, one column
+    // at a time, 128 3.4 against 3.8, 192 3.7 against 3.9, 512 6.65 against 6.0: from 192 on).
+    // A workgroup takes at most eight key / value heads, and fewer where their query heads make it more than 24 heads, up to 1024
+    // tokens (32 + 8 heads of 128: eight key / value heads 6.2 us at 1024 tokens and 8.8 at 2048, four 5.8 and 9.2, two 7.0 and 11.2;
+    // 32 + 32: sixteen 9.5 and 16.3, eight 9.0 and 14.1, four 11.2 and 18.5).
+    a.group = n_qh / n_kh;
+    a.kh = n_kh;
+    while (a.kh % 2 == 0 && (a.kh > 8 || (rows <= 1024 && a.kh * (a.group + 1) > 24))) a.kh /= 2;
+    const size_t lds_bytes = ((size_t)((cos_dim + 3) & ~3) + (size_t)a.kh * hd) * 4;
+    const bool tables = rows >= (vec == 1 ? 192 : 128) && lds_bytes <= 32 * 1024 && rows <= 0x7fffffffLL && n_kh / a.kh <= 65535;
     if (!tables && vec == 8) vec = 2;
     a.per_head = half / vec;
-    a.group = n_qh / n_kh;
     const int64_t per_row = (int64_t)(n_qh + n_kh) * a.per_head, blocks = (per_row + 255) / 256;
     if (!tables && (per_row > 0x7fffff00LL || rows * blocks > 0x7fffffffLL)) return UNIQL_E_SHAPE;
     a.rows = (unsigned)rows;
