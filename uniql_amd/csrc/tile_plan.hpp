@@ -42,10 +42,11 @@ static inline size_t tile_part_bytes(int m, int n, const TilePlan& plan) {
 // adding one costs the tall tiles 4 to 8 us a round.  Of another 6250 calls the plan with the smallest time here took 1.003 x
 // the best plan's time on average.
 // The exchange of 64- (one quartet), 96- and 128-row tiles since its slots are read in batches: of 300 drawn calls of 65 to 700
-// rows whose plan that changed (96-row tiles with 2 to 7 splits in place of shorter ones, mostly) 282 are faster, by 12 % on
+// rows whose plan that changed (96-row tiles with 2 to 7 splits in place of shorter ones, mostly) 284 are no slower, 12 % faster on
 // average (14336 -> 6144 at 84 rows 35.6 -> 27.9 us, 12160 -> 4096 at 66 27.2 -> 21.4, 4096 -> 11264 at 96 20.8 -> 19.3), and 8
-// slower by more than 4 %.  Kept above what is measured (1 us for two splits, 2 for eight) for 64-row tiles, so that one quartet
-// does not replace two, whose sums are half as long chains, and as it was for 32-row tiles, up to 64 rows the other kernel's rivals.
+// slower by more than 5 % (most of them 1024 columns over more than 10000 rows).  Kept above what is measured (1 us for two splits,
+// 2 for eight) for 64-row tiles, so that one quartet does not replace two, whose sums are half as long chains, and as it was for
+// 32-row tiles, up to 64 rows the other kernel's rivals.
 struct LaunchFit {
     double full, full_g;        // a whole round: constant, per K group
     double split, split_each;   // the exchange between K splits (partial tiles' stores, count, the last one's reading of all of them)
