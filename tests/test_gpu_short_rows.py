@@ -12,7 +12,7 @@ PLANS = [(s << 8) | (mt << 16) | (kw << 20) for mt, kw in ((1, 1), (1, 2), (2, 1
 
 
 @pytest.mark.parametrize("plan", PLANS)
-@pytest.mark.parametrize("groups,missing", [(2, 8), (2, 120), (3, 64), (4, 72), (6, 56), (12, 16), (14, 104)])
+@pytest.mark.parametrize("groups,missing", [(1, 24), (2, 8), (2, 120), (3, 64), (4, 72), (6, 56), (12, 16), (14, 104)])
 def test_short_rows(gpu, plan, groups, missing):
     from uniql_amd import ops
     m, k, n = 300, 128 * groups, 256
