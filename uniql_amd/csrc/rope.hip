@@ -25,8 +25,8 @@ struct RopeArgs {
     int seq_len, cos_batch, n_qh, n_kh, hd, index_bytes;
     unsigned rows;
     int per_head, group;                       // work items of a head, query heads of a key / value head
-    int kh;                                    // key / value heads of a workgroup
     unsigned per_head_inverse, group_inverse;  // 2^32 / divisor, rounded up: quotients without a division
+    int kh;                                    // key / value heads of a workgroup
 };
 constexpr unsigned kRopeGridRows = 65535;
 
