@@ -390,14 +390,13 @@ __global__ __launch_bounds__(64 * WAVES, WAVES / 4) void w4a16_mid_kernel(const 
         // 128-column kernel's exchange (w4a16_tile.hip); no workgroup barrier, since nobody else's stores matter.
         constexpr int kSlotBytes = WAVES * UT * 2048;
         char* tile = reinterpret_cast<char*>(a.part) + (size_t)strip * a.splits * kSlotBytes;
-        const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(tile, 0, (unsigned)(a.splits * kSlotBytes), 0x00020000);
+        // (The slot is the descriptor's base and not a scalar offset, as in that kernel: see there.)
+        const __amdgpu_buffer_rsrc_t slot_rsrc = __builtin_amdgcn_make_buffer_rsrc(tile + (size_t)split * kSlotBytes, 0, (unsigned)kSlotBytes, 0x00020000);
         const uint32_t mine = (uint32_t)(UT * 2048 * w) + 16u * (uint32_t)lane;
 #pragma unroll
         for (int t = 0; t < UT; ++t) {
-            __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, lo[t]), rsrc, mine + 2048u * t,
-                                                   (uint32_t)(split * kSlotBytes), kMidDeviceScope);
-            __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, hi[t]), rsrc, mine + 2048u * t + 1024u,
-                                                   (uint32_t)(split * kSlotBytes), kMidDeviceScope);
+            __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, lo[t]), slot_rsrc, mine + 2048u * t, 0, kMidDeviceScope);
+            __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, hi[t]), slot_rsrc, mine + 2048u * t + 1024u, 0, kMidDeviceScope);
         }
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         unsigned long long* count = a.accum + WAVES * (size_t)strip + w;

@@ -464,8 +464,6 @@ __global__ __launch_bounds__(256 * KW, 1) void w4a16_tile_kernel(const TileArgs 
     const int tile = mblock * nstrips + strip_of_launch;
     constexpr int T = 256 * KW, UPT = 512 / T, kSlotBytes = ROWS * 512;
     char* part_tile = split_k ? reinterpret_cast<char*>(a.part) + (size_t)tile * a.splits * kSlotBytes : nullptr;
-    // (The slot is the descriptor's base and not a scalar offset: with a scalar offset in a register the compiler puts no wait
-    // state between a 16-byte store and the next instruction, and one that overwrites the stored registers changed what was stored.)
     // The residual of a thread's units, requested in front of the exchange between the waves or of the slots' reading: a
     // round trip in all, not one for every unit.
     u32x4 ahead[MT][UPT];
@@ -479,6 +477,8 @@ __global__ __launch_bounds__(256 * KW, 1) void w4a16_tile_kernel(const TileArgs 
         }
     };
     if (!split_k) request_residual();
+    // (The slot is the descriptor's base and not a scalar offset: with a scalar offset in a register the compiler puts no wait
+    // state between a 16-byte store and the next instruction, and one that overwrites the stored registers changed what was stored.)
     const __amdgpu_buffer_rsrc_t part_rsrc = __builtin_amdgcn_make_buffer_rsrc(part_tile + (size_t)split * kSlotBytes, 0, split_k ? (unsigned)kSlotBytes : 0u, kRsrcFlags);
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) {
