@@ -73,6 +73,17 @@ extern "C" int rule_left_for_nothing(int n, int k, int lo, int hi) {
     }
     return bad;
 }
+
+// Products that enter one accumulator one after another, at most, in a call of m rows.
+extern "C" int longest_chain(int m, int n, int k) {
+    const LinearPlan plan = call_plan(m, n, k, k >= 256, (size_t)12 << 20, 0);
+    int longest = 0;
+    for (int i = 0; i < plan.parts; ++i) {
+        const int chain = plan.part[i].wide ? k : tile_chain(plan.part[i].tile);
+        longest = chain > longest ? chain : longest;
+    }
+    return longest;
+}
 """
 
 
@@ -114,3 +125,12 @@ def test_the_search_rates_one_and_two_quartets(plans, n):
 def test_calls_that_run_as_two_launches(plans, m, k, n, head):
     """the sizes at which the GPU tests of two launches look at their results do run as two"""
     assert plans.first_of_two(m, n, k) == head
+
+
+@pytest.mark.parametrize("m,k,n,chain", [(459, 10752, 2048, 672), (275, 13056, 3072, 832), (277, 9984, 3200, 640), (281, 11776, 2176, 512),
+                                         (462, 11264, 2048, 704), (1985, 14336, 512, 896),        # 64-row tiles of two quartets
+                                         (3558, 12672, 3968, 3168), (2132, 13440, 14976, 3360)])  # 128-column kernel alone
+def test_sums_get_no_longer_for_a_gain_of_a_few_per_cent(plans, m, k, n, chain):
+    """sizes at which taller tiles with K split, or the 256 x 256 kernel with such tiles behind it, are expected to be a little
+    faster than a plan whose sums are shorter chains of products"""
+    assert plans.longest_chain(m, n, k) <= chain

@@ -81,6 +81,14 @@ static inline int fit_index(int mt, int quartets) { return mt <= 2 ? 2 * (mt - 1
 static inline double tile_us(int mt, int quartets, int64_t wgs, int g, int splits) {
     return launch_us(kLaunchFits[fit_index(mt, quartets)], wgs, g, splits);
 }
+// us by which a launch with K split has to be faster than one whose sums are shorter chains of products to be taken in its
+// place: sums get no longer, and so no further from exact ones, for a gain of a few per cent (10752 -> 2048 at 459 rows, chains
+// of 896 in place of 672: 34.9 us against 35.7; 12672 -> 3968 at 3558, of 12672 in place of 3168: 328 against 356).  What the exchange
+// cost these heights before its slots were read in batches.
+static inline double longer_chain_us(const TilePlan& p) {
+    if (p.splits <= 1 || p.quartets == 2 || p.mtiles < 2) return 0.0;
+    return p.mtiles == 2 ? 0.26 * p.splits : p.mtiles == 3 ? 0.58 + 1.07 * p.splits : 1.48 * p.splits;
+}
 static inline double wide_us(int m, int n, int k) {
     return launch_us(kLaunchFits[6], (int64_t)(n / 256) * ((m + 255) / 256), k / 128, 1);
 }
@@ -177,6 +185,10 @@ static inline bool one_round(int m, int n, const TilePlan& p) {
 static inline RowPart best_launch(int m, int n, int k, bool wide_ok, size_t part_cap) {
     const RowPart rule = rule_launch(m, n, k, wide_ok);
     RowPart p = {m, false, tile_plan(m, n, k, 0, 0, 0, part_cap)};
+    if (p.tile.mtiles >= 3 && p.tile.splits > 1) {
+        const TilePlan shorter = tile_plan(m, n, k, 0, 2, 2, part_cap);
+        if (tile_chain(shorter) < tile_chain(p.tile) && shorter.us <= p.tile.us + longer_chain_us(p.tile)) p.tile = shorter;
+    }
     const double wide = wide_ok ? wide_us(m, n, k) : p.tile.us;
     if (wide < p.tile.us) {
         p.wide = true;
@@ -213,7 +225,7 @@ static inline LinearPlan linear_plan(int m, int n, int k, bool wide_ok, size_t p
         const RowPart head = best_launch(128 * j, n, k, wide_ok, part_cap);
         if (head.tile.us + 2.0 >= us) continue;
         const RowPart tail = best_launch(m - 128 * j, n, k, wide_ok, part_cap);
-        const double both = head.tile.us + tail.tile.us + 2.0;
+        const double both = head.tile.us + tail.tile.us + 2.0 + (head.wide && !plan.part[0].wide ? longer_chain_us(tail.tile) : 0.0);
         if (both < 0.98 * us) {
             us = both / 0.98;
             plan.parts = 2;
@@ -249,7 +261,7 @@ static inline LinearPlan call_plan(int m, int n, int k, bool wide_ok, size_t par
         const RowPart head = best_launch(m, c, k, wide_ok && c % 256 == 0, part_cap);
         if (head.tile.us + 2.0 >= us) continue;
         const RowPart tail = best_launch(m, n - c, k, wide_ok && (n - c) % 256 == 0, part_cap);
-        const double both = head.tile.us + tail.tile.us + 2.0;
+        const double both = head.tile.us + tail.tile.us + 2.0 + (head.wide && !plan.part[0].wide ? longer_chain_us(tail.tile) : 0.0);
         if (both < gain * us) {
             us = both / gain;
             plan.parts = 2;
