@@ -84,6 +84,13 @@ extern "C" int longest_chain(int m, int n, int k) {
     }
     return longest;
 }
+
+// Height and K splits of a call that runs as one launch; 0 0 where it runs as two.
+extern "C" void one_launch(int m, int n, int k, int* plan) {
+    const LinearPlan p = call_plan(m, n, k, k >= 256, (size_t)12 << 20, 0);
+    plan[0] = p.parts == 1 ? p.part[0].tile.mtiles : 0;
+    plan[1] = p.parts == 1 ? p.part[0].tile.splits : 0;
+}
 """
 
 
@@ -134,3 +141,13 @@ def test_sums_get_no_longer_for_a_gain_of_a_few_per_cent(plans, m, k, n, chain):
     """sizes at which taller tiles with K split, or the 256 x 256 kernel with such tiles behind it, are expected to be a little
     faster than a plan whose sums are shorter chains of products"""
     assert plans.longest_chain(m, n, k) <= chain
+
+
+@pytest.mark.parametrize("m,k,n,mtiles,splits", [(1563, 10624, 384, 2, 3), (1326, 6784, 768, 2, 2), (3025, 7424, 512, 2, 1),
+                                                 (96, 6272, 6656, 3, 4)])
+def test_many_rows_and_few_columns_stay_on_fewer_splits(plans, m, k, n, mtiles, splits):
+    """with at least as many rows as columns taller tiles with more splits were slower than expected (24.4 -> 32.9 us at the first
+    of these); with fewer they are what is chosen"""
+    plan = (ctypes.c_int * 2)()
+    plans.one_launch(m, n, k, plan)
+    assert tuple(plan) == (mtiles, splits)

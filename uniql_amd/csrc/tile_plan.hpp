@@ -43,8 +43,8 @@ static inline size_t tile_part_bytes(int m, int n, const TilePlan& plan) {
 // the best plan's time on average.
 // The exchange of 64- (one quartet), 96- and 128-row tiles since its slots are read in batches: of 300 drawn calls of 65 to 700
 // rows whose plan that changed (96-row tiles with 2 to 7 splits in place of shorter ones, mostly) 284 are no slower, 12 % faster on
-// average (14336 -> 6144 at 84 rows 35.6 -> 27.9 us, 12160 -> 4096 at 66 27.2 -> 21.4, 4096 -> 11264 at 96 20.8 -> 19.3), and 8
-// slower by more than 5 % (most of them 1024 columns over more than 10000 rows).  Kept above what is measured (1 us for two splits,
+// average (14336 -> 6144 at 84 rows 35.6 -> 27.9 us, 12160 -> 4096 at 66 27.2 -> 21.4, 4096 -> 11264 at 96 20.8 -> 19.3; calls with more
+// rows than columns: tile_us).  Kept above what is measured (1 us for two splits,
 // 2 for eight) for 64-row tiles, so that one quartet does not replace two, whose sums are half as long chains, and as it was for
 // 32-row tiles, up to 64 rows the other kernel's rivals.
 struct LaunchFit {
@@ -78,16 +78,23 @@ static inline double launch_us(const LaunchFit& f, int64_t wgs, int g, int split
     return us + (full > 0 ? f.after + l.behind * per_g * g : l.alone + per_g * g);
 }
 static inline int fit_index(int mt, int quartets) { return mt <= 2 ? 2 * (mt - 1) + (quartets - 1) : mt + 1; }
-static inline double tile_us(int mt, int quartets, int64_t wgs, int g, int splits) {
-    return launch_us(kLaunchFits[fit_index(mt, quartets)], wgs, g, splits);
+// What the exchange cost more before its slots were read in batches, and in two places still counts for.
+static inline double former_exchange_us(int mt, int quartets, int splits) {
+    if (splits <= 1 || quartets == 2 || mt < 2) return 0.0;
+    return mt == 2 ? -0.091 + 0.262 * splits : mt == 3 ? 0.58 + 1.068 * splits : 1.48 * splits;
+}
+// With at least as many rows as columns (activations of four times the weights' bytes and more) taller tiles with more splits are
+// no gain: of 438 drawn calls of 33 to 4096 rows whose plan the lower ratings change, the 293 with fewer rows than columns are
+// 1.07 x as fast and 16 of them slower by more than 5 %, of the 145 others, 1.00 x as fast, 38 are, by up to a third (10624 -> 384 at
+// 1563 rows 24.4 -> 32.9 us, 6784 -> 768 at 1326 24.1 -> 31.5, 7424 -> 512 at 3025 32.9 -> 42.6).
+static inline double tile_us(int mt, int quartets, int m, int n, int64_t wgs, int g, int splits) {
+    return launch_us(kLaunchFits[fit_index(mt, quartets)], wgs, g, splits) + (m >= n ? former_exchange_us(mt, quartets, splits) : 0.0);
 }
 // us by which a launch with K split has to be faster than one whose sums are shorter chains of products to be taken in its
 // place: sums get no longer, and so no further from exact ones, for a gain of a few per cent (10752 -> 2048 at 459 rows, chains
-// of 896 in place of 672: 34.9 us against 35.7; 12672 -> 3968 at 3558, of 12672 in place of 3168: 328 against 356).  What the exchange
-// cost these heights before its slots were read in batches.
-static inline double longer_chain_us(const TilePlan& p) {
-    if (p.splits <= 1 || p.quartets == 2 || p.mtiles < 2) return 0.0;
-    return p.mtiles == 2 ? 0.26 * p.splits : p.mtiles == 3 ? 0.58 + 1.07 * p.splits : 1.48 * p.splits;
+// of 896 in place of 672: 34.9 us against 35.7; 12672 -> 3968 at 3558, of 12672 in place of 3168: 328 against 356).
+static inline double longer_chain_us(int m, int n, const TilePlan& p) {
+    return m >= n ? 0.0 : former_exchange_us(p.mtiles, p.quartets, p.splits);  // there it is part of the plan's time
 }
 static inline double wide_us(int m, int n, int k) {
     return launch_us(kLaunchFits[6], (int64_t)(n / 256) * ((m + 255) / 256), k / 128, 1);
@@ -116,7 +123,7 @@ static inline TilePlan tile_plan(int m, int n, int k, int splits_override, int m
             for (int kw = 1; kw <= 2; ++kw) {
                 if (kw == 2 ? !two_ok || (kw_override & 1) : two_ok && kw_override == 2) continue;
                 TilePlan p = {mt, splits, kw == 2 ? gps2 : gps1, kw, 0.0};
-                p.us = tile_us(mt, kw, tiles * splits, p.gps, splits);
+                p.us = tile_us(mt, kw, m, n, tiles * splits, p.gps, splits);
                 const bool fits = splits == 1 || splits_override > 0 || tile_part_bytes(m, n, p) <= part_cap;
                 if (fits && p.us < best.us) best = p;
             }
@@ -170,7 +177,7 @@ static inline RowPart rule_launch(int m, int n, int k, bool wide_ok) {
     p.quartets = even_g && p.mtiles <= 2 && tiles * ceil_div_i(G, p.gps) <= 256 ? 2 : 1;
     if (p.quartets == 2) p.gps += p.gps & 1;
     p.splits = ceil_div_i(G, p.gps);
-    p.us = tile_us(p.mtiles, p.quartets, tiles * p.splits, p.gps, p.splits);
+    p.us = tile_us(p.mtiles, p.quartets, m, n, tiles * p.splits, p.gps, p.splits);
     return RowPart{m, false, p};
 }
 
@@ -187,7 +194,7 @@ static inline RowPart best_launch(int m, int n, int k, bool wide_ok, size_t part
     RowPart p = {m, false, tile_plan(m, n, k, 0, 0, 0, part_cap)};
     if (p.tile.mtiles >= 3 && p.tile.splits > 1) {
         const TilePlan shorter = tile_plan(m, n, k, 0, 2, 2, part_cap);
-        if (tile_chain(shorter) < tile_chain(p.tile) && shorter.us <= p.tile.us + longer_chain_us(p.tile)) p.tile = shorter;
+        if (tile_chain(shorter) < tile_chain(p.tile) && shorter.us <= p.tile.us + longer_chain_us(m, n, p.tile)) p.tile = shorter;
     }
     const double wide = wide_ok ? wide_us(m, n, k) : p.tile.us;
     if (wide < p.tile.us) {
@@ -225,7 +232,7 @@ static inline LinearPlan linear_plan(int m, int n, int k, bool wide_ok, size_t p
         const RowPart head = best_launch(128 * j, n, k, wide_ok, part_cap);
         if (head.tile.us + 2.0 >= us) continue;
         const RowPart tail = best_launch(m - 128 * j, n, k, wide_ok, part_cap);
-        const double both = head.tile.us + tail.tile.us + 2.0 + (head.wide && !plan.part[0].wide ? longer_chain_us(tail.tile) : 0.0);
+        const double both = head.tile.us + tail.tile.us + 2.0 + (head.wide && !plan.part[0].wide ? longer_chain_us(m - 128 * j, n, tail.tile) : 0.0);
         if (both < 0.98 * us) {
             us = both / 0.98;
             plan.parts = 2;
@@ -261,7 +268,7 @@ static inline LinearPlan call_plan(int m, int n, int k, bool wide_ok, size_t par
         const RowPart head = best_launch(m, c, k, wide_ok && c % 256 == 0, part_cap);
         if (head.tile.us + 2.0 >= us) continue;
         const RowPart tail = best_launch(m, n - c, k, wide_ok && (n - c) % 256 == 0, part_cap);
-        const double both = head.tile.us + tail.tile.us + 2.0 + (head.wide && !plan.part[0].wide ? longer_chain_us(tail.tile) : 0.0);
+        const double both = head.tile.us + tail.tile.us + 2.0 + (head.wide && !plan.part[0].wide ? longer_chain_us(m, n - c, tail.tile) : 0.0);
         if (both < gain * us) {
             us = both / gain;
             plan.parts = 2;
