@@ -55,3 +55,44 @@ def test_short_rows_on_the_plan_of_the_call(gpu, m):
         if "bias" in kw:
             kw = dict(bias=torch.randn(n, device=gpu, generator=torch.Generator(device=gpu).manual_seed(m)).half())
         assert torch.equal(ops.w4a16_linear(x, b, s, ws, n, k, **kw), ops.w4a16_linear(padded, b, s, ws, n, k, **kw))
+
+
+@pytest.mark.parametrize("m,k_in,n,flags", [(300, 2040, 1536, 0), (100, 1992, 512, 0), (2000, 4008, 4096, 0), (300, 2040, 256, F_TILED | 1 << 8 | 2 << 16 | 1 << 20)])
+def test_short_rows_take_no_scratch_memory_for_a_copy(gpu, m, k_in, n, flags):
+    """a call holds its result and what whole rows of the same layer take: the copy that is not made has no room either"""
+    import ctypes
+
+    from uniql_amd import _capi, ops
+    k = (k_in + 127) // 128 * 128
+    p = make_linear_problem(m, k, n, seed=m)
+    x, b, s = to_gpu(p, gpu)
+    ws = workspace_for(n, gpu)
+    x = x[:, :k_in].contiguous()
+    y = torch.empty((m, n), dtype=torch.float16, device=gpu)
+    ops.w4a16_linear(x, b, s, ws, n, k, flags=flags, out=y)    # the exchange words are there now
+    acc, tmp = ctypes.c_size_t(0), ctypes.c_size_t(0)
+    assert _capi.load().uniql_w4a16_linear_workspace(m, n, k, k, 0, flags, ctypes.byref(acc), ctypes.byref(tmp)) == 0
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    torch.cuda.reset_peak_memory_stats()
+    before = torch.cuda.memory_allocated()
+    ops.w4a16_linear(x, b, s, ws, n, k, flags=flags, out=y)
+    assert torch.cuda.max_memory_allocated() - before <= (tmp.value + 511) // 512 * 512
+
+
+@pytest.mark.parametrize("m", [17, 24])
+def test_short_rows_too_far_apart(gpu, m):
+    """2^24 values and more from one row to the next: copied in front of the tiled kernels, whose offsets have 32 bits"""
+    from uniql_amd import ops
+    k, k_in, n, apart = 512, 488, 256, 1 << 24
+    p = make_linear_problem(m, k, n, seed=m)
+    x, b, s = to_gpu(p, gpu)
+    ws = workspace_for(n, gpu)
+    far = torch.empty((m - 1) * apart + k_in, dtype=x.dtype, device=gpu).as_strided((m, k_in), (apart, 1))
+    far.copy_(x[:, :k_in])
+    padded = torch.zeros((m, k), dtype=x.dtype, device=gpu)
+    padded[:, :k_in] = x[:, :k_in]
+    plan = F_TILED | 1 << 8 | 1 << 16 | 1 << 20
+    assert torch.equal(ops.w4a16_linear(far, b, s, ws, n, k, flags=plan), ops.w4a16_linear(padded, b, s, ws, n, k, flags=plan))
+    torch.testing.assert_close(ops.w4a16_linear(far, b, s, ws, n, k), ops.w4a16_linear(padded, b, s, ws, n, k, flags=plan),
+                               rtol=2 ** -9, atol=2 ** -9)  # another plan's order of fp32 sums: a rounding to fp16 apart, below 1 the same absolutely

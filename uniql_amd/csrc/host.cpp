@@ -67,7 +67,7 @@ struct Linear {
     int size_n, size_k, n_out, groups, had_block;
     float had_scale;
     bool silu_mul;
-    std::map<std::tuple<int64_t, int64_t, unsigned>, std::pair<size_t, size_t>> needs;   // (m, k_in, flags) -> accum, temp bytes
+    std::map<std::tuple<int64_t, int64_t, unsigned>, std::pair<size_t, size_t>> needs;   // (m, columns asked for, flags) -> accum, temp bytes
 };
 
 // The call on x [m, k_in]; `sizes`: the shape of a new output.  Without the interpreter lock.
@@ -114,15 +114,19 @@ Tensor run(Linear& p, Tensor x, std::optional<Tensor> residual, bool relu2, bool
     }
     if (m == 0) return y;
     if (out_f32) flags |= UNIQL_F_OUT_F32;
+    const int64_t lda = m > 1 ? x.stride(0) : std::max<int64_t>((k_in + 7) / 8 * 8, 8);
+    // Rows shorter than K are read as they are, like whole ones, unless they are rotated first or too far apart for the tiled
+    // kernels' offsets; only then is there a copy of them to ask scratch memory for (4000 rows of 9000: 73 MB).
+    const int64_t k_asked = p.had_block == 0 && lda < (1LL << 24) ? p.size_k : k_in;
     size_t need_acc, need_tmp;
     Tensor accum, temp;
     {
         const py::gil_scoped_acquire lock;
-        const auto key = std::make_tuple(m, k_in, flags);
+        const auto key = std::make_tuple(m, k_asked, flags);
         auto hit = p.needs.find(key);
         if (hit == p.needs.end()) {
             size_t acc = 0, tmp = 0;
-            check(p_workspace((int)m, p.size_n, p.size_k, (int)k_in, p.had_block, flags, &acc, &tmp), "uniql_w4a16_linear_workspace");
+            check(p_workspace((int)m, p.size_n, p.size_k, (int)k_asked, p.had_block, flags, &acc, &tmp), "uniql_w4a16_linear_workspace");
             if (p.needs.size() > 4096) p.needs.clear();
             hit = p.needs.emplace(key, std::make_pair(acc, tmp)).first;
         }
@@ -131,7 +135,6 @@ Tensor run(Linear& p, Tensor x, std::optional<Tensor> residual, bool relu2, bool
         if (need_acc) accum = accumulator(py::cast(x.device()), need_acc, stream).cast<Tensor>();
     }
     if (need_tmp) temp = new_output({(int64_t)need_tmp}, at::kByte, x);
-    const int64_t lda = m > 1 ? x.stride(0) : std::max<int64_t>((k_in + 7) / 8 * 8, 8);
     const int code = p_linear(x.data_ptr(), lda, (int)k_in, p.B.data_ptr(), p.s.data_ptr(), p.bias ? p.bias->data_ptr() : nullptr, res_ptr,
                               ldr, y.data_ptr(), ldd, (int)n_out,
                               p.silu_mul ? UNIQL_EPI_SILU_MUL : (relu2 ? UNIQL_EPI_RELU2 : UNIQL_EPI_NONE),
