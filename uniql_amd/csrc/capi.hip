@@ -184,18 +184,17 @@ static MidPlan mid_for_few_rows(int m, int n, int k, int had_block, unsigned fla
     return n / 128 < 144 && (k <= 8192 || n >= 3072) ? mid_plan(m, n, k, 0, part_cap) : kNoMid;
 }
 
-// In place of a launch of the tiled kernels, where it is expected to be faster; padded: the tiled kernels need a
-// zero-padded copy of the rows first (2 us; rows too far apart for them).  Over a short K of fewer than 12 groups the tiled kernels' expected times are the
-// better ones from 33 rows on.  Plans that add longer chains of products than the tiled kernel's own are left out: a sum
+// In place of a launch of the tiled kernels, where it is expected to be faster.  Over a short K of fewer than 12 groups the tiled
+// kernels' expected times are the better ones from 33 rows on.  Plans that add longer chains of products than the tiled kernel's own are left out: a sum
 // is no less exact here than there (8192 -> 512 at 56 rows with two groups a wave: 1.1 x the distance from float64).
 // Drawn calls: 17 to 32 rows 1.26 x faster on average, 33 to 48 1.17, 49 to 64 1.03.
-static MidPlan mid_for_tiles(const RowPart& part, int n, int k, bool padded, unsigned flags, size_t part_cap) {
+static MidPlan mid_for_tiles(const RowPart& part, int n, int k, unsigned flags, size_t part_cap) {
     if (part.rows < kMidMinRows || part.rows > kMidMaxRows) return kNoMid;
     if (((flags >> 16) & 0xfu) == 9) return mid_plan(part.rows, n, k, (int)((flags >> 8) & 0xffu), part_cap);  // asked for
     if (part.rows <= kStreamMaxM || (part.rows > 32 && k < 12 * 128)) return kNoMid;
     if ((flags & UNIQL_F_FORCE_TILED) || ((flags >> 8) & 0x3fffu) != 0) return kNoMid;
     const MidPlan p = mid_plan(part.rows, n, k, 0, part_cap, tile_chain(part.tile));
-    return p.upw > 0 && p.us < part.tile.us + (padded ? 2.0 : 0.0) ? p : kNoMid;
+    return p.upw > 0 && p.us < part.tile.us ? p : kNoMid;
 }
 
 // basic: neither the kernel for 9 to 64 rows nor columns in two launches, for callers whose scratch memory is enough for the
@@ -227,14 +226,9 @@ static LinearNeeds linear_needs(int m, int n, int k, int k_in, int64_t lda, int 
     } else {
         q.plan = basic ? linear_plan(m, n, k, wide_shape_ok(m, n, k, groups, q.ld_kernel), part_cap, tune)
                        : call_plan(m, n, k, wide_shape_ok(m, n & ~255, k, groups, q.ld_kernel), part_cap, tune);
-        const bool one = q.plan.parts == 1;
         for (int i = 0; i < q.plan.parts; ++i)
             if (!basic && q.plan.head_columns == 0 && mid_shape_ok(q.plan.part[i].rows, n, k, q.rotate_first ? k : lda))
-                q.mid[i] = mid_for_tiles(q.plan.part[i], n, k, one && q.pad_first && !q.rotate_first, flags, part_cap);
-        if (one && q.mid[0].upw > 0 && !q.rotate_first) {  // that kernel guards its own loads
-            q.pad_first = false;
-            q.ld_kernel = lda;
-        }
+                q.mid[i] = mid_for_tiles(q.plan.part[i], n, k, flags, part_cap);
     }
     for (int i = 0; i < q.plan.parts; ++i) {
         const RowPart& part = q.plan.part[i];
@@ -268,8 +262,7 @@ static void call_workspace(int m, int n, int k, int had_block, unsigned flags, s
         const size_t a = plan_accum_bytes(plan, n), p = plan_part_bytes(plan, n);
         *accum = a > *accum ? a : *accum;
         *part = p > *part ? p : *part;
-        for (int i = 0; i < plan.parts; ++i)
-            for (int padded = 0; padded < 2; ++padded) most(plan.part[i].rows, mid_for_tiles(plan.part[i], n, k, padded != 0, flags, kPartialCap));
+        for (int i = 0; i < plan.parts; ++i) most(plan.part[i].rows, mid_for_tiles(plan.part[i], n, k, flags, kPartialCap));
     }
 }
 
