@@ -360,6 +360,7 @@ __global__ __launch_bounds__(64 * WAVES, WAVES / 4) void w4a16_mid_kernel(const 
     u32x4 ahead[UT];
     auto request_residual = [&]() __attribute__((always_inline)) {
         if constexpr (EXT) {
+            if (!a.epi.residual_vec) return;  // uniform
             const __amdgpu_buffer_rsrc_t rows = residual_rows(a.epi, 0, a.M, 128 * strip);
 #pragma unroll
             for (int t = 0; t < UT; ++t) ahead[t] = residual_load(a.epi, rows, 4 * (w + t * WAVES) + kq, 8 * slot);

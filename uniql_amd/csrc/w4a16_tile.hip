@@ -469,6 +469,9 @@ __global__ __launch_bounds__(256 * KW, 1) void w4a16_tile_kernel(const TileArgs 
     u32x4 ahead[MT][UPT];
     auto request_residual = [&]() __attribute__((always_inline)) {
         if constexpr (EXT == 1) {
+            // uniform; loads through an empty descriptor take their turn in the address path as well (in 128-row tiles the
+            // branch spills 32 registers)
+            if (MT < 4 && !a.epi.residual_vec) return;
             const __amdgpu_buffer_rsrc_t rows = residual_rows(a.epi, m0, a.M, 128 * strip);
 #pragma unroll
             for (int mt = 0; mt < MT; ++mt)
