@@ -204,7 +204,6 @@ int embedding_quantize_launch(const void* W, int64_t ldw, void* packed, void* sc
     };
     if (words <= 256) rows(w4_embedding_quantize_rows_kernel<4>);
     else if (words <= 512) rows(w4_embedding_quantize_rows_kernel<8>);
-    else if (words <= 640) rows(w4_embedding_quantize_rows_kernel<10>);
     else if (words <= 1024) rows(w4_embedding_quantize_rows_kernel<16>);
     else
         hipLaunchKernelGGL(w4_embedding_quantize_kernel, dim3((unsigned)vocab), dim3(256), 0, stream,
