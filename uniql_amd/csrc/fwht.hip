@@ -680,11 +680,16 @@ static int fwht_column_pairs(const void* x, void* y, int cols, float scale, hipS
 }
 template <typename T, int LOG2L>
 static int fwht_columns_go(const void* x, void* y, int cols, float scale, hipStream_t stream) {
+    // 16-bit values of 4096 rows in tiles of sixteen columns where those are faster from memory: us with eight columns and with
+    // sixteen.  Not below 2560 columns, where they leave more than three in eight compute units idle (2048: 19.3 and 25.3; 2304: 23.7 and
+    // 24.5; 2560: 28.2 and 27.4; 2816: 29.3 and 26.4; 3328: 30.1 and 26.6; 4096: 35.2 and 30.6), and not from 273 to 384 tiles, where a few
+    // compute units get a second one (4352: 36.4 and 35.9; 4608: 41.7 and 42.9; 5120: 42.2 and 46.8; 6144: 48.8 and 51.0; 6152: 44.2 and
+    // 38.4).  Further on the workgroups of a compute unit are out of step, and one tile more than there are places for costs nothing
+    // that shows (8192, 512 tiles: 76.0 and 57.2; 8200: 54.9 and 55.5; 8448: 64.1 and 51.5; 9216: 68.3 and 58.4; 12296: 83.8 and 74.3; 16392:
+    // 117.6 and 112.7).  A matrix that is in the caches with its result is a little faster in eight columns up to 4352 (2560: 21.5 and
+    // 23.1; 3072: 21.8 and 23.3; 3328: 22.5 and 22.4; 4096: 24.2 and 24.6), not further on (7168: 38.4 and 33.4; 8192: 49.7 and 34.2).
     if constexpr (LOG2L == 12 && sizeof(T) == 2)
         if (cols >= 2560 && cols < (1 << 21) && !(cols > 4352 && cols <= 6144)) return fwht_column_pairs<T>(x, y, cols, scale, stream);
-    // 16-bit values of 4096 rows in tiles of sixteen columns from 2560 columns on, where they keep more than half of the compute
-    // units busy (2048: 22 us, 18.4 with eight columns; 2560: 27.5 and 28.2), and not from 4353 to 6144, where a few compute
-    // units get a second one (5120: 48 us and 42.7).
     // Else the widest tiles of which every compute unit gets one: eight waves, two workgroups a compute unit; sixteen for fp32
     // over 4096 rows, where eight columns are a full sector and only one workgroup's stores fit beside the other's loads
     // (4096 x 14336: 150 us against 165; fp16 102 either way); four for few columns of 1024 rows (x 4096: 8.5 us against 9.3).
@@ -760,8 +765,8 @@ __global__ __launch_bounds__(256) void fwht_composite_kernel(const T* __restrict
 // chunks of more than 512 values have one or two bits left for the workgroup.  Then the base matrix across the chunks with
 // its signs as constants, on pairs of neighbouring columns; the terms are added in ascending order, starting from zero, as
 // fwht_composite_kernel does: the same bits.  Outputs whose first signs agree share the sums of those terms: with the outputs
-// in the order of their signs, quarter by quarter, 639 additions a column in place of 784 (28), 1134 of 1600 (40), 333 of 400
-// (20), 112 of 144 (12).
+// in the order of their signs, quarter by quarter, 644 additions a column in place of 784 (28), 1135 of 1600 (40), 335 of 400
+// (20), 124 of 144 (12).
 // What bounds it: the additions (a SIMD takes one of a wave in 2.4 clocks; the matrix unit's fp32 forms, tried, hold the
 // vector unit up for as long as the additions take) and eight passes of the row through LDS, each about as long as the memory
 // time, and at most two rows of 14336 in a compute unit's LDS to overlap them.  So the workgroups stay, and request their next
