@@ -161,6 +161,26 @@ def test_cut_columns_many_groups_per_workgroup(gpu):
     assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
 
 
+def test_cuts_and_quantising_refuse_what_no_call_can_take(gpu):
+    """runs that are not six values each, widths that 32 bits do not hold: an error with its reason, nothing allocated or launched"""
+    from uniql_amd import ops
+    (w, s), _, _ = _packed_layer(gpu, 256, 512, torch.Generator().manual_seed(1))
+    x = torch.zeros((512, 256), dtype=torch.float16, device=gpu)
+    torch.cuda.synchronize()
+    torch.cuda.reset_peak_memory_stats()
+    before = torch.cuda.memory_allocated()
+    with pytest.raises(RuntimeError, match="six values"):
+        ops.w4a16_cut_columns(w, s, 512, 256, [(0, 1, 512, 512, 512)])
+    for width in (1 << 31, -(1 << 32)):
+        with pytest.raises(RuntimeError, match="kept width"):
+            ops.w4a16_cut_columns(w, s, 512, 256, [(0, 1, 512, 512, 512, 0)], pad_out=width)
+        with pytest.raises(RuntimeError, match="kept sizes"):
+            ops.w4a16_cut_rows(w, s, 512, 256, 1, 256, 256, 512, pad_out=width)
+        with pytest.raises(RuntimeError, match="larger than a call can take"):
+            ops.w4a16_quantize(x, None, pad_out=width)
+    assert torch.cuda.max_memory_allocated() == before
+
+
 @pytest.mark.parametrize("n,n_real,pad", [(128, 128, 0), (256, 200, 56), (256, 130, 126), (256, 60, 324)])
 @pytest.mark.parametrize("k,units,full,kept", [(256, 1, 0, 129), (512, 4, 128, 108), (1280, 10, 128, 77), (1280, 37, 33, 31)])
 @pytest.mark.parametrize("per_column", [False, True])

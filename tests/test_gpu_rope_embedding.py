@@ -125,6 +125,18 @@ def test_embedding_quantize_rows_in_registers(gpu, d):
     assert torch.equal(scales.view(torch.int16), want_scales.view(torch.int16))
 
 
+@pytest.mark.parametrize("d,apart", [(8, 16), (520, 528), (2048, 4096), (2056, 8192), (4104, 5120), (8184, 8192)])
+def test_embedding_quantize_rows_apart(gpu, d, apart):
+    """a table whose rows are cut out of wider ones: what lies between them counts for nothing, not even a NaN"""
+    from uniql_amd import ops
+    rows = 37
+    table = torch.full((rows, apart), float("nan"), dtype=torch.float16, device=gpu)
+    w = torch.randn((rows, d), device=gpu, generator=torch.Generator(device=gpu).manual_seed(d)).half()
+    table[:, :d] = w
+    got, want = ops.w4_embedding_quantize(table[:, :d]), ops.w4_embedding_quantize(w)
+    assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
+
+
 def test_embedding_quantize_hand_computed_ties(gpu):
     """The device quantiser on the rows whose codes are worked out by hand in
     tests/test_oracle_golden.py::test_embedding_quantize_rounding_ties_by_hand (fp16 rounding of

@@ -96,3 +96,18 @@ def test_short_rows_too_far_apart(gpu, m):
     assert torch.equal(ops.w4a16_linear(far, b, s, ws, n, k, flags=plan), ops.w4a16_linear(padded, b, s, ws, n, k, flags=plan))
     torch.testing.assert_close(ops.w4a16_linear(far, b, s, ws, n, k), ops.w4a16_linear(padded, b, s, ws, n, k, flags=plan),
                                rtol=2 ** -9, atol=2 ** -9)  # another plan's order of fp32 sums: a rounding to fp16 apart, below 1 the same absolutely
+
+
+@pytest.mark.parametrize("m,k_in,n", [(25, 1744, 28032), (29, 9664, 15360), (17, 14280, 9216), (19, 3752, 26752)])
+def test_short_rows_up_to_32_stay_in_the_kernel_for_9_to_64(gpu, m, k_in, n):
+    """sizes at which the tiled kernels are rated a little better, as they are for whole rows: the other kernel's bits, not theirs"""
+    from uniql_amd import ops
+    k = (k_in + 127) // 128 * 128
+    g = torch.Generator(device=gpu).manual_seed(m)
+    b = torch.randint(-2 ** 31, 2 ** 31 - 1, (k // 16, 2 * n), dtype=torch.int32, device=gpu, generator=g)
+    s = (0.004 + 0.016 * torch.rand((k // 128, n), device=gpu, generator=g)).half()
+    x = torch.randn((m, k_in), device=gpu, generator=g).half()
+    ws = workspace_for(n, gpu)
+    got = ops.w4a16_linear(x, b, s, ws, n, k)
+    assert torch.equal(got, ops.w4a16_linear(x, b, s, ws, n, k, flags=9 << 16))
+    assert not torch.equal(got, ops.w4a16_linear(x, b, s, ws, n, k, flags=F_TILED))

@@ -188,13 +188,17 @@ static MidPlan mid_for_few_rows(int m, int n, int k, int had_block, unsigned fla
 // kernels' expected times are the better ones from 33 rows on.  Plans that add longer chains of products than the tiled kernel's own are left out: a sum
 // is no less exact here than there (8192 -> 512 at 56 rows with two groups a wave: 1.1 x the distance from float64).
 // Drawn calls: 17 to 32 rows 1.26 x faster on average, 33 to 48 1.17, 49 to 64 1.03.
-static MidPlan mid_for_tiles(const RowPart& part, int n, int k, unsigned flags, size_t part_cap) {
+// short_rows: fewer columns of X than K.  Up to 32 rows the tiled kernels' form for those is slower than its expected time: of 49
+// drawn calls of 17 to 32 rows for which the tiled kernels are rated up to 2 us better 35 are faster here by more than 2 % and 4
+// there (1744 -> 28032 at 25 rows 9.4 us against 11.5, 14280 -> 9216 at 17 21.2 against 22.4), of 27 of 33 to 48 rows 5 and 13, of 324 of
+// more 29 and 211.
+static MidPlan mid_for_tiles(const RowPart& part, int n, int k, bool short_rows, unsigned flags, size_t part_cap) {
     if (part.rows < kMidMinRows || part.rows > kMidMaxRows) return kNoMid;
     if (((flags >> 16) & 0xfu) == 9) return mid_plan(part.rows, n, k, (int)((flags >> 8) & 0xffu), part_cap);  // asked for
     if (part.rows <= kStreamMaxM || (part.rows > 32 && k < 12 * 128)) return kNoMid;
     if ((flags & UNIQL_F_FORCE_TILED) || ((flags >> 8) & 0x3fffu) != 0) return kNoMid;
     const MidPlan p = mid_plan(part.rows, n, k, 0, part_cap, tile_chain(part.tile));
-    return p.upw > 0 && p.us < part.tile.us ? p : kNoMid;
+    return p.upw > 0 && p.us < part.tile.us + (short_rows && part.rows <= 32 ? 2.0 : 0.0) ? p : kNoMid;
 }
 
 // basic: neither the kernel for 9 to 64 rows nor columns in two launches, for callers whose scratch memory is enough for the
@@ -228,7 +232,7 @@ static LinearNeeds linear_needs(int m, int n, int k, int k_in, int64_t lda, int 
                        : call_plan(m, n, k, wide_shape_ok(m, n & ~255, k, groups, q.ld_kernel), part_cap, tune);
         for (int i = 0; i < q.plan.parts; ++i)
             if (!basic && q.plan.head_columns == 0 && mid_shape_ok(q.plan.part[i].rows, n, k, q.rotate_first ? k : lda))
-                q.mid[i] = mid_for_tiles(q.plan.part[i], n, k, flags, part_cap);
+                q.mid[i] = mid_for_tiles(q.plan.part[i], n, k, k_in != k && !q.rotate_first, flags, part_cap);
     }
     for (int i = 0; i < q.plan.parts; ++i) {
         const RowPart& part = q.plan.part[i];
@@ -262,7 +266,9 @@ static void call_workspace(int m, int n, int k, int had_block, unsigned flags, s
         const size_t a = plan_accum_bytes(plan, n), p = plan_part_bytes(plan, n);
         *accum = a > *accum ? a : *accum;
         *part = p > *part ? p : *part;
-        for (int i = 0; i < plan.parts; ++i) most(plan.part[i].rows, mid_for_tiles(plan.part[i], n, k, flags, kPartialCap));
+        for (int i = 0; i < plan.parts; ++i)
+            for (int short_rows = 0; short_rows < 2; ++short_rows)
+                most(plan.part[i].rows, mid_for_tiles(plan.part[i], n, k, short_rows != 0, flags, kPartialCap));
     }
 }
 

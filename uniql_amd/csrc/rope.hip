@@ -295,8 +295,8 @@ int rope_indices_launch(void* q, int64_t q_row_stride, void* k, int64_t k_row_st
     // own values, two columns at a time: more threads in flight hide the dependent index -> table loads better than wide
     // accesses do (32 + 8 heads of 108: 96 tokens 3.15 us against 3.1, 128 3.4 against 3.1, 192 4.1 against 3.3; of 126, one column
     // at a time, 128 3.4 against 3.8, 192 3.7 against 3.9, 512 6.65 against 6.0: from 192 on).
-    // A workgroup takes at most eight key / value heads, and fewer where their query heads make it more than 24 heads, up to 1024
-    // tokens (32 + 8 heads of 128: eight key / value heads 6.2 us at 1024 tokens and 8.8 at 2048, four 5.8 and 9.2, two 7.0 and 11.2;
+    // A token's key / value heads are halved between workgroups while their number is even and a workgroup has more than eight, or, up
+    // to 1024 tokens, more than 24 heads with its query heads (an odd number, as 9 or 5 x 9 heads, stays together: 32 + 8 heads of 128: eight key / value heads 6.2 us at 1024 tokens and 8.8 at 2048, four 5.8 and 9.2, two 7.0 and 11.2;
     // 32 + 32: sixteen 9.5 and 16.3, eight 9.0 and 14.1, four 11.2 and 18.5).
     a.group = n_qh / n_kh;
     a.kh = n_kh;
