@@ -62,3 +62,27 @@ def test_gated_stores_end_at_the_width(gpu, m, flags, n_out):
     # the kernel's silu is fp32 with the device's expf: its fp16 rounding may fall to the neighbour, then the product's too
     assert float((dense.float() - want.float()).abs().max()) <= 2.0 ** -9 * float(want.float().abs().max())
     assert float((dense != want).float().mean()) < 0.01
+
+
+@pytest.mark.parametrize("n_out", [512, 504, 508, 385])
+@pytest.mark.parametrize("m,flags", [(12, 0), (40, 0), (131, F_TILED | 1 << 8 | 2 << 16 | 1 << 20), (131, F_TILED | 3 << 8 | 3 << 16), (300, F_TILED | 8 << 16)])
+def test_float32_results_with_a_bias(gpu, m, flags, n_out):
+    """the sum and the bias added once in fp32, also from a bias that is not 16-byte aligned, then the rest of the epilogue"""
+    from uniql_amd import ops
+    k, n = 12 * 128, 512
+    p = make_linear_problem(m, k, n, seed=m + n_out)
+    x, b, s = to_gpu(p, gpu)
+    ws = workspace_for(n, gpu)
+    g = torch.Generator(device=gpu).manual_seed(n_out)
+    bias = torch.randn(n_out + 1, device=gpu, generator=g).half()
+    residual = torch.randn((m, n_out), device=gpu, generator=g).half()
+    y32 = ops.w4a16_linear(x, b, s, ws, n, k, out_f32=True, flags=flags)[:, :n_out]
+    for aligned in (bias[:n_out], bias[1:]):
+        want = y32 + aligned.float()
+        call = dict(out_features=n_out, bias=aligned, out_f32=True, flags=flags)
+        assert torch.equal(ops.w4a16_linear(x, b, s, ws, n, k, **call), want)
+        assert torch.equal(ops.w4a16_linear(x, b, s, ws, n, k, residual=residual, **call), want + residual.float())
+        assert torch.equal(ops.w4a16_linear(x, b, s, ws, n, k, relu2=True, **call), want.clamp_min(0) ** 2)
+        wide = torch.zeros((m, 520), dtype=torch.float32, device=gpu)
+        ops.w4a16_linear(x, b, s, ws, n, k, out=wide[:, :n_out], **call)
+        assert torch.equal(wide[:, :n_out], want) and not wide[:, n_out:].any()

@@ -136,11 +136,13 @@ __device__ __forceinline__ half_t finish_half_gated(const Epilogue& e, int n, fl
     return (half_t)((float)a16 * (float)u16);
 }
 
+// ADDS_BIAS: false where a float32 value has its bias already
+template <bool ADDS_BIAS = true>
 __device__ __forceinline__ void finish_store(const Epilogue& e, void* D, int m, int n, float v) {
     if (n >= e.n_store) return;
     const size_t o = e.offset(m, n);
     if (e.out_f32) {
-        if (e.bias) v += (float)e.bias[n];
+        if (ADDS_BIAS && e.bias) v += (float)e.bias[n];
         if (e.relu2) v = v > 0.f ? v * v : 0.f;
         if (e.residual) v += (float)e.residual[(size_t)m * e.ldr + n];
         reinterpret_cast<float*>(D)[o] = v;
@@ -218,7 +220,13 @@ __device__ __forceinline__ void store_eight(const Epilogue& e, void* D, int m, i
     const int left = e.n_store - n0;
     if (left <= 0) return;
     if (e.out_f32) {
-        if (e.vec_ok && left >= 8 && !e.bias && !e.residual && !e.relu2) {
+        if (e.bias) {
+            float b[8];
+            load_eight(e.bias + n0, (reinterpret_cast<uintptr_t>(e.bias) & 15u) == 0, left, b);
+            lo += f4{b[0], b[1], b[2], b[3]};
+            hi += f4{b[4], b[5], b[6], b[7]};
+        }
+        if (e.vec_ok && left >= 8 && !e.residual && !e.relu2) {
             float* d = reinterpret_cast<float*>(D) + (size_t)m * e.ldd + n0;
             *reinterpret_cast<f4*>(d) = lo;
             *reinterpret_cast<f4*>(d + 4) = hi;
@@ -226,7 +234,7 @@ __device__ __forceinline__ void store_eight(const Epilogue& e, void* D, int m, i
         }
 #pragma clang loop unroll(disable)
         for (int i = 0; i < 8; ++i) {
-            finish_store(e, D, m, n0 + i, lo[0]);
+            finish_store<false>(e, D, m, n0 + i, lo[0]);
             shift_down(lo, hi);
         }
         return;
