@@ -31,3 +31,10 @@ def test_rows_and_heads(gpu, b, hq, hk, s, d, D, index_dtype):
                       torch.from_numpy(idx).to(index_dtype).to(gpu))
     assert np.array_equal(qt.cpu().numpy().view(np.uint16), want_q.transpose(0, 2, 1, 3).view(np.uint16))
     assert np.array_equal(kt.cpu().numpy().view(np.uint16), want_k.transpose(0, 2, 1, 3).view(np.uint16))
+
+
+# halves of a workgroup's heads that are just enough for a workgroup of their own, and just not: 128 work items; 768 entries beyond 1024 tokens
+@pytest.mark.parametrize("b,hq,hk,s,d,D", [(1, 32, 32, 1030, 48, 64), (1, 32, 32, 1030, 46, 64), (1, 32, 32, 1024, 64, 128), (1, 30, 30, 200, 64, 128),
+                                           (1, 40, 40, 300, 64, 128), (1, 40, 10, 1025, 128, 128), (3, 48, 12, 343, 128, 128)])
+def test_halves_that_are_enough_for_a_workgroup(gpu, b, hq, hk, s, d, D):
+    test_rows_and_heads(gpu, b, hq, hk, s, d, D, torch.uint8)

@@ -296,11 +296,17 @@ int rope_indices_launch(void* q, int64_t q_row_stride, void* k, int64_t k_row_st
     // accesses do (32 + 8 heads of 108: 96 tokens 3.15 us against 3.1, 128 3.4 against 3.1, 192 4.1 against 3.3; of 126, one column
     // at a time, 128 3.4 against 3.8, 192 3.7 against 3.9, 512 6.65 against 6.0: from 192 on).
     // A token's key / value heads are halved between workgroups while their number is even and a workgroup has more than eight, or, up
-    // to 1024 tokens, more than 24 heads with its query heads (an odd number, as 9 or 5 x 9 heads, stays together: 32 + 8 heads of 128: eight key / value heads 6.2 us at 1024 tokens and 8.8 at 2048, four 5.8 and 9.2, two 7.0 and 11.2;
-    // 32 + 32: sixteen 9.5 and 16.3, eight 9.0 and 14.1, four 11.2 and 18.5).
+    // to 1024 tokens, more than 24 heads with its query heads (an odd number, as 9 or 5 x 9 heads, stays together: 32 + 8 heads of
+    // 128: eight key / value heads 6.2 us at 1024 tokens and 8.8 at 2048, four 5.8 and 9.2, two 7.0 and 11.2; 32 + 32: sixteen 9.5 and
+    // 16.3, eight 9.0 and 14.1, four 11.2 and 18.5), and while half of them is enough for a workgroup: 128 work items, and beyond 1024
+    // tokens 768 gathered entries (heads of 64: 32 + 32 at 2048 tokens sixteen 8.2, eight 10.2; 40 + 40 forty 9.6, twenty 9.5, five 15.7;
+    // 40 + 10 at 4096 ten 9.1, five 10.8; 40 + 40 of 96 at 4096 forty 27.5, ten 21.8, five 30.4).
     a.group = n_qh / n_kh;
     a.kh = n_kh;
-    while (a.kh % 2 == 0 && (a.kh > 8 || (rows <= 1024 && a.kh * (a.group + 1) > 24))) a.kh /= 2;
+    const int64_t items = (int64_t)(a.group + 1) * (half / vec);  // of a key / value head and its query heads
+    while (a.kh % 2 == 0 && (a.kh > 8 || (rows <= 1024 && a.kh * (a.group + 1) > 24)) && a.kh / 2 * items >= 128 &&
+           (rows <= 1024 || (int64_t)(a.kh / 2) * hd >= 768))
+        a.kh /= 2;
     const size_t lds_bytes = ((size_t)((cos_dim + 3) & ~3) + (size_t)a.kh * hd) * 4;
     const bool tables = rows >= (vec == 1 ? 192 : 128) && lds_bytes <= 32 * 1024 && rows <= 0x7fffffffLL && n_kh / a.kh <= 65535;
     if (!tables && vec == 8) vec = 2;
