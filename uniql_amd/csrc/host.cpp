@@ -4,8 +4,8 @@
 //
 // Bound by what it costs to get a launch out: at one token the kernels take 4-5 us, and the same checks in Python with
 // a ctypes call of 26 arguments took 14.2 us per W4A16B16O16Linear call, 10.9 per embedding lookup and 9.6 per
-// rotation; the seven cuts of a pruned decoder layer, 53 us of kernels, took 77 (54 now), quantising
-// 14336 x 4096 39 (35 now; the kernel: 29).  The checks, their messages and the order in which they are made are those of uniql_amd.ops, which
+// rotation; the seven cuts of a pruned decoder layer, 53 us of kernels, took 81 (58 to 60 now), quantising
+// 14336 x 4096 39 (36 now; the kernel: 29).  The checks, their messages and the order in which they are made are those of uniql_amd.ops, which
 // validates a layer's own tensors once (prepare_linear) and hands the functions' addresses over (bind).
 // Nothing of a call is kept: no address of an input, no check, no output.  A layer's sizes -> scratch sizes map belongs to
 // the layer's handle and is a pure function of its key.  The interpreter lock is given up for the whole call - copies of

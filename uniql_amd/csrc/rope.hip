@@ -300,7 +300,8 @@ int rope_indices_launch(void* q, int64_t q_row_stride, void* k, int64_t k_row_st
     // 128: eight key / value heads 6.2 us at 1024 tokens and 8.8 at 2048, four 5.8 and 9.2, two 7.0 and 11.2; 32 + 32: sixteen 9.5 and
     // 16.3, eight 9.0 and 14.1, four 11.2 and 18.5), and while half of them is enough for a workgroup: 128 work items, and beyond 1024
     // tokens 768 gathered entries (heads of 64: 32 + 32 at 2048 tokens sixteen 8.2, eight 10.2; 40 + 40 forty 9.6, twenty 9.5, five 15.7;
-    // 40 + 10 at 4096 ten 9.1, five 10.8; 40 + 40 of 96 at 4096 forty 27.5, ten 21.8, five 30.4).
+    // 40 + 10 at 4096 ten 9.1, five 10.8; 40 + 40 of 96 at 4096 forty 27.5, ten 21.8, five 30.4).  Left: 64 + 8 heads of 128 at 1024 tokens,
+    // eight 6.9, two as here 7.6 (at 2048 11.6 either way).
     a.group = n_qh / n_kh;
     a.kh = n_kh;
     const int64_t items = (int64_t)(a.group + 1) * (half / vec);  // of a key / value head and its query heads
